@@ -64,11 +64,58 @@ __global__ __launch_bounds__(256) void fill_i32_kernel(int32_t* __restrict__ out
 }
 
 // "rmsnorm": y = x / sqrt(mean(x^2) + eps) * w per row, one workgroup per row
-// (src/backends/rocm/rocm_kernels_basic.cpp:1586-1616).  The sum of squares is a strided fma chain
-// per thread, a butterfly inside each wavefront and the four wavefront sums in order: the
-// reference's tree adds the same partials in another order, so results agree to rounding.
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                      float* __restrict__ y, uint64_t cols, float eps) {
+// (src/backends/rocm/rocm_kernels_basic.cpp:1586-1616).  The sum of squares is an fma chain per
+// thread, a butterfly inside each wavefront and the wavefronts' sums in order: the reference's tree
+// adds the same partials in another order, so results agree to rounding.
+//
+// Bound by latency for a few rows (one row is 40 KB at 5120) and by HBM for many.  The row stays in
+// registers, V float4 a thread, so it is read once, and every load of x and w is under way before the
+// first is needed; with one element a load and the row read a second time a row of 5120 took 16 us
+// (2048 rows: 28 us), 20 dependent trips to memory a thread.
+template <int V>
+__global__ __launch_bounds__(1024) void rmsnorm_kernel(const float4* __restrict__ x, const float4* __restrict__ w,
+                                                       float4* __restrict__ y, uint32_t cols4, float eps) {
+  __shared__ float part[16];
+  const float4* xr = x + static_cast<uint64_t>(blockIdx.x) * cols4;
+  float4* yr = y + static_cast<uint64_t>(blockIdx.x) * cols4;
+  float4 v[V], g[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const uint32_t c = threadIdx.x + j * blockDim.x;
+    v[j] = c < cols4 ? xr[c] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const uint32_t c = threadIdx.x + j * blockDim.x;
+    g[j] = w[c < cols4 ? c : 0u];
+  }
+  float sum = 0.0f;
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    sum = fmaf(v[j].x, v[j].x, sum);
+    sum = fmaf(v[j].y, v[j].y, sum);
+    sum = fmaf(v[j].z, v[j].z, sum);
+    sum = fmaf(v[j].w, v[j].w, sum);
+  }
+  sum = wave_sum_last(sum);
+  if ((threadIdx.x & 63u) == 63u) part[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  float total = 0.0f;
+  for (uint32_t i = 0; i < blockDim.x / 64u; ++i) total += part[i];
+  const float gain = 1.0f / sqrtf(total / static_cast<float>(cols4 * 4u) + eps);
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const uint32_t c = threadIdx.x + j * blockDim.x;
+    if (c < cols4) {
+      yr[c] = float4{v[j].x * gain * g[j].x, v[j].y * gain * g[j].y, v[j].z * gain * g[j].z, v[j].w * gain * g[j].w};
+    }
+  }
+}
+
+// Rows whose length is no multiple of four (their starts are not aligned) or that do not fit the
+// registers of one workgroup.
+__global__ __launch_bounds__(256) void rmsnorm_any_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                          float* __restrict__ y, uint64_t cols, float eps) {
   __shared__ float part[4];
   const float* xr = x + static_cast<uint64_t>(blockIdx.x) * cols;
   float* yr = y + static_cast<uint64_t>(blockIdx.x) * cols;
@@ -597,7 +644,28 @@ hipError_t launch_fill_i32(int32_t* out, int32_t value, uint64_t n, hipStream_t 
 
 hipError_t launch_rmsnorm(const float* x, const float* w, float* y, uint64_t rows, uint64_t cols, float eps,
                           hipStream_t stream) {
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3(static_cast<uint32_t>(rows)), dim3(256), 0, stream, x, w, y, cols, eps);
+  constexpr uint64_t kMaxThreads = 1024, kMaxV = 8;
+  if (cols % 4 != 0 || cols / 4 > kMaxThreads * kMaxV) {
+    hipLaunchKernelGGL(rmsnorm_any_kernel, dim3(static_cast<uint32_t>(rows)), dim3(256), 0, stream, x, w, y, cols, eps);
+    return hipGetLastError();
+  }
+  // Few rows: as many threads as one load each keeps busy.  From two rows a CU: 256 threads and the
+  // loads of several rows side by side on a CU.
+  const uint32_t cols4 = static_cast<uint32_t>(cols / 4);
+  const uint32_t most = rows >= 512 && cols4 <= 256 * kMaxV ? 256 : kMaxThreads;
+  uint32_t v = 1;
+  while (v * most < cols4) v *= 2;
+  const uint32_t per = (cols4 + v - 1) / v, threads = (per + 63) / 64 * 64;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(rows)), dim3(threads), 0, stream, reinterpret_cast<const float4*>(x),
+                       reinterpret_cast<const float4*>(w), reinterpret_cast<float4*>(y), cols4, eps);
+  };
+  switch (v) {
+    case 1: go(rmsnorm_kernel<1>); break;
+    case 2: go(rmsnorm_kernel<2>); break;
+    case 4: go(rmsnorm_kernel<4>); break;
+    default: go(rmsnorm_kernel<8>); break;
+  }
   return hipGetLastError();
 }
 
