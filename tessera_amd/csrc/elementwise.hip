@@ -433,57 +433,170 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(const float* __restrict__
   }
 }
 
-// "top_k_rows" (src/backends/rocm/rocm_kernels_basic.cpp:3176-3243): per-row top-k of
-// `vocab` fp32 logits in descending order, one workgroup per row.  Pass p selects the
-// largest value not yet taken; ties go to the earlier column inside a thread's strided
-// share and to the lower thread across threads, as in the reference's strict-greater merge.
-__global__ __launch_bounds__(256) void top_k_rows_kernel(const float* __restrict__ logits,
-                                                         uint32_t* __restrict__ ids,
-                                                         float* __restrict__ vals, uint64_t vocab,
-                                                         uint32_t top_k, uint64_t row_base) {
-  __shared__ float rv[256];
-  __shared__ uint32_t ri[256];
-  __shared__ uint32_t rown[256];
-  const uint32_t tid = threadIdx.x;
-  const float* row = logits + (row_base + blockIdx.x) * vocab;
-  // Columns this thread has already given away: they are the thread's largest, in order, so
-  // "not yet taken" is "smaller than the last one given, or equal to it at a later column".
-  float last_v = 0.0f;
-  uint64_t last_c = 0;
-  bool any = false;
+// "top_k_rows" (src/backends/rocm/rocm_kernels_basic.cpp:3176-3243): per-row top-k of `vocab` fp32
+// logits in descending order.  Ties go as in the reference's merge of 256 strided shares: to the lower
+// share (column mod 256), inside a share to the earlier column.  A value and that order make one 64-bit
+// key, larger first, no two alike; 0 is no key.  NaN ranks below everything.
+__device__ __forceinline__ uint64_t top_k_key(float v, uint32_t column) {
+  uint32_t bits = bit_cast<uint32_t>(v == 0.0f ? 0.0f : v);    // -0 and +0 tie
+  bits = (bits & 0x80000000u) ? ~bits : bits | 0x80000000u;
+  if (v != v) bits = 0u;
+  return static_cast<uint64_t>(bits) << 32 | (~((column & 255u) << 23 | column >> 8));
+}
+__device__ __forceinline__ uint32_t top_k_column(uint64_t key) {
+  const uint32_t tie = ~static_cast<uint32_t>(key);
+  return (tie >> 23 & 255u) | (tie & 0x7FFFFFu) << 8;
+}
+
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ uint64_t dpp_max_u64(uint64_t v) {
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRowMask, 0xF, false));
+  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v >> 32), kCtrl, kRowMask, 0xF, false));
+  const uint64_t moved = static_cast<uint64_t>(hi) << 32 | lo;
+  return moved > v ? moved : v;
+}
+// Largest key of the wavefront, the same in every lane (the row steps of wave_sum_last).
+__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
+  v = dpp_max_u64<0xB1, 0xF>(v);
+  v = dpp_max_u64<0x4E, 0xF>(v);
+  v = dpp_max_u64<0x141, 0xF>(v);
+  v = dpp_max_u64<0x140, 0xF>(v);
+  v = dpp_max_u64<0x142, 0xA>(v);
+  v = dpp_max_u64<0x143, 0xC>(v);
+  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(v), 63);
+  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(v >> 32), 63);
+  return static_cast<uint64_t>(hi) << 32 | lo;
+}
+
+// Up to 64 * V columns (a router's experts): one wavefront a row, the row in registers, one
+// wavefront-wide maximum per place.  No memory is touched between the places: 256 columns, 8 places
+// took 10.4 us with a pass over the row and a tree through LDS for each.
+template <int V>
+__global__ __launch_bounds__(256) void top_k_short_rows_kernel(const float* __restrict__ logits, uint32_t* __restrict__ ids,
+                                                               float* __restrict__ vals, uint32_t rows, uint32_t vocab,
+                                                               uint32_t top_k, uint64_t row_base) {
+  const uint32_t lane = threadIdx.x & 63u, r = blockIdx.x * 4u + (threadIdx.x >> 6);
+  if (r >= rows) return;
+  const float* row = logits + (row_base + r) * vocab;
+  uint64_t key[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const uint32_t c = lane + 64u * j;
+    key[j] = c < vocab ? top_k_key(row[c], c) : 0ull;
+  }
+  uint32_t mine = 0u;
   for (uint32_t p = 0; p < top_k; ++p) {
-    float best = -INFINITY;
-    uint64_t best_c = ~0ull;
-    for (uint64_t c = tid; c < vocab; c += 256u) {
-      const float v = row[c];
-      const bool open = !any || v < last_v || (v == last_v && c > last_c);
-      if (open && (best_c == ~0ull || v > best)) {
-        best = v;
-        best_c = c;
-      }
-    }
-    rv[tid] = best_c != ~0ull ? best : -INFINITY;
-    ri[tid] = best_c != ~0ull ? static_cast<uint32_t>(best_c) : 0u;
-    rown[tid] = tid;
+    uint64_t best = key[0];
+#pragma unroll
+    for (int j = 1; j < V; ++j) best = key[j] > best ? key[j] : best;
+    best = wave_max_u64(best);
+#pragma unroll
+    for (int j = 0; j < V; ++j) key[j] = key[j] == best ? 0ull : key[j];
+    if (lane == p) mine = top_k_column(best);
+  }
+  if (lane < top_k) {
+    ids[static_cast<size_t>(r) * top_k + lane] = mine;
+    vals[static_cast<size_t>(r) * top_k + lane] = row[mine];
+  }
+}
+
+// Longer rows (an output head's vocabulary): one workgroup of sixteen wavefronts a row, the row read
+// once.  From the first tile it takes a bound that at least top_k columns reach -- the top_k-th of the
+// two largest thread maxima of each wavefront -- and from then on a column is looked at again only if
+// it reaches the bound: those keys go to a list in LDS (some tens of a row in no particular order).  A
+// list that grows past kKeep is cut down by the same rule over its own entries.  At the end every entry
+// counts the entries above it, which is its place.  One workgroup and no scratch memory, so launches on
+// different streams stay independent; one CU reads a row of 131072 in about 10 us, where one pass over
+// the row for each of 8 places took 850 us.
+constexpr uint32_t kTopKThreads = 1024, kTopKPerTile = 8, kTopKTile = kTopKThreads * kTopKPerTile;
+constexpr uint32_t kTopKKeep = 1024, kTopKList = kTopKKeep + kTopKTile;
+
+__global__ __launch_bounds__(kTopKThreads) void top_k_long_rows_kernel(const float* __restrict__ logits,
+                                                                       uint32_t* __restrict__ ids, float* __restrict__ vals,
+                                                                       uint32_t vocab, uint32_t top_k, uint64_t row_base) {
+  __shared__ uint64_t list[kTopKList];
+  __shared__ uint64_t wave_top[32];
+  __shared__ uint64_t bound_s;
+  __shared__ uint32_t count_s;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const float* row = logits + (row_base + blockIdx.x) * vocab;
+
+  // The top_k-th largest of every wavefront's two largest thread maxima; the same in every thread.
+  auto bound_of = [&](uint64_t thread_max) {
+    const uint64_t first = wave_max_u64(thread_max);
+    const uint64_t second = wave_max_u64(thread_max == first ? 0ull : thread_max);
+    if (lane == 0u) wave_top[wave * 2u] = first, wave_top[wave * 2u + 1u] = second;
     __syncthreads();
-    for (uint32_t s = 128u; s > 0u; s >>= 1) {
-      if (tid < s && rv[tid + s] > rv[tid]) {
-        rv[tid] = rv[tid + s];
-        ri[tid] = ri[tid + s];
-        rown[tid] = rown[tid + s];
+    if (tid < 32u) {
+      const uint64_t mine = wave_top[tid];
+      uint32_t above = 0u;
+      for (uint32_t i = 0; i < 32u; ++i) above += (wave_top[i] > mine || (wave_top[i] == mine && i < tid)) ? 1u : 0u;
+      if (above == top_k - 1u) bound_s = mine;
+    }
+    if (tid == 0u) count_s = 0u;
+    __syncthreads();
+    return bound_s;
+  };
+
+  uint64_t bound = 0ull;
+  float next[kTopKPerTile];
+  auto load = [&](uint32_t tile) {
+#pragma unroll
+    for (uint32_t j = 0; j < kTopKPerTile; ++j) {
+      const uint64_t c = static_cast<uint64_t>(tile) * kTopKTile + tid + j * kTopKThreads;
+      next[j] = row[c < vocab ? c : vocab - 1u];
+    }
+  };
+  load(0);
+  const uint32_t tiles = (vocab + kTopKTile - 1u) / kTopKTile;
+  for (uint32_t t = 0; t < tiles; ++t) {
+    uint64_t key[kTopKPerTile];
+#pragma unroll
+    for (uint32_t j = 0; j < kTopKPerTile; ++j) {
+      const uint32_t c = t * kTopKTile + tid + j * kTopKThreads;
+      key[j] = c < vocab ? top_k_key(next[j], c) : 0ull;
+    }
+    if (t + 1u < tiles) load(t + 1u);
+    if (t == 0u) {
+      uint64_t most = 0ull;
+#pragma unroll
+      for (uint32_t j = 0; j < kTopKPerTile; ++j) most = key[j] > most ? key[j] : most;
+      bound = bound_of(most);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kTopKPerTile; ++j) {
+      if (key[j] >= bound && key[j] != 0ull) list[atomicAdd(&count_s, 1u)] = key[j];
+    }
+    lds_barrier();
+    uint32_t count = count_s;
+    lds_barrier();
+    while (count > kTopKKeep) {   // every wavefront holds entries here, so each round drops some
+      uint64_t held[kTopKList / kTopKThreads];
+      uint64_t most = 0ull;
+#pragma unroll
+      for (uint32_t j = 0; j < kTopKList / kTopKThreads; ++j) {
+        held[j] = tid + j * kTopKThreads < count ? list[tid + j * kTopKThreads] : 0ull;
+        most = held[j] > most ? held[j] : most;
+      }
+      bound = bound_of(most);
+#pragma unroll
+      for (uint32_t j = 0; j < kTopKList / kTopKThreads; ++j) {
+        if (held[j] >= bound && held[j] != 0ull) list[atomicAdd(&count_s, 1u)] = held[j];
       }
       __syncthreads();
+      count = count_s;
+      __syncthreads();
     }
-    if (tid == 0u) {
-      vals[static_cast<size_t>(blockIdx.x) * top_k + p] = rv[0];
-      ids[static_cast<size_t>(blockIdx.x) * top_k + p] = ri[0];
-    }
-    const uint32_t owner = rown[0];
-    __syncthreads();
-    if (tid == owner && best_c != ~0ull) {
-      last_v = best;
-      last_c = best_c;
-      any = true;
+  }
+  const uint32_t count = count_s;
+  if (tid < count) {
+    const uint64_t mine = list[tid];
+    uint32_t above = 0u;
+    for (uint32_t i = 0; i < count; ++i) above += list[i] > mine ? 1u : 0u;
+    if (above < top_k) {
+      const uint32_t c = top_k_column(mine);
+      ids[static_cast<size_t>(blockIdx.x) * top_k + above] = c;
+      vals[static_cast<size_t>(blockIdx.x) * top_k + above] = row[c];
     }
   }
 }
@@ -807,8 +920,17 @@ hipError_t launch_moe_gate(const float* vals, const float* x, const float* w, fl
 
 hipError_t launch_top_k_rows(const float* logits, uint32_t* ids, float* vals, uint32_t rows,
                              uint64_t vocab, uint32_t top_k, uint64_t row_base, hipStream_t stream) {
-  hipLaunchKernelGGL(top_k_rows_kernel, dim3(rows), dim3(256), 0, stream, logits, ids, vals, vocab, top_k,
-                     row_base);
+  // Up to 512 columns fit the registers of one wavefront; a workgroup of sixteen has a tile of 8192 to
+  // itself beyond that.
+  const uint32_t v = static_cast<uint32_t>(vocab);
+  const dim3 four_rows((rows + 3u) / 4u);
+  if (vocab <= 256) {
+    hipLaunchKernelGGL(top_k_short_rows_kernel<4>, four_rows, dim3(256), 0, stream, logits, ids, vals, rows, v, top_k, row_base);
+  } else if (vocab <= 512) {
+    hipLaunchKernelGGL(top_k_short_rows_kernel<8>, four_rows, dim3(256), 0, stream, logits, ids, vals, rows, v, top_k, row_base);
+  } else {
+    hipLaunchKernelGGL(top_k_long_rows_kernel, dim3(rows), dim3(kTopKThreads), 0, stream, logits, ids, vals, v, top_k, row_base);
+  }
   return hipGetLastError();
 }
 

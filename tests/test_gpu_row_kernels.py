@@ -29,3 +29,43 @@ def test_rmsnorm_edges(backend, rows, cols):
     # halved by the square root
     bound = max(2e-6, cols * 2.0 ** -25)
     assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 1e-30)) <= bound
+
+
+def top_k_want(row, top_k):
+    """Descending; ties to the lower share (column mod 256), inside a share to the earlier column."""
+    c = np.arange(row.size)
+    order = np.lexsort((c // 256, c % 256, -row.astype(np.float64)))[:top_k]
+    return order.astype(np.uint32), row[order]
+
+
+# a wavefront a row up to 256 and up to 512 columns, then a workgroup a row: less than a tile of 8192, one
+# tile, one column more, many tiles with a remainder.  Sorted rows and rows of few different values are the
+# ones whose candidates outgrow the list.
+@pytest.mark.parametrize("kind", ["normal", "rising", "falling", "ties", "equal", "infinite"])
+@pytest.mark.parametrize("rows,vocab,top_k", [(1, 1, 1), (5, 64, 8), (3, 256, 32), (6, 257, 3), (2, 512, 32), (2, 513, 32), (3, 1000, 1),
+                                              (2, 8192, 8), (1, 8193, 32), (2, 70001, 32), (1, 131072, 8), (1, 151936, 17)])
+def test_top_k_edges(backend, rows, vocab, top_k, kind):
+    g = synth.rng(vocab + top_k)
+    x = g.standard_normal((rows + 1, vocab)).astype(np.float32)
+    if kind in ("rising", "falling"):
+        x = np.sort(x, axis=1)
+        x = x if kind == "rising" else x[:, ::-1].copy()
+    elif kind == "ties":
+        x = np.round(x * 2) / 2          # holds -0.0 and 0.0, which tie
+    elif kind == "equal":
+        x[:] = -1.25
+    elif kind == "infinite":
+        x[:, ::3] = -np.inf
+        x[:, vocab // 2] = np.inf
+    dx = backend.Upload(x)
+    di, dv = backend.Upload(np.full(rows * top_k, 0xFFFFFFFF, np.uint32)), backend.AllocateBuffer(4 * rows * top_k)
+    if kind == "infinite" and np.isfinite(x[0]).sum() + 1 < top_k:
+        top_k = 1
+    run(backend, "top_k_rows", [dx, di, dv], [rows, vocab, top_k, 1])   # rows 1.. of the buffer
+    backend.Synchronize()
+    ids = backend.CopyD2H(di, dtype=np.uint32)[:rows * top_k].reshape(rows, top_k)
+    vals = backend.CopyD2H(dv, dtype=np.float32)[:rows * top_k].reshape(rows, top_k)
+    for r in range(rows):
+        want_ids, want_vals = top_k_want(x[r + 1], top_k)
+        assert np.array_equal(ids[r], want_ids), r
+        assert np.array_equal(vals[r].view(np.uint32), want_vals.view(np.uint32)), r
