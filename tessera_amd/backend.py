@@ -153,6 +153,10 @@ class Backend:
 
     def __init__(self, lib_path: str = LIB_PATH, stream: int = 0):
         self._lib = load_library(lib_path)
+        from . import _native   # built beside the kernel library (csrc/Makefile)
+        self._launch = _native.launch
+        self._entry = C.cast(self._lib.qmm_launch, C.c_void_p).value
+        self._entry_static = C.cast(self._lib.qmm_launch_static, C.c_void_p).value
         self._device_index = 0
         self._stream = C.c_void_p(stream)
         self._ready = False
@@ -244,15 +248,10 @@ class Backend:
         """``no_alloc=True`` goes through ``qmm_launch_static`` (not in the reference): the same
         launch with every kernel's scratch taken from the library's static device array, for
         callers that may not allocate device memory."""
-        nb, ns = len(launch.buffers), len(launch.scalars)
-        grid = (C.c_uint32 * 3)(launch.grid_x, launch.grid_y, launch.grid_z)
-        block = (C.c_uint32 * 3)(launch.block_x, launch.block_y, launch.block_z)
-        bufs = (C.c_void_p * max(nb, 1))(*[b.Handle() for b in launch.buffers])
-        sizes = (C.c_size_t * max(nb, 1))(*[b.Size() for b in launch.buffers])
-        scal = (C.c_uint64 * max(ns, 1))(*[int(s) & 0xFFFFFFFFFFFFFFFF for s in launch.scalars])
-        entry = self._lib.qmm_launch_static if no_alloc else self._lib.qmm_launch
-        self._check(entry(kernel.Handle(), grid, block, bufs, sizes, nb, scal, ns, self._stream),
-                    f"LaunchKernel({kernel.Id()})")
+        code = self._launch(self._entry_static if no_alloc else self._entry, kernel.Handle(), launch,
+                            self._stream.value or 0)
+        if code != 0:
+            self._check(code, f"LaunchKernel({kernel.Id()})")
 
     def WorkspaceBytes(self, kernel: Kernel, scalars: Sequence[int]) -> int:
         """Scratch a launch of ``kernel`` with these scalars needs (``qmm_workspace_bytes``)."""
