@@ -1,0 +1,655 @@
+// Softmax attention over a key/value cache: the "attention" ids, their flash-decoding forms and the
+// merge of those.  Contracts: include/tessera/backend.hpp:162-179,284-333,429-475,679-705; CPU
+// statements src/core/numerics/attention.cpp.
+//
+// Precision.  Scores and sums are fp32 in every variant.  Where the contraction runs on the fp16
+// matrix instruction, the fp32 side (queries, then weights) enters as two fp16 terms hi + lo of a value
+// brought near 2^8 resp. 2^14 by a power of two -- 22 significant bits -- and the cache's side enters
+// exactly: an fp16 number, or the integer or E4M3 code, whose scale multiplies the fp32 score (keys) or
+// the fp32 weight (values).
+
+#include <type_traits>
+
+#include "qmm_device.hpp"
+#include "qmm_kernels.hpp"
+
+namespace qmm {
+namespace {
+
+// How keys and values are stored.  The quantized kinds hold codes and one fp32 scale per key row (all
+// kv heads of a position), and an element is code * scale as in AttentionQ8Ref / AttentionQ4Ref /
+// AttentionFp8Ref (src/core/numerics/attention.cpp:45-121).
+enum class KvKind { F32, F16, Q8, Q4, Fp8 };
+constexpr int kv_bits(KvKind k) { return k == KvKind::F32 ? 32 : k == KvKind::F16 ? 16 : k == KvKind::Q4 ? 4 : 8; }
+constexpr bool kv_quantized(KvKind k) { return k == KvKind::Q8 || k == KvKind::Q4 || k == KvKind::Fp8; }
+
+// SPLIT (the flash-decoding ids, src/backends/rocm/rocm_kernels_basic.cpp:275-440): the part s of
+// (row, head) is chunk s of ceil(span / split) keys of the row's key range; it leaves the unnormalized
+// sum, the chunk's largest score and its sum of weights in pacc / pmax / psum at index
+// (row * heads + head) * split + s (an empty chunk: 0, -1e30, 0); attention_combine_kernel merges them.
+struct SplitOut {
+  float *pacc, *pmax, *psum;
+  uint64_t split;   // 0: no parts, `out` receives the rows
+};
+
+struct AttentionArgs {
+  const float* q;
+  const void *k, *v;
+  const float *k_scale, *v_scale;
+  float* out;
+  SplitOut part;
+  uint64_t n, q_base, row_base, window;
+  uint32_t heads, kv_heads, head_dim, causal;
+};
+
+// Keys [start, last] that query row i sees.
+__device__ __forceinline__ void key_range(const AttentionArgs& a, uint64_t i, uint64_t& start, uint64_t& last) {
+  const uint64_t pos = a.q_base + i;
+  last = a.causal != 0 ? (pos >= a.n ? a.n - 1 : pos) : a.n - 1;
+  start = 0;
+  if (a.causal != 0) {
+    start = (a.window != 0 && pos + 1 > a.window) ? pos + 1 - a.window : 0;
+    if (start > last) start = last;
+  }
+}
+// Chunk s of that range; false: the chunk is empty.
+__device__ __forceinline__ bool key_chunk(const AttentionArgs& a, uint64_t s, uint64_t& start, uint64_t& last) {
+  const uint64_t chunk = (last + 1 - start + a.part.split - 1) / a.part.split;
+  start += s * chunk;
+  if (start > last) return false;
+  last = start + chunk - 1 < last ? start + chunk - 1 : last;
+  return true;
+}
+
+// ---- few query rows: one workgroup per (row, kv head, chunk) -------------------------------------
+//
+// Bound by reading the cache.  A kv head's keys and values are read once for all the query heads that
+// share it (up to eight a workgroup; sixteen over an fp32 cache), each wavefront taking every NW-th tile
+// of 32 keys on its own, with no barrier and no LDS before the final merge of the wavefronts:
+//   S^T = K Q^T on v_mfma_f32_16x16x32_f16, keys as matrix rows, columns 2h and 2h + 1 the hi and lo
+//   term of head h, so a lane ends up with scores of 4 + 4 keys of its column and its neighbour's
+//   column is the other term.  O^T = V^T P^T takes those lanes' weights as they stand (slots 8g..8g+3
+//   of lane group g are keys 4g.. of the tile's first half, the next four of its second half), and a
+//   lane reads whole runs of eight keys' values, of which a byte permute per register pair makes the
+//   key-major operand: no transposition through LDS.
+// The loads of a tile's keys are under way during the previous tile's softmax and values, its values'
+// during the scores.  Over an fp32 cache the same shape runs on v_mfma_f32_16x16x4_f32, tiles of 16 keys.
+template <int BYTES>
+__device__ __forceinline__ void load_run(const uint8_t* p, uint32_t (&r)[(BYTES + 3) / 4]) {
+  if constexpr (BYTES == 2) {
+    r[0] = *reinterpret_cast<const uint16_t*>(p);
+  } else if constexpr (BYTES == 4) {
+    r[0] = *reinterpret_cast<const uint32_t*>(p);
+  } else if constexpr (BYTES == 8) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    r[0] = v.x, r[1] = v.y;
+  } else {
+#pragma unroll
+    for (int i = 0; i < BYTES / 16; ++i) {
+      const uint4 v = load_u4(p + 16 * i);
+      r[4 * i] = v.x, r[4 * i + 1] = v.y, r[4 * i + 2] = v.z, r[4 * i + 3] = v.w;
+    }
+  }
+}
+
+__device__ __forceinline__ half2_t as_half2(uint32_t v) { return bit_cast<half2_t>(v); }
+__device__ __forceinline__ uint32_t as_bits(half2_t v) { return bit_cast<uint32_t>(v); }
+// Two bytes 128 + code in the low bytes of halves -> the codes as fp16 (1024 + u is the half 0x6400 | u).
+__device__ __forceinline__ uint32_t halves_from_biased_bytes(uint32_t v) {
+  return as_bits(as_half2(v | 0x64006400u) - half2_t{static_cast<_Float16>(1152.0f), static_cast<_Float16>(1152.0f)});
+}
+// Two nibbles in the low bits of halves (two's complement) -> the codes as fp16.
+__device__ __forceinline__ uint32_t halves_from_nibbles(uint32_t v) {
+  return as_bits(as_half2((v & 0x000F000Fu) ^ 0x64086408u) - half2_t{static_cast<_Float16>(1032.0f), static_cast<_Float16>(1032.0f)});
+}
+__device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
+
+// Eight elements of one key (`w`: their run) as a matrix operand, in the order kq_dim.
+template <KvKind KV>
+__device__ __forceinline__ half8_t key_operand(const uint32_t* w) {
+  uint4 r;
+  if constexpr (KV == KvKind::F16) {
+    r = uint4{w[0], w[1], w[2], w[3]};
+  } else if constexpr (KV == KvKind::Q8) {
+    const uint32_t a = w[0] ^ 0x80808080u, b = w[1] ^ 0x80808080u;
+    r = uint4{halves_from_biased_bytes(perm(0, a, 0x0C010C00)), halves_from_biased_bytes(perm(0, a, 0x0C030C02)),
+              halves_from_biased_bytes(perm(0, b, 0x0C010C00)), halves_from_biased_bytes(perm(0, b, 0x0C030C02))};
+  } else if constexpr (KV == KvKind::Q4) {
+    const uint32_t a = perm(0, w[0], 0x0C010C00), b = perm(0, w[0], 0x0C030C02);
+    r = uint4{halves_from_nibbles(a), halves_from_nibbles(a >> 4), halves_from_nibbles(b), halves_from_nibbles(b >> 4)};
+  } else {
+    r = uint4{as_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[0], 1.0f, false)), as_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[0], 1.0f, true)),
+              as_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[1], 1.0f, false)), as_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[1], 1.0f, true))};
+  }
+  return bit_cast<half8_t>(r);
+}
+// The element of a run of eight that sits in slot e of key_operand: 4-bit codes come low nibbles of two
+// bytes first.
+template <KvKind KV>
+__device__ constexpr int kq_dim(int e) {
+  if (KV != KvKind::Q4) return e;
+  const int order[8] = {0, 2, 1, 3, 4, 6, 5, 7};
+  return order[e];
+}
+
+// Element j of the runs of two keys as a pair of fp16 numbers (the first key in the low half).
+template <KvKind KV>
+__device__ __forceinline__ uint32_t value_pair(const uint32_t* k0, const uint32_t* k1, int j) {
+  if constexpr (KV == KvKind::F16) {
+    return perm(k1[j / 2], k0[j / 2], (j & 1) ? 0x07060302u : 0x05040100u);
+  } else if constexpr (KV == KvKind::Q8) {
+    const uint32_t b = static_cast<uint32_t>(j & 3);
+    return halves_from_biased_bytes(perm(k1[j / 4], k0[j / 4], 0x0C000C00u | ((4u + b) << 16) | b) ^ 0x00800080u);
+  } else if constexpr (KV == KvKind::Q4) {
+    const uint32_t b = static_cast<uint32_t>(j & 7) / 2u;
+    const uint32_t t = perm(k1[j / 8], k0[j / 8], 0x0C000C00u | ((4u + b) << 16) | b);
+    return halves_from_nibbles((j & 1) ? t >> 4 : t);
+  } else {
+    const uint32_t b = static_cast<uint32_t>(j & 3);
+    return as_bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(perm(k1[j / 4], k0[j / 4], 0x0C0C0000u | ((4u + b) << 8) | b), 1.0f, false));
+  }
+}
+
+// Maximum / sum over the four groups of sixteen lanes; every lane returns it.
+__device__ __forceinline__ float groups_max(float v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(bit_cast<uint32_t>(v), bit_cast<uint32_t>(v), false, false);
+  v = fmaxf(bit_cast<float>(a[0]), bit_cast<float>(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(bit_cast<uint32_t>(v), bit_cast<uint32_t>(v), false, false);
+  return fmaxf(bit_cast<float>(b[0]), bit_cast<float>(b[1]));
+}
+__device__ __forceinline__ float groups_sum(float v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(bit_cast<uint32_t>(v), bit_cast<uint32_t>(v), false, false);
+  v = bit_cast<float>(a[0]) + bit_cast<float>(a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(bit_cast<uint32_t>(v), bit_cast<uint32_t>(v), false, false);
+  return bit_cast<float>(b[0]) + bit_cast<float>(b[1]);
+}
+// The value of the neighbouring lane (lane ^ 1).
+__device__ __forceinline__ float other_term(float v) {
+  return bit_cast<float>(__builtin_amdgcn_update_dpp(0, bit_cast<int>(v), 0xB1, 0xF, 0xF, false));
+}
+// 2^(target - exponent of v) for v > 0, within what fp32 can hold.
+__device__ __forceinline__ float power_of_two_to(float v, int target) {
+  const int e = static_cast<int>(bit_cast<uint32_t>(v) >> 23 & 255u);
+  const int s = 254 + target - e;
+  return bit_cast<float>(static_cast<uint32_t>(s > 254 ? 254 : s < 1 ? 1 : s) << 23);
+}
+
+constexpr float kLog2E = 1.44269504088896340736f, kLn2 = 0.69314718055994530942f;
+
+template <KvKind KV, int DP, int NW>
+__global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArgs a) {
+  constexpr bool F32 = KV == KvKind::F32, QUANT = kv_quantized(KV);
+  constexpr int BITS = kv_bits(KV);
+  constexpr int HEADS = F32 ? 16 : 8, KEYS = F32 ? 16 : 32;        // query heads a workgroup, keys a tile
+  constexpr int CE = F32 ? 4 : 128 / BITS < DP / 4 ? 128 / BITS : DP / 4;   // elements of a key a lane loads at once
+  constexpr int RUNS = DP / (4 * CE);                              // such loads a key row
+  constexpr int STEPS = F32 ? DP / 4 : DP / 32;                    // matrix instructions over head_dim
+  constexpr int VE = DP / 16;                                      // elements of a value row a lane holds
+  constexpr int KW = CE * BITS / 32, VW = (VE * BITS + 31) / 32;   // dwords of those
+  constexpr int HALVES = KEYS / 16;
+  __shared__ float merge_m[NW][HEADS], merge_l[NW][HEADS];
+  __shared__ __align__(16) float merge_o[NW][HEADS][16][VE + 4];
+
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, r = lane & 15u, g = lane >> 4;
+  const uint32_t group = a.heads / a.kv_heads, blocks = (group + HEADS - 1) / HEADS;
+  const uint64_t split = a.part.split == 0 ? 1 : a.part.split;
+  uint64_t rest = blockIdx.x / split;
+  const uint64_t s_part = blockIdx.x % split;
+  const uint32_t hb = static_cast<uint32_t>(rest % blocks);
+  rest /= blocks;
+  const uint32_t kv = static_cast<uint32_t>(rest % a.kv_heads);
+  const uint64_t row = rest / a.kv_heads;
+  const uint32_t head0 = kv * group + hb * HEADS, here = group - hb * HEADS < HEADS ? group - hb * HEADS : HEADS;
+  const uint32_t D = a.head_dim;
+
+  uint64_t start, last;
+  key_range(a, row, start, last);
+  if (a.part.split != 0 && !key_chunk(a, s_part, start, last)) {   // workgroup-uniform
+    for (uint32_t i = t; i < here * D; i += NW * 64u) a.part.pacc[((row * a.heads + head0 + i / D) * split + s_part) * D + i % D] = 0.0f;
+    if (t < here) {
+      const uint64_t at = (row * a.heads + head0 + t) * split + s_part;
+      a.part.pmax[at] = -1e30f, a.part.psum[at] = 0.0f;
+    }
+    return;
+  }
+
+  const uint64_t stride = static_cast<uint64_t>(a.kv_heads) * D * BITS / 8;
+  const uint8_t* kb = static_cast<const uint8_t*>(a.k) + static_cast<uint64_t>(kv) * D * BITS / 8;
+  const uint8_t* vb = static_cast<const uint8_t*>(a.v) + static_cast<uint64_t>(kv) * D * BITS / 8;
+  uint32_t kr[HALVES][RUNS][KW], vr[4 * HALVES][VW];
+  float ksv[4 * HALVES], vsv[4 * HALVES];
+  // Rows past the range's end are read as its last row: finite numbers that get the weight 0.
+  auto key_at = [&](uint64_t j) { return j < last ? j : last; };
+  auto load_keys = [&](uint64_t j0) {
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+      const uint8_t* p = kb + key_at(j0 + 16 * h + r) * stride;
+#pragma unroll
+      for (int i = 0; i < RUNS; ++i) {
+        const uint32_t d = (i * 4 + g) * CE;
+        if (d < D) {
+          load_run<CE * BITS / 8>(p + d * BITS / 8, kr[h][i]);
+        } else {
+#pragma unroll
+          for (int w = 0; w < KW; ++w) kr[h][i][w] = 0u;
+        }
+      }
+    }
+    if constexpr (QUANT) {
+#pragma unroll
+      for (int e = 0; e < 4 * HALVES; ++e) ksv[e] = a.k_scale[key_at(j0 + 16 * (e / 4) + 4 * g + e % 4)];
+    }
+  };
+  auto load_values = [&](uint64_t j0) {
+#pragma unroll
+    for (int e = 0; e < 4 * HALVES; ++e) {
+      const uint64_t key = key_at(j0 + 16 * (e / 4) + 4 * g + e % 4);
+      if (r * VE < D) {
+        load_run<VE * BITS / 8>(vb + key * stride + r * VE * BITS / 8, vr[e]);
+      } else {
+#pragma unroll
+        for (int w = 0; w < VW; ++w) vr[e][w] = 0u;
+      }
+      if constexpr (QUANT) vsv[e] = a.v_scale[key];
+    }
+  };
+  const uint64_t first = start + wave * KEYS;
+  if (first <= last) {
+    load_keys(first);
+    load_values(first);
+  }
+
+  // The query operand: column r is head r (fp32) or the term r % 2 of head r / 2.
+  const uint32_t column_head = F32 ? r : r / 2u;
+  const float* qp = a.q + ((a.row_base + row) * a.heads + head0 + (column_head < here ? column_head : here - 1u)) * D;
+  float qf[F32 ? STEPS : 1];
+  half8_t qh[F32 ? 1 : STEPS];
+  float score_scale = kLog2E / sqrtf(static_cast<float>(D));
+  if constexpr (F32) {
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i) {
+      const uint32_t d = (i * 4 + g) * CE;
+      const float4 x = d < D ? *reinterpret_cast<const float4*>(qp + d) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+      qf[4 * i] = x.x, qf[4 * i + 1] = x.y, qf[4 * i + 2] = x.z, qf[4 * i + 3] = x.w;
+    }
+  } else {
+    float raw[STEPS][8], most = 0.0f;
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const uint32_t d = ((i * 8 / CE) * 4 + g) * CE + i * 8 % CE;
+      const float4 x = d < D ? *reinterpret_cast<const float4*>(qp + d) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+      const float4 y = d < D ? *reinterpret_cast<const float4*>(qp + d + 4) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+      raw[i][0] = x.x, raw[i][1] = x.y, raw[i][2] = x.z, raw[i][3] = x.w;
+      raw[i][4] = y.x, raw[i][5] = y.y, raw[i][6] = y.z, raw[i][7] = y.w;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(raw[i][e]));
+    }
+    most = groups_max(most);
+    const float up = power_of_two_to(most, 8);
+    score_scale /= up;
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = raw[i][kq_dim<KV>(e)] * up;
+        const _Float16 hi = static_cast<_Float16>(x);
+        qh[i][e] = (r & 1u) ? static_cast<_Float16>(x - static_cast<float>(hi)) : hi;
+      }
+    }
+  }
+
+  float4_t o[VE];
+#pragma unroll
+  for (int j = 0; j < VE; ++j) o[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  float run_max = -INFINITY, run_sum = 0.0f;
+  float value_most = 0.0f, value_up = F32 ? 1.0f : QUANT ? power_of_two_to(0.0f, 14) : 0x1p14f;
+  for (uint64_t j0 = first; j0 <= last; j0 += NW * KEYS) {
+    const bool more = j0 + NW * KEYS <= last;
+    float s[4 * HALVES];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+      float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+      if constexpr (F32) {
+        float4_t acc2 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < RUNS; ++i) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i][0]), qf[4 * i], acc, 0, 0, 0);
+          acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i][1]), qf[4 * i + 1], acc2, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i][2]), qf[4 * i + 2], acc, 0, 0, 0);
+          acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i][3]), qf[4 * i + 3], acc2, 0, 0, 0);
+        }
+        acc += acc2;
+      } else {
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(key_operand<KV>(&kr[h][i * 8 / CE][i * 8 % CE * BITS / 32]), qh[i], acc, 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float x = acc[e];
+        if constexpr (!F32) x += other_term(x);
+        x *= score_scale;
+        if constexpr (QUANT) x *= ksv[4 * h + e];
+        s[4 * h + e] = j0 + 16 * h + 4 * g + e <= last ? x : -INFINITY;
+      }
+    }
+    if (more) load_keys(j0 + NW * KEYS);
+
+    float most = s[0];
+#pragma unroll
+    for (int e = 1; e < 4 * HALVES; ++e) most = fmaxf(most, s[e]);
+    const float m_new = fmaxf(run_max, groups_max(most));
+    float corr = __builtin_amdgcn_exp2f(run_max - m_new);          // 0 on the first tile (run_max = -inf)
+    run_max = m_new;
+    float sum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4 * HALVES; ++e) {
+      s[e] = __builtin_amdgcn_exp2f(s[e] - m_new);
+      sum += s[e];
+    }
+    run_sum = fmaf(corr, run_sum, sum);
+    if constexpr (QUANT) {
+      // The values' scales enter the weights; the power of two follows the largest of them so far.
+      float vm = fabsf(vsv[0]);
+#pragma unroll
+      for (int e = 1; e < 4 * HALVES; ++e) vm = fmaxf(vm, fabsf(vsv[e]));
+      vm = groups_max(vm);
+      if (vm > value_most) {
+        value_most = vm;
+        const float up = power_of_two_to(vm, 14);
+        corr *= up / value_up;
+        value_up = up;
+      }
+#pragma unroll
+      for (int e = 0; e < 4 * HALVES; ++e) s[e] *= vsv[e] * value_up;
+    } else if constexpr (!F32) {
+#pragma unroll
+      for (int e = 0; e < 4 * HALVES; ++e) s[e] *= value_up;
+    }
+    if (__any(corr != 1.0f)) {
+#pragma unroll
+      for (int j = 0; j < VE; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[j][e] *= corr;
+      }
+    }
+    if constexpr (F32) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+#pragma unroll
+        for (int j = 0; j < VE; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(vr[e][j]), s[e], o[j], 0, 0, 0);
+      }
+    } else {
+      half8_t p;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const _Float16 hi = static_cast<_Float16>(s[e]);
+        p[e] = (r & 1u) ? static_cast<_Float16>(s[e] - static_cast<float>(hi)) : hi;
+      }
+#pragma unroll
+      for (int j = 0; j < VE; ++j) {
+        const uint4 w = {value_pair<KV>(vr[0], vr[1], j), value_pair<KV>(vr[2], vr[3], j),
+                         value_pair<KV>(vr[4 % (4 * HALVES)], vr[5 % (4 * HALVES)], j),
+                         value_pair<KV>(vr[6 % (4 * HALVES)], vr[7 % (4 * HALVES)], j)};
+        o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bit_cast<half8_t>(w), p, o[j], 0, 0, 0);
+      }
+    }
+    if (more) load_values(j0 + NW * KEYS);
+  }
+
+  // Merge of the wavefronts: everyone's sum under the largest score of all, added in wavefront order.
+  run_sum = groups_sum(run_sum);
+  const bool writer = F32 || (r & 1u) == 0u;
+  if (g == 0u && writer) merge_m[wave][column_head] = run_max, merge_l[wave][column_head] = run_sum;
+  __syncthreads();
+  float top = merge_m[0][column_head];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) top = fmaxf(top, merge_m[w][column_head]);
+  const float f = __builtin_amdgcn_exp2f(run_max - top) / value_up;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+#pragma unroll
+    for (int j = 0; j < VE; j += 4) {
+      float4 x;
+      float* xs = &x.x;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) xs[c] = (F32 ? o[j + c][e] : o[j + c][e] + other_term(o[j + c][e])) * f;
+      if (writer) *reinterpret_cast<float4*>(&merge_o[wave][column_head][4 * g + e][j]) = x;
+    }
+  }
+  __syncthreads();
+  for (uint32_t i = t; i < here * D; i += NW * 64u) {
+    const uint32_t h = i / D, d = i % D;
+    float m = merge_m[0][h];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m = fmaxf(m, merge_m[w][h]);
+    float sum = 0.0f, acc = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      sum = fmaf(__builtin_amdgcn_exp2f(merge_m[w][h] - m), merge_l[w][h], sum);
+      acc += merge_o[w][h][d / VE][d % VE];
+    }
+    if (a.part.split != 0) {
+      const uint64_t at = (row * a.heads + head0 + h) * split + s_part;
+      a.part.pacc[at * D + d] = acc;
+      if (d == 0) a.part.pmax[at] = m * kLn2, a.part.psum[at] = sum;
+    } else {
+      a.out[((a.row_base + row) * a.heads + head0 + h) * D + d] = acc / sum;
+    }
+  }
+}
+
+// ---- head sizes that the matrix kernels' 16-byte runs do not divide ------------------------------
+//
+// One workgroup of four wavefronts per (query row, head[, chunk]).  Keys are taken 64 at a time: a
+// wavefront forms the score of a key with its lanes across head_dim (coalesced key reads, a sum over the
+// wavefront), the first wavefront turns the 64 scores into weights against the running maximum, and
+// thread e accumulates weight * v[key][e] (coalesced value reads).
+template <KvKind KV>
+__global__ __launch_bounds__(256) void attention_any_kernel(AttentionArgs a) {
+  constexpr uint32_t kKeys = 64;
+  __shared__ float sc[kKeys], wt[kKeys], bc[2];
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+  const uint64_t split = a.part.split == 0 ? 1 : a.part.split, at = blockIdx.x, rest = at / split;
+  const uint64_t i = rest / a.heads, h = rest % a.heads, kv = h / (a.heads / a.kv_heads), D = a.head_dim;
+  uint64_t start, last;
+  key_range(a, i, start, last);
+  if (a.part.split != 0 && !key_chunk(a, at % split, start, last)) {   // workgroup-uniform
+    if (t < D) a.part.pacc[at * D + t] = 0.0f;
+    if (t == 0) a.part.pmax[at] = -1e30f, a.part.psum[at] = 0.0f;
+    return;
+  }
+  const float scale = 1.0f / sqrtf(static_cast<float>(D));
+  const uint64_t qb = ((a.row_base + i) * a.heads + h) * D;
+  auto kv_at = [&](const void* base, const float* row_scale, uint64_t key, uint64_t idx) {
+    if constexpr (KV == KvKind::F16) {
+      return half_bits_to_float(static_cast<const uint16_t*>(base)[idx]);
+    } else if constexpr (KV == KvKind::F32) {
+      return static_cast<const float*>(base)[idx];
+    } else if constexpr (KV == KvKind::Q8) {
+      return static_cast<float>(static_cast<const int8_t*>(base)[idx]) * row_scale[key];
+    } else if constexpr (KV == KvKind::Q4) {
+      const int nib = (static_cast<const uint8_t*>(base)[idx >> 1] >> ((idx & 1u) * 4u)) & 0xF;
+      return static_cast<float>((nib & 8) ? nib - 16 : nib) * row_scale[key];
+    } else {
+      return e4m3_to_float(static_cast<const uint8_t*>(base)[idx]) * row_scale[key];
+    }
+  };
+  float qr[4];                       // head_dim <= 256: up to four elements a lane
+#pragma unroll
+  for (int cc = 0; cc < 4; ++cc) qr[cc] = lane + 64u * cc < D ? a.q[qb + lane + 64u * cc] : 0.0f;
+
+  float run_max = -INFINITY, run_sum = 0.0f, acc = 0.0f;
+  for (uint64_t j0 = start; j0 <= last; j0 += kKeys) {
+    const uint32_t count = last - j0 + 1 < kKeys ? static_cast<uint32_t>(last - j0 + 1) : kKeys;
+    for (uint32_t kk = wave; kk < kKeys; kk += 4u) {
+      float dot = 0.0f;
+      if (kk < count) {
+        const uint64_t kb = ((j0 + kk) * a.kv_heads + kv) * D;
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) {
+          if (lane + 64u * cc < D) dot = fmaf(qr[cc], kv_at(a.k, a.k_scale, j0 + kk, kb + lane + 64u * cc), dot);
+        }
+      }
+      dot = wave_sum(dot);
+      if (lane == 0) sc[kk] = kk < count ? dot * scale : -INFINITY;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const float s = sc[lane];
+      const float m_new = fmaxf(run_max, wave_max(s));
+      const float w = lane < count ? expf(s - m_new) : 0.0f;
+      wt[lane] = w;
+      const float l = wave_sum(w);
+      if (lane == 0) {
+        bc[0] = m_new;
+        bc[1] = l;
+      }
+    }
+    __syncthreads();
+    const float m_new = bc[0];
+    const float corr = expf(run_max - m_new);      // 0 on the first tile (run_max = -inf)
+    run_sum = fmaf(corr, run_sum, bc[1]);
+    run_max = m_new;
+    if (t < D) {
+      float x = 0.0f;
+      for (uint32_t kk = 0; kk < count; ++kk) {
+        x = fmaf(wt[kk], kv_at(a.v, a.v_scale, j0 + kk, ((j0 + kk) * a.kv_heads + kv) * D + t), x);
+      }
+      acc = fmaf(corr, acc, x);
+    }
+    __syncthreads();
+  }
+  if (a.part.split != 0) {
+    if (t < D) a.part.pacc[at * D + t] = acc;
+    if (t == 0) a.part.pmax[at] = run_max, a.part.psum[at] = run_sum;
+  } else {
+    if (t < D) a.out[qb + t] = acc / run_sum;
+  }
+}
+
+// out[row][head] = sum_s w_s pacc_s / sum_s w_s psum_s with w_s = exp(pmax_s - max_s pmax_s)
+// (src/backends/rocm/rocm_kernels_basic.cpp:664-690).  One workgroup per (row, head); V consecutive
+// elements a lane, the parts dealt to the four wavefronts, several of a wavefront's loads in flight:
+// latency is all there is to 24 rows of 256 over 64 parts, which one chain of parts a thread took
+// 19 us over.
+template <int V>
+__global__ __launch_bounds__(256) void attention_combine_kernel(const float* __restrict__ pacc, const float* __restrict__ pmax,
+                                                                const float* __restrict__ psum, float* __restrict__ out,
+                                                                uint32_t head_dim, uint32_t split) {
+  __shared__ float num[4][256], den[4];
+  const uint64_t at = blockIdx.x, base = at * split;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, e0 = lane * V;
+  float top = -1e30f;
+  for (uint32_t s = lane; s < split; s += 64u) top = fmaxf(top, pmax[base + s]);
+  top = wave_max(top);
+  float n[V] = {}, d = 0.0f;
+#pragma unroll 8
+  for (uint32_t s = wave; s < split; s += 4u) {
+    const float w = expf(pmax[base + s] - top);
+    d = fmaf(w, psum[base + s], d);
+#pragma unroll
+    for (int c = 0; c < V; ++c) {
+      if (e0 + c < head_dim) n[c] = fmaf(w, pacc[(base + s) * head_dim + e0 + c], n[c]);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < V; ++c) num[wave][e0 + c] = n[c];
+  if (lane == 0) den[wave] = d;
+  __syncthreads();
+  if (threadIdx.x < head_dim) {
+    const uint32_t e = threadIdx.x;
+    out[at * head_dim + e] = (((num[0][e] + num[1][e]) + num[2][e]) + num[3][e]) / (((den[0] + den[1]) + den[2]) + den[3]);
+  }
+}
+
+// ---- dispatch ------------------------------------------------------------------------------------
+
+template <KvKind KV>
+hipError_t launch_rows(const AttentionArgs& a, uint64_t m, hipStream_t stream) {
+  constexpr uint32_t kHeads = KV == KvKind::F32 ? 16 : 8;
+  const uint32_t group = a.heads / a.kv_heads, blocks = (group + kHeads - 1) / kHeads;
+  const uint64_t split = a.part.split == 0 ? 1 : a.part.split;
+  const dim3 grid(static_cast<uint32_t>(m * a.kv_heads * blocks * split));
+  // Four wavefronts a workgroup take 128 keys at once; where a workgroup has more to do and the
+  // registers allow it, eight.
+  const bool wide = a.n / split > 160;
+  auto go = [&](auto kernel, uint32_t waves) { hipLaunchKernelGGL(kernel, grid, dim3(waves * 64u), 0, stream, a); };
+  if (a.head_dim <= 64) {
+    wide ? go(attention_rows_kernel<KV, 64, 8>, 8) : go(attention_rows_kernel<KV, 64, 4>, 4);
+  } else if (a.head_dim <= 128) {
+    wide ? go(attention_rows_kernel<KV, 128, 8>, 8) : go(attention_rows_kernel<KV, 128, 4>, 4);
+  } else {
+    go(attention_rows_kernel<KV, 256, 4>, 4);
+  }
+  return hipGetLastError();
+}
+
+// kind: 0 fp32, 1 fp16 keys and values; 2 int8, 3 4-bit, 4 E4M3 codes with one scale per key row.
+hipError_t launch_attention_as(uint32_t kind, const AttentionArgs& a, uint64_t m, hipStream_t stream) {
+  auto go = [&](auto tag) {
+    constexpr KvKind KV = decltype(tag)::value;
+    // The runs that the lanes load divide a head's row: 16 bytes of a key (a quarter of the padded row
+    // where that is less), a sixteenth of the padded row of a value.
+    const uint32_t padded = a.head_dim <= 64 ? 64 : a.head_dim <= 128 ? 128 : 256;
+    const uint32_t run = KV == KvKind::F32 ? 4 : 128u / kv_bits(KV) < padded / 4 ? 128u / kv_bits(KV) : padded / 4;
+    if (a.head_dim % run == 0 && a.head_dim % (padded / 16) == 0) return launch_rows<KV>(a, m, stream);
+    const uint64_t parts = a.part.split == 0 ? 1 : a.part.split;
+    hipLaunchKernelGGL(attention_any_kernel<KV>, dim3(static_cast<uint32_t>(m * a.heads * parts)), dim3(256), 0, stream, a);
+    return hipGetLastError();
+  };
+  switch (kind) {
+    case 0: return go(std::integral_constant<KvKind, KvKind::F32>{});
+    case 1: return go(std::integral_constant<KvKind, KvKind::F16>{});
+    case 2: return go(std::integral_constant<KvKind, KvKind::Q8>{});
+    case 3: return go(std::integral_constant<KvKind, KvKind::Q4>{});
+    default: return go(std::integral_constant<KvKind, KvKind::Fp8>{});
+  }
+}
+
+AttentionArgs args_of(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale, float* out,
+                      uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t row_base,
+                      uint64_t window, bool causal) {
+  return AttentionArgs{q, k, v, k_scale, v_scale, out, SplitOut{}, n, q_base, row_base, window, static_cast<uint32_t>(heads),
+                       static_cast<uint32_t>(kv_heads), static_cast<uint32_t>(head_dim), causal ? 1u : 0u};
+}
+
+}  // namespace
+
+hipError_t launch_attention(const float* q, const void* k, const void* v, float* out, uint64_t m, uint64_t n, uint64_t heads,
+                            uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t row_base, uint64_t window,
+                            bool kv_f16, bool causal, hipStream_t stream) {
+  return launch_attention_as(kv_f16 ? 1u : 0u, args_of(q, k, v, nullptr, nullptr, out, n, heads, kv_heads, head_dim, q_base, row_base,
+                                                       window, causal), m, stream);
+}
+
+// kind: 0 int8, 1 4-bit, 2 E4M3 keys and values with one scale per key row; always causal.
+hipError_t launch_attention_quant(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
+                                  float* out, uint64_t m, uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
+                                  uint64_t q_base, uint64_t row_base, uint64_t window, uint32_t kind, hipStream_t stream) {
+  return launch_attention_as(2u + kind, args_of(q, k, v, k_scale, v_scale, out, n, heads, kv_heads, head_dim, q_base, row_base, window,
+                                                true), m, stream);
+}
+
+// The split-N form: kv_kind as launch_attention_as (0 fp32, 1 fp16, 2.. quantized with scales).
+hipError_t launch_attention_split(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
+                                  float* pacc, float* pmax, float* psum, uint64_t m, uint64_t n, uint64_t heads,
+                                  uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t window, uint32_t kv_kind,
+                                  bool causal, uint64_t split, hipStream_t stream) {
+  AttentionArgs a = args_of(q, k, v, k_scale, v_scale, nullptr, n, heads, kv_heads, head_dim, q_base, 0, window, causal);
+  a.part = SplitOut{pacc, pmax, psum, split};
+  return launch_attention_as(kv_kind, a, m, stream);
+}
+
+hipError_t launch_attention_combine(const float* pacc, const float* pmax, const float* psum, float* out, uint64_t m,
+                                    uint64_t heads, uint64_t head_dim, uint64_t split, hipStream_t stream) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(m * heads)), dim3(256), 0, stream, pacc, pmax, psum, out,
+                       static_cast<uint32_t>(head_dim), static_cast<uint32_t>(split));
+  };
+  head_dim <= 64 ? go(attention_combine_kernel<1>) : head_dim <= 128 ? go(attention_combine_kernel<2>) : go(attention_combine_kernel<4>);
+  return hipGetLastError();
+}
+
+}  // namespace qmm

@@ -1,6 +1,6 @@
 // The non-matmul pieces of a transformer block that sit between the projections, as plain correct
-// kernels so that a trunk can run on this backend end to end: rotary embeddings, softmax attention
-// over a key/value cache, the query/gate split of gated attention.  Contracts:
+// kernels so that a trunk can run on this backend end to end: rotary embeddings, the quantizers of a
+// key/value cache, the query/gate split of gated attention (attention itself: attention.hip).  Contracts:
 // include/tessera/backend.hpp:162-179,378-390; CPU statements src/core/numerics/attention.cpp.
 // None of them is tuned: they move kilobytes where the projections move megabytes.
 
@@ -29,146 +29,6 @@ __global__ __launch_bounds__(256) void rope_kernel(float* __restrict__ data, con
   const float x1 = base[j], x2 = base[j + pairs];
   base[j] = x1 * c - x2 * s;
   base[j + pairs] = x1 * s + x2 * c;
-}
-
-// One workgroup of four wavefronts per (query row, head).  Keys are taken 64 at a time: a
-// wavefront forms the score of a key with its lanes across head_dim (coalesced key reads, a DPP
-// sum), the first wavefront turns the 64 scores into weights against the running maximum, and
-// thread e accumulates weight * v[key][e] (coalesced value reads): the usual running softmax, so
-// the result differs from AttentionRef (src/core/numerics/attention.cpp:158-225) in summation
-// order only.
-// KV: how keys and values are stored.  The quantized kinds hold codes and one fp32 scale per key
-// row (all kv heads of a position), and an element is code * scale as in AttentionQ8Ref /
-// AttentionQ4Ref / AttentionFp8Ref (src/core/numerics/attention.cpp:45-121).
-enum class KvKind { F32, F16, Q8, Q4, Fp8 };
-
-// SPLIT (the flash-decoding ids, src/backends/rocm/rocm_kernels_basic.cpp:275-440): workgroup
-// (row, head, s) covers chunk s of ceil(span / split) keys of the row's key range and leaves the
-// unnormalized sum, the chunk's largest score and its sum of weights in pacc / pmax / psum at
-// index (row * heads + head) * split + s (an empty chunk: 0, -1e30, 0); attention_combine_kernel
-// merges them.
-struct SplitOut {
-  float *pacc, *pmax, *psum;
-  uint64_t split;
-};
-
-template <KvKind KV, bool SPLIT>
-__global__ __launch_bounds__(256) void attention_kernel(const float* __restrict__ q, const void* __restrict__ k,
-                                                        const void* __restrict__ v, const float* __restrict__ k_scale,
-                                                        const float* __restrict__ v_scale, float* __restrict__ out,
-                                                        SplitOut part, uint64_t n, uint64_t heads, uint64_t kv_heads,
-                                                        uint64_t head_dim, uint64_t q_base, uint64_t row_base, uint64_t window,
-                                                        uint64_t causal) {
-  constexpr uint32_t kKeys = 64;
-  __shared__ float sc[kKeys], wt[kKeys], bc[2];
-  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-  const uint64_t g = blockIdx.x, rest = SPLIT ? g / part.split : g;
-  const uint64_t i = rest / heads, h = rest % heads, kv = h / (heads / kv_heads);
-  const uint64_t pos = q_base + i;
-  uint64_t last = causal != 0 ? (pos >= n ? n - 1 : pos) : n - 1;
-  uint64_t start = 0;
-  if (causal != 0) {
-    start = (window != 0 && pos + 1 > window) ? pos + 1 - window : 0;
-    if (start > last) start = last;
-  }
-  if constexpr (SPLIT) {
-    const uint64_t chunk = (last + 1 - start + part.split - 1) / part.split;
-    const uint64_t cstart = start + (g % part.split) * chunk;
-    if (cstart > last) {   // workgroup-uniform
-      if (t < head_dim) part.pacc[g * head_dim + t] = 0.0f;
-      if (t == 0) part.pmax[g] = -1e30f, part.psum[g] = 0.0f;
-      return;
-    }
-    last = cstart + chunk - 1 < last ? cstart + chunk - 1 : last;
-    start = cstart;
-  }
-  const float scale = 1.0f / sqrtf(static_cast<float>(head_dim));
-  const uint64_t qb = ((row_base + i) * heads + h) * head_dim;
-  auto kv_at = [&](const void* base, const float* row_scale, uint64_t key, uint64_t idx) {
-    if constexpr (KV == KvKind::F16) {
-      return half_bits_to_float(static_cast<const uint16_t*>(base)[idx]);
-    } else if constexpr (KV == KvKind::F32) {
-      return static_cast<const float*>(base)[idx];
-    } else if constexpr (KV == KvKind::Q8) {
-      return static_cast<float>(static_cast<const int8_t*>(base)[idx]) * row_scale[key];
-    } else if constexpr (KV == KvKind::Q4) {
-      const int nib = (static_cast<const uint8_t*>(base)[idx >> 1] >> ((idx & 1u) * 4u)) & 0xF;
-      return static_cast<float>((nib & 8) ? nib - 16 : nib) * row_scale[key];
-    } else {
-      return e4m3_to_float(static_cast<const uint8_t*>(base)[idx]) * row_scale[key];
-    }
-  };
-  float qr[4];                       // head_dim <= 256: up to four elements a lane
-#pragma unroll
-  for (int cc = 0; cc < 4; ++cc) qr[cc] = lane + 64u * cc < head_dim ? q[qb + lane + 64u * cc] : 0.0f;
-
-  float run_max = -INFINITY, run_sum = 0.0f, acc = 0.0f;
-  for (uint64_t j0 = start; j0 <= last; j0 += kKeys) {
-    const uint32_t count = last - j0 + 1 < kKeys ? static_cast<uint32_t>(last - j0 + 1) : kKeys;
-    for (uint32_t kk = wave; kk < kKeys; kk += 4u) {
-      float dot = 0.0f;
-      if (kk < count) {
-        const uint64_t kb = ((j0 + kk) * kv_heads + kv) * head_dim;
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) {
-          if (lane + 64u * cc < head_dim) dot = fmaf(qr[cc], kv_at(k, k_scale, j0 + kk, kb + lane + 64u * cc), dot);
-        }
-      }
-      dot = wave_sum(dot);
-      if (lane == 0) sc[kk] = kk < count ? dot * scale : -INFINITY;
-    }
-    __syncthreads();
-    if (wave == 0) {
-      const float s = sc[lane];
-      const float m_new = fmaxf(run_max, wave_max(s));
-      const float w = lane < count ? expf(s - m_new) : 0.0f;
-      wt[lane] = w;
-      const float l = wave_sum(w);
-      if (lane == 0) {
-        bc[0] = m_new;
-        bc[1] = l;
-      }
-    }
-    __syncthreads();
-    const float m_new = bc[0];
-    const float corr = expf(run_max - m_new);      // 0 on the first tile (run_max = -inf)
-    run_sum = fmaf(corr, run_sum, bc[1]);
-    run_max = m_new;
-    if (t < head_dim) {
-      float a = 0.0f;
-      for (uint32_t kk = 0; kk < count; ++kk) {
-        a = fmaf(wt[kk], kv_at(v, v_scale, j0 + kk, ((j0 + kk) * kv_heads + kv) * head_dim + t), a);
-      }
-      acc = fmaf(corr, acc, a);
-    }
-    __syncthreads();
-  }
-  if constexpr (SPLIT) {
-    if (t < head_dim) part.pacc[g * head_dim + t] = acc;
-    if (t == 0) part.pmax[g] = run_max, part.psum[g] = run_sum;
-  } else {
-    if (t < head_dim) out[qb + t] = acc / run_sum;
-  }
-}
-
-// out[row][head] = sum_s w_s pacc_s / sum_s w_s psum_s with w_s = exp(pmax_s - max_s pmax_s)
-// (src/backends/rocm/rocm_kernels_basic.cpp:664-690).  One workgroup per (row, head).
-__global__ __launch_bounds__(256) void attention_combine_kernel(const float* __restrict__ pacc, const float* __restrict__ pmax,
-                                                                const float* __restrict__ psum, float* __restrict__ out,
-                                                                uint64_t head_dim, uint64_t split) {
-  const uint64_t g = blockIdx.x, base = g * split;
-  const uint32_t e = threadIdx.x;
-  float top = -1e30f;
-  for (uint64_t s = 0; s < split; ++s) top = fmaxf(top, pmax[base + s]);
-  if (e < head_dim) {
-    float num = 0.0f, den = 0.0f;
-    for (uint64_t s = 0; s < split; ++s) {
-      const float w = expf(pmax[base + s] - top);
-      num = fmaf(w, pacc[(base + s) * head_dim + e], num);
-      den = fmaf(w, psum[base + s], den);
-    }
-    out[g * head_dim + e] = num / den;
-  }
 }
 
 __global__ __launch_bounds__(256) void qgate_split_kernel(const float* __restrict__ fused, float* __restrict__ q,
@@ -243,60 +103,6 @@ hipError_t launch_rope(float* data, const uint64_t* pos3, uint64_t rows, uint64_
                        uint64_t pos_base, float theta, uint64_t sec_t, uint64_t sec_h, hipStream_t stream) {
   hipLaunchKernelGGL(rope_kernel, blocks_for(rows * heads * (rope_dim / 2)), dim3(256), 0, stream, data, pos3, rows, heads,
                      head_dim, rope_dim, pos_base, theta, sec_t, sec_h);
-  return hipGetLastError();
-}
-
-namespace {
-// kind: 0 fp32, 1 fp16 keys and values; 2 int8, 3 4-bit, 4 E4M3 codes with one scale per key row.
-template <bool SPLIT>
-hipError_t launch_attention_as(uint32_t kind, dim3 grid, const float* q, const void* k, const void* v, const float* k_scale,
-                               const float* v_scale, float* out, SplitOut part, uint64_t n, uint64_t heads, uint64_t kv_heads,
-                               uint64_t head_dim, uint64_t q_base, uint64_t row_base, uint64_t window, bool causal,
-                               hipStream_t stream) {
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, q, k, v, k_scale, v_scale, out, part, n, heads, kv_heads, head_dim,
-                       q_base, row_base, window, causal ? 1ull : 0ull);
-  };
-  switch (kind) {
-    case 0: go(attention_kernel<KvKind::F32, SPLIT>); break;
-    case 1: go(attention_kernel<KvKind::F16, SPLIT>); break;
-    case 2: go(attention_kernel<KvKind::Q8, SPLIT>); break;
-    case 3: go(attention_kernel<KvKind::Q4, SPLIT>); break;
-    default: go(attention_kernel<KvKind::Fp8, SPLIT>); break;
-  }
-  return hipGetLastError();
-}
-}  // namespace
-
-hipError_t launch_attention(const float* q, const void* k, const void* v, float* out, uint64_t m, uint64_t n, uint64_t heads,
-                            uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t row_base, uint64_t window,
-                            bool kv_f16, bool causal, hipStream_t stream) {
-  return launch_attention_as<false>(kv_f16 ? 1u : 0u, dim3(static_cast<uint32_t>(m * heads)), q, k, v, nullptr, nullptr, out,
-                                    SplitOut{}, n, heads, kv_heads, head_dim, q_base, row_base, window, causal, stream);
-}
-
-// kind: 0 int8, 1 4-bit, 2 E4M3 keys and values with one scale per key row; always causal.
-hipError_t launch_attention_quant(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
-                                  float* out, uint64_t m, uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
-                                  uint64_t q_base, uint64_t row_base, uint64_t window, uint32_t kind, hipStream_t stream) {
-  return launch_attention_as<false>(2u + kind, dim3(static_cast<uint32_t>(m * heads)), q, k, v, k_scale, v_scale, out, SplitOut{},
-                                    n, heads, kv_heads, head_dim, q_base, row_base, window, true, stream);
-}
-
-// The split-N form: kv_kind as launch_attention_as (0 fp32, 1 fp16, 2.. quantized with scales).
-hipError_t launch_attention_split(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
-                                  float* pacc, float* pmax, float* psum, uint64_t m, uint64_t n, uint64_t heads,
-                                  uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t window, uint32_t kv_kind,
-                                  bool causal, uint64_t split, hipStream_t stream) {
-  return launch_attention_as<true>(kv_kind, dim3(static_cast<uint32_t>(m * heads * split)), q, k, v, k_scale, v_scale, nullptr,
-                                   SplitOut{pacc, pmax, psum, split}, n, heads, kv_heads, head_dim, q_base, 0, window, causal,
-                                   stream);
-}
-
-hipError_t launch_attention_combine(const float* pacc, const float* pmax, const float* psum, float* out, uint64_t m,
-                                    uint64_t heads, uint64_t head_dim, uint64_t split, hipStream_t stream) {
-  hipLaunchKernelGGL(attention_combine_kernel, dim3(static_cast<uint32_t>(m * heads)), dim3(256), 0, stream, pacc, pmax, psum, out,
-                     head_dim, split);
   return hipGetLastError();
 }
 

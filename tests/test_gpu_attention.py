@@ -1,0 +1,125 @@
+"""Attention over every kind of cache at the edges of its dispatch: head sizes around the padded sizes of
+the matrix kernels (64, 128, 256) and ones their loads do not divide, query heads per key head around the
+columns of a matrix instruction, key counts around the tiles, a value scale of zero, rising and falling
+scales.  Against the oracle's restatements; bound as in test_gpu_trunk.py (sums in another order)."""
+import numpy as np
+import pytest
+
+import oracle
+from tessera_amd import synth
+from util import run
+
+pytestmark = pytest.mark.gpu
+
+KINDS = {"f32": 0, "f16": 1, "q8": 2, "q4": 3, "fp8": 4}
+
+
+def cache(g, kind, n, width, gain=None):
+    """Keys or values as the cache holds them: (elements or codes, scales or None)."""
+    x = g.standard_normal((n, width)).astype(np.float32)
+    if gain is not None:
+        x *= gain[:, None].astype(np.float32)
+    if kind == "f32":
+        return x, None
+    if kind == "f16":
+        return x.astype(np.float16), None
+    if kind == "fp8":
+        return oracle.quantize_fp8_pack(x, n, width)
+    return oracle.quantize_kv(x, n, width, 8 if kind == "q8" else 4)
+
+
+def attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, q_base, window, row_base=0, causal=1, split=0):
+    """The attention id of the cache kind, or its split form and the merge; rows of the whole batch buffer."""
+    total = q.shape[0]
+    dq, dk, dv = backend.Upload(q), backend.Upload(k), backend.Upload(v)
+    scales = [] if ks is None else [backend.Upload(ks), backend.Upload(vs)]
+    dout = backend.Upload(np.full((total, heads * head_dim), 7.0, np.float32))
+    tail = [window, int(kind == "f16"), causal] if ks is None else [window, KINDS[kind] - 2]
+    base = "attention" if ks is None else f"attention_{kind}"
+    if not split:
+        run(backend, base, [dq, dk, dv, *scales, dout], [m, n, heads, kv_heads, head_dim, q_base, row_base, *tail], grid=(m * heads, 1, 1))
+    else:
+        parts = [backend.AllocateBuffer(4 * m * heads * split * w) for w in (head_dim, 1, 1)]
+        run(backend, base + "_split", [dq, dk, dv, *scales, *parts], [m, n, heads, kv_heads, head_dim, q_base, *tail, split],
+            grid=(m * heads * split, 1, 1))
+        run(backend, "attention_combine", [*parts, dout], [m, heads, head_dim, split], grid=(m * heads, 1, 1))
+    backend.Synchronize()
+    return backend.CopyD2H(dout, dtype=np.float32).reshape(total, heads * head_dim)
+
+
+def expected(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, q_base, window, causal=1):
+    if ks is None:
+        return oracle.attention(q, k, v, m, n, heads, kv_heads, head_dim, q_base, window, kind == "f16", bool(causal))
+    return oracle.attention_quant(q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, kind, q_base, window)
+
+
+CASES = [
+    # m, n, heads, kv_heads, head_dim, q_base, window
+    (1, 1, 1, 1, 64, 0, 0),
+    (1, 31, 4, 4, 64, 30, 0),            # one head a key head, a tile less one key
+    (1, 33, 8, 1, 128, 32, 0),           # all eight columns
+    (2, 128, 9, 1, 128, 126, 0),         # nine heads: a second block of one
+    (1, 129, 17, 1, 64, 128, 0),         # three blocks; over fp32 two of sixteen
+    (1, 300, 16, 4, 64, 299, 0),
+    (3, 517, 24, 4, 256, 514, 0),
+    (1, 700, 6, 2, 256, 699, 250),       # window
+    (2, 90, 6, 3, 96, 88, 0),            # padded to 128
+    (2, 90, 4, 2, 80, 88, 0),            # divides the runs of some kinds only
+    (2, 70, 4, 2, 160, 60, 0),           # padded to 256
+    (1, 45, 2, 1, 16, 44, 0),
+    (2, 50, 2, 1, 24, 48, 0),
+    (2, 50, 8, 4, 34, 48, 0),            # no kind's runs
+]
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("case", CASES)
+def test_attention_edges(backend, kind, case):
+    m, n, heads, kv_heads, head_dim, q_base, window = case
+    g = synth.rng(n * 7 + head_dim + KINDS[kind])
+    width = kv_heads * head_dim
+    q = g.standard_normal((m + 3, heads * head_dim)).astype(np.float32)
+    k, ks = cache(g, kind, n, width)
+    v, vs = cache(g, kind, n, width)
+    want = expected(kind, q[2:2 + m], k, v, ks, vs, m, n, heads, kv_heads, head_dim, q_base, window)
+    bound = 2e-6 * max(1.0, np.max(np.abs(want)))
+    got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, q_base, window, row_base=2)
+    assert np.max(np.abs(got[2:2 + m] - want)) <= bound
+    assert np.all(got[:2] == 7.0) and np.all(got[2 + m:] == 7.0)
+    for split in (1, 3, 7):
+        got = attend(backend, kind, np.ascontiguousarray(q[2:2 + m]), k, v, ks, vs, m, n, heads, kv_heads, head_dim, q_base, window,
+                     split=split)
+        assert np.max(np.abs(got - want)) <= 2 * bound, split
+
+
+@pytest.mark.parametrize("kind", ["q8", "q4", "fp8"])
+@pytest.mark.parametrize("shape", ["rising", "falling", "zeros", "tiny"])
+def test_attention_value_scales_over_many_binades(backend, kind, shape):
+    """The values' scales enter the weights under a power of two that follows the largest so far."""
+    m, n, heads, kv_heads, head_dim = 2, 400, 6, 2, 128
+    g = synth.rng(900 + len(shape))
+    gain = {"rising": np.exp2(np.linspace(-40, 10, n)), "falling": np.exp2(np.linspace(10, -40, n)),
+            "zeros": np.where(np.arange(n) < 200, 0.0, 1.0), "tiny": np.full(n, 1e-30)}[shape]
+    q = g.standard_normal((m, heads * head_dim)).astype(np.float32)
+    k, ks = cache(g, kind, n, kv_heads * head_dim)
+    v, vs = cache(g, kind, n, kv_heads * head_dim, gain)
+    want = expected(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0)
+    got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0)
+    assert np.max(np.abs(got - want)) <= 4e-6 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("gain", [2.0 ** -60, 2.0 ** 40])
+def test_attention_query_magnitudes(backend, kind, gain):
+    """Queries far from 1 (their keys far the other way where the cache can hold that, else scores near zero
+    or a one-hot softmax): the power of two under which they enter is undone exactly."""
+    m, n, heads, kv_heads, head_dim = 1, 150, 4, 2, 64
+    g = synth.rng(77)
+    q = (g.standard_normal((m, heads * head_dim)) * gain).astype(np.float32)
+    k, ks = cache(g, kind, n, kv_heads * head_dim)
+    if kind == "f32":
+        k = (k / np.float32(gain)).astype(np.float32)
+    v, vs = cache(g, kind, n, kv_heads * head_dim)
+    want = expected(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - 1, 0)
+    got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - 1, 0)
+    assert np.max(np.abs(got - want)) <= 4e-6 * max(1.0, np.max(np.abs(want)))
