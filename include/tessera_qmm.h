@@ -180,7 +180,8 @@ size_t qmm_static_scratch_bytes(void);
  * (256-byte aligned) to use for every later qmm_launch on any stream, in stream order, until it
  * is replaced or cleared with (NULL, 0); while one is set, qmm_launch allocates nothing and a
  * launch that needs more returns InvalidArgument.  The caller must not free or replace the
- * block while launches that use it are in flight. */
+ * block while launches that use it are in flight.  ("gemm_fp8" is the exception to the refusal: with less
+ * than it asks for it runs its slower passes that need none.) */
 qmm_status qmm_workspace_bytes(qmm_kernel kernel, const uint64_t* scalars, size_t nscalars, size_t* out_bytes);
 qmm_status qmm_set_workspace(void* device_ptr, size_t bytes);
 

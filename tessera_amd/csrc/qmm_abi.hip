@@ -166,6 +166,7 @@ void* decode_scratch(const LaunchCtx& c) {
 constexpr uint64_t kQ4KGemmMinRows = 17;
 constexpr uint64_t kQ4KTensorRowsDefault = 64;
 std::atomic<uint64_t> g_q4k_tensor_rows{kQ4KTensorRowsDefault};
+constexpr uint64_t kFp8GemmMinRows = 17;     // below: E4M3 terms on a large matrix, else the VALU GEMV passes
 constexpr uint64_t kMxfp4GemmMinRows = 17;   // below: the VALU GEMV passes, exact fp32 order
 constexpr uint64_t kQ4KFewRowsMinWeights = uint64_t{16} << 20;
 constexpr uint64_t kQ4KRows16MinRows = 3;      // from here the 16x16x32 kernel, below the 4x4x4 one
@@ -1025,6 +1026,19 @@ qmm_status run_gemm_fp8(const LaunchCtx& c) {
                                             c.ptr<float>(3), decode_scratch(c), static_cast<uint32_t>(m),
                                             static_cast<uint32_t>(n), static_cast<uint32_t>(k), false, c.stream));
   }
+  // More rows: the weights as fp16 on the matrix cores against two fp16 terms of each row (gemm_fp8.hip).  Where
+  // the scratch for the terms cannot be had (a workspace of the caller's that is too small, growth while the
+  // stream is captured) the multiply-add passes below need none.
+  if (m >= kFp8GemmMinRows && qmm::gemm_fp8_f16_supported(m, n, k)) {
+    const size_t bytes = qmm::gemm_fp8_f16_workspace_bytes(m, n, k);
+    void* ws = bytes <= kDecodeScratchBytes ? decode_scratch(c) : nullptr;
+    if (ws != nullptr || workspace(c, bytes, &ws) == QMM_OK) {
+      return map_hip(qmm::launch_fp8_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<const float>(2),
+                                              c.ptr<float>(3), ws, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
+                                              static_cast<uint32_t>(k), c.stream));
+    }
+    g_last_error.clear();
+  }
   return map_hip(qmm::launch_fp8_gemv(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<const float>(2),
                                       c.ptr<float>(3), static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                       static_cast<uint32_t>(k), c.stream));
@@ -1526,6 +1540,12 @@ qmm_status qmm_workspace_bytes(qmm_kernel kernel, const uint64_t* scalars, size_
   } else if (id == "gemm_mxfp4" || id == "gemm_mxfp4_batched") {
     const uint64_t m = sc(0), k = sc(2);
     if (m >= kMxfp4GemmMinRows && qmm::gemm_mxfp4_f32_supported(m, k)) *out_bytes = qmm::gemm_mxfp4_f32_workspace_bytes(m, k);
+  } else if (id == "gemm_fp8") {
+    const uint64_t m = sc(0), n = sc(1), k = sc(2);
+    if (n != 0 && m >= kFp8GemmMinRows && qmm::gemm_fp8_f16_supported(m, n, k)) {
+      const size_t bytes = qmm::gemm_fp8_f16_workspace_bytes(m, n, k);
+      if (bytes > kDecodeScratchBytes) *out_bytes = bytes;
+    }
   } else if (starts("gemm_q5k") || starts("gemm_q6k")) {
     const uint64_t m = sc(0), n = sc(1), k = sc(2);
     if (m >= kQ4KGemmMinRows && qmm::gemm_kquant_f16_supported(m, n, k)) *out_bytes = qmm::gemm_kquant_f16_workspace_bytes(m, n, k);
