@@ -38,6 +38,8 @@
 // of the matrix whether or not that is a multiple of 16 rows: the CUs then stream equal byte counts,
 // which is what sets the duration of a launch that is bound by memory.
 
+#include <type_traits>
+
 #include "i8_limbs.hpp"
 #include "qmm_device.hpp"
 #include "qmm_kernels.hpp"
@@ -376,6 +378,201 @@ __global__ __launch_bounds__(WMAX * 64) void kquant_rows_kernel(KqArgs p) {
   }
 }
 
+// ---- the same sums with the weights streamed through LDS ------------------------------------------------------
+// A wavefront owns ONE 256-wide block column of its workgroup's K part, keeps the activations' operands for it in
+// registers from start to end, and walks the workgroup's 16-row tiles: the kernel above converts every block of K
+// for its four to five tiles, which with five rows takes as long as the tiles' sums.  A unit (16 rows x one block) comes by coalesced 16-byte direct loads into a private ring of LDS
+// slots, RING - 1 units ahead; a lane then reads the registers that the kernel above loads from memory with
+// 2-byte-aligned 8-byte accesses to sixteen rows at once.  Up to eight activation rows a pass in every format.
+// K parts leave their sums in a scratch buffer that a reduce launch adds in part order.  Bound by vector issue
+// (Q6_K, 5 rows: about 260 instructions a unit, three wavefronts a SIMD; eight wavefronts instead of twelve were
+// 41.6 us against 33.3 on 5120 x 17408, whose 73 MB take 14 us at the rate of a copy).  The rule that picks this
+// form and both sides' figures: kquant_rows_stream in qmm_abi.hip.
+template <class F>
+struct KqUnit {   // pieces of 16 bytes from the 16-byte boundary at or below the block's start
+  static constexpr uint32_t kPieces = F::kBlock % 16u == 0u ? F::kBlock / 16u : F::kBlock / 16u + 1u;
+  static constexpr uint32_t kRow = kPieces * 16u, kBytes = 16u * kRow;
+  static constexpr int kLoads = (16u * kPieces + 63u) / 64u;
+};
+
+struct KqStreamArgs {
+  const uint8_t* w;
+  const uint8_t* w_end;    // one past the matrix (`w` may point into its middle)
+  const float* x;
+  float* out;              // [parts][m][ld], ld = n when there is one part
+  uint32_t m, n, nblk, parts, groups, tiles_per_wg, tiles_per_sync, ld;
+};
+
+__device__ __forceinline__ void kq_direct16(const void* base, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+
+// Sums over the lane groups (16 lanes each) of NA sets' values; register q of the result holds, in lane group g,
+// row 4 q + 2 (g & 1) + (g >> 1) of the pass.
+__device__ __forceinline__ float swap32_add(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(bit_cast<uint32_t>(a), bit_cast<uint32_t>(b), false, false);
+  return bit_cast<float>(r[0]) + bit_cast<float>(r[1]);
+}
+__device__ __forceinline__ float swap16_add(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(bit_cast<uint32_t>(a), bit_cast<uint32_t>(b), false, false);
+  return bit_cast<float>(r[0]) + bit_cast<float>(r[1]);
+}
+template <class F, int NA, int NQ>
+__device__ __forceinline__ void kq_rows_of(const float (&val)[NA], float (&res)[NQ]) {
+  auto at = [&](int s) { return s < NA ? val[s < NA ? s : 0] : 0.0f; };
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if constexpr (F::kRowsPerSet == 2) res[q] = swap16_add(at(2 * q), at(2 * q + 1));
+    else res[q] = swap16_add(swap32_add(at(4 * q), at(4 * q + 1)), swap32_add(at(4 * q + 2), at(4 * q + 3)));
+  }
+}
+
+template <class F, int NA, int RING, int WMAX>
+__global__ __launch_bounds__(WMAX * 64) void kquant_rows_stream_kernel(KqStreamArgs p) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  using U = KqUnit<F>;
+  constexpr int kRows = NA * F::kRowsPerSet, kQuads = (kRows + 3) / 4;
+  const uint32_t lane = threadIdx.x & 63u, ln = lane & 15u, g = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t waves = blockDim.x >> 6;
+  // K part i has blocks [i nblk / parts, (i + 1) nblk / parts); wavefronts past its columns leave before any barrier
+  const uint32_t part = blockIdx.x / p.groups, wg = blockIdx.x - part * p.groups;
+  const uint32_t b0 = part * p.nblk / p.parts, cols = (part + 1u) * p.nblk / p.parts - b0;
+  const uint32_t tiles_total = (p.n + 15u) >> 4, tile0 = wg * p.tiles_per_wg;
+  if (wave >= cols || tile0 >= tiles_total) return;
+  const uint32_t tiles = tiles_total - tile0 < p.tiles_per_wg ? tiles_total - tile0 : p.tiles_per_wg;
+  const uint32_t col = b0 + wave, row_bytes = p.nblk * F::kBlock, row0 = tile0 * 16u;
+
+  uint8_t* ring = lds + wave * (RING * U::kBytes);
+  const uint32_t ring_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)ring));
+  uint8_t* slot = lds + waves * (RING * U::kBytes) + wave * kSlot;
+  float* table = reinterpret_cast<float*>(lds + waves * (RING * U::kBytes + kSlot));   // [tiles per sync][cols][4 kQuads][16]
+
+  // the activations of the column, in registers before the first weights are asked for
+  float4_t xr[kRows];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    const uint32_t src = static_cast<uint32_t>(r) < p.m ? r : 0u;
+    xr[r] = *reinterpret_cast<const float4_t*>(p.x + (static_cast<size_t>(src) * p.nblk + col) * 256u + lane * 4u);
+  }
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) asm volatile("" : "+v"(xr[r]));
+
+  uint32_t piece_row[U::kLoads], piece_off[U::kLoads];
+#pragma unroll
+  for (int i = 0; i < U::kLoads; ++i) {
+    uint32_t pc = i * 64u + lane;
+    pc = pc < 16u * U::kPieces ? pc : 16u * U::kPieces - 1u;
+    piece_row[i] = pc / U::kPieces;
+    piece_off[i] = (pc - piece_row[i] * U::kPieces) * 16u;
+  }
+  constexpr bool kShifted = F::kBlock % 16u != 0u;
+  const uint8_t* unit0 = p.w + static_cast<size_t>(row0) * row_bytes + static_cast<size_t>(col) * F::kBlock;
+  uint32_t issued = 0, fill = 0;
+  auto next_unit = [&]() {
+    // (past the last tile the last one again, so that outstanding loads are counted exactly; nobody reads it)
+    const uint32_t tl = issued < tiles ? issued : tiles - 1u;
+    const uint8_t* base = unit0 + static_cast<size_t>(tl * 16u) * row_bytes;
+    const uint32_t last = p.n - 1u - (row0 + tl * 16u);         // rows past the matrix: the last row, never stored
+    const uint32_t mis = kShifted ? static_cast<uint32_t>(reinterpret_cast<uintptr_t>(base)) & 15u : 0u;
+    base -= mis;
+    // A block's last piece may reach past the matrix's end, at its last block only: then the whole piece before is
+    // brought in its place, and the bytes are put right before they are read.
+    const int64_t room = kShifted ? reinterpret_cast<intptr_t>(p.w_end) / 16 * 16 - 16 - reinterpret_cast<intptr_t>(base) : 0;
+    const uint32_t end_off = room < 0xFFFFFFFFll ? static_cast<uint32_t>(room) : 0xFFFFFFFFu;
+    const uint32_t dst = ring_addr + fill * U::kBytes;
+#pragma unroll
+    for (int i = 0; i < U::kLoads; ++i) {
+      const uint32_t row_off = (piece_row[i] < last ? piece_row[i] : last) * row_bytes;
+      uint32_t off = row_off + piece_off[i];
+      if (kShifted) {
+        off = ((row_off + mis) & ~15u) + piece_off[i];
+        off = off < end_off ? off : end_off;
+      }
+      if (i + 1 < U::kLoads || 16u * U::kPieces % 64u == 0u || lane < 16u * U::kPieces % 64u) kq_direct16(base, off, dst + i * 1024u);
+    }
+    ++issued;
+    fill = fill + 1u == RING ? 0u : fill + 1u;
+  };
+#pragma unroll
+  for (int i = 0; i < RING; ++i) next_unit();
+
+  int4v_t A[NA][4];
+  typename F::Ctx ctx[NA];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    if (static_cast<uint32_t>(r) < p.m) convert_block(make_float4(xr[r][0], xr[r][1], xr[r][2], xr[r][3]), lane, slot);
+    F::fetch(A[r / F::kRowsPerSet], ctx[r / F::kRowsPerSet], slot, r, p.m, lane);
+  }
+
+  float* out = p.out + static_cast<size_t>(part) * p.m * p.ld;
+  const uint32_t quad_row = 2u * (g & 1u) + (g >> 1);
+  uint32_t read = 0;
+  for (uint32_t g0 = 0; g0 < tiles; g0 += p.tiles_per_sync) {
+    const uint32_t in_group = tiles - g0 < p.tiles_per_sync ? tiles - g0 : p.tiles_per_sync;
+    for (uint32_t ti = 0; ti < in_group; ++ti) {
+      // RING - 1 later units may still be under way (stores of the sums only make the wait longer)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 1) * U::kLoads) : "memory");
+      uint8_t* unit = ring + read * U::kBytes;
+      read = read + 1u == RING ? 0u : read + 1u;
+      uint32_t row = ln, shift = 0;
+      if (kShifted) {
+        const uint32_t last = p.n - 1u - (row0 + (g0 + ti) * 16u);
+        const uintptr_t start = reinterpret_cast<uintptr_t>(unit0) + static_cast<size_t>((g0 + ti) * 16u) * row_bytes;
+        row = ln < last ? ln : last;
+        shift = (static_cast<uint32_t>(start) + row * row_bytes) & 15u;
+        const uint32_t over = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p.w_end)) & 15u;
+        const uint8_t* block_end = reinterpret_cast<const uint8_t*>(start) + static_cast<size_t>(last < 15u ? last : 15u) * row_bytes + F::kBlock;
+        if (over != 0u && block_end == p.w_end) {     // the matrix's last block: its bytes past the last whole piece
+          if (lane < over / 2u) {
+            *reinterpret_cast<uint16_t*>(unit + last * U::kRow + (U::kPieces - 1u) * 16u + lane * 2u) =
+                reinterpret_cast<const uint16_t*>(p.w_end - over)[lane];
+          }
+          asm volatile("" ::: "memory");   // read below in this order (a wavefront's LDS accesses keep theirs)
+        }
+      }
+      typename F::Unit u;
+      F::read(u, unit + row * U::kRow + shift, g);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      next_unit();
+      float val[NA], res[kQuads];
+      F::template dot<NA>(u, A, ctx, val, lane);
+      kq_rows_of<F>(val, res);
+      float* dst = table + ((ti * cols + wave) * (4 * kQuads) + quad_row) * 16u + ln;
+#pragma unroll
+      for (int q = 0; q < kQuads; ++q) dst[q * 64] = res[q];
+    }
+    lds_barrier();
+    for (uint32_t o = threadIdx.x; o < in_group * kQuads * 64u; o += cols * 64u) {
+      const uint32_t nn = o & 15u, r = (o >> 4) % (4u * kQuads), ti = o / (64u * kQuads);
+      const uint32_t row = row0 + (g0 + ti) * 16u + nn;
+      if (r >= p.m || row >= p.n) continue;
+      float sum = 0.0f;
+      for (uint32_t wv = 0; wv < cols; ++wv) sum += table[((ti * cols + wv) * (4u * kQuads) + r) * 16u + nn];   // wavefront order
+      out[static_cast<size_t>(r) * p.ld + row] = sum;
+    }
+    if (g0 + p.tiles_per_sync < tiles) lds_barrier();      // the table is written again
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct load may outlive its workgroup
+}
+
+// The parts' sums of `cols` columns in part order: c[r][col] = sum over parts of part[.][r][col].
+__global__ __launch_bounds__(256) void kq_reduce_kernel(const float* __restrict__ part, float* __restrict__ c, uint32_t cols,
+                                                        uint32_t m, uint32_t parts, size_t ldc) {
+  const uint32_t col = blockIdx.x * 256u + threadIdx.x, r = blockIdx.y;
+  if (col >= cols) return;
+  const size_t region = static_cast<size_t>(m) * cols;
+  const float* src = part + static_cast<size_t>(r) * cols + col;
+  float sum = 0.0f;
+  for (uint32_t i = 0; i < parts; ++i) sum += src[i * region];
+  c[r * ldc + col] = sum;
+}
+
+// Most wavefronts of a streaming workgroup: three a SIMD while the operands of NA sets leave the registers for it.
+template <class F, int NA>
+constexpr int kq_stream_waves() { return NA <= 6 ? 12 : 8; }
+
 struct KqPlan {
   uint32_t waves, rows_per_wg, workgroups, lds;
 };
@@ -458,13 +655,122 @@ hipError_t kq_launch_rows(const float* a, const uint8_t* w, float* c, uint32_t m
   return hipSuccess;
 }
 
+constexpr uint32_t kKqRing = 3;
+
+template <class F, int NA>
+uint32_t kq_stream_lds(uint32_t waves, uint32_t tiles_per_sync) {
+  constexpr uint32_t quads = (NA * F::kRowsPerSet + 3) / 4;
+  return waves * (kKqRing * KqUnit<F>::kBytes + kSlot + tiles_per_sync * quads * 256u);
+}
+
+// K parts and tiles a workgroup.  The launch lasts as long as the SIMD with the most wavefronts works: each
+// converts its activations (`prologue`, in tiles' worth of work, and the first trip to memory), then does the
+// workgroup's tiles; every part more is a region more to write and add up.
+template <class F, int NA>
+void kq_stream_plan(uint32_t n, uint32_t nblk, uint32_t cus, uint32_t& parts, uint32_t& groups, uint32_t& per) {
+  constexpr uint32_t wmax = kq_stream_waves<F, NA>();
+  const uint32_t tiles = (n + 15u) / 16u, fewest = (nblk + wmax - 1u) / wmax;
+  uint32_t best = ~0u;
+  for (uint32_t q = fewest; q <= nblk && q <= fewest + 8u; ++q) {
+    const uint32_t cols = (nblk + q - 1u) / q, on_simd = (cols + 3u) / 4u;
+    uint32_t grp = cus / q;
+    grp = grp == 0u ? 1u : (grp > tiles ? tiles : grp);
+    const uint32_t t = (tiles + grp - 1u) / grp, rounds = (q * ((tiles + t - 1u) / t) + cus - 1u) / cus;
+    const uint32_t cost = (on_simd * (2u + NA + 2u * t) * rounds) * 4u + (q > 1u ? 24u + 2u * q : 0u);
+    if (cost < best) best = cost, parts = q, per = t, groups = (tiles + t - 1u) / t;
+  }
+}
+
+template <class F, int NA>
+hipError_t kq_stream(const float* a, const uint8_t* w, const uint8_t* w_end, float* c, float* ws, uint32_t m, uint32_t n, size_t ldc,
+                     uint32_t nblk, uint32_t parts, uint32_t groups, uint32_t per, hipStream_t stream) {
+  const uint32_t waves = (nblk + parts - 1u) / parts;
+  uint32_t sync = (kKqLdsLimit - kq_stream_lds<F, NA>(waves, 0)) / (kq_stream_lds<F, NA>(waves, 1) - kq_stream_lds<F, NA>(waves, 0));
+  sync = sync > per ? per : sync;
+  const uint32_t meets = (per + sync - 1u) / sync;
+  sync = (per + meets - 1u) / meets;
+  const KqStreamArgs args{w, w_end, a, parts > 1u ? ws : c, m, n, nblk, parts, groups, per, sync,
+                          parts > 1u ? n : static_cast<uint32_t>(ldc)};
+  hipLaunchKernelGGL((kquant_rows_stream_kernel<F, NA, kKqRing, kq_stream_waves<F, NA>()>), dim3(parts * groups), dim3(waves * 64u),
+                     (kq_stream_lds<F, NA>(waves, sync)), stream, args);
+  if (parts > 1u) {
+    hipLaunchKernelGGL(kq_reduce_kernel, dim3((n + 255u) / 256u, m), dim3(256), 0, stream, ws, c, n, m, parts, ldc);
+  }
+  return hipGetLastError();
+}
+
+// One pass of up to eight rows, over as many ranges of weight rows as the scratch for the parts' sums asks for.
+template <class F, int NA>
+hipError_t kq_stream_rows(const float* a, const uint8_t* w, float* c, float* ws, size_t ws_bytes, uint32_t m, uint32_t n, uint32_t nblk,
+                          hipStream_t stream) {
+  const size_t row_bytes = static_cast<size_t>(nblk) * F::kBlock;
+  const uint32_t cus = static_cast<uint32_t>(num_cus());
+  const uint8_t* w_end = w + row_bytes * n;
+  uint32_t parts = 1, groups = 1, per = 1;
+  kq_stream_plan<F, NA>(n, nblk, cus, parts, groups, per);
+  const uint32_t cap = static_cast<uint32_t>(ws_bytes / 4u / parts / m / 16u * 16u);
+  if (parts == 1u || n <= cap) return kq_stream<F, NA>(a, w, w_end, c, ws, m, n, n, nblk, parts, groups, per, stream);
+  if (cap == 0u) return hipErrorInvalidValue;
+  for (uint32_t n0 = 0; n0 < n; n0 += cap) {
+    const uint32_t nc = n - n0 < cap ? n - n0 : cap;
+    const uint32_t g = (nc + 16u * per - 1u) / (16u * per);
+    const hipError_t e = kq_stream<F, NA>(a, w + row_bytes * n0, w_end, c + n0, ws, m, nc, n, nblk, parts, g, per, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+template <class F>
+hipError_t kq_stream_all(const float* a, const uint8_t* w, float* c, void* ws, size_t ws_bytes, uint32_t m, uint32_t n, uint32_t k,
+                         hipStream_t stream) {
+  const uint32_t nblk = k / 256u, passes = (m + 7u) / 8u, per_pass = (m + passes - 1u) / passes;
+  for (uint32_t r0 = 0; r0 < m; r0 += per_pass) {
+    const uint32_t mr = m - r0 < per_pass ? m - r0 : per_pass, sets = (mr + F::kRowsPerSet - 1u) / F::kRowsPerSet;
+    const float* ar = a + static_cast<size_t>(r0) * k;
+    float *cr = c + static_cast<size_t>(r0) * n, *part = static_cast<float*>(ws);
+    hipError_t e = hipErrorInvalidValue;
+    auto with = [&](auto na) {
+      if (sets <= na.value && e == hipErrorInvalidValue) e = kq_stream_rows<F, na.value>(ar, w, cr, part, ws_bytes, mr, n, nblk, stream);
+    };
+    with(std::integral_constant<int, 1>{}), with(std::integral_constant<int, 2>{});
+    with(std::integral_constant<int, 3>{}), with(std::integral_constant<int, 4>{});
+    if constexpr (F::kRowsPerSet == 1) {
+      with(std::integral_constant<int, 5>{}), with(std::integral_constant<int, 6>{}), with(std::integral_constant<int, 8>{});
+    }
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+template <class F, int NA>
+hipError_t kq_stream_prepare() {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(kquant_rows_stream_kernel<F, NA, kKqRing, kq_stream_waves<F, NA>()>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kKqLdsLimit));
+}
+
+template <class F>
+hipError_t kq_stream_prepare_format() {
+  hipError_t e;
+  if ((e = kq_stream_prepare<F, 1>()) != hipSuccess) return e;
+  if ((e = kq_stream_prepare<F, 2>()) != hipSuccess) return e;
+  if ((e = kq_stream_prepare<F, 3>()) != hipSuccess) return e;
+  if ((e = kq_stream_prepare<F, 4>()) != hipSuccess) return e;
+  if constexpr (F::kRowsPerSet == 1) {
+    if ((e = kq_stream_prepare<F, 5>()) != hipSuccess) return e;
+    if ((e = kq_stream_prepare<F, 6>()) != hipSuccess) return e;
+    if ((e = kq_stream_prepare<F, 8>()) != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 template <class F>
 hipError_t kq_prepare_format() {
   hipError_t e;
   if ((e = kq_prepare_one<F, 1>()) != hipSuccess) return e;
   if ((e = kq_prepare_one<F, 2>()) != hipSuccess) return e;
   if ((e = kq_prepare_one<F, 3>()) != hipSuccess) return e;
-  return kq_prepare_one<F, 4>();
+  if ((e = kq_prepare_one<F, 4>()) != hipSuccess) return e;
+  return hipSuccess;
 }
 
 }  // namespace
@@ -473,7 +779,15 @@ hipError_t gemv_kquant_rows_prepare() {
   hipError_t e;
   if ((e = kq_prepare_format<Sub32Format<false>>()) != hipSuccess) return e;
   if ((e = kq_prepare_format<Sub32Format<true>>()) != hipSuccess) return e;
-  return kq_prepare_format<Q6KFormat>();
+  if ((e = kq_prepare_format<Q6KFormat>()) != hipSuccess) return e;
+  if ((e = kq_stream_prepare_format<Sub32Format<true>>()) != hipSuccess) return e;
+  return kq_stream_prepare_format<Q6KFormat>();
+}
+
+hipError_t launch_kquant_rows_stream(uint32_t bits, const float* a, const uint8_t* w, float* c, void* ws, size_t ws_bytes, uint32_t m,
+                                     uint32_t n, uint32_t k, hipStream_t stream) {
+  if (bits == 5u) return kq_stream_all<Sub32Format<true>>(a, w, c, ws, ws_bytes, m, n, k, stream);
+  return bits == 6u ? kq_stream_all<Q6KFormat>(a, w, c, ws, ws_bytes, m, n, k, stream) : hipErrorInvalidValue;
 }
 
 bool gemv_kquant_rows_supported(uint64_t m, uint64_t n, uint64_t k) {

@@ -717,6 +717,23 @@ qmm_status kquant_prefill(const LaunchCtx& c, uint32_t block_bytes, uint64_t m, 
   return st;
 }
 
+constexpr uint64_t kKquantStreamMaxK = uint64_t{1} << 17;   // 64 K parts: the scratch holds 8192 weight rows' sums
+// Up to 16 rows of Q5_K or Q6_K (`bits`) on the streaming form of the int8 kernel, which leaves partial sums of its
+// K parts in the decode scratch.  Against the form that has all of K in a workgroup it converts a block's
+// activations once instead of once a workgroup and takes up to eight rows of Q6_K a pass instead of four, but
+// pays a reduce launch: Q6_K 5120 x 17408, 5 rows 79 -> 33 us, 3 rows 40 -> 29; 6144 x 5120, 5 rows 28 -> 20, but
+// 3 rows 14.5 -> 16; 513 x 1280, 5 rows 10 -> 9.  Q5_K, which had eight rows a pass: 5120 x 17408, 8 rows 57 -> 27,
+// 2 rows 21 -> 18.5; 1024 x 5120, 8 rows 15 -> 11; 2047 x 2048, 8 rows 8.4 -> 10 (the other form stays).
+qmm_status kquant_rows_stream(const LaunchCtx& c, uint32_t bits, float* out, uint64_t m, uint64_t n, uint64_t k) {
+  void* ws = decode_scratch(c);
+  if (ws == nullptr) {
+    g_last_error = "Q5_K / Q6_K: decode scratch missing";
+    return QMM_DEVICE_ERROR;
+  }
+  return map_hip(qmm::launch_kquant_rows_stream(bits, c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, ws, kDecodeScratchBytes,
+                                                static_cast<uint32_t>(m), static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
+}
+
 // ---- Q5_K ---------------------------------------------------------------------
 // "gemm_q5k", "gemm_q5k_batched", "gemm_q5k_vec", "gemm_q5k_rows{R}": as the Q6_K ids below, with
 // 176-byte blocks (include/tessera/backend.hpp:202-206,524-536; rocm_backend.cpp:95-101).
@@ -736,8 +753,10 @@ qmm_status q5k_matmul(const LaunchCtx& c, uint64_t m, uint64_t n, uint64_t k, ui
   // (17408 x 5120: 2 rows 17.6 us against 30.3 on a multiply-add pass per row, 8 rows 31 against 121).
   const bool one_pass = m >= 2 && qmm::gemv_kquant_rows_supported(m, n, k);
   const auto launch = one_pass ? qmm::launch_q5k_rows_i8 : qmm::launch_q5k_gemv;
-  qmm_status st = map_hip(launch(c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, static_cast<uint32_t>(m),
-                                 static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
+  qmm_status st = m >= 2 && m <= 16 && k <= kKquantStreamMaxK && (k > 8192 || (m >= 5 && k >= 4096)) && qmm::gemv_kquant_rows_supported(m, n, k)
+                      ? kquant_rows_stream(c, 5, out, m, n, k)
+                      : map_hip(launch(c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, static_cast<uint32_t>(m),
+                                       static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
   if (st == QMM_OK && split > 1) st = map_hip(qmm::launch_fill_f32(out + m * n, 0.0f, (split - 1) * m * n, c.stream));
   return st;
 }
@@ -790,8 +809,10 @@ qmm_status q6k_matmul(const LaunchCtx& c, uint64_t m, uint64_t n, uint64_t k, ui
   // two rows stay on the multiply-add pass, 26 against 29 us).
   const bool one_pass = m >= 3 && qmm::gemv_kquant_rows_supported(m, n, k);
   const auto launch = one_pass ? qmm::launch_q6k_rows_i8 : qmm::launch_q6k_gemv;
-  qmm_status st = map_hip(launch(c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, static_cast<uint32_t>(m),
-                                 static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
+  qmm_status st = m >= 2 && m <= 16 && k <= kKquantStreamMaxK && (k > 8192 || m >= 5) && qmm::gemv_kquant_rows_supported(m, n, k)
+                      ? kquant_rows_stream(c, 6, out, m, n, k)
+                      : map_hip(launch(c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, static_cast<uint32_t>(m),
+                                       static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
   if (st == QMM_OK && split > 1) st = map_hip(qmm::launch_fill_f32(out + m * n, 0.0f, (split - 1) * m * n, c.stream));
   return st;
 }

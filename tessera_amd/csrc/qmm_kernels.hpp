@@ -176,6 +176,10 @@ hipError_t moe_q4k_prepare();           // once per device, from qmm_init (moe_q
 // Q4_K / Q5_K / Q6_K x a few fp32 rows in one pass over the weights on the int8 matrix cores
 // (gemv_kquant_rows.hip); any m, taken some rows a pass (eight, eight, four).
 hipError_t gemv_kquant_rows_prepare();   // once per device, from qmm_init
+// Q5_K, Q6_K (`bits` = 5, 6): weights streamed through LDS, K cut into parts whose sums go to `ws` (any size that holds
+// 16 weight rows' sums), up to eight rows a pass.
+hipError_t launch_kquant_rows_stream(uint32_t bits, const float* a, const uint8_t* w, float* c, void* ws, size_t ws_bytes, uint32_t m,
+                                     uint32_t n, uint32_t k, hipStream_t stream);
 bool gemv_kquant_rows_supported(uint64_t m, uint64_t n, uint64_t k);
 hipError_t launch_q4k_rows_i8(const float* a, const uint8_t* w, float* c, uint32_t m, uint32_t n, uint32_t k,
                               hipStream_t stream);

@@ -195,3 +195,36 @@ def test_q4k_non_finite_values_stay_in_their_row(backend):
     assert not np.isfinite(got[1]).any()
     assert not np.isfinite(got[:, bad_rows]).any()
     assert rel_err(got[[0, 2]][:, good], ref[:, good]) <= TOL
+
+
+@pytest.mark.parametrize("fmt", ["q5k", "q6k"])
+@pytest.mark.parametrize("m,n,k", [(5, 1, 4096), (6, 17, 8448), (8, 129, 4352), (10, 2051, 5120), (12, 47, 12544), (3, 333, 12800),
+                                   (2, 16, 131072), (15, 30, 9984)])
+def test_streamed_rows_match_oracle(backend, fmt, m, n, k):
+    """The streaming form: K parts with one to twelve block columns, a last tile of one row, matrices that end
+    inside a 16-byte piece (n * k / 256 no multiple of eight), passes of unequal rows, and nothing past C."""
+    make, ref_fn, _, _ = FORMATS[fmt]
+    g = synth.rng(7800 + 13 * m + n + k)
+    w, a = make(g, n, k), synth.activations_f32(g, m, k)
+    da, dw, dc = backend.Upload(a), backend.Upload(w), backend.Upload(np.full(m * n + 32, 3.0, np.float32))
+    run(backend, f"gemm_{fmt}", [da, dw, dc], [m, n, k], grid=ref_grid_vec(m, n))
+    backend.Synchronize()
+    out = backend.CopyD2H(dc, dtype=np.float32)
+    ref = ref_fn(a, w, m, n, k, threads=True)
+    assert np.all(out[m * n:] == 3.0)
+    got = out[:m * n].reshape(m, n)
+    assert rel_err(got, ref) <= TOL, (fmt, m, n, k, rel_err(got, ref))
+    assert rms_err(got, ref) < 5e-5, (fmt, m, n, k, rms_err(got, ref))
+
+
+def test_streamed_rows_in_ranges_of_weight_rows(backend):
+    """More partial sums than the scratch holds: the weight rows are taken a range at a time.  41 distinct rows,
+    repeated, so that every range begins at another one of them."""
+    m, n, k, distinct = 8, 8209, 131072, 41
+    g = synth.rng(7900)
+    rows = synth.q6k_weights(g, distinct, k).reshape(distinct, -1)
+    w = rows[np.arange(n) % distinct].reshape(-1)
+    a = synth.activations_f32(g, m, k)
+    ref = oracle.gemm_q6k(a, rows.reshape(-1), m, distinct, k, threads=True)
+    got = gemm(backend, "gemm_q6k", a, w, m, n, k)
+    assert rms_err(got, ref[:, np.arange(n) % distinct]) < 2e-4
