@@ -17,7 +17,7 @@
  *     tessera::StatusCode (include/tessera/types.hpp:36-48);
  *   - no exceptions cross the boundary;
  *   - device memory: qmm_alloc allocates what the caller asks for; qmm_init allocates the 16 MB
- *     scratch of the decode-sized kernels once; prefill-sized launches (Q4_K/Q5_K/Q6_K from 17
+ *     scratch of the decode-sized kernels once and reserves 256 MB for the blocks below; prefill-sized launches (Q4_K/Q5_K/Q6_K from 17
  *     rows, the grouped routed-expert ids) need a workspace, which is the caller's when one was
  *     set with qmm_set_workspace and otherwise a library-owned block that qmm_launch grows on
  *     demand with hipMalloc.  A block that a launch has used is never freed (growth allocates a
@@ -25,6 +25,16 @@
  *     recorded into a HIP graph keeps a valid pointer); growth while `stream` is being captured
  *     returns InvalidArgument with a message: grow before capturing, or set a workspace.
  *     qmm_launch_static never allocates.
+ *   - streams: launches that use the decode scratch or the workspace share it, so the caller orders
+ *     them (one stream, or events).  Every other launch is independent of launches on other streams;
+ *     "gemm_fp8" from 17 rows and "gemm_q5k*" / "gemm_q6k*" with 2..16 rows, which also hand
+ *     intermediate results from one kernel to the next, keep them in blocks of their own: 32 MB for
+ *     the eager launches of each stream, and what they need for each capture and stream that records
+ *     them.  Blocks come out of the 256 MB that qmm_init reserves, then out of slabs of 128 MB, 2 GB in
+ *     all; while a caller's workspace is set no slab is allocated.  They are not given back (a graph may
+ *     still use them), and a stream handle's block passes to the next stream with that handle: let a
+ *     stream's launches finish before it is destroyed.  A launch that gets no block, or is made on
+ *     hipStreamPerThread, runs kernels that need none (slower; sums in another order).
  */
 #ifndef TESSERA_QMM_H_
 #define TESSERA_QMM_H_
@@ -180,8 +190,7 @@ size_t qmm_static_scratch_bytes(void);
  * (256-byte aligned) to use for every later qmm_launch on any stream, in stream order, until it
  * is replaced or cleared with (NULL, 0); while one is set, qmm_launch allocates nothing and a
  * launch that needs more returns InvalidArgument.  The caller must not free or replace the
- * block while launches that use it are in flight.  ("gemm_fp8" is the exception to the refusal: with less
- * than it asks for it runs its slower passes that need none.) */
+ * block while launches that use it are in flight. */
 qmm_status qmm_workspace_bytes(qmm_kernel kernel, const uint64_t* scalars, size_t nscalars, size_t* out_bytes);
 qmm_status qmm_set_workspace(void* device_ptr, size_t bytes);
 

@@ -285,8 +285,9 @@ struct Fp8Plan {
 // another (two on a CU take as long as one after the other: 0.36 us a 64-wide step of 32 rows, 0.58 of 64, measured
 // with 1 to 4 a CU), then the launch that adds the parts and the traffic of their sums.
 // 17 x 6144 x 5120: one part 33, five 16 us; 300 x 512 x 5120: 54 and, with eight, 21 us.  A part keeps at least
-// four steps.  (Tiles of 128 rows were no faster up to 1024 rows and leave no registers for the sums.)
-Fp8Plan fp8_plan(uint32_t m, uint32_t n, uint32_t k) {
+// four steps, and the parts' sums fit `room` bytes.  (Tiles of 128 rows were no faster up to 1024 rows and leave no
+// registers for the sums.)
+Fp8Plan fp8_plan(uint32_t m, uint32_t n, uint32_t k, size_t room, float* estimate) {
   const uint32_t cus = static_cast<uint32_t>(num_cus()), steps = k / kStepK, tiles_n = (n + kBN - 1u) / kBN;
   Fp8Plan best{64u, 1u, steps};
   float best_us = 1e30f;
@@ -295,12 +296,14 @@ Fp8Plan fp8_plan(uint32_t m, uint32_t n, uint32_t k) {
     const float step_us = bm == 32u ? 0.36f : 0.58f;
     for (uint32_t parts = 1; parts == 1u || (parts <= 16u && steps / parts >= 4u); ++parts) {
       const uint32_t spp = (steps + parts - 1u) / parts, real = (steps + spp - 1u) / spp;
+      if (real > 1u && static_cast<size_t>(real) * m * n * 4 > room) break;
       const uint64_t rounds = (tiles * real + cus - 1u) / cus;
       float us = static_cast<float>(rounds) * static_cast<float>(spp) * step_us;
       if (real > 1u) us += 3.5f + static_cast<float>(real) * static_cast<float>(m) * static_cast<float>(n) * 1.6e-6f;
       if (us < best_us) best_us = us, best = Fp8Plan{bm, real, spp};
     }
   }
+  *estimate = best_us;
   return best;
 }
 
@@ -308,24 +311,37 @@ size_t terms_bytes(uint64_t m, uint64_t k) {
   return static_cast<size_t>(m) * k * 4 + ((static_cast<size_t>(m) * 4 + 255) & ~size_t{255});
 }
 
-}  // namespace
-
-bool gemm_fp8_f16_supported(uint64_t m, uint64_t n, uint64_t k) {
-  return m >= 17 && k % 64 == 0 && k <= (1u << 20) && n <= (1u << 30) && m <= 65535u && m * n < (1ull << 40);
+// Rows of one go: all where their terms fit the scratch, else the multiple of 64 (fewer where not even 64 fit)
+// with the smallest sum of estimates.  2048 x 6144 x 5120, whose terms take 42 MB, goes as two times 1024 rows,
+// as many rounds of tiles as in one go.
+constexpr size_t kScratch = gemm_fp8_f16_scratch_limit;
+uint32_t fp8_rows(uint32_t m, uint32_t n, uint32_t k) {
+  if (terms_bytes(m, k) <= kScratch) return m;
+  uint32_t most = static_cast<uint32_t>((kScratch - 256) / (static_cast<size_t>(k) * 4 + 4));
+  if (most < 64u) return most;
+  most = most / 64u * 64u;
+  uint32_t best = most;
+  float best_us = 1e30f;
+  for (uint32_t rows = most; rows >= 64u && rows * 2u >= most; rows -= 64u) {
+    float each = 0.0f, last = 0.0f;
+    fp8_plan(rows, n, k, kScratch - terms_bytes(rows, k), &each);
+    const uint32_t left = m % rows;
+    if (left != 0u) fp8_plan(left, n, k, kScratch - terms_bytes(left, k), &last);
+    const float us = static_cast<float>(m / rows) * each + last;
+    if (us < best_us) best_us = us, best = rows;
+  }
+  return best;
 }
 
-size_t gemm_fp8_f16_workspace_bytes(uint64_t m, uint64_t n, uint64_t k) {
-  const Fp8Plan pl = fp8_plan(static_cast<uint32_t>(m), static_cast<uint32_t>(n), static_cast<uint32_t>(k));
-  return terms_bytes(m, k) + (pl.parts > 1 ? static_cast<size_t>(pl.parts) * m * n * 4 : 0);
-}
-
-hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* workspace, uint32_t m,
-                               uint32_t n, uint32_t k, hipStream_t stream) {
-  const Fp8Plan pl = fp8_plan(m, n, k);
-  _Float16* a16 = static_cast<_Float16*>(workspace);
+// One go of m rows (their terms fit the scratch): the terms, the product, the parts' sums.
+hipError_t launch_rows(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch, uint32_t m, uint32_t n,
+                       uint32_t k, hipStream_t stream) {
+  float us;
+  const Fp8Plan pl = fp8_plan(m, n, k, kScratch - terms_bytes(m, k), &us);
+  _Float16* a16 = static_cast<_Float16*>(scratch);
   const size_t plane = static_cast<size_t>(m) * k;
   float* a_scale = reinterpret_cast<float*>(a16 + 2 * plane);
-  float* part = pl.parts > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + terms_bytes(m, k)) : nullptr;
+  float* part = pl.parts > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(scratch) + terms_bytes(m, k)) : nullptr;
   if (k <= 2048u) hipLaunchKernelGGL(rows_to_f16_terms_kernel<2>, dim3(m), dim3(256), 0, stream, a, a16, a_scale, k, plane);
   else if (k <= 8192u) hipLaunchKernelGGL(rows_to_f16_terms_kernel<8>, dim3(m), dim3(256), 0, stream, a, a16, a_scale, k, plane);
   else hipLaunchKernelGGL(rows_to_f16_terms_kernel<0>, dim3(m), dim3(256), 0, stream, a, a16, a_scale, k, plane);
@@ -348,6 +364,36 @@ hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_
     }
   }
   return hipGetLastError();
+}
+
+}  // namespace
+
+bool gemm_fp8_f16_supported(uint64_t m, uint64_t n, uint64_t k) {
+  return m >= 17 && k % 64 == 0 && k <= (1u << 20) && n <= (1u << 30) && m <= 65535u && m * n < (1ull << 40);
+}
+
+size_t gemm_fp8_f16_scratch_bytes(uint64_t m, uint64_t n, uint64_t k) {
+  const uint32_t rows = fp8_rows(static_cast<uint32_t>(m), static_cast<uint32_t>(n), static_cast<uint32_t>(k));
+  size_t most = 0;
+  for (const uint32_t part : {rows, static_cast<uint32_t>(m % rows)}) {
+    if (part == 0u) continue;
+    float us;
+    const Fp8Plan pl = fp8_plan(part, static_cast<uint32_t>(n), static_cast<uint32_t>(k), kScratch - terms_bytes(part, k), &us);
+    const size_t bytes = terms_bytes(part, k) + (pl.parts > 1 ? static_cast<size_t>(pl.parts) * part * n * 4 : 0);
+    most = bytes > most ? bytes : most;
+  }
+  return most;
+}
+
+hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch, uint32_t m,
+                               uint32_t n, uint32_t k, hipStream_t stream) {
+  const uint32_t rows = fp8_rows(m, n, k);
+  for (uint32_t r = 0; r < m; r += rows) {
+    const hipError_t e = launch_rows(a + static_cast<size_t>(r) * k, w, w_scale, c + static_cast<size_t>(r) * n, scratch,
+                                     m - r < rows ? m - r : rows, n, k, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace qmm

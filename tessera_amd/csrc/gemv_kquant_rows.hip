@@ -720,26 +720,57 @@ hipError_t kq_stream_rows(const float* a, const uint8_t* w, float* c, float* ws,
   return hipSuccess;
 }
 
+// `go` with the number of operand sets of the kernel that takes `rows` rows (at most eight).
+template <class F, class Go>
+void kq_stream_with_sets(uint32_t rows, Go&& go) {
+  const uint32_t sets = (rows + F::kRowsPerSet - 1u) / F::kRowsPerSet;
+  bool done = false;
+  auto with = [&](auto na) {
+    if (!done && sets <= na.value) done = true, go(na);
+  };
+  with(std::integral_constant<int, 1>{}), with(std::integral_constant<int, 2>{});
+  with(std::integral_constant<int, 3>{}), with(std::integral_constant<int, 4>{});
+  if constexpr (F::kRowsPerSet == 1) {
+    with(std::integral_constant<int, 5>{}), with(std::integral_constant<int, 6>{}), with(std::integral_constant<int, 8>{});
+  }
+}
+
+uint32_t kq_stream_rows_per_pass(uint32_t m) {
+  const uint32_t passes = (m + 7u) / 8u;
+  return (m + passes - 1u) / passes;
+}
+
 template <class F>
 hipError_t kq_stream_all(const float* a, const uint8_t* w, float* c, void* ws, size_t ws_bytes, uint32_t m, uint32_t n, uint32_t k,
                          hipStream_t stream) {
-  const uint32_t nblk = k / 256u, passes = (m + 7u) / 8u, per_pass = (m + passes - 1u) / passes;
+  const uint32_t nblk = k / 256u, per_pass = kq_stream_rows_per_pass(m);
   for (uint32_t r0 = 0; r0 < m; r0 += per_pass) {
-    const uint32_t mr = m - r0 < per_pass ? m - r0 : per_pass, sets = (mr + F::kRowsPerSet - 1u) / F::kRowsPerSet;
-    const float* ar = a + static_cast<size_t>(r0) * k;
-    float *cr = c + static_cast<size_t>(r0) * n, *part = static_cast<float*>(ws);
+    const uint32_t mr = m - r0 < per_pass ? m - r0 : per_pass;
     hipError_t e = hipErrorInvalidValue;
-    auto with = [&](auto na) {
-      if (sets <= na.value && e == hipErrorInvalidValue) e = kq_stream_rows<F, na.value>(ar, w, cr, part, ws_bytes, mr, n, nblk, stream);
-    };
-    with(std::integral_constant<int, 1>{}), with(std::integral_constant<int, 2>{});
-    with(std::integral_constant<int, 3>{}), with(std::integral_constant<int, 4>{});
-    if constexpr (F::kRowsPerSet == 1) {
-      with(std::integral_constant<int, 5>{}), with(std::integral_constant<int, 6>{}), with(std::integral_constant<int, 8>{});
-    }
+    kq_stream_with_sets<F>(mr, [&](auto na) {
+      e = kq_stream_rows<F, na.value>(a + static_cast<size_t>(r0) * k, w, c + static_cast<size_t>(r0) * n, static_cast<float*>(ws),
+                                      ws_bytes, mr, n, nblk, stream);
+    });
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+// The passes' rows differ by one at most, but another number of sets may mean another number of parts.
+template <class F>
+size_t kq_stream_scratch(size_t ws_bytes, uint32_t m, uint32_t n, uint32_t k) {
+  const uint32_t per_pass = kq_stream_rows_per_pass(m);
+  size_t most = 0;
+  for (const uint32_t rows : {per_pass, m % per_pass}) {
+    if (rows == 0u) continue;
+    kq_stream_with_sets<F>(rows, [&](auto na) {
+      uint32_t parts = 1, groups = 1, per = 1;
+      kq_stream_plan<F, na.value>(n, k / 256u, static_cast<uint32_t>(num_cus()), parts, groups, per);
+      const size_t bytes = parts > 1u ? static_cast<size_t>(parts) * rows * n * 4 : 0;
+      most = bytes > most ? bytes : most;
+    });
+  }
+  return most < ws_bytes ? most : ws_bytes;
 }
 
 template <class F, int NA>
@@ -788,6 +819,10 @@ hipError_t launch_kquant_rows_stream(uint32_t bits, const float* a, const uint8_
                                      uint32_t n, uint32_t k, hipStream_t stream) {
   if (bits == 5u) return kq_stream_all<Sub32Format<true>>(a, w, c, ws, ws_bytes, m, n, k, stream);
   return bits == 6u ? kq_stream_all<Q6KFormat>(a, w, c, ws, ws_bytes, m, n, k, stream) : hipErrorInvalidValue;
+}
+
+size_t kquant_rows_stream_scratch(uint32_t bits, size_t ws_bytes, uint32_t m, uint32_t n, uint32_t k) {
+  return bits == 5u ? kq_stream_scratch<Sub32Format<true>>(ws_bytes, m, n, k) : kq_stream_scratch<Q6KFormat>(ws_bytes, m, n, k);
 }
 
 bool gemv_kquant_rows_supported(uint64_t m, uint64_t n, uint64_t k) {

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "qmm_kernels.hpp"
+#include "stream_scratch.hpp"
 
 namespace {
 
@@ -154,6 +155,65 @@ void* decode_scratch(const LaunchCtx& c) {
   static_assert(kDecodeScratchBytes <= kStaticScratchBytes, "the static scratch holds the decode scratch");
   return c.no_alloc ? g_static_scratch[g_device] : g_decode_scratch;
 }
+
+// Scratch of "gemm_fp8" and of Q5_K / Q6_K with a few rows, whose calls on different streams are independent of
+// one another: see stream_scratch.hpp.  qmm_init reserves the first slab; later ones are allocated under the
+// relaxed capture mode, which permits it while a stream is captured, unless the caller has handed over a workspace
+// (then a launch allocates nothing).
+qmm::StreamScratch g_stream_scratch;
+
+class StreamBlock {
+ public:
+  StreamBlock(const LaunchCtx& c, size_t bytes) {
+    if (c.no_alloc) {
+      ptr_ = bytes <= kStaticScratchBytes ? g_static_scratch[g_device] : nullptr;
+      return;
+    }
+    if (bytes == 0 || c.stream == hipStreamPerThread) return;   // (the latter: one handle, another stream in each thread)
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(c.stream, &status, &id) != hipSuccess) {
+      (void)hipGetLastError();                    // the null stream beside another stream's capture
+      status = hipStreamCaptureStatusNone;
+    }
+    if (status == hipStreamCaptureStatusInvalidated) return;
+    block_ = g_stream_scratch.find(status == hipStreamCaptureStatusActive ? id + 1 : 0, c.stream, bytes, grow);
+    if (block_ == nullptr) return;
+    block_->busy.lock();
+    ptr_ = block_->ptr;
+  }
+  ~StreamBlock() {
+    if (block_ != nullptr) block_->busy.unlock();
+  }
+  StreamBlock(const StreamBlock&) = delete;
+  StreamBlock& operator=(const StreamBlock&) = delete;
+  void* get() const { return ptr_; }
+
+  static void* grow(size_t bytes) {
+    {
+      std::lock_guard<std::mutex> lock(g_workspace_mutex);
+      if (g_user_workspace != nullptr) return nullptr;
+    }
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    void* fresh = nullptr;
+    if (hipMalloc(&fresh, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      fresh = nullptr;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return fresh;
+  }
+
+ private:
+  qmm::ScratchBlock* block_ = nullptr;
+  void* ptr_ = nullptr;
+};
+static_assert(qmm::gemm_fp8_f16_scratch_limit <= qmm::StreamScratch::kBlockBytes &&
+              qmm::gemm_fp8_f16_scratch_limit <= kStaticScratchBytes && kDecodeScratchBytes <= qmm::StreamScratch::kBlockBytes);
 
 // Q4_K regimes by activation rows.  One row and small matrices: the VALU GEMV.  2..16 rows of a
 // matrix with at least kQ4KFewRowsMinWeights weights: the exact few-row MFMA kernels (weights read
@@ -719,19 +779,20 @@ qmm_status kquant_prefill(const LaunchCtx& c, uint32_t block_bytes, uint64_t m, 
 
 constexpr uint64_t kKquantStreamMaxK = uint64_t{1} << 17;   // 64 K parts: the scratch holds 8192 weight rows' sums
 // Up to 16 rows of Q5_K or Q6_K (`bits`) on the streaming form of the int8 kernel, which leaves partial sums of its
-// K parts in the decode scratch.  Against the form that has all of K in a workgroup it converts a block's
+// K parts in the stream's scratch block.  Against the form that has all of K in a workgroup it converts a block's
 // activations once instead of once a workgroup and takes up to eight rows of Q6_K a pass instead of four, but
 // pays a reduce launch: Q6_K 5120 x 17408, 5 rows 79 -> 33 us, 3 rows 40 -> 29; 6144 x 5120, 5 rows 28 -> 20, but
 // 3 rows 14.5 -> 16; 513 x 1280, 5 rows 10 -> 9.  Q5_K, which had eight rows a pass: 5120 x 17408, 8 rows 57 -> 27,
 // 2 rows 21 -> 18.5; 1024 x 5120, 8 rows 15 -> 11; 2047 x 2048, 8 rows 8.4 -> 10 (the other form stays).
-qmm_status kquant_rows_stream(const LaunchCtx& c, uint32_t bits, float* out, uint64_t m, uint64_t n, uint64_t k) {
-  void* ws = decode_scratch(c);
-  if (ws == nullptr) {
-    g_last_error = "Q5_K / Q6_K: decode scratch missing";
-    return QMM_DEVICE_ERROR;
-  }
-  return map_hip(qmm::launch_kquant_rows_stream(bits, c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, ws, kDecodeScratchBytes,
-                                                static_cast<uint32_t>(m), static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
+// A stream without a block takes the other form, which needs no scratch: false, and nothing is launched.
+bool kquant_rows_stream(const LaunchCtx& c, uint32_t bits, float* out, uint64_t m, uint64_t n, uint64_t k, qmm_status* st) {
+  const uint32_t m32 = static_cast<uint32_t>(m), n32 = static_cast<uint32_t>(n), k32 = static_cast<uint32_t>(k);
+  const size_t need = qmm::kquant_rows_stream_scratch(bits, kDecodeScratchBytes, m32, n32, k32);   // 0: K in one part
+  const StreamBlock block(c, need);
+  if (need != 0 && block.get() == nullptr) return false;
+  *st = map_hip(qmm::launch_kquant_rows_stream(bits, c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, block.get(),
+                                               kDecodeScratchBytes, m32, n32, k32, c.stream));
+  return true;
 }
 
 // ---- Q5_K ---------------------------------------------------------------------
@@ -753,10 +814,13 @@ qmm_status q5k_matmul(const LaunchCtx& c, uint64_t m, uint64_t n, uint64_t k, ui
   // (17408 x 5120: 2 rows 17.6 us against 30.3 on a multiply-add pass per row, 8 rows 31 against 121).
   const bool one_pass = m >= 2 && qmm::gemv_kquant_rows_supported(m, n, k);
   const auto launch = one_pass ? qmm::launch_q5k_rows_i8 : qmm::launch_q5k_gemv;
-  qmm_status st = m >= 2 && m <= 16 && k <= kKquantStreamMaxK && (k > 8192 || (m >= 5 && k >= 4096)) && qmm::gemv_kquant_rows_supported(m, n, k)
-                      ? kquant_rows_stream(c, 5, out, m, n, k)
-                      : map_hip(launch(c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, static_cast<uint32_t>(m),
-                                       static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
+  const bool stream = m >= 2 && m <= 16 && k <= kKquantStreamMaxK && (k > 8192 || (m >= 5 && k >= 4096)) &&
+                      qmm::gemv_kquant_rows_supported(m, n, k);
+  qmm_status st = QMM_OK;
+  if (!stream || !kquant_rows_stream(c, 5, out, m, n, k, &st)) {
+    st = map_hip(launch(c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
+                        static_cast<uint32_t>(k), c.stream));
+  }
   if (st == QMM_OK && split > 1) st = map_hip(qmm::launch_fill_f32(out + m * n, 0.0f, (split - 1) * m * n, c.stream));
   return st;
 }
@@ -809,10 +873,12 @@ qmm_status q6k_matmul(const LaunchCtx& c, uint64_t m, uint64_t n, uint64_t k, ui
   // two rows stay on the multiply-add pass, 26 against 29 us).
   const bool one_pass = m >= 3 && qmm::gemv_kquant_rows_supported(m, n, k);
   const auto launch = one_pass ? qmm::launch_q6k_rows_i8 : qmm::launch_q6k_gemv;
-  qmm_status st = m >= 2 && m <= 16 && k <= kKquantStreamMaxK && (k > 8192 || m >= 5) && qmm::gemv_kquant_rows_supported(m, n, k)
-                      ? kquant_rows_stream(c, 6, out, m, n, k)
-                      : map_hip(launch(c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, static_cast<uint32_t>(m),
-                                       static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
+  const bool stream = m >= 2 && m <= 16 && k <= kKquantStreamMaxK && (k > 8192 || m >= 5) && qmm::gemv_kquant_rows_supported(m, n, k);
+  qmm_status st = QMM_OK;
+  if (!stream || !kquant_rows_stream(c, 6, out, m, n, k, &st)) {
+    st = map_hip(launch(c.ptr<const float>(0), c.ptr<const uint8_t>(1), out, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
+                        static_cast<uint32_t>(k), c.stream));
+  }
   if (st == QMM_OK && split > 1) st = map_hip(qmm::launch_fill_f32(out + m * n, 0.0f, (split - 1) * m * n, c.stream));
   return st;
 }
@@ -1047,18 +1113,16 @@ qmm_status run_gemm_fp8(const LaunchCtx& c) {
                                             c.ptr<float>(3), decode_scratch(c), static_cast<uint32_t>(m),
                                             static_cast<uint32_t>(n), static_cast<uint32_t>(k), false, c.stream));
   }
-  // More rows: the weights as fp16 on the matrix cores against two fp16 terms of each row (gemm_fp8.hip).  Where
-  // the scratch for the terms cannot be had (a workspace of the caller's that is too small, growth while the
-  // stream is captured) the multiply-add passes below need none.
+  // More rows: the weights as fp16 on the matrix cores against two fp16 terms of each row (gemm_fp8.hip), in the
+  // stream's own scratch block, as many rows at a time as fit it: the same kernels and bits whatever ran before,
+  // whatever workspace is set and under capture.  A stream without a block runs the multiply-add passes below.
   if (m >= kFp8GemmMinRows && qmm::gemm_fp8_f16_supported(m, n, k)) {
-    const size_t bytes = qmm::gemm_fp8_f16_workspace_bytes(m, n, k);
-    void* ws = bytes <= kDecodeScratchBytes ? decode_scratch(c) : nullptr;
-    if (ws != nullptr || workspace(c, bytes, &ws) == QMM_OK) {
+    const StreamBlock block(c, qmm::gemm_fp8_f16_scratch_bytes(m, n, k));
+    if (block.get() != nullptr) {
       return map_hip(qmm::launch_fp8_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<const float>(2),
-                                              c.ptr<float>(3), ws, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
+                                              c.ptr<float>(3), block.get(), static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                               static_cast<uint32_t>(k), c.stream));
     }
-    g_last_error.clear();
   }
   return map_hip(qmm::launch_fp8_gemv(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<const float>(2),
                                       c.ptr<float>(3), static_cast<uint32_t>(m), static_cast<uint32_t>(n),
@@ -1408,6 +1472,7 @@ qmm_status qmm_init(int device) {
       return map_hip(e);
     }
   }
+  (void)g_stream_scratch.reserve(StreamBlock::grow);   // (without it the ids that use it run kernels that need none)
   return QMM_OK;
 }
 
@@ -1561,12 +1626,6 @@ qmm_status qmm_workspace_bytes(qmm_kernel kernel, const uint64_t* scalars, size_
   } else if (id == "gemm_mxfp4" || id == "gemm_mxfp4_batched") {
     const uint64_t m = sc(0), k = sc(2);
     if (m >= kMxfp4GemmMinRows && qmm::gemm_mxfp4_f32_supported(m, k)) *out_bytes = qmm::gemm_mxfp4_f32_workspace_bytes(m, k);
-  } else if (id == "gemm_fp8") {
-    const uint64_t m = sc(0), n = sc(1), k = sc(2);
-    if (n != 0 && m >= kFp8GemmMinRows && qmm::gemm_fp8_f16_supported(m, n, k)) {
-      const size_t bytes = qmm::gemm_fp8_f16_workspace_bytes(m, n, k);
-      if (bytes > kDecodeScratchBytes) *out_bytes = bytes;
-    }
   } else if (starts("gemm_q5k") || starts("gemm_q6k")) {
     const uint64_t m = sc(0), n = sc(1), k = sc(2);
     if (m >= kQ4KGemmMinRows && qmm::gemm_kquant_f16_supported(m, n, k)) *out_bytes = qmm::gemm_kquant_f16_workspace_bytes(m, n, k);

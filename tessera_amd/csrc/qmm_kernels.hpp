@@ -106,10 +106,12 @@ bool gemm_fp8_f32_rows_supported(uint64_t m, uint64_t n, uint64_t k);
 hipError_t gemm_fp8_f32_rows_prepare();
 hipError_t launch_fp8_f32_rows(const float* a, const uint8_t* w, const float* wscale, float* c, void* workspace,
                                uint32_t m, uint32_t n, uint32_t k, bool block_scales, hipStream_t stream);
-// "gemm_fp8" from 17 rows up (gemm_fp8.hip): fp16 weights on the fly against two fp16 terms of each row.
+// "gemm_fp8" from 17 rows up (gemm_fp8.hip): fp16 weights on the fly against two fp16 terms of each row, as many
+// rows at a time as gemm_fp8_f16_scratch_limit bytes of scratch hold.
+constexpr size_t gemm_fp8_f16_scratch_limit = size_t{32} << 20;
 bool gemm_fp8_f16_supported(uint64_t m, uint64_t n, uint64_t k);
-size_t gemm_fp8_f16_workspace_bytes(uint64_t m, uint64_t n, uint64_t k);
-hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* workspace,
+size_t gemm_fp8_f16_scratch_bytes(uint64_t m, uint64_t n, uint64_t k);
+hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch,
                                uint32_t m, uint32_t n, uint32_t k, hipStream_t stream);
 size_t gemm_mxfp4_f32_workspace_bytes(uint64_t m, uint64_t k);
 hipError_t launch_mxfp4_f32_gemm(const float* a, const uint8_t* w, float* c, void* workspace, uint32_t m,
@@ -177,7 +179,8 @@ hipError_t moe_q4k_prepare();           // once per device, from qmm_init (moe_q
 // (gemv_kquant_rows.hip); any m, taken some rows a pass (eight, eight, four).
 hipError_t gemv_kquant_rows_prepare();   // once per device, from qmm_init
 // Q5_K, Q6_K (`bits` = 5, 6): weights streamed through LDS, K cut into parts whose sums go to `ws` (any size that holds
-// 16 weight rows' sums), up to eight rows a pass.
+// 16 weight rows' sums), up to eight rows a pass.  kquant_rows_stream_scratch: what one pass takes of `ws_bytes`.
+size_t kquant_rows_stream_scratch(uint32_t bits, size_t ws_bytes, uint32_t m, uint32_t n, uint32_t k);
 hipError_t launch_kquant_rows_stream(uint32_t bits, const float* a, const uint8_t* w, float* c, void* ws, size_t ws_bytes, uint32_t m,
                                      uint32_t n, uint32_t k, hipStream_t stream);
 bool gemv_kquant_rows_supported(uint64_t m, uint64_t n, uint64_t k);
