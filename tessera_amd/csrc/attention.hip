@@ -176,6 +176,13 @@ __device__ __forceinline__ float power_of_two_to(float v, int target) {
 
 constexpr float kLog2E = 1.44269504088896340736f, kLn2 = 0.69314718055994530942f;
 
+// What weights are taken relative to: the largest score, or 0 where every score so far is -inf (the weights
+// are then 0, not exp(-inf + inf)).
+__device__ __forceinline__ float reference_score(float largest) { return largest == -INFINITY ? 0.0f : largest; }
+// A second term's sum where the cache's side may hold infinities: infinity times the (possibly zero or
+// negative) second term says nothing that the first term's sum does not.
+__device__ __forceinline__ float finite_or_zero(float v) { return __builtin_isfinite(v) ? v : 0.0f; }
+
 template <KvKind KV, int DP, int NW>
 __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArgs a) {
   constexpr bool F32 = KV == KvKind::F32, QUANT = kv_quantized(KV);
@@ -328,6 +335,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float x = acc[e];
+        if constexpr (KV == KvKind::F16) x = (r & 1u) ? finite_or_zero(x) : x;
         if constexpr (!F32) x += other_term(x);
         x *= score_scale;
         if constexpr (QUANT) x *= ksv[4 * h + e];
@@ -340,12 +348,13 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 #pragma unroll
     for (int e = 1; e < 4 * HALVES; ++e) most = fmaxf(most, s[e]);
     const float m_new = fmaxf(run_max, groups_max(most));
-    float corr = __builtin_amdgcn_exp2f(run_max - m_new);          // 0 on the first tile (run_max = -inf)
+    const float m_ref = reference_score(m_new);
+    float corr = __builtin_amdgcn_exp2f(run_max - m_ref);          // 0 on the first tile (run_max = -inf)
     run_max = m_new;
     float sum = 0.0f;
 #pragma unroll
     for (int e = 0; e < 4 * HALVES; ++e) {
-      s[e] = __builtin_amdgcn_exp2f(s[e] - m_new);
+      s[e] = __builtin_amdgcn_exp2f(s[e] - m_ref);
       sum += s[e];
     }
     run_sum = fmaf(corr, run_sum, sum);
@@ -372,6 +381,18 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
       for (int j = 0; j < VE; ++j) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[j][e] *= corr;
+      }
+    }
+    if constexpr (!QUANT) {
+      // Rows past the range's end stand for no key: infinite elements of the one read in their place would
+      // not vanish under the weight 0.
+      if (j0 + KEYS - 1 > last) {
+#pragma unroll
+        for (int e = 0; e < 4 * HALVES; ++e) {
+          const bool none = j0 + 16 * (e / 4) + 4 * g + e % 4 > last;
+#pragma unroll
+          for (int w = 0; w < VW; ++w) vr[e][w] = none ? 0u : vr[e][w];
+        }
       }
     }
     if constexpr (F32) {
@@ -406,7 +427,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
   float top = merge_m[0][column_head];
 #pragma unroll
   for (int w = 1; w < NW; ++w) top = fmaxf(top, merge_m[w][column_head]);
-  const float f = __builtin_amdgcn_exp2f(run_max - top) / value_up;
+  const float f = __builtin_amdgcn_exp2f(run_max - reference_score(top)) / value_up;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
 #pragma unroll
@@ -414,7 +435,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
       float4 x;
       float* xs = &x.x;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) xs[c] = (F32 ? o[j + c][e] : o[j + c][e] + other_term(o[j + c][e])) * f;
+      for (int c = 0; c < 4; ++c) {
+        float own = o[j + c][e];
+        if constexpr (KV == KvKind::F16) own = (r & 1u) ? finite_or_zero(own) : own;
+        xs[c] = (F32 ? own : own + other_term(own)) * f;
+      }
       if (writer) *reinterpret_cast<float4*>(&merge_o[wave][column_head][4 * g + e][j]) = x;
     }
   }
@@ -425,9 +450,10 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 #pragma unroll
     for (int w = 1; w < NW; ++w) m = fmaxf(m, merge_m[w][h]);
     float sum = 0.0f, acc = 0.0f;
+    const float m_ref = reference_score(m);
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      sum = fmaf(__builtin_amdgcn_exp2f(merge_m[w][h] - m), merge_l[w][h], sum);
+      sum = fmaf(__builtin_amdgcn_exp2f(merge_m[w][h] - m_ref), merge_l[w][h], sum);
       acc += merge_o[w][h][d / VE][d % VE];
     }
     if (a.part.split != 0) {
@@ -499,7 +525,7 @@ __global__ __launch_bounds__(256) void attention_any_kernel(AttentionArgs a) {
     if (wave == 0) {
       const float s = sc[lane];
       const float m_new = fmaxf(run_max, wave_max(s));
-      const float w = lane < count ? expf(s - m_new) : 0.0f;
+      const float w = lane < count ? expf(s - reference_score(m_new)) : 0.0f;
       wt[lane] = w;
       const float l = wave_sum(w);
       if (lane == 0) {
@@ -509,7 +535,7 @@ __global__ __launch_bounds__(256) void attention_any_kernel(AttentionArgs a) {
     }
     __syncthreads();
     const float m_new = bc[0];
-    const float corr = expf(run_max - m_new);      // 0 on the first tile (run_max = -inf)
+    const float corr = expf(run_max - reference_score(m_new));      // 0 on the first tile (run_max = -inf)
     run_sum = fmaf(corr, run_sum, bc[1]);
     run_max = m_new;
     if (t < D) {

@@ -123,3 +123,76 @@ def test_attention_query_magnitudes(backend, kind, gain):
     want = expected(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - 1, 0)
     got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - 1, 0)
     assert np.max(np.abs(got - want)) <= 4e-6 * max(1.0, np.max(np.abs(want)))
+
+
+# spans of keys of score -inf: one, the last one, whole tiles of every kernel, the first 64 and more, a whole part
+@pytest.mark.parametrize("kind", ["f32", "f16"])
+@pytest.mark.parametrize("head_dim", [64, 128, 256, 34])
+@pytest.mark.parametrize("spans", [[(7, 8)], [(299, 300)], [(0, 40), (64, 96)], [(0, 100)], [(150, 300)]])
+def test_attention_keys_of_infinite_score(backend, kind, head_dim, spans):
+    """A key with an infinite element whose score is -inf has the weight 0: the rest of the row is as without it."""
+    m, n, heads, kv_heads = 2, 301, 6, 2
+    g = synth.rng(1200 + head_dim)
+    q = g.standard_normal((m, heads * head_dim)).astype(np.float32)
+    k, _ = cache(g, kind, n, kv_heads * head_dim)
+    v, _ = cache(g, kind, n, kv_heads * head_dim)
+    q, k = q.reshape(m, heads, head_dim), k.reshape(n, kv_heads, head_dim)
+    q[:, :, 3] = np.abs(q[:, :, 3]) + np.float32(0.1)
+    q[0, 0, 3] = 1.0                                   # (no second term)
+    q[0, 1, 3] = 0.1                                   # (a negative one)
+    q[:, :, 5] = -q[:, :, 3]
+    out = np.zeros(n, bool)
+    for lo, hi in spans:
+        out[lo:hi] = True
+    k[out, :, 3] = -np.inf
+    k[out[:, None] & (np.arange(kv_heads) == 1), 5] = np.inf
+    q, k = q.reshape(m, -1), k.reshape(n, -1)
+    want = expected(kind, q, k, v, None, None, m, n, heads, kv_heads, head_dim, n - m, 0)
+    assert np.isfinite(want).all()
+    bound = 2e-6 * max(1.0, np.max(np.abs(want)))
+    for split in (0, 1, 4):
+        got = attend(backend, kind, q, k, v, None, None, m, n, heads, kv_heads, head_dim, n - m, 0, split=split)
+        assert np.max(np.abs(got - want)) <= 2 * bound, split
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16"])
+@pytest.mark.parametrize("head_dim", [64, 256, 34])
+@pytest.mark.parametrize("n", [1, 33, 290])
+def test_attention_infinite_values(backend, kind, head_dim, n):
+    """An infinite value makes its own element of the rows that see it infinite, with its sign, and no other;
+    also as the last key, whose row stands in for the keys past the end."""
+    heads, kv_heads, m = 6, 2, min(2, n)
+    g = synth.rng(1300 + n + head_dim)
+    q = (0.1 * g.standard_normal((m, heads * head_dim))).astype(np.float32)
+    k, _ = cache(g, kind, n, kv_heads * head_dim)
+    v, _ = cache(g, kind, n, kv_heads * head_dim)
+    v = v.reshape(n, kv_heads, head_dim)
+    v[n // 2, 0, 1] = np.inf
+    v[n - 1, 1, 9] = -np.inf
+    v = v.reshape(n, -1)
+    want = expected(kind, q, k, v, None, None, m, n, heads, kv_heads, head_dim, n - m, 0)
+    assert not np.isnan(want).any() and np.isinf(want).any()
+    for split in (0, 3):
+        got = attend(backend, kind, q, k, v, None, None, m, n, heads, kv_heads, head_dim, n - m, 0, split=split)
+        inf = np.isinf(want)
+        assert np.array_equal(got[inf], want[inf]), split
+        assert np.max(np.abs(got[~inf] - want[~inf])) <= 4e-6, split
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16"])
+def test_attention_nan_stays_in_its_rows(backend, kind):
+    """A NaN in a query spoils that row's head, one in a key the rows that see it, one in a value their element."""
+    m, n, heads, kv_heads, head_dim = 4, 90, 4, 2, 64
+    g = synth.rng(1400)
+    q = g.standard_normal((m, heads * head_dim)).astype(np.float32)
+    k, _ = cache(g, kind, n, kv_heads * head_dim)
+    v, _ = cache(g, kind, n, kv_heads * head_dim)
+    q[0, 70] = np.nan                       # row 0, head 1
+    k[88, 5] = np.nan                       # rows 2 and 3, heads 0 and 1
+    v[87, 64 + 6] = np.nan                  # rows 1 to 3, heads 2 and 3, element 6
+    got = attend(backend, kind, q, k, v, None, None, m, n, heads, kv_heads, head_dim, n - m, 0).reshape(m, heads, head_dim)
+    bad = np.zeros(got.shape, bool)
+    bad[0, 1] = True
+    bad[2:, :2] = True
+    bad[1:, 2:, 6] = True
+    assert np.array_equal(np.isnan(got), bad)
