@@ -3,10 +3,13 @@
 // statements src/core/numerics/attention.cpp.
 //
 // Precision.  Scores and sums are fp32 in every variant.  Where the contraction runs on the fp16
-// matrix instruction, the fp32 side (queries, then weights) enters as two fp16 terms hi + lo of a value
-// brought near 2^8 resp. 2^14 by a power of two -- 22 significant bits -- and the cache's side enters
-// exactly: an fp16 number, or the integer or E4M3 code, whose scale multiplies the fp32 score (keys) or
-// the fp32 weight (values).
+// matrix instruction, the fp32 side (queries, then weights times the values' scales) enters as two fp16
+// terms of a value x that a power of two brings below 2^15: hi = RN16(x), lo = RN16(2^11 (x - hi)), whose
+// sums meet as hi + 2^-11 lo.  That misses x by at most 2^-23 of itself while |x| >= 2^-14 and by 2^-36
+// below.  A query element is brought under its head's largest and keeps that precision down to 2^-28 of it; a
+// weight, under the largest of the row so far, down to 2^-18 of it, and what is smaller is off by 2^-40 of it.
+// The cache's side enters exactly: an fp16 number, or the integer or E4M3 code, whose scale multiplies
+// the fp32 score (keys) or the fp32 weight (values).
 
 #include <type_traits>
 
@@ -268,6 +271,13 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 
   // The query operand: column r is head r (fp32) or the term r % 2 of head r / 2.
   const uint32_t column_head = F32 ? r : r / 2u;
+  const bool second = !F32 && (r & 1u) != 0u;                      // this lane's column is a second term
+  const float term_down = second ? 0x1p-11f : 1.0f;
+  // Two terms of x, this lane's: hi, or 2^11 (x - hi).
+  auto term_of = [&](float x) {
+    const _Float16 hi = static_cast<_Float16>(x);
+    return second ? static_cast<_Float16>((x - static_cast<float>(hi)) * 0x1p11f) : hi;
+  };
   const float* qp = a.q + ((a.row_base + row) * a.heads + head0 + (column_head < here ? column_head : here - 1u)) * D;
   float qf[F32 ? STEPS : 1];
   half8_t qh[F32 ? 1 : STEPS];
@@ -292,15 +302,13 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
       for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(raw[i][e]));
     }
     most = groups_max(most);
-    const float up = power_of_two_to(most, 8);
+    const float up = power_of_two_to(most, 14);
     score_scale /= up;
 #pragma unroll
     for (int i = 0; i < STEPS; ++i) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float x = raw[i][kq_dim<KV>(e)] * up;
-        const _Float16 hi = static_cast<_Float16>(x);
-        qh[i][e] = (r & 1u) ? static_cast<_Float16>(x - static_cast<float>(hi)) : hi;
+        qh[i][e] = term_of(raw[i][kq_dim<KV>(e)] * up);
       }
     }
   }
@@ -309,7 +317,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 #pragma unroll
   for (int j = 0; j < VE; ++j) o[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
   float run_max = -INFINITY, run_sum = 0.0f;
-  float value_most = 0.0f, value_up = F32 ? 1.0f : QUANT ? power_of_two_to(0.0f, 14) : 0x1p14f;
+  float lane_most = 0.0f, value_up = F32 ? 1.0f : QUANT ? power_of_two_to(0.0f, 14) : 0x1p14f;
   for (uint64_t j0 = first; j0 <= last; j0 += NW * KEYS) {
     const bool more = j0 + NW * KEYS <= last;
     float s[4 * HALVES];
@@ -335,8 +343,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float x = acc[e];
-        if constexpr (KV == KvKind::F16) x = (r & 1u) ? finite_or_zero(x) : x;
-        if constexpr (!F32) x += other_term(x);
+        if constexpr (KV == KvKind::F16) x = second ? finite_or_zero(x) : x;
+        if constexpr (!F32) {
+          x *= term_down;
+          x += other_term(x);
+        }
         x *= score_scale;
         if constexpr (QUANT) x *= ksv[4 * h + e];
         s[4 * h + e] = j0 + 16 * h + 4 * g + e <= last ? x : -INFINITY;
@@ -359,19 +370,28 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
     }
     run_sum = fmaf(corr, run_sum, sum);
     if constexpr (QUANT) {
-      // The values' scales enter the weights; the power of two follows the largest of them so far.
-      float vm = fabsf(vsv[0]);
+      // The values' scales enter the weights.  The power of two keeps the largest contribution so far between
+      // 2^4 and 2^15.  It is looked at when a new largest score has made the old contributions smaller, and when a
+      // scale of this tile would leave the range under the largest weight, 1 (known before the weights are).
+      float scale_most = fabsf(vsv[0]);
 #pragma unroll
-      for (int e = 1; e < 4 * HALVES; ++e) vm = fmaxf(vm, fabsf(vsv[e]));
-      vm = groups_max(vm);
-      if (vm > value_most) {
-        value_most = vm;
-        const float up = power_of_two_to(vm, 14);
-        corr *= up / value_up;
-        value_up = up;
+      for (int e = 1; e < 4 * HALVES; ++e) scale_most = fmaxf(scale_most, fabsf(vsv[e]));
+      lane_most *= corr;
+#pragma unroll
+      for (int e = 0; e < 4 * HALVES; ++e) {
+        s[e] *= vsv[e];
+        lane_most = fmaxf(lane_most, fabsf(s[e]));
+      }
+      if (__any(corr != 1.0f || !(scale_most * value_up < 0x1p15f))) {
+        const float largest = groups_max(lane_most), scaled = largest * value_up;
+        if (largest > 0.0f && !(scaled >= 0x1p4f && scaled < 0x1p15f)) {
+          const float up = power_of_two_to(largest, 12);
+          corr *= up / value_up;
+          value_up = up;
+        }
       }
 #pragma unroll
-      for (int e = 0; e < 4 * HALVES; ++e) s[e] *= vsv[e] * value_up;
+      for (int e = 0; e < 4 * HALVES; ++e) s[e] *= value_up;
     } else if constexpr (!F32) {
 #pragma unroll
       for (int e = 0; e < 4 * HALVES; ++e) s[e] *= value_up;
@@ -404,10 +424,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
     } else {
       half8_t p;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const _Float16 hi = static_cast<_Float16>(s[e]);
-        p[e] = (r & 1u) ? static_cast<_Float16>(s[e] - static_cast<float>(hi)) : hi;
-      }
+      for (int e = 0; e < 8; ++e) p[e] = term_of(s[e]);
 #pragma unroll
       for (int j = 0; j < VE; ++j) {
         const uint4 w = {value_pair<KV>(vr[0], vr[1], j), value_pair<KV>(vr[2], vr[3], j),
@@ -421,7 +438,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 
   // Merge of the wavefronts: everyone's sum under the largest score of all, added in wavefront order.
   run_sum = groups_sum(run_sum);
-  const bool writer = F32 || (r & 1u) == 0u;
+  const bool writer = !second;
   if (g == 0u && writer) merge_m[wave][column_head] = run_max, merge_l[wave][column_head] = run_sum;
   __syncthreads();
   float top = merge_m[0][column_head];
@@ -437,7 +454,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         float own = o[j + c][e];
-        if constexpr (KV == KvKind::F16) own = (r & 1u) ? finite_or_zero(own) : own;
+        if constexpr (KV == KvKind::F16) own = second ? finite_or_zero(own) : own;
+        own *= term_down;
         xs[c] = (F32 ? own : own + other_term(own)) * f;
       }
       if (writer) *reinterpret_cast<float4*>(&merge_o[wave][column_head][4 * g + e][j]) = x;

@@ -196,3 +196,62 @@ def test_attention_nan_stays_in_its_rows(backend, kind):
     bad[2:, :2] = True
     bad[1:, 2:, 6] = True
     assert np.array_equal(np.isnan(got), bad)
+
+
+def attention_f64(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, q_base):
+    """softmax(Q K^T / sqrt(head_dim)) V in float64, causal, over the numbers that the cache holds."""
+    if ks is not None:
+        k, v = (oracle.dequant_kv(c, np.ones(n, np.float32), n, kv_heads * head_dim, kind).astype(np.float64) *
+                np.asarray(s, np.float64)[:, None] for c, s in ((k, ks), (v, vs)))
+    k, v = (np.asarray(x, np.float64).reshape(n, kv_heads, head_dim) for x in (k, v))
+    q, out = q.astype(np.float64).reshape(m, heads, head_dim), np.empty((m, heads, head_dim))
+    for i in range(m):
+        for h in range(heads):
+            s = k[:q_base + i + 1, h // (heads // kv_heads)] @ q[i, h] / np.sqrt(head_dim)
+            p = np.exp(s - s.max())
+            out[i, h] = p @ v[:q_base + i + 1, h // (heads // kv_heads)] / p.sum()
+    return out.reshape(m, heads * head_dim)
+
+
+@pytest.mark.parametrize("kind", ["q8", "q4", "fp8"])
+@pytest.mark.parametrize("at", [3, 200, 399])
+@pytest.mark.parametrize("binades", [12, 20, 30, 45, 60])
+def test_attention_weight_on_a_small_value_scale(backend, kind, at, binades):
+    """All the weight on one key whose value scale is 2^-binades of the others', which have none: the result keeps
+    its precision however large the scales of what does not contribute."""
+    m, n, heads, kv_heads, head_dim = 1, 400, 6, 2, 128
+    g = synth.rng(1500 + binades)
+    q = g.standard_normal((m, heads * head_dim)).astype(np.float32)
+    k = (0.01 * g.standard_normal((n, kv_heads, head_dim))).astype(np.float32)
+    for h in range(kv_heads):                                    # along every head of the group
+        k[at, h] = q.reshape(heads, head_dim)[h * 3:h * 3 + 3].mean(axis=0) * 150.0
+    k = k.reshape(n, -1)
+    k, ks = (oracle.quantize_fp8_pack(k, n, kv_heads * head_dim) if kind == "fp8" else
+             oracle.quantize_kv(k, n, kv_heads * head_dim, 8 if kind == "q8" else 4))
+    v, vs = cache(g, kind, n, kv_heads * head_dim)
+    vs[at] *= np.float32(2.0 ** -binades)
+    want = attention_f64(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m)
+    assert np.max(np.abs(want)) < 8.0 * 2.0 ** -binades         # (the others' weights vanish)
+    for split in (0, 4):
+        got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0, split=split)
+        assert np.max(np.abs(got - want)) <= 1e-6 * np.max(np.abs(want)), split
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+def test_attention_query_range_inside_a_head(backend, kind):
+    """One query element 2^18 times the others, on a dimension where every key is zero: the scores come from the
+    small ones alone and keep their precision."""
+    m, n, heads, kv_heads, head_dim = 2, 400, 6, 2, 128
+    g = synth.rng(1600)
+    q = g.standard_normal((m, heads, head_dim)).astype(np.float32)
+    q[:, :, 17] = 2.0 ** 18
+    q = q.reshape(m, -1)
+    k = g.standard_normal((n, kv_heads, head_dim)).astype(np.float32)
+    k[:, :, 17] = 0.0
+    k, ks = {"f32": lambda x: (x, None), "f16": lambda x: (x.astype(np.float16), None),
+             "fp8": lambda x: oracle.quantize_fp8_pack(x, n, kv_heads * head_dim)}.get(
+                 kind, lambda x: oracle.quantize_kv(x, n, kv_heads * head_dim, 8 if kind == "q8" else 4))(k.reshape(n, -1))
+    v, vs = cache(g, kind, n, kv_heads * head_dim)
+    want = attention_f64(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m)
+    got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0)
+    assert np.max(np.abs(got - want)) <= 2e-6 * max(1.0, np.max(np.abs(want)))
