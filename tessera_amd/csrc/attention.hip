@@ -194,10 +194,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
   constexpr int CE = F32 ? 4 : 128 / BITS < DP / 4 ? 128 / BITS : DP / 4;   // elements of a key a lane loads at once
   constexpr int RUNS = DP / (4 * CE);                              // such loads a key row
   constexpr int STEPS = F32 ? DP / 4 : DP / 32;                    // matrix instructions over head_dim
+  constexpr int CHAINS = F32 ? STEPS / 4 : STEPS / 2 < 1 ? 1 : STEPS / 2;   // sums of a score
   constexpr int VE = DP / 16;                                      // elements of a value row a lane holds
   constexpr int KW = CE * BITS / 32, VW = (VE * BITS + 31) / 32;   // dwords of those
   constexpr int HALVES = KEYS / 16;
-  __shared__ float merge_m[NW][HEADS], merge_l[NW][HEADS];
+  __shared__ float merge_m[NW][HEADS], merge_l[NW][HEADS], merge_scale[HEADS];
   __shared__ __align__(16) float merge_o[NW][HEADS][16][VE + 4];
 
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, r = lane & 15u, g = lane >> 4;
@@ -281,6 +282,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
   const float* qp = a.q + ((a.row_base + row) * a.heads + head0 + (column_head < here ? column_head : here - 1u)) * D;
   float qf[F32 ? STEPS : 1];
   half8_t qh[F32 ? 1 : STEPS];
+  // A column's scores are kept as the matrix instructions leave them, s; score_scale s is in units of log2.  Only
+  // differences from the largest are brought to those units, so that rounding goes with their size.
   float score_scale = kLog2E / sqrtf(static_cast<float>(D));
   if constexpr (F32) {
 #pragma unroll
@@ -302,7 +305,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
       for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(raw[i][e]));
     }
     most = groups_max(most);
-    const float up = power_of_two_to(most, 14);
+    const float up = most == 0.0f ? 1.0f : power_of_two_to(most, 14);
     score_scale /= up;
 #pragma unroll
     for (int i = 0; i < STEPS; ++i) {
@@ -323,49 +326,63 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
     float s[4 * HALVES];
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) {
-      float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-      if constexpr (F32) {
-        float4_t acc2 = {0.0f, 0.0f, 0.0f, 0.0f};
+      // One matrix instruction after another on one sum rounds at every step: CHAINS sums, added pairwise.
+      float4_t sums[CHAINS];
 #pragma unroll
-        for (int i = 0; i < RUNS; ++i) {
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i][0]), qf[4 * i], acc, 0, 0, 0);
-          acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i][1]), qf[4 * i + 1], acc2, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i][2]), qf[4 * i + 2], acc, 0, 0, 0);
-          acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i][3]), qf[4 * i + 3], acc2, 0, 0, 0);
-        }
-        acc += acc2;
-      } else {
+      for (int c = 0; c < CHAINS; ++c) sums[c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int i = 0; i < STEPS; ++i) {
+      for (int i = 0; i < STEPS; ++i) {
+        float4_t& acc = sums[i * CHAINS / STEPS];
+        if constexpr (F32) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(kr[h][i / 4][i % 4]), qf[i], acc, 0, 0, 0);
+        } else {
           acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(key_operand<KV>(&kr[h][i * 8 / CE][i * 8 % CE * BITS / 32]), qh[i], acc, 0, 0, 0);
         }
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float x = acc[e];
-        if constexpr (KV == KvKind::F16) x = second ? finite_or_zero(x) : x;
-        if constexpr (!F32) {
-          x *= term_down;
-          x += other_term(x);
-        }
-        x *= score_scale;
-        if constexpr (QUANT) x *= ksv[4 * h + e];
-        s[4 * h + e] = j0 + 16 * h + 4 * g + e <= last ? x : -INFINITY;
+      for (int c = CHAINS / 2; c > 0; c /= 2) {
+#pragma unroll
+        for (int i = 0; i < c; ++i) sums[i] += sums[i + c];
       }
+      const float4_t acc = sums[0];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[4 * h + e] = acc[e] * term_down;
+    }
+    float own[4 * HALVES], all = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4 * HALVES; ++e) {
+      own[e] = s[e];
+      if constexpr (!F32) s[e] += other_term(s[e]);
+      if constexpr (QUANT) s[e] *= ksv[e];
+      all += s[e];
     }
     if (more) load_keys(j0 + NW * KEYS);
+    if constexpr (KV == KvKind::F16) {
+      if (__any(!(fabsf(all) < INFINITY))) {       // infinities among the keys
+#pragma unroll
+        for (int e = 0; e < 4 * HALVES; ++e) {
+          const float x = second ? finite_or_zero(own[e]) : own[e];
+          s[e] = x + other_term(x);
+        }
+      }
+    }
+    const bool past = j0 + KEYS - 1 > last;        // the range ends inside this tile
+    if (past) {
+#pragma unroll
+      for (int e = 0; e < 4 * HALVES; ++e) s[e] = j0 + 16 * (e / 4) + 4 * g + e % 4 <= last ? s[e] : -INFINITY;
+    }
 
     float most = s[0];
 #pragma unroll
     for (int e = 1; e < 4 * HALVES; ++e) most = fmaxf(most, s[e]);
     const float m_new = fmaxf(run_max, groups_max(most));
     const float m_ref = reference_score(m_new);
-    float corr = __builtin_amdgcn_exp2f(run_max - m_ref);          // 0 on the first tile (run_max = -inf)
+    float corr = __builtin_amdgcn_exp2f((run_max - m_ref) * score_scale);   // 0 on the first tile (run_max = -inf)
     run_max = m_new;
     float sum = 0.0f;
 #pragma unroll
     for (int e = 0; e < 4 * HALVES; ++e) {
-      s[e] = __builtin_amdgcn_exp2f(s[e] - m_ref);
+      s[e] = __builtin_amdgcn_exp2f((s[e] - m_ref) * score_scale);
       sum += s[e];
     }
     run_sum = fmaf(corr, run_sum, sum);
@@ -406,7 +423,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
     if constexpr (!QUANT) {
       // Rows past the range's end stand for no key: infinite elements of the one read in their place would
       // not vanish under the weight 0.
-      if (j0 + KEYS - 1 > last) {
+      if (past) {
 #pragma unroll
         for (int e = 0; e < 4 * HALVES; ++e) {
           const bool none = j0 + 16 * (e / 4) + 4 * g + e % 4 > last;
@@ -417,9 +434,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
     }
     if constexpr (F32) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
+      for (int j = 0; j < VE; ++j) {
+        float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};   // the tile's own sum, for the reason of CHAINS
 #pragma unroll
-        for (int j = 0; j < VE; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(vr[e][j]), s[e], o[j], 0, 0, 0);
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bit_cast<float>(vr[e][j]), s[e], acc, 0, 0, 0);
+        o[j] += acc;
       }
     } else {
       half8_t p;
@@ -440,11 +459,12 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
   run_sum = groups_sum(run_sum);
   const bool writer = !second;
   if (g == 0u && writer) merge_m[wave][column_head] = run_max, merge_l[wave][column_head] = run_sum;
+  if (t < 16u && writer) merge_scale[column_head] = score_scale;
   __syncthreads();
   float top = merge_m[0][column_head];
 #pragma unroll
   for (int w = 1; w < NW; ++w) top = fmaxf(top, merge_m[w][column_head]);
-  const float f = __builtin_amdgcn_exp2f(run_max - reference_score(top)) / value_up;
+  const float f = __builtin_amdgcn_exp2f((run_max - reference_score(top)) * score_scale) / value_up;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
 #pragma unroll
@@ -468,16 +488,16 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 #pragma unroll
     for (int w = 1; w < NW; ++w) m = fmaxf(m, merge_m[w][h]);
     float sum = 0.0f, acc = 0.0f;
-    const float m_ref = reference_score(m);
+    const float m_ref = reference_score(m), scale = merge_scale[h];
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      sum = fmaf(__builtin_amdgcn_exp2f(merge_m[w][h] - m_ref), merge_l[w][h], sum);
+      sum = fmaf(__builtin_amdgcn_exp2f((merge_m[w][h] - m_ref) * scale), merge_l[w][h], sum);
       acc += merge_o[w][h][d / VE][d % VE];
     }
     if (a.part.split != 0) {
       const uint64_t at = (row * a.heads + head0 + h) * split + s_part;
       a.part.pacc[at * D + d] = acc;
-      if (d == 0) a.part.pmax[at] = m * kLn2, a.part.psum[at] = sum;
+      if (d == 0) a.part.pmax[at] = m * scale * kLn2, a.part.psum[at] = sum;
     } else {
       a.out[((a.row_base + row) * a.heads + head0 + h) * D + d] = acc / sum;
     }

@@ -255,3 +255,23 @@ def test_attention_query_range_inside_a_head(backend, kind):
     want = attention_f64(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m)
     got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0)
     assert np.max(np.abs(got - want)) <= 2e-6 * max(1.0, np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("split", [0, 8])
+def test_attention_rounding_of_long_heads(backend, kind, split):
+    """Scores of standard deviation 4 over head_dim 256.  A weight's relative error is its score's error.  Sums of
+    at most 64 products and pairwise sums of those round like a chain of about 14 terms, each step by
+    2^-24 * 0.42 of the score in the root mean square: sqrt(14) * 0.42 * 2^-24 * 4 = 3.7e-7; one running sum over the
+    head, or two, are at 8e-7 and more.  The sums over the keys add 2e-7."""
+    m, n, heads, kv_heads, head_dim = 1, 1200, 24, 4, 256
+    errors = []
+    for seed in range(6):
+        g = synth.rng(1700 + seed)
+        q = (4.0 * g.standard_normal((m, heads * head_dim))).astype(np.float32)
+        k, ks = cache(g, kind, n, kv_heads * head_dim)
+        v, vs = cache(g, kind, n, kv_heads * head_dim)
+        want = attention_f64(kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m)
+        got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0, split=split)
+        errors.append(np.linalg.norm(got - want) / np.linalg.norm(want))
+    assert np.sqrt(np.mean(np.square(errors))) <= 1.3 * np.hypot(3.7e-7, 2e-7)
