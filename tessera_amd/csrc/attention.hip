@@ -496,8 +496,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
     }
     if (a.part.split != 0) {
       const uint64_t at = (row * a.heads + head0 + h) * split + s_part;
-      a.part.pacc[at * D + d] = acc;
-      if (d == 0) a.part.pmax[at] = m * scale * kLn2, a.part.psum[at] = sum;
+      // The part's largest score in natural units is rounded; the sums move by what that took from it.
+      const float natural = scale * kLn2, largest = m * natural;
+      const float moved = m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(fmaf(m, natural, -largest) * kLog2E);
+      a.part.pacc[at * D + d] = acc * moved;
+      if (d == 0) a.part.pmax[at] = largest, a.part.psum[at] = sum * moved;
     } else {
       a.out[((a.row_base + row) * a.heads + head0 + h) * D + d] = acc / sum;
     }

@@ -275,3 +275,25 @@ def test_attention_rounding_of_long_heads(backend, kind, split):
         got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0, split=split)
         errors.append(np.linalg.norm(got - want) / np.linalg.norm(want))
     assert np.sqrt(np.mean(np.square(errors))) <= 1.3 * np.hypot(3.7e-7, 2e-7)
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16"])
+def test_attention_parts_of_large_scores(backend, kind):
+    """Scores near 400, exact in fp32 and in natural units (one element a query, head_dim 64): what is left is the
+    rounding of differences up to 6, 6 * 2^-23, and of the weights.  A part's largest score rounded apart from its
+    sums would cost 400 * 2^-25 = 1.2e-5."""
+    m, n, heads, kv_heads, head_dim = 1, 640, 4, 2, 64
+    g = synth.rng(1800)
+    q = np.zeros((m, heads, head_dim), np.float32)
+    q[:, :, 11] = 1.0
+    k = g.standard_normal((n, kv_heads, head_dim)).astype(np.float32)
+    k[:, :, 11] = 2.0 * np.round(8.0 * 200.0 + 12.0 * g.uniform(-1.0, 1.0, (n, kv_heads)))   # (exact in fp16)
+    k = k.reshape(n, -1)
+    k = k.astype(np.float16) if kind == "f16" else k
+    v, _ = cache(g, kind, n, kv_heads * head_dim)
+    q = q.reshape(m, -1)
+    want = attention_f64(kind, q, k, v, None, None, m, n, heads, kv_heads, head_dim, n - m)
+    for split in (1, 5, 40):
+        got = attend(backend, kind, q, k, v, None, None, m, n, heads, kv_heads, head_dim, n - m, 0, split=split)
+        err = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert err <= 1.2e-6, (split, err)
