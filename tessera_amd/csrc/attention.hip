@@ -638,10 +638,11 @@ hipError_t launch_rows(const AttentionArgs& a, uint64_t m, hipStream_t stream) {
   constexpr uint32_t kHeads = KV == KvKind::F32 ? 16 : 8;
   const uint32_t group = a.heads / a.kv_heads, blocks = (group + kHeads - 1) / kHeads;
   const uint64_t split = a.part.split == 0 ? 1 : a.part.split;
-  const dim3 grid(static_cast<uint32_t>(m * a.kv_heads * blocks * split));
+  const uint64_t workgroups = m * a.kv_heads * blocks * split;
+  const dim3 grid(static_cast<uint32_t>(workgroups));
   // Four wavefronts a workgroup take 128 keys at once; where a workgroup has more to do and the
-  // registers allow it, eight.
-  const bool wide = a.n / split > 160;
+  // registers and the size of a grid allow it, eight.
+  const bool wide = a.n / split > 160 && workgroups < kMaxGridThreads / 512u;
   auto go = [&](auto kernel, uint32_t waves) { hipLaunchKernelGGL(kernel, grid, dim3(waves * 64u), 0, stream, a); };
   if (a.head_dim <= 64) {
     wide ? go(attention_rows_kernel<KV, 64, 8>, 8) : go(attention_rows_kernel<KV, 64, 4>, 4);

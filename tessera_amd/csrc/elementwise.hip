@@ -758,7 +758,8 @@ hipError_t launch_fill_i32(int32_t* out, int32_t value, uint64_t n, hipStream_t 
 hipError_t launch_rmsnorm(const float* x, const float* w, float* y, uint64_t rows, uint64_t cols, float eps,
                           hipStream_t stream) {
   constexpr uint64_t kMaxThreads = 1024, kMaxV = 8;
-  if (cols % 4 != 0 || cols / 4 > kMaxThreads * kMaxV) {
+  // (a launch has fewer than 2^32 threads: with 256 a row, up to 2^24 rows)
+  if (cols % 4 != 0 || cols / 4 > kMaxThreads * kMaxV || (cols / 4 > 256 * kMaxV && rows >= kMaxGridThreads / kMaxThreads)) {
     hipLaunchKernelGGL(rmsnorm_any_kernel, dim3(static_cast<uint32_t>(rows)), dim3(256), 0, stream, x, w, y, cols, eps);
     return hipGetLastError();
   }
@@ -929,7 +930,12 @@ hipError_t launch_top_k_rows(const float* logits, uint32_t* ids, float* vals, ui
   } else if (vocab <= 512) {
     hipLaunchKernelGGL(top_k_short_rows_kernel<8>, four_rows, dim3(256), 0, stream, logits, ids, vals, rows, v, top_k, row_base);
   } else {
-    hipLaunchKernelGGL(top_k_long_rows_kernel, dim3(rows), dim3(kTopKThreads), 0, stream, logits, ids, vals, v, top_k, row_base);
+    constexpr uint32_t kMost = static_cast<uint32_t>(kMaxGridThreads / kTopKThreads) - 1u;   // rows of one launch
+    for (uint32_t r = 0; r < rows; r += kMost) {
+      const size_t at = static_cast<size_t>(r) * top_k;
+      hipLaunchKernelGGL(top_k_long_rows_kernel, dim3(rows - r < kMost ? rows - r : kMost), dim3(kTopKThreads), 0, stream, logits,
+                         ids + at, vals + at, v, top_k, row_base + r);
+    }
   }
   return hipGetLastError();
 }

@@ -10,6 +10,8 @@
 
 namespace qmm {
 
+constexpr uint64_t kMaxGridThreads = uint64_t{1} << 32;   // a launch has fewer threads along each dimension
+
 void set_num_cus(int cus);
 int num_cus();
 

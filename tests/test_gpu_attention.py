@@ -4,6 +4,7 @@ columns of a matrix instruction, key counts around the tiles, a value scale of z
 scales.  Against the oracle's restatements; bound as in test_gpu_trunk.py (sums in another order)."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from tessera_amd import synth
@@ -297,3 +298,24 @@ def test_attention_parts_of_large_scores(backend, kind):
         got = attend(backend, kind, q, k, v, None, None, m, n, heads, kv_heads, head_dim, n - m, 0, split=split)
         err = np.linalg.norm(got - want) / np.linalg.norm(want)
         assert err <= 1.2e-6, (split, err)
+
+
+def test_attention_more_workgroups_than_one_grid_of_wide_ones(backend):
+    """2^23 workgroups of eight wavefronts are 2^32 threads, which one launch may not have: four wavefronts each."""
+    heads, head_dim, n = 32, 16, 200
+    m = (1 << 23) // heads + 3
+    g = synth.rng(1900)
+    k, _ = cache(g, "f16", n, heads * head_dim)
+    v, _ = cache(g, "f16", n, heads * head_dim)
+    q = torch.empty(m, heads * head_dim, device="cuda")
+    q.normal_(generator=torch.Generator(device="cuda").manual_seed(7))
+    out = torch.full((m, heads * head_dim), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    wrap = lambda t: backend.WrapBuffer(t.data_ptr(), t.numel() * t.element_size())
+    run(backend, "attention", [wrap(q), backend.Upload(k), backend.Upload(v), wrap(out)],
+        [m, n, heads, heads, head_dim, n, 0, 0, 1, 1], grid=(m * heads, 1, 1))
+    backend.Synchronize()
+    assert torch.isfinite(out).all()
+    rows = [0, 1, m // 2, m - 1]
+    want = expected("f16", q[rows].cpu().numpy(), k, v, None, None, len(rows), n, heads, heads, head_dim, n, 0)
+    assert np.max(np.abs(out[rows].cpu().numpy() - want)) <= 2e-6 * max(1.0, np.max(np.abs(want)))

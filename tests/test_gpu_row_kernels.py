@@ -2,6 +2,7 @@
 number of loads a thread or another loop takes over, against the oracle."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from tessera_amd import synth
@@ -69,3 +70,44 @@ def test_top_k_edges(backend, rows, vocab, top_k, kind):
         want_ids, want_vals = top_k_want(x[r + 1], top_k)
         assert np.array_equal(ids[r], want_ids), r
         assert np.array_equal(vals[r].view(np.uint32), want_vals.view(np.uint32)), r
+
+
+def test_top_k_more_rows_than_one_grid(backend):
+    """2^22 rows of a workgroup of 1024 are 2^32 threads, which one launch may not have: two launches."""
+    rows, vocab, top_k = (1 << 22) + 5, 513, 3
+    x = torch.empty(rows, vocab, device="cuda")
+    x.normal_(generator=torch.Generator(device="cuda").manual_seed(5))
+    ids = torch.full((rows, top_k), -1, dtype=torch.int32, device="cuda")
+    vals = torch.empty(rows, top_k, device="cuda")
+    torch.cuda.synchronize()
+    wrap = lambda t: backend.WrapBuffer(t.data_ptr(), t.numel() * t.element_size())
+    run(backend, "top_k_rows", [wrap(x), wrap(ids), wrap(vals)], [rows, vocab, top_k, 0])
+    backend.Synchronize()
+    assert (ids >= 0).all()
+    some = list(range(4)) + list(range((1 << 22) - 6, rows))
+    for r in some:
+        want_ids, want_vals = top_k_want(x[r].cpu().numpy(), top_k)
+        assert np.array_equal(ids[r].cpu().numpy().astype(np.uint32), want_ids), r
+        assert np.array_equal(vals[r].cpu().numpy(), want_vals), r
+
+
+def test_rmsnorm_more_rows_than_one_grid_of_wide_workgroups(backend):
+    """2^22 rows too long for a workgroup of 256 to hold, in place: 138 GB, on the loop that reads a row twice."""
+    rows, cols = (1 << 22) + 1, 8196
+    if torch.cuda.mem_get_info()[0] < 150 << 30:
+        pytest.skip("needs 150 GB")
+    x = torch.empty(rows * cols, device="cuda")
+    x.normal_(generator=torch.Generator(device="cuda").manual_seed(6))
+    w = torch.ones(cols, device="cuda")
+    some = [0, 1 << 21, rows - 1]
+    before = {r: x[r * cols:(r + 1) * cols].cpu().numpy() for r in some}
+    torch.cuda.synchronize()
+    wrap = lambda t: backend.WrapBuffer(t.data_ptr(), t.numel() * t.element_size())
+    eps = np.float32(1e-6)
+    run(backend, "rmsnorm", [wrap(x), wrap(w), wrap(x)], [rows, cols, int(eps.view(np.uint32))])
+    backend.Synchronize()
+    for r in some:
+        want = oracle.rmsnorm(before[r][None], np.ones(cols, np.float32), 1, cols, float(eps))[0]
+        assert np.max(np.abs(x[r * cols:(r + 1) * cols].cpu().numpy() - want)) <= 2e-5, r
+    del x
+    torch.cuda.empty_cache()
