@@ -4,9 +4,9 @@
 //
 // Precision.  The contract is fp32 activations and exact weights.  Every E4M3 code is an fp16 number, so the
 // weights are converted in registers without loss; a row of A becomes two fp16 terms under a power of two that
-// brings its largest magnitude to [2^14, 2^15): hi = RN16(x / s), lo = RN16(x / s - hi).  That keeps 22 bits of
-// every element down to 2^-28 of the row's largest and 2^-39 of the largest below that.  Products of an 11-bit
-// and a 4-bit significand are exact; v_mfma_f32_32x32x16_f16 adds them up, and its additions are what costs
+// brings its largest magnitude to [2^14, 2^15): hi = RN16(x / s), lo = RN16(2^11 (x / s - hi)), x / s = hi + 2^-11 lo.
+// That misses an element by at most 2^-23 of itself down to 2^-28 of the row's largest, and by 2^-50 of the
+// largest below.  Products of an 11-bit and a 4-bit significand are exact; v_mfma_f32_32x32x16_f16 adds them up, and its additions are what costs
 // precision: one chain of both terms over 5120 weights was measured at 6.2e-7 of the float64 result in the
 // 2-norm, against 1.2e-7 for the multiply-add kernel's short chains.  So an output has four sums: the second
 // term's products, 2^-11 as large, in one of their own, the first term's for 128 weights at a time, those of 1024,
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256) void rows_to_f16_terms_kernel(const float* __r
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       hi[i] = static_cast<_Float16>(x[i]);
-      const float rest = x[i] - static_cast<float>(hi[i]);
+      const float rest = (x[i] - static_cast<float>(hi[i])) * 0x1p11f;
       lo[i] = static_cast<_Float16>(fabsf(x[i]) < 65504.0f ? rest : 0.0f);   // (NaN compares false)
     }
     *reinterpret_cast<half4_t*>(out + g * 4u) = hi;
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_kernel(const _Float16* __rest
   };
 
   // Four sums an output: `run` takes the first term's products of kRunSteps steps and is then added to `acc`, which
-  // takes kAccSteps steps and is added to `total`; `low` takes the second term's, 2^-11 as large, from end to end.
+  // takes kAccSteps steps and is added to `total`; `low` takes the second term's, worth 2^-11 each, from end to end.
   float16_t total[kTI][kTJ], acc[kTI][kTJ], run[kTI][kTJ], low[kTI][kTJ];
 #pragma unroll
   for (int i = 0; i < kTI; ++i)
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_kernel(const _Float16* __rest
       for (int e = 0; e < 16; ++e) {
         const uint32_t row = m0 + wave_m * WM + i * 32u + (e >> 2) * 8u + kg * 4u + (e & 3u);
         if (row >= m || col >= n) continue;
-        const float sum = total[i][j][e] + (acc[i][j][e] + (run[i][j][e] + low[i][j][e]));
+        const float sum = total[i][j][e] + (acc[i][j][e] + fmaf(low[i][j][e], 0x1p-11f, run[i][j][e]));
         out[static_cast<size_t>(row) * n + col] = part != nullptr ? sum : sum * a_scale[row] * ws;
       }
   }

@@ -1,5 +1,5 @@
 """FP8 E4M3 weights ("gemm_fp8") times 17 rows and more on the fp16 matrix instruction: the codes are exact in
-fp16, an fp32 row goes in as two fp16 terms (22 bits of every element down to 2^-28 of the row's largest).
+fp16, an fp32 row goes in as two fp16 terms (2^-23 of every element down to 2^-28 of the row's largest).
 Reference kernel src/backends/rocm/rocm_kernels_basic.cpp:1039-1064, CPU GemmFp8Ref.
 
 Bound, in units of an output's root sum of squared products (the size it has before its products cancel): the
@@ -49,7 +49,7 @@ def test_matches_float64(backend, m, n, k):
     a = synth.activations_f32(g, m, k)
     a[m // 2] *= np.float32(2.0 ** 100)      # rows keep scales of their own
     a[m - 1] *= np.float32(2.0 ** -110)
-    a[0, : k // 2] *= np.float32(2.0 ** -20)  # and elements far below a row's largest their precision
+    a[0, : k // 2] *= np.float32(2.0 ** -20)
     assert within(fp8_gemm(backend, a, codes, scales, m, n, k), *exact(a, codes, scales, n, k), k)
 
 
@@ -101,3 +101,23 @@ def test_small_caller_workspace_still_runs(backend):
     fast = fp8_gemm(backend, a, codes, scales, m, n, k)
     want = exact(a[:64], codes, scales, n, k)
     assert within(slow[:64], *want, k) and within(fast[:64], *want, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 130, 1024), (64, 300, 5120)])
+@pytest.mark.parametrize("binades", [10, 17, 20, 24, 28])
+def test_elements_far_below_the_row_s_largest(backend, m, n, k, binades):
+    """Weights that are zero on a row's largest elements: the output comes from the others alone, 2^-binades as
+    large, and keeps their precision."""
+    g = synth.rng(6400 + binades)
+    codes, scales = synth.fp8_weights(g, n, k)
+    a = synth.activations_f32(g, m, k)
+    largest = np.arange(0, k, 16)
+    a = np.clip(a, -4.0, 4.0)
+    a[:, largest] = 4.0 * np.sign(a[:, largest] + np.float32(0.5))
+    rest = np.setdiff1d(np.arange(k), largest)
+    small = a[:, rest]
+    a[:, rest] = np.sign(small) * np.clip(np.abs(small), 1.0, 4.0) * np.float32(2.0 ** -binades)
+    codes = codes.reshape(n, k).copy()
+    codes[:, largest] = 0
+    codes = codes.reshape(-1)
+    assert within(fp8_gemm(backend, a, codes, scales, m, n, k), *exact(a, codes, scales, n, k), k)
