@@ -56,6 +56,16 @@ bool method(PyObject* owner, PyObject* name, uint64_t* out) {
   return ok;
 }
 
+// The elements that owner.name has now, as a new tuple: what the loops over them call may run Python code, and that
+// (or another thread meanwhile) may change the list.
+PyObject* snapshot(PyObject* owner, PyObject* name) {
+  PyObject* list = PyObject_GetAttr(owner, name);
+  if (list == nullptr) return nullptr;
+  PyObject* items = PySequence_Tuple(list);
+  Py_DECREF(list);
+  return items;
+}
+
 PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t count) {
   if (count != 4) {
     PyErr_SetString(PyExc_TypeError, "launch(entry, kernel, launch, stream)");
@@ -74,36 +84,23 @@ PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t count) {
   void* handles[QMM_MAX_BOUND_BUFFERS];
   size_t sizes[QMM_MAX_BOUND_BUFFERS];
   uint64_t scalars[QMM_MAX_SCALARS];
-  PyObject* list = PyObject_GetAttr(args[2], s_buffers);
-  if (list == nullptr) return nullptr;
-  PyObject* items = PySequence_Fast(list, "buffers must be a sequence");
-  Py_DECREF(list);
+  PyObject* items = snapshot(args[2], s_buffers);
   if (items == nullptr) return nullptr;
-  const Py_ssize_t nbuffers = PySequence_Fast_GET_SIZE(items);
+  const Py_ssize_t nbuffers = PyTuple_GET_SIZE(items);
   bool ok = true;
   for (Py_ssize_t i = 0; ok && i < nbuffers && i < QMM_MAX_BOUND_BUFFERS; ++i) {
-    PyObject* buffer = PySequence_Fast_GET_ITEM(items, i);
-    Py_INCREF(buffer);
+    PyObject* buffer = PyTuple_GET_ITEM(items, i);
     ok = method(buffer, s_handle, &v);
     handles[i] = reinterpret_cast<void*>(v);
     ok = ok && method(buffer, s_size, &v);
     sizes[i] = static_cast<size_t>(v);
-    Py_DECREF(buffer);
   }
   Py_DECREF(items);
   if (!ok) return nullptr;
-  list = PyObject_GetAttr(args[2], s_scalars);
-  if (list == nullptr) return nullptr;
-  items = PySequence_Fast(list, "scalars must be a sequence");
-  Py_DECREF(list);
+  items = snapshot(args[2], s_scalars);
   if (items == nullptr) return nullptr;
-  const Py_ssize_t nscalars = PySequence_Fast_GET_SIZE(items);
-  for (Py_ssize_t i = 0; ok && i < nscalars && i < QMM_MAX_SCALARS; ++i) {
-    PyObject* scalar = PySequence_Fast_GET_ITEM(items, i);
-    Py_INCREF(scalar);
-    ok = whole(scalar, &scalars[i]);
-    Py_DECREF(scalar);
-  }
+  const Py_ssize_t nscalars = PyTuple_GET_SIZE(items);
+  for (Py_ssize_t i = 0; ok && i < nscalars && i < QMM_MAX_SCALARS; ++i) ok = whole(PyTuple_GET_ITEM(items, i), &scalars[i]);
   Py_DECREF(items);
   if (!ok) return nullptr;
   qmm_status status;
