@@ -148,13 +148,35 @@ class KernelLaunch:
     scalars: list = field(default_factory=list)
 
 
+_ENTRY = C.CFUNCTYPE(C.c_int32, C.c_size_t, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32), C.POINTER(C.c_void_p),
+                     C.POINTER(C.c_size_t), C.c_size_t, C.POINTER(C.c_uint64), C.c_size_t, C.c_void_p)
+
+
+def _launch_ctypes(entry: int, kernel: int, launch: KernelLaunch, stream: int) -> int:
+    """``_native.launch`` over ctypes, 2.4 us a launch slower: for an interpreter that the extension
+    was not built for (``make -C tessera_amd/csrc PYTHON=...`` builds it)."""
+    mask = 0xFFFFFFFFFFFFFFFF
+    pairs = [((b.Handle() or 0) & mask, (b.Size() or 0) & mask) for b in tuple(launch.buffers)]
+    scalars = [int(s) & mask for s in tuple(launch.scalars)]
+    grid = (C.c_uint32 * 3)(*[int(v) & 0xFFFFFFFF for v in (launch.grid_x, launch.grid_y, launch.grid_z)])
+    block = (C.c_uint32 * 3)(*[int(v) & 0xFFFFFFFF for v in (launch.block_x, launch.block_y, launch.block_z)])
+    nb, ns = len(pairs), len(scalars)
+    handles = (C.c_void_p * max(nb, 1))(*[h for h, _ in pairs])
+    sizes = (C.c_size_t * max(nb, 1))(*[s for _, s in pairs])
+    return _ENTRY(entry)(kernel, grid, block, handles, sizes, nb, (C.c_uint64 * max(ns, 1))(*scalars), ns, stream)
+
+
+try:
+    from ._native import launch as _launch_arrays   # built beside the kernel library (csrc/Makefile)
+except ImportError:
+    _launch_arrays = _launch_ctypes
+
+
 class Backend:
     """The MI355X backend: ``Name() == "mi355x"``; one instance per process."""
 
     def __init__(self, lib_path: str = LIB_PATH, stream: int = 0):
         self._lib = load_library(lib_path)
-        from . import _native   # built beside the kernel library (csrc/Makefile)
-        self._launch = _native.launch
         self._entry = C.cast(self._lib.qmm_launch, C.c_void_p).value
         self._entry_static = C.cast(self._lib.qmm_launch_static, C.c_void_p).value
         self._device_index = 0
@@ -248,8 +270,8 @@ class Backend:
         """``no_alloc=True`` goes through ``qmm_launch_static`` (not in the reference): the same
         launch with every kernel's scratch taken from the library's static device array, for
         callers that may not allocate device memory."""
-        code = self._launch(self._entry_static if no_alloc else self._entry, kernel.Handle(), launch,
-                            self._stream.value or 0)
+        code = _launch_arrays(self._entry_static if no_alloc else self._entry, kernel.Handle(), launch,
+                              self._stream.value or 0)
         if code != 0:
             self._check(code, f"LaunchKernel({kernel.Id()})")
 

@@ -1,18 +1,21 @@
 """The Python side of a launch (tessera_amd/host/pylaunch.cpp): what arrives at the C entry point.  The entry here
 is a callback, so no device and no library call is needed."""
 import ctypes
+import os
+import subprocess
+import sys
+import sysconfig
 
 import numpy as np
 import pytest
 
-from tessera_amd import KernelLaunch
+from tessera_amd import KernelLaunch, backend as backend_module
 
-native = pytest.importorskip("tessera_amd._native")
-
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ENTRY = ctypes.CFUNCTYPE(ctypes.c_int32, ctypes.c_size_t, ctypes.POINTER(ctypes.c_uint32), ctypes.POINTER(ctypes.c_uint32),
                          ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_size_t), ctypes.c_size_t,
                          ctypes.POINTER(ctypes.c_uint64), ctypes.c_size_t, ctypes.c_void_p)
-LAUNCHES = [native.launch]
+LAUNCHES = [backend_module._launch_arrays, backend_module._launch_ctypes]   # (the first is the extension's, see below)
 
 
 class FakeBuffer:
@@ -79,3 +82,22 @@ def test_errors_of_the_arguments_are_raised(launch):
     for bad in (KernelLaunch(buffers=[object()]), KernelLaunch(scalars=["x"]), KernelLaunch(scalars=5), KernelLaunch(grid_x=None)):
         with pytest.raises((AttributeError, ValueError, TypeError)):
             arrived(launch, 1, bad, 0)
+
+
+def test_extension_is_built_for_this_interpreter():
+    """Its file carries the interpreter's tag, so that no other loads it."""
+    from tessera_amd import _native
+    assert backend_module._launch_arrays is _native.launch
+    assert _native.__file__.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def test_launches_without_the_extension():
+    """An interpreter that the extension was not built for still launches, through ctypes."""
+    program = ("import sys; sys.modules['tessera_amd._native'] = None\n"
+               "import tessera_amd; from tessera_amd import backend as b\n"
+               "assert b._launch_arrays is b._launch_ctypes\n"
+               "be = tessera_amd.Backend(); k = be.LoadKernel('gemm_q4k')\n"
+               "try:\n    be.LaunchKernel(k, tessera_amd.KernelLaunch(buffers=[be.WrapBuffer(0x1000, 1 << 20)] * 17, scalars=[1, 1, 256]))\n"
+               "except tessera_amd.StatusError as e:\n    assert e.code == tessera_amd.StatusCode.InvalidArgument; print('refused')\n")
+    out = subprocess.run([sys.executable, "-c", program], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert out.stdout.strip() == "refused", out.stderr
