@@ -548,25 +548,35 @@ __global__ __launch_bounds__(WMAX * 64) void kquant_rows_stream_kernel(KqStreamA
       const uint32_t nn = o & 15u, r = (o >> 4) % (4u * kQuads), ti = o / (64u * kQuads);
       const uint32_t row = row0 + (g0 + ti) * 16u + nn;
       if (r >= p.m || row >= p.n) continue;
-      float sum = 0.0f;
-      for (uint32_t wv = 0; wv < cols; ++wv) sum += table[((ti * cols + wv) * (4u * kQuads) + r) * 16u + nn];   // wavefront order
-      out[static_cast<size_t>(r) * p.ld + row] = sum;
+      float sums[4] = {0.0f, 0.0f, 0.0f, 0.0f};      // every fourth wavefront's: short sums round less
+      for (uint32_t w0 = 0; w0 < cols; w0 += 4u) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+          if (w0 + i < cols) sums[i] += table[((ti * cols + w0 + i) * (4u * kQuads) + r) * 16u + nn];
+        }
+      }
+      out[static_cast<size_t>(r) * p.ld + row] = (sums[0] + sums[1]) + (sums[2] + sums[3]);
     }
     if (g0 + p.tiles_per_sync < tiles) lds_barrier();      // the table is written again
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct load may outlive its workgroup
 }
 
-// The parts' sums of `cols` columns in part order: c[r][col] = sum over parts of part[.][r][col].
+// The parts' sums of `cols` columns: c[r][col] = sum over parts of part[.][r][col], every fourth part's apart.
 __global__ __launch_bounds__(256) void kq_reduce_kernel(const float* __restrict__ part, float* __restrict__ c, uint32_t cols,
                                                         uint32_t m, uint32_t parts, size_t ldc) {
   const uint32_t col = blockIdx.x * 256u + threadIdx.x, r = blockIdx.y;
   if (col >= cols) return;
   const size_t region = static_cast<size_t>(m) * cols;
   const float* src = part + static_cast<size_t>(r) * cols + col;
-  float sum = 0.0f;
-  for (uint32_t i = 0; i < parts; ++i) sum += src[i * region];
-  c[r * ldc + col] = sum;
+  float sums[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (uint32_t i0 = 0; i0 < parts; i0 += 4u) {
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) {
+      if (i0 + i < parts) sums[i] += src[(i0 + i) * region];
+    }
+  }
+  c[r * ldc + col] = (sums[0] + sums[1]) + (sums[2] + sums[3]);
 }
 
 // Most wavefronts of a streaming workgroup: three a SIMD while the operands of NA sets leave the registers for it.

@@ -228,3 +228,25 @@ def test_streamed_rows_in_ranges_of_weight_rows(backend):
     ref = oracle.gemm_q6k(a, rows.reshape(-1), m, distinct, k, threads=True)
     got = gemm(backend, "gemm_q6k", a, w, m, n, k)
     assert rms_err(got, ref[:, np.arange(n) % distinct]) < 2e-4
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [("q6k", 8, 1024, 17408), ("q6k", 16, 512, 8704), ("q5k", 8, 1024, 17408)])
+def test_streamed_sums_round_no_more_than_the_other_form_s(backend, fmt, m, n, k):
+    """The same integer sums, added over the block columns and K parts in fp32: against float64 no further off than
+    the form that a stream without scratch runs, which is the per-thread stream (handle 2); 3 % for the sample."""
+    make, _, deq, _ = FORMATS[fmt]
+    errors = {0: [], 2: []}
+    try:
+        for seed in range(4):
+            g = synth.rng(8000 + m + seed)
+            w, a = make(g, n, k), synth.activations_f32(g, m, k)
+            want = a.astype(np.float64) @ deq(w).reshape(n, k).astype(np.float64).T
+            for stream in errors:
+                backend.SetStream(stream)
+                got = gemm(backend, f"gemm_{fmt}_batched", a, w, m, n, k)
+                errors[stream].append(np.linalg.norm(got - want) / np.linalg.norm(want))
+    finally:
+        backend.SetStream(0)
+    streamed, plain = (np.sqrt(np.mean(np.square(e))) for e in errors.values())
+    print(fmt, m, n, k, streamed, plain)
+    assert streamed <= 1.03 * plain, (streamed, plain)
