@@ -28,9 +28,9 @@
  *   - streams: launches that use the decode scratch or the workspace share it, so the caller orders
  *     them (one stream, or events).  Every other launch is independent of launches on other streams;
  *     "gemm_fp8" from 17 rows and "gemm_q5k*" / "gemm_q6k*" with 2..16 rows, which also hand
- *     intermediate results from one kernel to the next, keep them in blocks of their own: 32 MB for
- *     the eager launches of each stream, and what they need for each capture and stream that records
- *     them.  Blocks come out of the 256 MB that qmm_init reserves, then out of slabs of 128 MB, 2 GB in
+ *     intermediate results from one kernel to the next, keep them in blocks of their own: 16 MB for
+ *     the eager launches of each stream (128 MB more where a "gemm_fp8" call does not fit), and what
+ *     they need for each capture and stream that records them.  Blocks come out of the 256 MB that qmm_init reserves, then out of slabs of 128 MB, 2 GB in
  *     all; while a caller's workspace is set no slab is allocated.  They are not given back (a graph may
  *     still use them), and a stream handle's block passes to the next stream with that handle: let a
  *     stream's launches finish before it is destroyed.  A launch that gets no block, or is made on

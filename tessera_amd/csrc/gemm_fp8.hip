@@ -312,21 +312,21 @@ size_t terms_bytes(uint64_t m, uint64_t k) {
 }
 
 // Rows of one go: all where their terms fit the scratch, else the multiple of 64 (fewer where not even 64 fit)
-// with the smallest sum of estimates.  2048 x 6144 x 5120, whose terms take 42 MB, goes as two times 1024 rows,
-// as many rounds of tiles as in one go.
-constexpr size_t kScratch = gemm_fp8_f16_scratch_limit;
-uint32_t fp8_rows(uint32_t m, uint32_t n, uint32_t k) {
-  if (terms_bytes(m, k) <= kScratch) return m;
-  uint32_t most = static_cast<uint32_t>((kScratch - 256) / (static_cast<size_t>(k) * 4 + 4));
+// with the smallest sum of estimates.  The limit of 128 MB costs nothing up to 8192 rows; with 32 MB 300 x 5120 x
+// 17408, whose terms take 21 MB, has no room for the sums of K parts (162 us, without a limit 137), with 64 MB 512
+// rows have room for some of them only (220, without 201).
+uint32_t fp8_rows(uint32_t m, uint32_t n, uint32_t k, size_t limit) {
+  if (terms_bytes(m, k) <= limit) return m;
+  uint32_t most = static_cast<uint32_t>((limit - 256) / (static_cast<size_t>(k) * 4 + 4));
   if (most < 64u) return most;
   most = most / 64u * 64u;
   uint32_t best = most;
   float best_us = 1e30f;
   for (uint32_t rows = most; rows >= 64u && rows * 2u >= most; rows -= 64u) {
     float each = 0.0f, last = 0.0f;
-    fp8_plan(rows, n, k, kScratch - terms_bytes(rows, k), &each);
+    fp8_plan(rows, n, k, limit - terms_bytes(rows, k), &each);
     const uint32_t left = m % rows;
-    if (left != 0u) fp8_plan(left, n, k, kScratch - terms_bytes(left, k), &last);
+    if (left != 0u) fp8_plan(left, n, k, limit - terms_bytes(left, k), &last);
     const float us = static_cast<float>(m / rows) * each + last;
     if (us < best_us) best_us = us, best = rows;
   }
@@ -334,10 +334,10 @@ uint32_t fp8_rows(uint32_t m, uint32_t n, uint32_t k) {
 }
 
 // One go of m rows (their terms fit the scratch): the terms, the product, the parts' sums.
-hipError_t launch_rows(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch, uint32_t m, uint32_t n,
-                       uint32_t k, hipStream_t stream) {
+hipError_t launch_rows(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch, size_t limit, uint32_t m,
+                       uint32_t n, uint32_t k, hipStream_t stream) {
   float us;
-  const Fp8Plan pl = fp8_plan(m, n, k, kScratch - terms_bytes(m, k), &us);
+  const Fp8Plan pl = fp8_plan(m, n, k, limit - terms_bytes(m, k), &us);
   _Float16* a16 = static_cast<_Float16*>(scratch);
   const size_t plane = static_cast<size_t>(m) * k;
   float* a_scale = reinterpret_cast<float*>(a16 + 2 * plane);
@@ -372,24 +372,24 @@ bool gemm_fp8_f16_supported(uint64_t m, uint64_t n, uint64_t k) {
   return m >= 17 && k % 64 == 0 && k <= (1u << 20) && n <= (1u << 30) && m <= 65535u && m * n < (1ull << 40);
 }
 
-size_t gemm_fp8_f16_scratch_bytes(uint64_t m, uint64_t n, uint64_t k) {
-  const uint32_t rows = fp8_rows(static_cast<uint32_t>(m), static_cast<uint32_t>(n), static_cast<uint32_t>(k));
+size_t gemm_fp8_f16_scratch_bytes(uint64_t m, uint64_t n, uint64_t k, size_t limit) {
+  const uint32_t rows = fp8_rows(static_cast<uint32_t>(m), static_cast<uint32_t>(n), static_cast<uint32_t>(k), limit);
   size_t most = 0;
   for (const uint32_t part : {rows, static_cast<uint32_t>(m % rows)}) {
     if (part == 0u) continue;
     float us;
-    const Fp8Plan pl = fp8_plan(part, static_cast<uint32_t>(n), static_cast<uint32_t>(k), kScratch - terms_bytes(part, k), &us);
+    const Fp8Plan pl = fp8_plan(part, static_cast<uint32_t>(n), static_cast<uint32_t>(k), limit - terms_bytes(part, k), &us);
     const size_t bytes = terms_bytes(part, k) + (pl.parts > 1 ? static_cast<size_t>(pl.parts) * part * n * 4 : 0);
     most = bytes > most ? bytes : most;
   }
   return most;
 }
 
-hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch, uint32_t m,
-                               uint32_t n, uint32_t k, hipStream_t stream) {
-  const uint32_t rows = fp8_rows(m, n, k);
+hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch, size_t limit,
+                               uint32_t m, uint32_t n, uint32_t k, hipStream_t stream) {
+  const uint32_t rows = fp8_rows(m, n, k, limit);
   for (uint32_t r = 0; r < m; r += rows) {
-    const hipError_t e = launch_rows(a + static_cast<size_t>(r) * k, w, w_scale, c + static_cast<size_t>(r) * n, scratch,
+    const hipError_t e = launch_rows(a + static_cast<size_t>(r) * k, w, w_scale, c + static_cast<size_t>(r) * n, scratch, limit,
                                      m - r < rows ? m - r : rows, n, k, stream);
     if (e != hipSuccess) return e;
   }

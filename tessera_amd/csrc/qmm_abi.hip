@@ -212,8 +212,7 @@ class StreamBlock {
   qmm::ScratchBlock* block_ = nullptr;
   void* ptr_ = nullptr;
 };
-static_assert(qmm::gemm_fp8_f16_scratch_limit <= qmm::StreamScratch::kBlockBytes &&
-              qmm::gemm_fp8_f16_scratch_limit <= kStaticScratchBytes && kDecodeScratchBytes <= qmm::StreamScratch::kBlockBytes);
+static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock);
 
 // Q4_K regimes by activation rows.  One row and small matrices: the VALU GEMV.  2..16 rows of a
 // matrix with at least kQ4KFewRowsMinWeights weights: the exact few-row MFMA kernels (weights read
@@ -1117,11 +1116,12 @@ qmm_status run_gemm_fp8(const LaunchCtx& c) {
   // stream's own scratch block, as many rows at a time as fit it: the same kernels and bits whatever ran before,
   // whatever workspace is set and under capture.  A stream without a block runs the multiply-add passes below.
   if (m >= kFp8GemmMinRows && qmm::gemm_fp8_f16_supported(m, n, k)) {
-    const StreamBlock block(c, qmm::gemm_fp8_f16_scratch_bytes(m, n, k));
+    const size_t limit = c.no_alloc ? kStaticScratchBytes : qmm::StreamScratch::kBlockBytes;
+    const StreamBlock block(c, qmm::gemm_fp8_f16_scratch_bytes(m, n, k, limit));
     if (block.get() != nullptr) {
       return map_hip(qmm::launch_fp8_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<const float>(2),
-                                              c.ptr<float>(3), block.get(), static_cast<uint32_t>(m), static_cast<uint32_t>(n),
-                                              static_cast<uint32_t>(k), c.stream));
+                                              c.ptr<float>(3), block.get(), limit, static_cast<uint32_t>(m),
+                                              static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
     }
   }
   return map_hip(qmm::launch_fp8_gemv(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<const float>(2),

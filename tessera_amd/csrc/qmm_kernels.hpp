@@ -109,11 +109,10 @@ hipError_t gemm_fp8_f32_rows_prepare();
 hipError_t launch_fp8_f32_rows(const float* a, const uint8_t* w, const float* wscale, float* c, void* workspace,
                                uint32_t m, uint32_t n, uint32_t k, bool block_scales, hipStream_t stream);
 // "gemm_fp8" from 17 rows up (gemm_fp8.hip): fp16 weights on the fly against two fp16 terms of each row, as many
-// rows at a time as gemm_fp8_f16_scratch_limit bytes of scratch hold.
-constexpr size_t gemm_fp8_f16_scratch_limit = size_t{32} << 20;
+// rows at a time as `limit` bytes of scratch hold (32 MB or more); gemm_fp8_f16_scratch_bytes: what it takes of them.
 bool gemm_fp8_f16_supported(uint64_t m, uint64_t n, uint64_t k);
-size_t gemm_fp8_f16_scratch_bytes(uint64_t m, uint64_t n, uint64_t k);
-hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch,
+size_t gemm_fp8_f16_scratch_bytes(uint64_t m, uint64_t n, uint64_t k, size_t limit);
+hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch, size_t limit,
                                uint32_t m, uint32_t n, uint32_t k, hipStream_t stream);
 size_t gemm_mxfp4_f32_workspace_bytes(uint64_t m, uint64_t k);
 hipError_t launch_mxfp4_f32_gemm(const float* a, const uint8_t* w, float* c, void* workspace, uint32_t m,

@@ -25,7 +25,9 @@ struct ScratchBlock {
 
 class StreamScratch {
  public:
-  static constexpr size_t kBlockBytes = size_t{32} << 20;     // a stream's eager block; no call asks for more
+  // A stream's eager blocks: one of 16 MB, which all few-row calls fit, and one of 128 MB for what does not fit it.
+  // No call asks for more.
+  static constexpr size_t kSmallBlock = size_t{16} << 20, kBlockBytes = size_t{128} << 20;
   static constexpr size_t kFirstSlab = size_t{256} << 20, kSlab = size_t{128} << 20, kMaxBytes = size_t{2} << 30;
   static constexpr size_t kGrain = size_t{512} << 10;         // a capture's block is a multiple of this
 
@@ -40,20 +42,21 @@ class StreamScratch {
       if (b.capture == capture && b.stream == stream && b.bytes >= bytes) return &b;
     }
     if (count_ == kMaxBlocks) return nullptr;
-    const size_t size = capture == 0 ? kBlockBytes : (bytes + kGrain - 1) / kGrain * kGrain;
-    if (left_ < size) {
+    const size_t size = capture != 0 ? (bytes + kGrain - 1) / kGrain * kGrain : bytes <= kSmallBlock ? kSmallBlock : kBlockBytes;
+    unsigned char* from = next_;
+    if (left_ >= size) {
+      next_ += size;
+      left_ -= size;
+    } else {
       const size_t slab = total_ == 0 ? kFirstSlab : kSlab;
       if (total_ + slab > kMaxBytes) return nullptr;
-      void* fresh = grow(slab);
-      if (fresh == nullptr) return nullptr;
-      next_ = static_cast<unsigned char*>(fresh);
-      left_ = slab;
+      from = static_cast<unsigned char*>(grow(slab));
+      if (from == nullptr) return nullptr;
       total_ += slab;
+      if (slab - size > left_) next_ = from + size, left_ = slab - size;   // the larger rest serves the next owners
     }
     ScratchBlock& b = blocks_[count_++];
-    b.capture = capture, b.stream = stream, b.ptr = next_, b.bytes = size;
-    next_ += size;
-    left_ -= size;
+    b.capture = capture, b.stream = stream, b.ptr = from, b.bytes = size;
     return &b;
   }
 
@@ -71,6 +74,7 @@ class StreamScratch {
 
  private:
   static constexpr size_t kMaxBlocks = 4096;
+  static_assert(kBlockBytes <= kSlab && kSlab <= kFirstSlab);
   std::mutex mutex_;
   ScratchBlock blocks_[kMaxBlocks];
   size_t count_ = 0;

@@ -37,9 +37,11 @@ int main() {
   CHECK(s.reserve(grow) && taken == StreamScratch::kFirstSlab && s.reserve(grow) && taken == StreamScratch::kFirstSlab);
   ScratchBlock* a = s.find(0, stream(0), 5 * MB, grow);            // the null stream is an owner like any other
   ScratchBlock* b = s.find(0, stream(1), MB, grow);
-  CHECK(a && b && a != b && a->bytes == StreamScratch::kBlockBytes);
-  CHECK(s.find(0, stream(0), 32 * MB, grow) == a && s.find(0, stream(1), 1, grow) == b);
-  CHECK(s.find(0, stream(0), 32 * MB + 1, grow) == nullptr);
+  CHECK(a && b && a != b && a->bytes == StreamScratch::kSmallBlock);
+  CHECK(s.find(0, stream(0), 16 * MB, grow) == a && s.find(0, stream(1), 1, grow) == b);
+  ScratchBlock* large = s.find(0, stream(0), 16 * MB + 1, grow);   // besides the small one
+  CHECK(large && large != a && large->bytes == StreamScratch::kBlockBytes && s.find(0, stream(0), 128 * MB, grow) == large);
+  CHECK(s.find(0, stream(0), 128 * MB + 1, grow) == nullptr);
   // captures: own blocks, also on a stream that has an eager one; a larger need, another block
   ScratchBlock* c = s.find(7, stream(1), 3 * MB, grow);
   ScratchBlock* d = s.find(7, stream(2), 3 * MB, grow);
@@ -47,7 +49,7 @@ int main() {
   CHECK(c && d && e && s.find(7, stream(1), 2 * MB, grow) == c);
   ScratchBlock* f = s.find(7, stream(1), 4 * MB, grow);
   CHECK(f && f != c && s.find(7, stream(1), 4 * MB, grow) == f);
-  std::vector<ScratchBlock*> all{a, b, c, d, e, f};
+  std::vector<ScratchBlock*> all{a, b, large, c, d, e, f};
   // a caller's workspace is set: what was reserved is still given out, nothing is allocated
   closed = true;
   for (uintptr_t i = 3;; ++i) {
@@ -58,6 +60,10 @@ int main() {
   }
   CHECK(taken == StreamScratch::kFirstSlab && s.find(0, stream(1), MB, grow) == b);
   closed = false;
+  // a block that needs a slab of its own leaves the rest of the last one to others
+  ScratchBlock* whole = s.find(0, stream(900), 100 * MB, grow);
+  CHECK(whole && taken == StreamScratch::kFirstSlab + StreamScratch::kSlab);
+  all.push_back(whole);
   // and without one no more than the bound, however many owners ask
   for (uintptr_t i = 1000; i < 20000; ++i) {
     ScratchBlock* more = i % 2 ? s.find(0, stream(i), MB, grow) : s.find(i, stream(5), 700000, grow);
