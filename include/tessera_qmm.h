@@ -154,7 +154,14 @@ const char* qmm_kernel_name(size_t index);
  *   - "gemm_fp8" and "gemm_fp8_block" likewise: 2..16 rows of a matrix of 16 M weights or more with k a
  *     multiple of 512 run on the matrix cores (E4M3 weights as stored, activations to 16 significant
  *     bits, the matrix core's own accumulation: within 2e-4 of the rms output of the reference's fp32
- *     loop, 2e-3 with x20 outlier channels); other shapes on the vector unit in fp32.
+ *     loop, 2e-3 with x20 outlier channels).  "gemm_fp8" from 17 rows with k a multiple of 64 carries an
+ *     activation to 2^-23 of itself, down to 2^-28 of its row's largest (below, to 2^-50 of that largest), on
+ *     the matrix cores with sums kept short: no further from float64 than the fp32 loop.  Other shapes run
+ *     on the vector unit in fp32.
+ *   - the attention ids carry a query element to 2^-23 of itself down to 2^-28 of its head's largest, and
+ *     softmax weights likewise (over a quantized cache a weight times its value's scale, down to 2^-18 of
+ *     the row's largest); keys and values enter as the cache holds them, scores and sums are fp32.  Over
+ *     an fp32 cache everything is fp32.
  *   - "mfma_probe": buffer Out (workgroups * 256 floats); scalars kind (0 fp16 32x32x16, 1 scaled
  *     fp8 x fp4 32x32x64, 2 int8 16x16x64), random (0 constant operands, 1 hashed), iterations,
  *     workgroups.  "read_probe": a plain read of a buffer.  Measurement ids: the matrix-core and the

@@ -90,6 +90,17 @@ def test_mxfp4_fp32_rows(backend, name, m):
     assert np.array_equal(want, got), (name, m, need)
 
 
+# 1100 rows: their terms take 18 MB, more than the library's other fixed scratch
+@pytest.mark.parametrize("m,n,k", [(1, 520, 1024), (16, 4100, 4096), (17, 520, 1024), (300, 520, 1024), (1100, 130, 4096)])
+def test_fp8_rows_take_no_workspace(backend, m, n, k):
+    g = synth.rng(8350 + m)
+    codes, scales = synth.fp8_weights(g, n, k)
+    a = synth.activations_f32(g, m, k)
+    make = lambda: [backend.Upload(a), backend.Upload(codes), backend.Upload(scales), backend.AllocateBuffer(4 * m * n)]
+    want, got, need = outputs_with_exact_workspace(backend, "gemm_fp8", [m, n, k], make, 3)
+    assert need == 0 and np.array_equal(want, got), (m, need)
+
+
 @pytest.mark.parametrize("m", [1, 4, 32, 33, 200])
 @pytest.mark.parametrize("wperm", [0, 1])
 def test_w4a8_with_and_without_the_permuted_weights(backend, m, wperm):

@@ -17,7 +17,9 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # file -> kernels (substring of the mangled name) that must not use scratch memory
 NO_SCRATCH = {
     "gemv_q4k_rows16.hip": ["q4k_rows16_kernel"],
-    "gemv_kquant_rows.hip": ["kquant_rows_kernel"],
+    "gemv_kquant_rows.hip": ["kquant_rows_kernel", "kquant_rows_stream_kernel"],
+    "gemm_fp8.hip": ["fp8_gemm_kernel"],
+    "attention.hip": ["attention_rows_kernel"],
     "gemv_q4k_i8.hip": ["q4k_i8_gemv_kernel"],
 }
 
