@@ -36,15 +36,7 @@ constexpr int kMaxTerms = 4;                // E4M3 terms an fp32 activation is 
 constexpr int kKS = 128;                    // K per step: one 32-bit word of E8M0 bytes per weight row
 constexpr int kDmaPerStage = 13;            // direct loads a wavefront issues per stage (8 A, 4 B, 1 scales)
 
-// Direct HBM -> LDS load: lane p's `bytes` at global `base + voff` land at LDS address
-// lds_addr + p * bytes (base and lds_addr wave-uniform).  Issued as inline assembly so
-// that the waits stay under this file's control: the kernel waits for exactly the stage
-// it is about to publish (vmcnt counts direct loads in order) and keeps two younger
-// stages in flight across its LDS reads.
-__device__ __forceinline__ void direct_load16(const void* base, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
-}
+// direct_load16 with four bytes a lane.
 __device__ __forceinline__ void direct_load4(const void* base, uint32_t voff, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");

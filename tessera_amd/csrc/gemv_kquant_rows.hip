@@ -403,11 +403,6 @@ struct KqStreamArgs {
   uint32_t m, n, nblk, parts, groups, tiles_per_wg, tiles_per_sync, ld;
 };
 
-__device__ __forceinline__ void kq_direct16(const void* base, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
-}
-
 // Sums over the lane groups (16 lanes each) of NA sets' values; register q of the result holds, in lane group g,
 // row 4 q + 2 (g & 1) + (g >> 1) of the pass.
 __device__ __forceinline__ float swap32_add(float a, float b) {
@@ -490,7 +485,7 @@ __global__ __launch_bounds__(WMAX * 64) void kquant_rows_stream_kernel(KqStreamA
         off = ((row_off + mis) & ~15u) + piece_off[i];
         off = off < end_off ? off : end_off;
       }
-      if (i + 1 < U::kLoads || 16u * U::kPieces % 64u == 0u || lane < 16u * U::kPieces % 64u) kq_direct16(base, off, dst + i * 1024u);
+      if (i + 1 < U::kLoads || 16u * U::kPieces % 64u == 0u || lane < 16u * U::kPieces % 64u) direct_load16(base, off, dst + i * 1024u);
     }
     ++issued;
     fill = fill + 1u == RING ? 0u : fill + 1u;

@@ -36,11 +36,6 @@ typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kSlots = 33;      // 32 weight dwords per lane and super-block + 1 slot of sub-block sums
 
-__device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
-}
-
 // Power of two that brings a row with largest magnitude `amax` to [256, 512).
 __device__ __forceinline__ float prep_scale(float amax) {
   const uint32_t e = (bit_cast<uint32_t>(amax) >> 23) & 0xFFu;
@@ -205,17 +200,17 @@ __global__ __launch_bounds__(64) void q4k_gemv_mfma_kernel(const uint8_t* __rest
 #pragma unroll
     for (int i = 0; i < kWDma; ++i) {
       if (i + 1 < kWDma || kWGran % 64u == 0) {
-        dma16(wb, w_src[i], stage + i * 1024u);
+        direct_load16(wb, w_src[i], stage + i * 1024u);
       } else if (lane < kWGran % 64u) {
-        dma16(wb, w_src[i], stage + i * 1024u);
+        direct_load16(wb, w_src[i], stage + i * 1024u);
       }
     }
 #pragma unroll
     for (int i = 0; i < kXDma; ++i) {
       if (i + 1 < kXDma || kXGran % 64u == 0) {
-        dma16(xb, x_src[i], stage + kWBytes + i * 1024u);
+        direct_load16(xb, x_src[i], stage + kWBytes + i * 1024u);
       } else if (lane < kXGran % 64u) {
-        dma16(xb, x_src[i], stage + kWBytes + i * 1024u);
+        direct_load16(xb, x_src[i], stage + kWBytes + i * 1024u);
       }
     }
   };
@@ -408,9 +403,9 @@ __global__ __launch_bounds__(64 * kResWaves) void q4k_rows_resident_kernel(
     for (int i = 0; i < kItemDma; ++i) {
       const uint32_t off = src_sbo[i] < lim ? src_full[i] : src_first[i];
       if (i + 1 < kItemDma) {
-        dma16(base, off, dst + i * 1024u);
+        direct_load16(base, off, dst + i * 1024u);
       } else if (lane < (kItemBytes / 16u) % 64u) {
-        dma16(base, off, dst + i * 1024u);
+        direct_load16(base, off, dst + i * 1024u);
       }
     }
   };

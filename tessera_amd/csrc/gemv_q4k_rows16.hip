@@ -73,12 +73,6 @@ struct R16Args {
   R16Part part[kMaxParts];
 };
 
-// 16 bytes from base + voff straight into LDS at lds_addr + 16 * lane (no register in between).
-__device__ __forceinline__ void r16_dma16(const void* base, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
-}
-
 template <int kCtrl, int kRowMask>
 __device__ __forceinline__ uint32_t dpp_umax16(uint32_t v) {
   const uint32_t moved = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRowMask, 0xF, false));
@@ -213,9 +207,9 @@ __global__ __launch_bounds__(768) void q4k_rows16_kernel(R16Args p) {
     for (int i = 0; i < kKL; ++i) {
       const uint32_t off = (piece_row[i] < last ? piece_row[i] : last) * row_bytes + piece_off[i];
       if (i + 1 < kKL) {
-        r16_dma16(base, off, dst + i * 1024u);
+        direct_load16(base, off, dst + i * 1024u);
       } else if (lane < kTile * 9u - 128u) {
-        r16_dma16(base, off, dst + i * 1024u);
+        direct_load16(base, off, dst + i * 1024u);
       }
     }
     ++issued;

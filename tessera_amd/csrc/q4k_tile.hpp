@@ -10,11 +10,6 @@
 namespace qmm {
 namespace {
 
-__device__ __forceinline__ void direct_load16(const void* base, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
-}
-
 // Largest |v| over a 256-thread workgroup (every thread returns it).
 __device__ __forceinline__ float block_amax(float v, float* red) {
   v = wave_max(v);

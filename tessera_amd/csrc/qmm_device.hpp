@@ -138,6 +138,15 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Direct HBM -> LDS load: lane p's 16 bytes at base + voff land at LDS address lds_addr + 16 p (base and
+// lds_addr wave-uniform; base + voff 16-byte aligned), with no register in between.  Inline assembly, so that
+// the waits stay with the kernel: it waits for exactly what it is about to read (vmcnt counts direct loads in
+// order) and keeps younger loads in flight.
+__device__ __forceinline__ void direct_load16(const void* base, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+
 __device__ __forceinline__ uint4 load_u4(const void* p) {
   return *reinterpret_cast<const uint4*>(p);
 }
