@@ -6,12 +6,13 @@
 // weights are converted in registers without loss; a row of A becomes two fp16 terms under a power of two that
 // brings its largest magnitude to [2^14, 2^15): hi = RN16(x / s), lo = RN16(2^11 (x / s - hi)), x / s = hi + 2^-11 lo.
 // That misses an element by at most 2^-23 of itself down to 2^-28 of the row's largest, and by 2^-50 of the
-// largest below.  Products of an 11-bit and a 4-bit significand are exact; v_mfma_f32_32x32x16_f16 adds them up, and its additions are what costs
-// precision: one chain of both terms over 5120 weights was measured at 6.2e-7 of the float64 result in the
-// 2-norm, against 1.2e-7 for the multiply-add kernel's short chains.  So an output has four sums: the second
-// term's products, 2^-11 as large, in one of their own, the first term's for 128 weights at a time, those of 1024,
-// and the total.  Measured 0.92e-7 (k = 1024) to 1.06e-7 (k = 5120), the
-// multiply-add kernel 0.95e-7 and 1.21e-7.
+// largest below.  Products of an 11-bit and a 4-bit significand are exact; v_mfma_f32_32x32x16_f16 adds them up,
+// and its additions are what costs precision: one chain of both terms over 5120 weights was measured at 6.2e-7 of
+// the float64 result in the 2-norm, against 1.2e-7 for the multiply-add kernel's short chains.  So an output has
+// four sums: the second term's products, worth 2^-11 each, in one of their own, the first term's for 128 weights
+// at a time, those of 1024, and the total.  Measured 0.91e-7 (k = 1024) to 1.22e-7 (k = 17408), the multiply-add
+// kernel 0.94e-7 and 1.48e-7; with eight columns of the activations 1000 times the others 1.11e-7 and 1.35e-7
+// against 0.92e-7 and 1.44e-7 (64 weights at a time: 1.06e-7, but 58.4 us instead of 56.2 at 300 x 6144 x 5120).
 // (The scaled 8-bit instruction would take the codes as they are but aligns an instruction's products to the
 // largest before it adds them: 1.5e-5.)
 //
@@ -21,10 +22,10 @@
 // long) and the codes (128 x 64 bytes) travel HBM -> LDS by direct loads into a ring of stages; a wavefront
 // converts the codes of its columns once per stage and uses them against both terms of all its rows.  Whatever
 // part of the chip one round of tiles leaves idle is filled by splitting K (fp8_plan); the partial sums are added
-// in part order by a last launch: no atomics, the same bits every time.  What bounds it: the matrix cores are
-// busy 51 % of the cycles of 300 x 6144 x 5120 (2 x 2 m n k fp16 flops in 44 us), LDS reads and the step's
-// barrier take the rest; a short stack of rows is bound by the weight stream.
-// 300 x 6144 x 5120: 1109 -> 61 us against 75 four-row passes of the multiply-add kernel; 17 rows 68 -> 16 us.
+// in part order by a last launch: no atomics, the same bits every time.  What bounds it: at 300 x 6144 x 5120 the
+// matrix cores are busy 37 % of the product's cycles, vector instructions issue in 30 % and a wavefront waits in
+// 23 %, and with one wavefront a SIMD none of these overlap; a short stack of rows is bound by the weight stream.
+// 300 x 6144 x 5120: 1108 -> 56 us against 75 four-row passes of the multiply-add kernel; 17 rows 68 -> 16 us.
 
 #include "q4k_tile.hpp"
 #include "qmm_kernels.hpp"

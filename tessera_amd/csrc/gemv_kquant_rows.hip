@@ -381,13 +381,14 @@ __global__ __launch_bounds__(WMAX * 64) void kquant_rows_kernel(KqArgs p) {
 // ---- the same sums with the weights streamed through LDS ------------------------------------------------------
 // A wavefront owns ONE 256-wide block column of its workgroup's K part, keeps the activations' operands for it in
 // registers from start to end, and walks the workgroup's 16-row tiles: the kernel above converts every block of K
-// for its four to five tiles, which with five rows takes as long as the tiles' sums.  A unit (16 rows x one block) comes by coalesced 16-byte direct loads into a private ring of LDS
-// slots, RING - 1 units ahead; a lane then reads the registers that the kernel above loads from memory with
-// 2-byte-aligned 8-byte accesses to sixteen rows at once.  Up to eight activation rows a pass in every format.
-// K parts leave their sums in a scratch buffer that a reduce launch adds in part order.  Bound by vector issue
-// (Q6_K, 5 rows: about 260 instructions a unit, three wavefronts a SIMD; eight wavefronts instead of twelve were
-// 41.6 us against 33.3 on 5120 x 17408, whose 73 MB take 14 us at the rate of a copy).  The rule that picks this
-// form and both sides' figures: kquant_rows_stream in qmm_abi.hip.
+// for its four to five tiles, which with five rows takes as long as the tiles' sums.  A unit (16 rows x one block)
+// comes by coalesced 16-byte direct loads into a private ring of LDS slots, RING - 1 units ahead; a lane then reads
+// the registers that the kernel above loads from memory with 2-byte-aligned 8-byte accesses to sixteen rows at once.
+// Up to eight activation rows a pass in every format.  K parts leave their sums in a scratch buffer that a reduce
+// launch adds up.  Bound by vector issue and LDS: Q6_K, 5 rows of 5120 x 17408, 30 us where its 73 MB take 14 at the
+// rate of a copy: vector instructions issue in 54 % of the cycles (335 a unit, the activations' conversion
+// included), LDS is busy in 64 %, the matrix cores in 12 %.  The rule that picks this form and both sides' figures:
+// kquant_rows_stream in qmm_abi.hip.
 template <class F>
 struct KqUnit {   // pieces of 16 bytes from the 16-byte boundary at or below the block's start
   static constexpr uint32_t kPieces = F::kBlock % 16u == 0u ? F::kBlock / 16u : F::kBlock / 16u + 1u;
@@ -518,7 +519,8 @@ __global__ __launch_bounds__(WMAX * 64) void kquant_rows_stream_kernel(KqStreamA
         row = ln < last ? ln : last;
         shift = (static_cast<uint32_t>(start) + row * row_bytes) & 15u;
         const uint32_t over = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p.w_end)) & 15u;
-        const uint8_t* block_end = reinterpret_cast<const uint8_t*>(start) + static_cast<size_t>(last < 15u ? last : 15u) * row_bytes + F::kBlock;
+        const uint8_t* block_end =
+            reinterpret_cast<const uint8_t*>(start) + static_cast<size_t>(last < 15u ? last : 15u) * row_bytes + F::kBlock;
         if (over != 0u && block_end == p.w_end) {     // the matrix's last block: its bytes past the last whole piece
           if (lane < over / 2u) {
             *reinterpret_cast<uint16_t*>(unit + last * U::kRow + (U::kPieces - 1u) * 16u + lane * 2u) =
