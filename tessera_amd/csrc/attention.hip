@@ -359,6 +359,16 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
       if constexpr (QUANT) s[e] *= ksv[e];
       all += s[e];
     }
+    if constexpr (QUANT) {
+      // A key with an infinite scale is NaN where its code is 0; its score is formed from the codes' sum, which is not.
+      float scale_most = ksv[0];
+#pragma unroll
+      for (int e = 1; e < 4 * HALVES; ++e) scale_most = fmaxf(scale_most, ksv[e]);
+      if (__any(scale_most == INFINITY)) {
+#pragma unroll
+        for (int e = 0; e < 4 * HALVES; ++e) s[e] = ksv[e] == INFINITY ? NAN : s[e];
+      }
+    }
     if (more) load_keys(j0 + NW * KEYS);
     if constexpr (KV == KvKind::F16) {
       if (__any(!(fabsf(all) < INFINITY))) {       // infinities among the keys
@@ -372,7 +382,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
     const bool past = j0 + KEYS - 1 > last;        // the range ends inside this tile
     if (past) {
 #pragma unroll
-      for (int e = 0; e < 4 * HALVES; ++e) s[e] = j0 + 16 * (e / 4) + 4 * g + e % 4 <= last ? s[e] : -INFINITY;
+      for (int e = 0; e < 4 * HALVES; ++e) {
+        const bool none = j0 + 16 * (e / 4) + 4 * g + e % 4 > last;
+        s[e] = none ? -INFINITY : s[e];
+        if constexpr (QUANT) vsv[e] = none ? 0.0f : vsv[e];
+      }
     }
 
     float most = s[0];
@@ -477,7 +491,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         float own = o[j + c][e];
-        if constexpr (KV == KvKind::F16) own = second ? finite_or_zero(own) : own;
+        if constexpr (!F32) own = second ? finite_or_zero(own) : own;
         own *= term_down;
         xs[c] = (F32 ? own : own + other_term(own)) * f;
       }

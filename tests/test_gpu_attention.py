@@ -319,3 +319,39 @@ def test_attention_more_workgroups_than_one_grid_of_wide_ones(backend):
     rows = [0, 1, m // 2, m - 1]
     want = expected("f16", q[rows].cpu().numpy(), k, v, None, None, len(rows), n, heads, heads, head_dim, n, 0)
     assert np.max(np.abs(out[rows].cpu().numpy() - want)) <= 2e-6 * max(1.0, np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("kind", ["q8", "q4", "fp8"])
+@pytest.mark.parametrize("head_dim", [64, 256, 36])
+@pytest.mark.parametrize("at", [5, 200, 299])
+def test_attention_infinite_scales(backend, kind, head_dim, at):
+    """A key row with an infinite scale holds NaN wherever its code is 0 (what the quantizer leaves of a row with an
+    infinity), and spoils the rows that see it, whatever the sign of the codes' score; a value row's makes the elements
+    of its codes infinite or, for code 0, NaN, and no others.  Key 299 is the last, whose row also stands in for the
+    keys past the end."""
+    m, n, heads, kv_heads = 2, 300, 6, 2
+    g = synth.rng(1950 + head_dim)
+    q = (0.1 * g.standard_normal((m, heads * head_dim))).astype(np.float32)
+    k, ks = cache(g, kind, n, kv_heads * head_dim)
+    v, vs = cache(g, kind, n, kv_heads * head_dim)
+    k, v = (np.asarray(x).reshape(n, -1).copy() for x in (k, v))
+    k[at], v[at] = 0, 0
+    for h in range(kv_heads):                      # one code other than 0 in each head
+        byte = h * head_dim // (2 if kind == "q4" else 1) + 4
+        k[at, byte] = 0xF1 if kind == "fp8" else 0x09 if kind == "q4" else 0x81
+        v[at, byte] = k[at, byte]
+    bad = ks.copy()
+    bad[at] = np.inf
+    last = np.arange(m) + n - m
+    got = attend(backend, kind, q, k, v, bad, vs, m, n, heads, kv_heads, head_dim, n - m, 0).reshape(m, heads, head_dim)
+    assert np.array_equal(np.isnan(got), np.broadcast_to((last >= at)[:, None, None], got.shape))
+    bad = vs.copy()
+    bad[at] = np.inf
+    with np.errstate(invalid="ignore"):
+        want = expected(kind, q, k, v, ks, bad, m, n, heads, kv_heads, head_dim, n - m, 0)
+    for split in (0, 3):
+        got = attend(backend, kind, q, k, v, ks, bad, m, n, heads, kv_heads, head_dim, n - m, 0, split=split)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), split
+        assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]), split
+        some = np.isfinite(want)
+        assert np.max(np.abs(got[some] - want[some]), initial=0.0) <= 4e-6, split
