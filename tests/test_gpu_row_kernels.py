@@ -46,7 +46,7 @@ def top_k_want(row, top_k):
 # a wavefront a row up to 256 and up to 512 columns, then a workgroup a row: less than a tile of 8192, one
 # tile, one column more, many tiles with a remainder.  Sorted rows and rows of few different values are the
 # ones whose candidates outgrow the list.
-@pytest.mark.parametrize("kind", ["normal", "rising", "falling", "ties", "equal", "infinite"])
+@pytest.mark.parametrize("kind", ["normal", "rising", "falling", "ties", "equal", "infinite", "nan"])
 @pytest.mark.parametrize("rows,vocab,top_k", [(1, 1, 1), (5, 64, 8), (3, 256, 32), (6, 257, 3), (2, 512, 32), (2, 513, 32), (3, 1000, 1),
                                               (2, 8192, 8), (1, 8193, 32), (2, 70001, 32), (1, 131072, 8), (1, 151936, 17)])
 def test_top_k_edges(backend, rows, vocab, top_k, kind):
@@ -62,6 +62,8 @@ def test_top_k_edges(backend, rows, vocab, top_k, kind):
     elif kind == "infinite":
         x[:, ::3] = -np.inf
         x[:, vocab // 2] = np.inf
+    elif kind == "nan":
+        x[:, ::5] = np.nan               # below everything
     dx = backend.Upload(x)
     di, dv = backend.Upload(np.full(rows * top_k, 0xFFFFFFFF, np.uint32)), backend.AllocateBuffer(4 * rows * top_k)
     if kind == "infinite" and np.isfinite(x[0]).sum() + 1 < top_k:
