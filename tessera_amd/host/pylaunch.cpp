@@ -56,15 +56,32 @@ bool method(PyObject* owner, PyObject* name, uint64_t* out) {
   return ok;
 }
 
-// The elements that owner.name has now, as a new tuple: what the loops over them call may run Python code, and that
-// (or another thread meanwhile) may change the list.
-PyObject* snapshot(PyObject* owner, PyObject* name) {
-  PyObject* list = PyObject_GetAttr(owner, name);
-  if (list == nullptr) return nullptr;
-  PyObject* items = PySequence_Tuple(list);
-  Py_DECREF(list);
-  return items;
-}
+// The elements that owner.name has now, up to N of them held, and their whole number: what is called on them may run
+// Python code, and that (or another thread meanwhile) may change the list.  (A tuple of them costs 25 ns more.)
+template <int N>
+struct Snapshot {
+  PyObject* item[N];
+  Py_ssize_t held = 0, count = -1;   // count < 0: a Python error is set
+
+  Snapshot(PyObject* owner, PyObject* name) {
+    PyObject* list = PyObject_GetAttr(owner, name);
+    if (list == nullptr) return;
+    PyObject* items = PySequence_Fast(list, "buffers and scalars must be sequences");
+    Py_DECREF(list);
+    if (items == nullptr) return;
+    count = PySequence_Fast_GET_SIZE(items);
+    for (; held < count && held < N; ++held) {
+      item[held] = PySequence_Fast_GET_ITEM(items, held);
+      Py_INCREF(item[held]);
+    }
+    Py_DECREF(items);
+  }
+  ~Snapshot() {
+    for (Py_ssize_t i = 0; i < held; ++i) Py_DECREF(item[i]);
+  }
+  Snapshot(const Snapshot&) = delete;
+  Snapshot& operator=(const Snapshot&) = delete;
+};
 
 PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t count) {
   if (count != 4) {
@@ -84,29 +101,23 @@ PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t count) {
   void* handles[QMM_MAX_BOUND_BUFFERS];
   size_t sizes[QMM_MAX_BOUND_BUFFERS];
   uint64_t scalars[QMM_MAX_SCALARS];
-  PyObject* items = snapshot(args[2], s_buffers);
-  if (items == nullptr) return nullptr;
-  const Py_ssize_t nbuffers = PyTuple_GET_SIZE(items);
-  bool ok = true;
-  for (Py_ssize_t i = 0; ok && i < nbuffers && i < QMM_MAX_BOUND_BUFFERS; ++i) {
-    PyObject* buffer = PyTuple_GET_ITEM(items, i);
-    ok = method(buffer, s_handle, &v);
+  const Snapshot<QMM_MAX_BOUND_BUFFERS> buffer(args[2], s_buffers);
+  if (buffer.count < 0) return nullptr;
+  for (Py_ssize_t i = 0; i < buffer.held; ++i) {
+    if (!method(buffer.item[i], s_handle, &v)) return nullptr;
     handles[i] = reinterpret_cast<void*>(v);
-    ok = ok && method(buffer, s_size, &v);
+    if (!method(buffer.item[i], s_size, &v)) return nullptr;
     sizes[i] = static_cast<size_t>(v);
   }
-  Py_DECREF(items);
-  if (!ok) return nullptr;
-  items = snapshot(args[2], s_scalars);
-  if (items == nullptr) return nullptr;
-  const Py_ssize_t nscalars = PyTuple_GET_SIZE(items);
-  for (Py_ssize_t i = 0; ok && i < nscalars && i < QMM_MAX_SCALARS; ++i) ok = whole(PyTuple_GET_ITEM(items, i), &scalars[i]);
-  Py_DECREF(items);
-  if (!ok) return nullptr;
+  const Snapshot<QMM_MAX_SCALARS> scalar(args[2], s_scalars);
+  if (scalar.count < 0) return nullptr;
+  for (Py_ssize_t i = 0; i < scalar.held; ++i) {
+    if (!whole(scalar.item[i], &scalars[i])) return nullptr;
+  }
   qmm_status status;
   Py_BEGIN_ALLOW_THREADS
-  status = reinterpret_cast<Entry>(entry)(static_cast<qmm_kernel>(kernel), grid, block, handles, sizes, static_cast<size_t>(nbuffers),
-                                          scalars, static_cast<size_t>(nscalars), reinterpret_cast<void*>(stream));
+  status = reinterpret_cast<Entry>(entry)(static_cast<qmm_kernel>(kernel), grid, block, handles, sizes, static_cast<size_t>(buffer.count),
+                                          scalars, static_cast<size_t>(scalar.count), reinterpret_cast<void*>(stream));
   Py_END_ALLOW_THREADS
   return PyLong_FromLong(status);
 }
