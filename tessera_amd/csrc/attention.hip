@@ -41,7 +41,7 @@ struct AttentionArgs {
   const float *k_scale, *v_scale;
   float* out;
   SplitOut part;
-  uint64_t n, q_base, row_base, window;
+  uint64_t rows, n, q_base, row_base, window;
   uint32_t heads, kv_heads, head_dim, causal;
 };
 
@@ -77,12 +77,12 @@ __device__ __forceinline__ bool key_chunk(const AttentionArgs& a, uint64_t s, ui
 //   key-major operand: no transposition through LDS.
 // The loads of a tile's keys are under way during the previous tile's softmax and values, its values'
 // during the scores.  Over an fp32 cache the same shape runs on v_mfma_f32_16x16x4_f32, tiles of 16 keys.
-// One row against 9301 int8 keys of 4 heads of 256 in 64 parts: 16 us (one element a load: 86 us).  With many
-// rows, each reading the cache through L2, vector issue bounds it: 512 rows against 2512 fp16 keys 441 us (6.4 ms),
-// vector instructions in 52 % of the cycles, the matrix cores in 8 %, one wavefront a SIMD at this head size.
+// One row against 9301 int8 keys of 4 heads of 256 in 64 parts: 16 us (one element a load: 86 us).
 template <int BYTES>
 __device__ __forceinline__ void load_run(const uint8_t* p, uint32_t (&r)[(BYTES + 3) / 4]) {
-  if constexpr (BYTES == 2) {
+  if constexpr (BYTES == 1) {
+    r[0] = *p;
+  } else if constexpr (BYTES == 2) {
     r[0] = *reinterpret_cast<const uint16_t*>(p);
   } else if constexpr (BYTES == 4) {
     r[0] = *reinterpret_cast<const uint32_t*>(p);
@@ -189,11 +189,35 @@ __device__ __forceinline__ float reference_score(float largest) { return largest
 // negative) second term says nothing that the first term's sum does not.
 __device__ __forceinline__ float finite_or_zero(float v) { return __builtin_isfinite(v) ? v : 0.0f; }
 
+// Query heads a workgroup takes at once, and what its wavefronts hand to the merge.
+template <KvKind KV>
+constexpr int rows_heads() { return KV == KvKind::F32 ? 16 : 8; }
 template <KvKind KV, int DP, int NW>
-__global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArgs a) {
+struct RowsShared {
+  float m[NW][rows_heads<KV>()], l[NW][rows_heads<KV>()], scale[rows_heads<KV>()];
+  alignas(16) float o[NW][rows_heads<KV>()][16][DP / 16 + 4];
+};
+
+// A part without keys, of heads head0 .. head0 + here - 1 of a row.
+template <int THREADS>
+__device__ __forceinline__ void empty_part(const AttentionArgs& a, uint64_t row, uint32_t head0, uint32_t here, uint64_t s_part) {
+  const uint32_t t = threadIdx.x, D = a.head_dim;
+  const uint64_t split = a.part.split;
+  for (uint32_t i = t; i < here * D; i += THREADS) a.part.pacc[((row * a.heads + head0 + i / D) * split + s_part) * D + i % D] = 0.0f;
+  if (t < here) {
+    const uint64_t at = (row * a.heads + head0 + t) * split + s_part;
+    a.part.pmax[at] = -1e30f, a.part.psum[at] = 0.0f;
+  }
+}
+
+// Heads head0 .. head0 + here - 1 (at most rows_heads, all of key head kv) of query row `row` over keys start .. last:
+// part s_part of the row, or all of it.
+template <KvKind KV, int DP, int NW>
+__device__ __forceinline__ void attend_row(const AttentionArgs& a, uint64_t row, uint32_t kv, uint32_t head0, uint32_t here,
+                                           uint64_t start, uint64_t last, uint64_t s_part, RowsShared<KV, DP, NW>& merge) {
   constexpr bool F32 = KV == KvKind::F32, QUANT = kv_quantized(KV);
   constexpr int BITS = kv_bits(KV);
-  constexpr int HEADS = F32 ? 16 : 8, KEYS = F32 ? 16 : 32;        // query heads a workgroup, keys a tile
+  constexpr int KEYS = F32 ? 16 : 32;                              // keys a tile
   constexpr int CE = F32 ? 4 : 128 / BITS < DP / 4 ? 128 / BITS : DP / 4;   // elements of a key a lane loads at once
   constexpr int RUNS = DP / (4 * CE);                              // such loads a key row
   constexpr int STEPS = F32 ? DP / 4 : DP / 32;                    // matrix instructions over head_dim
@@ -201,31 +225,10 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
   constexpr int VE = DP / 16;                                      // elements of a value row a lane holds
   constexpr int KW = CE * BITS / 32, VW = (VE * BITS + 31) / 32;   // dwords of those
   constexpr int HALVES = KEYS / 16;
-  __shared__ float merge_m[NW][HEADS], merge_l[NW][HEADS], merge_scale[HEADS];
-  __shared__ __align__(16) float merge_o[NW][HEADS][16][VE + 4];
 
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, r = lane & 15u, g = lane >> 4;
-  const uint32_t group = a.heads / a.kv_heads, blocks = (group + HEADS - 1) / HEADS;
   const uint64_t split = a.part.split == 0 ? 1 : a.part.split;
-  uint64_t rest = blockIdx.x / split;
-  const uint64_t s_part = blockIdx.x % split;
-  const uint32_t hb = static_cast<uint32_t>(rest % blocks);
-  rest /= blocks;
-  const uint32_t kv = static_cast<uint32_t>(rest % a.kv_heads);
-  const uint64_t row = rest / a.kv_heads;
-  const uint32_t head0 = kv * group + hb * HEADS, here = group - hb * HEADS < HEADS ? group - hb * HEADS : HEADS;
   const uint32_t D = a.head_dim;
-
-  uint64_t start, last;
-  key_range(a, row, start, last);
-  if (a.part.split != 0 && !key_chunk(a, s_part, start, last)) {   // workgroup-uniform
-    for (uint32_t i = t; i < here * D; i += NW * 64u) a.part.pacc[((row * a.heads + head0 + i / D) * split + s_part) * D + i % D] = 0.0f;
-    if (t < here) {
-      const uint64_t at = (row * a.heads + head0 + t) * split + s_part;
-      a.part.pmax[at] = -1e30f, a.part.psum[at] = 0.0f;
-    }
-    return;
-  }
 
   const uint64_t stride = static_cast<uint64_t>(a.kv_heads) * D * BITS / 8;
   const uint8_t* kb = static_cast<const uint8_t*>(a.k) + static_cast<uint64_t>(kv) * D * BITS / 8;
@@ -475,12 +478,12 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
   // Merge of the wavefronts: everyone's sum under the largest score of all, added in wavefront order.
   run_sum = groups_sum(run_sum);
   const bool writer = !second;
-  if (g == 0u && writer) merge_m[wave][column_head] = run_max, merge_l[wave][column_head] = run_sum;
-  if (t < 16u && writer) merge_scale[column_head] = score_scale;
+  if (g == 0u && writer) merge.m[wave][column_head] = run_max, merge.l[wave][column_head] = run_sum;
+  if (t < 16u && writer) merge.scale[column_head] = score_scale;
   __syncthreads();
-  float top = merge_m[0][column_head];
+  float top = merge.m[0][column_head];
 #pragma unroll
-  for (int w = 1; w < NW; ++w) top = fmaxf(top, merge_m[w][column_head]);
+  for (int w = 1; w < NW; ++w) top = fmaxf(top, merge.m[w][column_head]);
   const float f = __builtin_amdgcn_exp2f((run_max - reference_score(top)) * score_scale) / value_up;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -495,21 +498,21 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
         own *= term_down;
         xs[c] = (F32 ? own : own + other_term(own)) * f;
       }
-      if (writer) *reinterpret_cast<float4*>(&merge_o[wave][column_head][4 * g + e][j]) = x;
+      if (writer) *reinterpret_cast<float4*>(&merge.o[wave][column_head][4 * g + e][j]) = x;
     }
   }
   __syncthreads();
   for (uint32_t i = t; i < here * D; i += NW * 64u) {
     const uint32_t h = i / D, d = i % D;
-    float m = merge_m[0][h];
+    float m = merge.m[0][h];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) m = fmaxf(m, merge_m[w][h]);
+    for (int w = 1; w < NW; ++w) m = fmaxf(m, merge.m[w][h]);
     float sum = 0.0f, acc = 0.0f;
-    const float m_ref = reference_score(m), scale = merge_scale[h];
+    const float m_ref = reference_score(m), scale = merge.scale[h];
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      sum = fmaf(__builtin_amdgcn_exp2f((merge_m[w][h] - m_ref) * scale), merge_l[w][h], sum);
-      acc += merge_o[w][h][d / VE][d % VE];
+      sum = fmaf(__builtin_amdgcn_exp2f((merge.m[w][h] - m_ref) * scale), merge.l[w][h], sum);
+      acc += merge.o[w][h][d / VE][d % VE];
     }
     if (a.part.split != 0) {
       const uint64_t at = (row * a.heads + head0 + h) * split + s_part;
@@ -520,6 +523,429 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
       if (d == 0) a.part.pmax[at] = largest, a.part.psum[at] = sum * moved;
     } else {
       a.out[((a.row_base + row) * a.heads + head0 + h) * D + d] = acc / sum;
+    }
+  }
+}
+
+template <KvKind KV, int DP, int NW>
+__global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArgs a) {
+  constexpr uint32_t kHeads = rows_heads<KV>();
+  __shared__ RowsShared<KV, DP, NW> merge;
+  const uint32_t group = a.heads / a.kv_heads, blocks = (group + kHeads - 1) / kHeads;
+  const uint64_t split = a.part.split == 0 ? 1 : a.part.split;
+  const uint64_t rest = blockIdx.x / split, row_kv = rest / blocks;
+  const uint32_t first = static_cast<uint32_t>(rest % blocks) * kHeads, kv = static_cast<uint32_t>(row_kv % a.kv_heads);
+  const uint32_t head0 = kv * group + first, here = group - first < kHeads ? group - first : kHeads;
+  const uint64_t row = row_kv / a.kv_heads, s_part = blockIdx.x % split;
+  uint64_t start, last;
+  key_range(a, row, start, last);
+  if (a.part.split != 0 && !key_chunk(a, s_part, start, last)) {   // workgroup-uniform
+    empty_part<NW * 64>(a, row, head0, here, s_part);
+    return;
+  }
+  attend_row<KV, DP, NW>(a, row, kv, head0, here, start, last, s_part, merge);
+}
+
+// ---- many query rows: a workgroup shares its keys among 64 (row, head) pairs ---------------------
+//
+// The pairs of a key head, `group` to a row, are the columns of the contractions.  A workgroup owns 64 of them
+// and walks the keys that any of them sees, 64 at a time: they are made fp16 (exactly: an fp16 number or a code)
+// once, on their way into LDS, keys row by row and values transposed, and every column's two terms meet the same
+// operand read.  Eight wavefronts, two a SIMD: four groups of 16 columns times two halves of a tile's keys, each
+// wavefront with its own running maximum and sums, merged at the end, and its queries' terms in registers.
+//   S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_16x16x32_f16, a lane's weights taken as they stand, as in
+//   attend_row, but with a column a pair and both of its terms in one lane.  Row r of block j of O^T stands for
+//   element VE r + j, so that a lane ends up with runs of a row of the result.
+// Both terms of a weight go into one sum: the second, x - hi as it is, is off by 2^-25 where it is an fp16
+// subnormal, with the largest weight at 2^14 (with values' scales, the largest contribution between 2^9 and 2^15):
+// 2^-34 of the largest at most.  A tile's contribution is summed by itself and added to the running sum, so that
+// rounding there goes with a few terms and not with the number of keys.
+// 512 rows of 24 heads of 256 on 2512 fp16 keys of 4: 119 us (432 with a workgroup a row and key head, which read each
+// key for six columns), int8 keys 125 (455).  It waits for LDS (28 % of the cycles busy there) and for the step's barrier;
+// vector issue takes 31 %, the matrix cores 20 %.
+// Infinities and NaN are not kept apart here.  Whatever meets one ends with a sum that is not finite, or sets
+// `special`; the workgroup's columns are then done again with attend_row.
+template <int DP>
+struct TileShared {
+  static constexpr uint32_t kKeyBytes = 64 * DP * 2, kStage = 2 * kKeyBytes;
+  alignas(16) uint8_t stage[2][kStage];        // 64 keys, then two times 32 keys' values transposed
+  float scales[2][2][64];                      // keys', values'
+  float most[64], sum[64], up[64];             // the second halves'
+  uint32_t special;
+};
+
+template <KvKind KV, int DP>
+__global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a) {
+  constexpr bool QUANT = kv_quantized(KV);
+  constexpr int BITS = kv_bits(KV);
+  constexpr int STEPS = DP / 32, CHAINS = STEPS / 2;               // matrix instructions of a score, its sums (as in attend_row)
+  constexpr int VE = DP / 16, RE = DP / 32;                        // elements of a row of the result, of a value run
+  constexpr int GROUP = DP == 256 ? 2 : 4;                                         // operands read at once
+  constexpr int CHUNKS = DP / 8;                                   // runs of eight elements of a key
+  constexpr int KLOADS = 64 * CHUNKS / 512;
+  constexpr int KW = 8 * BITS / 32, VW = (RE * BITS + 31) / 32;
+  using Shared = TileShared<DP>;
+  union Lds {
+    Shared tile;
+    RowsShared<KV, DP, 8> rows;
+    __device__ Lds() {}
+  };
+  __shared__ Lds lds;
+  Shared& sh = lds.tile;
+
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t r = lane & 15u, g = lane >> 4, col_group = wave & 3u, half = wave >> 2;
+  const uint32_t D = a.head_dim, group = a.heads / a.kv_heads;
+  const uint32_t split = a.part.split == 0 ? 1u : static_cast<uint32_t>(a.part.split), units = gridDim.x / a.kv_heads;
+  const uint32_t kv = blockIdx.x % a.kv_heads, unit = units - 1u - blockIdx.x / a.kv_heads, s_part = unit % split;
+  const uint64_t columns = a.rows * group;
+  const uint64_t c0 = static_cast<uint64_t>(unit / split) * 64;    // the longest first
+  const uint64_t c_end = c0 + 64 < columns ? c0 + 64 : columns;
+  const uint64_t col_any = c0 + col_group * 16 + r, col = col_any < c_end ? col_any : c_end - 1;
+  const uint64_t row = col / group;
+  const uint32_t head = kv * group + static_cast<uint32_t>(col % group);
+  uint64_t first_key, last_key;
+  key_range(a, row, first_key, last_key);
+  const uint32_t start = static_cast<uint32_t>(first_key), last = static_cast<uint32_t>(last_key);
+  key_range(a, c0 / group, first_key, last_key);
+  uint32_t wg_start = static_cast<uint32_t>(first_key);
+  const uint32_t first_row_last = static_cast<uint32_t>(last_key);
+  key_range(a, (c_end - 1) / group, first_key, last_key);
+  uint32_t wg_last = static_cast<uint32_t>(last_key);
+  const uint32_t last_row_start = static_cast<uint32_t>(first_key);
+  // Calls f(row, first head, heads) for the workgroup's columns, rows_heads of a row at most at a time.
+  auto for_rows = [&](auto f) {
+    for (uint64_t c = c0; c < c_end;) {
+      const uint32_t h = static_cast<uint32_t>(c % group);
+      uint32_t here = group - h < rows_heads<KV>() ? group - h : rows_heads<KV>();
+      if (here > c_end - c) here = static_cast<uint32_t>(c_end - c);
+      f(c / group, kv * group + h, here);
+      c += here;
+    }
+  };
+  if (split > 1u) {                                                // whole tiles of the workgroup's keys a part
+    const uint32_t chunk = ((wg_last - wg_start + split) / split + 63u) / 64u * 64u;
+    if (s_part * chunk > wg_last - wg_start) {
+      for_rows([&](uint64_t i, uint32_t head0, uint32_t here) { empty_part<512>(a, i, head0, here, s_part); });
+      return;
+    }
+    wg_start += s_part * chunk;
+    if (wg_last - wg_start >= chunk) wg_last = wg_start + chunk - 1u;
+  }
+
+  const uint64_t stride = static_cast<uint64_t>(a.kv_heads) * D * BITS / 8;
+  const uint8_t* kb = static_cast<const uint8_t*>(a.k) + static_cast<uint64_t>(kv) * D * BITS / 8;
+  const uint8_t* vb = static_cast<const uint8_t*>(a.v) + static_cast<uint64_t>(kv) * D * BITS / 8;
+  uint32_t kr[KLOADS][KW], vr[4][VW];
+  float sr = 0.0f;
+  // Values: elements RE v_run.., keys 4 v_four.. of the tile; lanes l and l + 16 write the halves of a chunk.
+  const uint32_t v_run = (lane & 15u) * 2u + (lane >> 5), v_four = half * 8u + (lane >> 4 & 1u) * 4u + col_group;
+  const uint32_t k_key = t / CHUNKS, k_chunk = t % CHUNKS;         // keys k_key + (512 / CHUNKS) i
+  // Elements past head_dim are read as the row's first: the queries are 0 there, of the result they are not stored.
+  const uint32_t k_elem = k_chunk * 8u < D ? k_chunk * BITS : 0u, v_elem = v_run * RE < D ? v_run * RE * BITS / 8 : 0u;
+  const uint32_t k_off = k_key * static_cast<uint32_t>(stride) + k_elem, v_off = v_four * 4u * static_cast<uint32_t>(stride) + v_elem;
+  auto fetch = [&](uint32_t j0) {
+    const uint32_t left = wg_last - j0;
+    const uint8_t *k_tile = kb + j0 * stride, *v_tile = vb + j0 * stride;
+    if (left >= 63u) {
+#pragma unroll
+      for (int i = 0; i < KLOADS; ++i) load_run<BITS>(k_tile + i * (512 / CHUNKS) * stride + k_off, kr[i]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) load_run<RE * BITS / 8>(v_tile + e * stride + v_off, vr[e]);
+    } else {
+      // The last tile: keys past the range's end are read as its last one; no column sees them.
+#pragma unroll
+      for (int i = 0; i < KLOADS; ++i) {
+        const uint32_t key = k_key + i * (512u / CHUNKS);
+        load_run<BITS>(k_tile + (key < left ? key : left) * stride + k_elem, kr[i]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t key = v_four * 4u + e;
+        load_run<RE * BITS / 8>(v_tile + (key < left ? key : left) * stride + v_elem, vr[e]);
+      }
+    }
+    if constexpr (QUANT) {
+      const uint32_t key = t & 63u;
+      if (t < 128u) sr = (t < 64u ? a.k_scale : a.v_scale)[j0 + (key < left ? key : left)];
+    }
+  };
+  // A key's row in LDS: its chunks of sixteen bytes at c ^ swizzle, so that neighbouring keys' chunks fall on
+  // different banks; 256 bytes hold 16 chunks.
+  auto key_swizzle = [](uint32_t key) { return CHUNKS >= 16 ? key & 15u : (key >> 1) & 7u; };
+  auto value_place = [](uint32_t row, uint32_t chunk) { return (row & 3u) * 256u + (row >> 2) * 64u + ((chunk ^ (row & 3u)) * 16u); };
+  auto stash = [&](uint32_t b) {
+    uint8_t* keys = sh.stage[b];
+#pragma unroll
+    for (int i = 0; i < KLOADS; ++i) {
+      const uint32_t key = k_key + i * (512u / CHUNKS);
+      *reinterpret_cast<half8_t*>(keys + key * (DP * 2u) + ((k_chunk ^ key_swizzle(key)) * 16u)) = key_operand<KV>(kr[i]);
+    }
+    // Row r of block j of a half's values: four chunks of sixteen bytes, chunk c of keys 4c.. and 16 + 4c.. at
+    // c ^ r % 4; the rows in the order 0, 4, 8, 12, 1, .., which with that puts sixteen lanes on sixteen bank groups.
+    const uint32_t vrow = v_run >> 1, four = v_four & 7u;
+    uint8_t* values = keys + Shared::kKeyBytes + half * (DP * 64u) + (v_run & 1u) * (RE * 1024u) + value_place(vrow, four & 3u) + (four >> 2) * 8u;
+#pragma unroll
+    for (int j = 0; j < RE; ++j) {
+      *reinterpret_cast<uint2*>(values + j * 1024u) = uint2{value_pair<KV>(vr[0], vr[1], j), value_pair<KV>(vr[2], vr[3], j)};
+    }
+    if constexpr (QUANT) {
+      if (t < 128u) {
+        sh.scales[b][t >> 6][t & 63u] = sr;
+        if (t < 64u && !(fabsf(sr) < INFINITY)) sh.special = 1u;   // such a key's score says nothing of its weight here
+      }
+    }
+  };
+
+  if (t == 0) sh.special = 0u;
+  fetch(wg_start);
+
+  // The queries' terms.
+  half8_t q_hi[STEPS], q_lo[STEPS];
+  float score_scale = kLog2E / sqrtf(static_cast<float>(D));
+  {
+    const float* qp = a.q + ((a.row_base + row) * a.heads + head) * D;
+    float raw[STEPS][8], most = 0.0f;
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const uint32_t d = i * 32u + g * 8u;
+      const float4 x = d < D ? *reinterpret_cast<const float4*>(qp + d) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+      const float4 y = d < D ? *reinterpret_cast<const float4*>(qp + d + 4) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+      raw[i][0] = x.x, raw[i][1] = x.y, raw[i][2] = x.z, raw[i][3] = x.w;
+      raw[i][4] = y.x, raw[i][5] = y.y, raw[i][6] = y.z, raw[i][7] = y.w;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(raw[i][e]));
+    }
+    most = groups_max(most);
+    const float up = most == 0.0f ? 1.0f : power_of_two_to(most, 14);
+    score_scale /= up;
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = raw[i][kq_dim<KV>(e)] * up;
+        const _Float16 hi = static_cast<_Float16>(v);
+        q_hi[i][e] = hi;
+        q_lo[i][e] = static_cast<_Float16>((v - static_cast<float>(hi)) * 0x1p11f);
+      }
+    }
+  }
+  __syncthreads();                                                 // `special` is set up
+  stash(0);
+  if (wg_last - wg_start >= 64u) fetch(wg_start + 64u);
+  __syncthreads();
+
+  float4_t o[VE];
+#pragma unroll
+  for (int j = 0; j < VE; ++j) o[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  float run_max = -INFINITY, run_sum = 0.0f;
+  float lane_most = 0.0f, value_up = QUANT ? power_of_two_to(0.0f, 14) : 0x1p14f;
+  const uint32_t key_row = (half * 32u + r) * (DP * 2u), key_swz = key_swizzle(r);
+  const uint32_t value_row = Shared::kKeyBytes + half * (DP * 64u) + value_place(r, g);
+  // A tile's loads are under way for the whole of the tile before it, and it goes to LDS after that one's scores.
+  for (uint32_t j0 = wg_start, b = 0; j0 <= wg_last; j0 += 64u, b ^= 1u) {
+    const uint8_t* stage = sh.stage[b];
+
+    // Element 4 h + e of a lane: key 16 h + 4 g + e of the wavefront's 32.  Operands are read a group ahead of
+    // their matrix instructions; the barriers keep the compiler from moving each read to its use.
+    float s[8];
+    float4_t hi[CHAINS], lo;
+    half8_t kf[2][GROUP];
+    auto read_keys = [&](int n, half8_t (&f)[GROUP]) {
+#pragma unroll
+      for (int i = 0; i < GROUP; ++i) {
+        const uint32_t h = (n * GROUP + i) / STEPS, step = (n * GROUP + i) % STEPS;
+        f[i] = *reinterpret_cast<const half8_t*>(stage + key_row + h * (16u * DP * 2u) + (((4u * step + g) ^ key_swz) * 16u));
+      }
+    };
+    read_keys(0, kf[0]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < 2 * STEPS / GROUP; ++n) {
+      if (n + 1 < 2 * STEPS / GROUP) read_keys(n + 1, kf[(n + 1) & 1]);
+#pragma unroll
+      for (int i = 0; i < GROUP; ++i) {
+        const int h = (n * GROUP + i) / STEPS, step = (n * GROUP + i) % STEPS;
+        if (step == 0) {
+          lo = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int c = 0; c < CHAINS; ++c) hi[c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        hi[step % CHAINS] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[n & 1][i], q_hi[step], hi[step % CHAINS], 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[n & 1][i], q_lo[step], lo, 0, 0, 0);
+        if (step == STEPS - 1) {
+#pragma unroll
+          for (int c = CHAINS / 2; c > 0; c /= 2) {
+#pragma unroll
+            for (int x = 0; x < c; ++x) hi[x] += hi[x + c];
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[4 * h + e] = fmaf(lo[e], 0x1p-11f, hi[0][e]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (wg_last - j0 >= 64u) stash(b ^ 1u);
+    if (wg_last - j0 >= 128u) fetch(j0 + 128u);
+    half8_t vf[2][GROUP];
+    auto read_values = [&](int n, half8_t (&f)[GROUP]) {
+#pragma unroll
+      for (int i = 0; i < GROUP; ++i) f[i] = *reinterpret_cast<const half8_t*>(stage + value_row + (n * GROUP + i) * 1024u);
+    };
+    read_values(0, vf[0]);
+    float vsv[8];
+    if constexpr (QUANT) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t at = half * 32u + h * 16u + g * 4u;
+        const float4 ks = *reinterpret_cast<const float4*>(&sh.scales[b][0][at]), vs = *reinterpret_cast<const float4*>(&sh.scales[b][1][at]);
+        s[4 * h] *= ks.x, s[4 * h + 1] *= ks.y, s[4 * h + 2] *= ks.z, s[4 * h + 3] *= ks.w;
+        vsv[4 * h] = vs.x, vsv[4 * h + 1] = vs.y, vsv[4 * h + 2] = vs.z, vsv[4 * h + 3] = vs.w;
+      }
+    }
+    if (j0 + 63 > first_row_last || j0 < last_row_start) {         // some column does not see some key of the tile
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t key = j0 + half * 32u + 16u * (e / 4) + 4u * g + e % 4;
+        s[e] = key >= start && key <= last ? s[e] : -INFINITY;
+      }
+    }
+    float most = s[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) most = fmaxf(most, s[e]);
+    const float m_new = fmaxf(run_max, groups_max(most));
+    const float m_ref = reference_score(m_new);
+    float corr = __builtin_amdgcn_exp2f((run_max - m_ref) * score_scale);   // 0 on the first tile (run_max = -inf)
+    run_max = m_new;
+    float sum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      s[e] = __builtin_amdgcn_exp2f((s[e] - m_ref) * score_scale);
+      sum += s[e];
+    }
+    run_sum = fmaf(corr, run_sum, sum);
+    if constexpr (QUANT) {
+      // As in attend_row: the power of two follows the largest contribution.
+      float scale_most = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) scale_most = fmaxf(scale_most, fabsf(vsv[e]));
+      lane_most *= corr;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        s[e] *= vsv[e];
+        lane_most = fmaxf(lane_most, fabsf(s[e]));
+      }
+      if (__any(corr != 1.0f || !(scale_most * value_up < 0x1p15f))) {
+        const float largest = groups_max(lane_most), scaled = largest * value_up;
+        if (largest > 0.0f && !(scaled >= 0x1p9f && scaled < 0x1p15f)) {
+          const float up = power_of_two_to(largest, 13);
+          corr *= up / value_up;
+          value_up = up;
+        }
+      }
+    }
+    half8_t p_hi, p_lo;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = s[e] * value_up;
+      const _Float16 hi = static_cast<_Float16>(x);
+      p_hi[e] = hi;
+      p_lo[e] = static_cast<_Float16>(x - static_cast<float>(hi));
+    }
+    if (__any(corr != 1.0f)) {
+#pragma unroll
+      for (int j = 0; j < VE; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[j][e] *= corr;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < VE / GROUP; ++n) {
+      if (n + 1 < VE / GROUP) read_values(n + 1, vf[(n + 1) & 1]);
+      float4_t acc[GROUP];
+#pragma unroll
+      for (int i = 0; i < GROUP; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n & 1][i], p_lo, float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < GROUP; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n & 1][i], p_hi, acc[i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < GROUP; ++i) o[n * GROUP + i] += acc[i];
+    }
+    __syncthreads();
+  }
+
+  // Merge of the two halves' sums under the larger maximum; the lanes' shares of the sum of weights first.
+  run_sum = groups_sum(run_sum);
+  float* other = reinterpret_cast<float*>(sh.stage[0]) + col_group * (VE * 256u) + lane;
+  const uint32_t at = col_group * 16u + r;
+  if (half == 1u) {
+    if (g == 0u) sh.most[at] = run_max, sh.sum[at] = run_sum, sh.up[at] = value_up;
+#pragma unroll
+    for (int j = 0; j < VE; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) other[(j * 4 + e) * 64] = o[j][e];
+  }
+  __syncthreads();
+  if (half == 0u) {
+    const float m1 = sh.most[at], most = fmaxf(run_max, m1), top = reference_score(most);
+    const float w0 = __builtin_amdgcn_exp2f((run_max - top) * score_scale), w1 = __builtin_amdgcn_exp2f((m1 - top) * score_scale);
+    const float total = fmaf(w1, sh.sum[at], w0 * run_sum);
+    const float f0 = w0 / value_up, f1 = w1 / sh.up[at];
+    bool finite = fabsf(total) < INFINITY && (split > 1u || total != 0.0f);
+#pragma unroll
+    for (int j = 0; j < VE; ++j) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = fmaf(other[(j * 4 + e) * 64], f1, o[j][e] * f0);
+        finite = finite && fabsf(x) < INFINITY;
+        other[(j * 4 + e) * 64] = x;
+      }
+    }
+    if (!finite) sh.special = 1u;
+    if (g == 0u) sh.most[at] = most, sh.sum[at] = total;
+  }
+  __syncthreads();
+  // (the results only now: `out` may be q's memory, which attend_row reads)
+  if (__builtin_amdgcn_readfirstlane(sh.special) != 0u) {          // workgroup-uniform
+    for_rows([&](uint64_t i, uint32_t head0, uint32_t here) {
+      uint64_t row_start, row_last;
+      key_range(a, i, row_start, row_last);
+      if (split > 1u) {
+        row_start = row_start > wg_start ? row_start : wg_start, row_last = row_last < wg_last ? row_last : wg_last;
+        if (row_start > row_last) {
+          empty_part<512>(a, i, head0, here, s_part);
+          return;
+        }
+      }
+      __syncthreads();
+      attend_row<KV, DP, 8>(a, i, kv, head0, here, row_start, row_last, s_part, lds.rows);
+    });
+    return;
+  }
+  if (col_any >= c_end) return;
+  const float total = sh.sum[at];
+  float* out = a.out + ((a.row_base + row) * a.heads + head) * D;
+  float factor = 1.0f;
+  if (split > 1u) {
+    const uint64_t part = (row * a.heads + head) * split + s_part;
+    out = a.part.pacc + part * D;
+    // The part's largest score in natural units is rounded; the sums move by what that took from it.
+    const float most = sh.most[at], natural = score_scale * kLn2, largest = most * natural;
+    factor = most == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(fmaf(most, natural, -largest) * kLog2E);
+    if (g == 0u && half == 0u) a.part.pmax[part] = fmaxf(largest, -1e30f), a.part.psum[part] = total * factor;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t e = half * 2u + i, d = (g * 4u + e) * VE;
+#pragma unroll
+    for (int j = 0; j < VE; j += 4) {
+      float x[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float sum = other[((j + v) * 4 + e) * 64];
+        x[v] = split > 1u ? sum * factor : sum / total;
+      }
+      if (d + j < D) *reinterpret_cast<float4*>(out + d + j) = float4{x[0], x[1], x[2], x[3]};
     }
   }
 }
@@ -671,19 +1097,31 @@ hipError_t launch_rows(const AttentionArgs& a, uint64_t m, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// The runs that the lanes of the matrix kernels load divide a head's row: 16 bytes of a key (a quarter of the padded
+// row where that is less), a sixteenth of the padded row of a value.
+constexpr uint32_t padded_head(uint32_t head_dim) { return head_dim <= 64 ? 64 : head_dim <= 128 ? 128 : 256; }
+template <KvKind KV>
+bool runs_fit(uint32_t head_dim) {
+  const uint32_t padded = padded_head(head_dim);
+  const uint32_t run = KV == KvKind::F32 ? 4 : 128u / kv_bits(KV) < padded / 4 ? 128u / kv_bits(KV) : padded / 4;
+  return head_dim % run == 0 && head_dim % (padded / 16) == 0;
+}
+
+uint64_t tile_units(uint64_t m, uint64_t heads, uint64_t kv_heads) { return (m * (heads / kv_heads) + 63) / 64 * kv_heads; }
+
+// `a.part.split` parts of the keys (0: one, into `a.out`) for each 64 (row, head) pairs.
+template <KvKind KV>
+hipError_t launch_tiles(const AttentionArgs& a, hipStream_t stream) {
+  const uint64_t split = a.part.split == 0 ? 1 : a.part.split;
+  const dim3 grid(static_cast<uint32_t>(tile_units(a.rows, a.heads, a.kv_heads) * split));
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, a); };
+  a.head_dim <= 64 ? go(attention_tile_kernel<KV, 64>) : a.head_dim <= 128 ? go(attention_tile_kernel<KV, 128>) : go(attention_tile_kernel<KV, 256>);
+  return hipGetLastError();
+}
+
 // kind: 0 fp32, 1 fp16 keys and values; 2 int8, 3 4-bit, 4 E4M3 codes with one scale per key row.
-hipError_t launch_attention_as(uint32_t kind, const AttentionArgs& a, uint64_t m, hipStream_t stream) {
-  auto go = [&](auto tag) {
-    constexpr KvKind KV = decltype(tag)::value;
-    // The runs that the lanes load divide a head's row: 16 bytes of a key (a quarter of the padded row
-    // where that is less), a sixteenth of the padded row of a value.
-    const uint32_t padded = a.head_dim <= 64 ? 64 : a.head_dim <= 128 ? 128 : 256;
-    const uint32_t run = KV == KvKind::F32 ? 4 : 128u / kv_bits(KV) < padded / 4 ? 128u / kv_bits(KV) : padded / 4;
-    if (a.head_dim % run == 0 && a.head_dim % (padded / 16) == 0) return launch_rows<KV>(a, m, stream);
-    const uint64_t parts = a.part.split == 0 ? 1 : a.part.split;
-    hipLaunchKernelGGL(attention_any_kernel<KV>, dim3(static_cast<uint32_t>(m * a.heads * parts)), dim3(256), 0, stream, a);
-    return hipGetLastError();
-  };
+template <class Go>
+auto with_kind(uint32_t kind, Go&& go) {
   switch (kind) {
     case 0: return go(std::integral_constant<KvKind, KvKind::F32>{});
     case 1: return go(std::integral_constant<KvKind, KvKind::F16>{});
@@ -693,28 +1131,69 @@ hipError_t launch_attention_as(uint32_t kind, const AttentionArgs& a, uint64_t m
   }
 }
 
+hipError_t launch_attention_as(uint32_t kind, const AttentionArgs& a, uint64_t m, hipStream_t stream) {
+  return with_kind(kind, [&](auto tag) {
+    constexpr KvKind KV = decltype(tag)::value;
+    if (runs_fit<KV>(a.head_dim)) return launch_rows<KV>(a, m, stream);
+    const uint64_t parts = a.part.split == 0 ? 1 : a.part.split;
+    hipLaunchKernelGGL(attention_any_kernel<KV>, dim3(static_cast<uint32_t>(m * a.heads * parts)), dim3(256), 0, stream, a);
+    return hipGetLastError();
+  });
+}
+
 AttentionArgs args_of(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale, float* out,
                       uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t row_base,
-                      uint64_t window, bool causal) {
-  return AttentionArgs{q, k, v, k_scale, v_scale, out, SplitOut{}, n, q_base, row_base, window, static_cast<uint32_t>(heads),
+                      uint64_t window, bool causal, uint64_t rows) {
+  return AttentionArgs{q, k, v, k_scale, v_scale, out, SplitOut{}, rows, n, q_base, row_base, window, static_cast<uint32_t>(heads),
                        static_cast<uint32_t>(kv_heads), static_cast<uint32_t>(head_dim), causal ? 1u : 0u};
 }
 
 }  // namespace
 
-hipError_t launch_attention(const float* q, const void* k, const void* v, float* out, uint64_t m, uint64_t n, uint64_t heads,
-                            uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t row_base, uint64_t window,
-                            bool kv_f16, bool causal, hipStream_t stream) {
-  return launch_attention_as(kv_f16 ? 1u : 0u, args_of(q, k, v, nullptr, nullptr, out, n, heads, kv_heads, head_dim, q_base, row_base,
-                                                       window, causal), m, stream);
+uint64_t attention_parts(uint32_t kind, uint64_t m, uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
+                         uint64_t q_base, uint64_t window, bool causal, const void* out, uint64_t most_parts) {
+  if (kind == 0 || m < 17 || n >= (1u << 31) || reinterpret_cast<uintptr_t>(out) % 16 != 0) return 0;
+  const uint32_t dim = static_cast<uint32_t>(head_dim);
+  if (!with_kind(kind, [&](auto tag) { return runs_fit<decltype(tag)::value>(dim); })) return 0;
+  if (kv_heads * head_dim * 2 >= (1u << 25)) return 0;             // a tile's rows lie within 2^31 bytes
+  // Sides measured (us, rows' kernel / this one): in parts 17 rows of 24 heads of 256 on 2000 fp16 keys 47 / 30, 40 rows of
+  // 32 of 128 on 2000 int8 keys 53 / 24, but 64 rows of 24 of 256 on 300 keys 17 / 27, 100 rows of 8 of 64 on 500 keys
+  // 10 / 13: the line lies at some 24 M elements of keys met.  In one part: 300 rows of 8 heads of 128 with keys of their own
+  // 152 / 40, 256 rows of 16 of 64 on 100 keys 17 / 12, 100 rows of 8 of 64 on 500 keys 10 / 16.
+  const uint64_t units = tile_units(m, heads, kv_heads), cus = static_cast<uint64_t>(num_cus());
+  if (units >= kMaxGridThreads / 512u) return 0;
+  uint64_t keys = causal && q_base + m < n ? q_base + m : n;
+  if (causal && window != 0 && window < keys) keys = window;
+  uint64_t parts = cus / units < keys / 256 ? cus / units : keys / 256;
+  if (parts > most_parts) parts = most_parts;
+  while (parts > 1 && attention_parts_bytes(m, heads, head_dim, parts) > kAttentionPartsMost) --parts;
+  const uint64_t row_units = m * kv_heads * ((heads / kv_heads + 7) / 8);   // workgroups of the rows' kernel
+  if (parts > 1 && row_units * padded_head(dim) >= (24u << 20) / keys) return parts;
+  return row_units >= 400 ? 1 : 0;
 }
 
-// kind: 0 int8, 1 4-bit, 2 E4M3 keys and values with one scale per key row; always causal.
-hipError_t launch_attention_quant(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
-                                  float* out, uint64_t m, uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
-                                  uint64_t q_base, uint64_t row_base, uint64_t window, uint32_t kind, hipStream_t stream) {
-  return launch_attention_as(2u + kind, args_of(q, k, v, k_scale, v_scale, out, n, heads, kv_heads, head_dim, q_base, row_base, window,
-                                                true), m, stream);
+size_t attention_parts_bytes(uint64_t m, uint64_t heads, uint64_t head_dim, uint64_t parts) {
+  return parts < 2 ? 0 : static_cast<size_t>(m * heads * parts * (head_dim + 2) * 4);
+}
+
+// kind: 0 fp32, 1 fp16 keys and values; 2 int8, 3 4-bit, 4 E4M3 codes with one scale per key row (always causal).
+hipError_t launch_attention(uint32_t kind, const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
+                            float* out, uint64_t m, uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
+                            uint64_t q_base, uint64_t row_base, uint64_t window, bool causal, uint64_t parts, void* scratch,
+                            hipStream_t stream) {
+  AttentionArgs a = args_of(q, k, v, k_scale, v_scale, out, n, heads, kv_heads, head_dim, q_base, row_base, window, causal, m);
+  if (parts == 0) return launch_attention_as(kind, a, m, stream);
+  if (parts > 1) {
+    float* acc = static_cast<float*>(scratch);
+    float* most = acc + m * heads * parts * head_dim;
+    a.part = SplitOut{acc, most, most + m * heads * parts, parts};
+  }
+  const hipError_t e = with_kind(kind, [&](auto tag) {
+    if constexpr (decltype(tag)::value == KvKind::F32) return hipErrorInvalidValue;
+    else return launch_tiles<decltype(tag)::value>(a, stream);
+  });
+  if (e != hipSuccess || parts == 1) return e;
+  return launch_attention_combine(a.part.pacc, a.part.pmax, a.part.psum, out + row_base * heads * head_dim, m, heads, head_dim, parts, stream);
 }
 
 // The split-N form: kv_kind as launch_attention_as (0 fp32, 1 fp16, 2.. quantized with scales).
@@ -722,7 +1201,7 @@ hipError_t launch_attention_split(const float* q, const void* k, const void* v, 
                                   float* pacc, float* pmax, float* psum, uint64_t m, uint64_t n, uint64_t heads,
                                   uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t window, uint32_t kv_kind,
                                   bool causal, uint64_t split, hipStream_t stream) {
-  AttentionArgs a = args_of(q, k, v, k_scale, v_scale, nullptr, n, heads, kv_heads, head_dim, q_base, 0, window, causal);
+  AttentionArgs a = args_of(q, k, v, k_scale, v_scale, nullptr, n, heads, kv_heads, head_dim, q_base, 0, window, causal, m);
   a.part = SplitOut{pacc, pmax, psum, split};
   return launch_attention_as(kv_kind, a, m, stream);
 }

@@ -156,7 +156,7 @@ void* decode_scratch(const LaunchCtx& c) {
   return c.no_alloc ? g_static_scratch[g_device] : g_decode_scratch;
 }
 
-// Scratch of "gemm_fp8" and of Q5_K / Q6_K with a few rows, whose calls on different streams are independent of
+// Scratch of "gemm_fp8", of Q5_K / Q6_K with a few rows and of "attention" with few columns, whose calls on different streams are independent of
 // one another: see stream_scratch.hpp.  qmm_init reserves the first slab; later ones are allocated under the
 // relaxed capture mode, which permits it while a stream is captured, unless the caller has handed over a workspace
 // (then a launch allocates nothing).
@@ -212,7 +212,7 @@ class StreamBlock {
   qmm::ScratchBlock* block_ = nullptr;
   void* ptr_ = nullptr;
 };
-static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock);
+static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock && qmm::kAttentionPartsMost <= qmm::StreamScratch::kSmallBlock);
 
 // Q4_K regimes by activation rows.  One row and small matrices: the VALU GEMV.  2..16 rows of a
 // matrix with at least kQ4KFewRowsMinWeights weights: the exact few-row MFMA kernels (weights read
@@ -490,13 +490,32 @@ qmm_status run_rope_common(const LaunchCtx& c, bool multimodal) {
 qmm_status run_rope(const LaunchCtx& c) { return run_rope_common(c, false); }
 qmm_status run_mrope(const LaunchCtx& c) { return run_rope_common(c, true); }
 
+// What "attention" and its quantized forms do once their buffers are known to fit.  The keys' parts, where a call has
+// too few rows to fill the chip, lie in the stream's scratch block; without one they stay in one part.
+qmm_status attend(const LaunchCtx& c, uint32_t kind, const float* k_scale, const float* v_scale, float* out, bool causal) {
+  const uint64_t m = c.sc[0], n = c.sc[1], heads = c.sc[2], kv_heads = c.sc[3], head_dim = c.sc[4], q_base = c.sc[5],
+                 row_base = c.sc[6], window = c.sc[7];
+  auto go = [&](uint64_t parts, void* scratch) {
+    return map_hip(qmm::launch_attention(kind, c.ptr<const float>(0), c.ptr<const void>(1), c.ptr<const void>(2), k_scale, v_scale,
+                                         out, m, n, heads, kv_heads, head_dim, q_base, row_base, window, causal, parts, scratch, c.stream));
+  };
+  auto plan = [&](uint64_t most) { return qmm::attention_parts(kind, m, n, heads, kv_heads, head_dim, q_base, window, causal, out, most); };
+  const uint64_t parts = plan(64);
+  if (parts > 1) {
+    const StreamBlock block(c, qmm::attention_parts_bytes(m, heads, head_dim, parts));
+    if (block.get() != nullptr) return go(parts, block.get());
+    return go(plan(1), nullptr);
+  }
+  return go(parts, nullptr);
+}
+
 // "attention": buffers Q (rows x heads*head_dim fp32), K, V (n x kv_heads*head_dim, fp32 or fp16), Out
 // (as Q); scalars m, n, heads, kv_heads, head_dim, q_base, row_base, window, kv_f16, causal
 // (include/tessera/backend.hpp:167-179,429-440).  Q and Out hold at least row_base + m rows.
 qmm_status run_attention(const LaunchCtx& c) {
   if (!counts(c, 4, 10)) return bad("attention: expects 4 buffers and 10 scalars");
   const uint64_t m = c.sc[0], n = c.sc[1], heads = c.sc[2], kv_heads = c.sc[3], head_dim = c.sc[4], q_base = c.sc[5],
-                 row_base = c.sc[6], window = c.sc[7], kv_f16 = c.sc[8], causal = c.sc[9];
+                 row_base = c.sc[6], kv_f16 = c.sc[8], causal = c.sc[9];
   if (m == 0 || n == 0 || heads == 0 || kv_heads == 0 || head_dim == 0 || heads % kv_heads != 0) {
     return bad("attention: m, n, heads, kv_heads, head_dim must be non-zero and heads a multiple of kv_heads");
   }
@@ -510,8 +529,7 @@ qmm_status run_attention(const LaunchCtx& c) {
   if (!c.fits(0, q_bytes) || !c.fits(1, kv_bytes) || !c.fits(2, kv_bytes) || !c.fits(3, q_bytes)) {
     return bad("attention: a buffer is smaller than the scalars require");
   }
-  return map_hip(qmm::launch_attention(c.ptr<const float>(0), c.ptr<const void>(1), c.ptr<const void>(2), c.ptr<float>(3), m, n,
-                                       heads, kv_heads, head_dim, q_base, row_base, window, kv_f16 == 1, causal == 1, c.stream));
+  return attend(c, static_cast<uint32_t>(kv_f16), nullptr, nullptr, c.ptr<float>(3), causal == 1);
 }
 
 // "attention_q8", "attention_q4", "attention_fp8": buffers q, K and V codes (n x kv_heads*head_dim int8
@@ -521,7 +539,7 @@ qmm_status run_attention(const LaunchCtx& c) {
 qmm_status run_attention_quant(const LaunchCtx& c, uint32_t kind) {
   if (!counts(c, 6, 9)) return bad("attention_q8/q4/fp8: expects 6 buffers and 9 scalars");
   const uint64_t m = c.sc[0], n = c.sc[1], heads = c.sc[2], kv_heads = c.sc[3], head_dim = c.sc[4], q_base = c.sc[5],
-                 row_base = c.sc[6], window = c.sc[7];
+                 row_base = c.sc[6];
   if (m == 0 || n == 0 || heads == 0 || kv_heads == 0 || head_dim == 0 || heads % kv_heads != 0 || c.sc[8] > 2) {
     return bad("attention_q8/q4/fp8: m, n, heads, kv_heads, head_dim must be non-zero, heads a multiple of kv_heads, kind 0..2");
   }
@@ -538,9 +556,7 @@ qmm_status run_attention_quant(const LaunchCtx& c, uint32_t kind) {
       !c.fits(4, static_cast<u128>(n) * 4) || !c.fits(5, q_bytes)) {
     return bad("attention_q8/q4/fp8: a buffer is smaller than the scalars require");
   }
-  return map_hip(qmm::launch_attention_quant(c.ptr<const float>(0), c.ptr<const void>(1), c.ptr<const void>(2),
-                                             c.ptr<const float>(3), c.ptr<const float>(4), c.ptr<float>(5), m, n, heads,
-                                             kv_heads, head_dim, q_base, row_base, window, kind, c.stream));
+  return attend(c, 2u + kind, c.ptr<const float>(3), c.ptr<const float>(4), c.ptr<float>(5), true);
 }
 qmm_status run_attention_q8(const LaunchCtx& c) { return run_attention_quant(c, 0); }
 qmm_status run_attention_q4(const LaunchCtx& c) { return run_attention_quant(c, 1); }

@@ -231,12 +231,16 @@ hipError_t launch_moe_scale_add(const float* a, const float* b, const float* f, 
 // pos3 null: "rope" (positions pos_base + row); else "mrope" (per-row (t, h, w) triples, section sizes).
 hipError_t launch_rope(float* data, const uint64_t* pos3, uint64_t rows, uint64_t heads, uint64_t head_dim, uint64_t rope_dim,
                        uint64_t pos_base, float theta, uint64_t sec_t, uint64_t sec_h, hipStream_t stream);
-hipError_t launch_attention(const float* q, const void* k, const void* v, float* out, uint64_t m, uint64_t n, uint64_t heads,
-                            uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t row_base, uint64_t window,
-                            bool kv_f16, bool causal, hipStream_t stream);
-hipError_t launch_attention_quant(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
-                                  float* out, uint64_t m, uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
-                                  uint64_t q_base, uint64_t row_base, uint64_t window, uint32_t kind, hipStream_t stream);
+// attention_parts: how "attention" runs a call. 0: the rows' kernels; else the kernel that shares keys among rows, its
+// keys in that many parts (at most `most_parts`), which attention_parts_bytes of `scratch` hold where there are two or more.
+constexpr size_t kAttentionPartsMost = size_t{16} << 20;
+uint64_t attention_parts(uint32_t kind, uint64_t m, uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
+                         uint64_t q_base, uint64_t window, bool causal, const void* out, uint64_t most_parts);
+size_t attention_parts_bytes(uint64_t m, uint64_t heads, uint64_t head_dim, uint64_t parts);
+hipError_t launch_attention(uint32_t kind, const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
+                            float* out, uint64_t m, uint64_t n, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
+                            uint64_t q_base, uint64_t row_base, uint64_t window, bool causal, uint64_t parts, void* scratch,
+                            hipStream_t stream);
 hipError_t launch_attention_split(const float* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
                                   float* pacc, float* pmax, float* psum, uint64_t m, uint64_t n, uint64_t heads,
                                   uint64_t kv_heads, uint64_t head_dim, uint64_t q_base, uint64_t window, uint32_t kv_kind,

@@ -1,0 +1,89 @@
+"""Attention with many query rows, where 64 (row, head) pairs share a workgroup's keys: pairs around 64, key counts
+around 64, windows, padded head sizes, the keys in one part and in several.  Against the oracle, and against the rows'
+kernels (the same call sixteen rows at a time) where the cache or the queries hold infinities or NaN."""
+import numpy as np
+import pytest
+
+from tessera_amd import synth
+from test_gpu_attention import KINDS, attend, cache, expected
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # m, n, heads, kv_heads, head_dim, q_base, window
+    (410, 410, 2, 1, 64, 0, 0),          # 820 pairs: the last workgroup has 52
+    (101, 449, 4, 4, 128, 348, 0),       # a pair a row; one key more than seven tiles
+    (203, 300, 6, 2, 256, 97, 70),       # a window shorter than two tiles
+    (137, 140, 9, 3, 96, 3, 0),          # padded to 128; rows across workgroups
+    (401, 200, 1, 1, 64, 100, 0),        # rows past the last key
+    (33, 2100, 24, 4, 256, 2067, 0),     # parts of the keys
+    (40, 1100, 8, 8, 128, 1060, 0),
+    (70, 1300, 8, 8, 64, 1230, 820),     # parts of which early rows see none of the last, late rows little of the first
+    (20, 1537, 16, 4, 160, 1517, 0),     # padded to 256
+]
+
+
+@pytest.mark.parametrize("kind", ["f16", "q8", "q4", "fp8"])
+@pytest.mark.parametrize("case", CASES)
+def test_attention_tiles(backend, kind, case):
+    m, n, heads, kv_heads, head_dim, q_base, window = case
+    g = synth.rng(n + head_dim + KINDS[kind])
+    width = kv_heads * head_dim
+    q = g.standard_normal((m + 3, heads * head_dim)).astype(np.float32)
+    k, ks = cache(g, kind, n, width)
+    v, vs = cache(g, kind, n, width)
+    want = expected(kind, q[2:2 + m], k, v, ks, vs, m, n, heads, kv_heads, head_dim, q_base, window)
+    got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, q_base, window, row_base=2)
+    # sums in another order, as test_gpu_attention.py (twice it where parts are merged)
+    assert np.max(np.abs(got[2:2 + m] - want)) <= 4e-6 * max(1.0, np.max(np.abs(want)))
+    assert np.all(got[:2] == 7.0) and np.all(got[2 + m:] == 7.0)
+
+
+def test_attention_tiles_not_causal(backend):
+    m, n, heads, kv_heads, head_dim = 101, 203, 4, 4, 128
+    g = synth.rng(5)
+    q = g.standard_normal((m, heads * head_dim)).astype(np.float32)
+    k, v = (cache(g, "f16", n, kv_heads * head_dim)[0] for _ in range(2))
+    want = expected("f16", q, k, v, None, None, m, n, heads, kv_heads, head_dim, 0, 0, causal=0)
+    got = attend(backend, "f16", q, k, v, None, None, m, n, heads, kv_heads, head_dim, 0, 0, causal=0)
+    assert np.max(np.abs(got - want)) <= 2e-6 * max(1.0, np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("shape", [(101, 449, 4, 4, 128), (33, 2100, 24, 4, 256), (410, 410, 2, 1, 64)])
+@pytest.mark.parametrize("what", ["key", "key-", "value", "value nan", "query", "key scale", "value scale", "zeros"])
+def test_attention_tiles_special_values(backend, shape, what):
+    m, n, heads, kv_heads, head_dim = shape
+    kind = "q8" if "scale" in what else "f16"
+    g = synth.rng(n)
+    q = g.standard_normal((m, heads * head_dim)).astype(np.float32)
+    k, ks = cache(g, kind, n, kv_heads * head_dim)
+    v, vs = cache(g, kind, n, kv_heads * head_dim)
+    at = n - m // 2                       # some rows see it, some do not
+    if what == "key":
+        k[at, 3] = np.inf
+    elif what == "key-":
+        k[at, :head_dim] = -np.inf
+    elif what == "value":
+        v[at, 5] = np.inf
+    elif what == "value nan":
+        v[at, 5] = np.nan
+    elif what == "query":
+        q[m // 2, 7] = np.inf
+    elif what == "key scale":
+        ks[at] = np.inf
+    elif what == "value scale":
+        vs[at] = np.inf
+    else:
+        q[m // 3] = 0.0
+        k[:] = 0
+    got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0)
+    want = np.empty_like(got)
+    for r in range(0, m, 16):
+        rows = min(16, m - r)
+        want[r:r + rows] = attend(backend, kind, np.ascontiguousarray(q[r:r + rows]), k, v, ks, vs, rows, n, heads, kv_heads,
+                                  head_dim, n - m + r, 0)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want))
+    fine = np.isfinite(want)
+    assert np.array_equal(got[~fine & ~np.isnan(want)], want[~fine & ~np.isnan(want)])
+    assert np.max(np.abs(got[fine] - want[fine]), initial=0.0) <= 4e-6 * max(1.0, np.max(np.abs(want[fine]), initial=0.0))
