@@ -156,7 +156,7 @@ void* decode_scratch(const LaunchCtx& c) {
   return c.no_alloc ? g_static_scratch[g_device] : g_decode_scratch;
 }
 
-// Scratch of "gemm_fp8", of Q5_K / Q6_K with a few rows and of "attention" with few columns, whose calls on different streams are independent of
+// Scratch of "gemm_fp8", of Q5_K / Q6_K with a few rows and of "attention" with few columns and of "gemm_mxfp4" from 17 rows, whose calls on different streams are independent of
 // one another: see stream_scratch.hpp.  qmm_init reserves the first slab; later ones are allocated under the
 // relaxed capture mode, which permits it while a stream is captured, unless the caller has handed over a workspace
 // (then a launch allocates nothing).
@@ -940,9 +940,15 @@ qmm_status run_gemm_mxfp4(const LaunchCtx& c) {
   // scale) and the fp32 rows as a short sum of E4M3 terms (gemm_mxfp4.hip).
   if (m >= kMxfp4GemmMinRows && m <= 0xFFFFFFFFull && n <= 0xFFFFFFFFull && qmm::gemm_mxfp4_f32_supported(m, k)) {
     void* ws = nullptr;
+    const size_t ws_bytes = (qmm::gemm_mxfp4_f32_workspace_bytes(m, k) + 255) / 256 * 256;
     const qmm_status st = workspace(c, qmm::gemm_mxfp4_f32_workspace_bytes(m, k), &ws);
     if (st != QMM_OK) return st;
-    return map_hip(qmm::launch_mxfp4_f32_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<float>(2), ws,
+    // The shared tiles' blocks: the stream's scratch block, or what the static array has left behind the workspace.
+    const size_t parts_bytes = qmm::gemm_mxfp4_f32_parts_bytes(m, n, k);
+    const StreamBlock block(c, c.no_alloc && parts_bytes != 0 ? ws_bytes + parts_bytes : parts_bytes);
+    float* parts = parts_bytes == 0 ? nullptr : static_cast<float*>(block.get());
+    if (parts != nullptr && c.no_alloc) parts += ws_bytes / 4;
+    return map_hip(qmm::launch_mxfp4_f32_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<float>(2), ws, parts,
                                               static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                               static_cast<uint32_t>(k), c.stream));
   }
