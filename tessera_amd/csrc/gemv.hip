@@ -1427,20 +1427,14 @@ __global__ __launch_bounds__(256) void gemv_smallk_kernel(typename Codec::Args a
   const uint32_t t = threadIdx.x, lane = t & 63u;
   const uint32_t rows_per_wave = 64u / cpr;
   const uint32_t chunk = lane % cpr, sub = lane / cpr;
-  typename Codec::template X<R> x;
-  if constexpr (Codec::kStageX) {
-    Codec::template load_x<R>(args, chunk, true, x, GlobalX{args.a, args.k});
-  } else {
-    Codec::template load_x<R>(args, chunk, true, x, 0);
-  }
   const Lane ln = Codec::make_lane(args, cpr, chunk, 0u);
   const uint32_t wave_global = blockIdx.x * (blockDim.x >> 6) + (t >> 6);
   const uint32_t waves_total = gridDim.x * (blockDim.x >> 6);
   const uint32_t groups = (n + rows_per_wave - 1) / rows_per_wave;
-  for (uint32_t g0 = wave_global; g0 < groups; g0 += waves_total * U) {
-    typename Codec::Frag frag[U];
-    bool ok[U];
-    uint32_t rows[U];
+  typename Codec::Frag frag[U];
+  bool ok[U];
+  uint32_t rows[U];
+  auto fetch = [&](uint32_t g0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t grp = g0 + u * waves_total;
@@ -1448,6 +1442,18 @@ __global__ __launch_bounds__(256) void gemv_smallk_kernel(typename Codec::Args a
       ok[u] = grp < groups && rows[u] < n;
       Codec::load(args, ln, ok[u] ? rows[u] : 0u, cpr, frag[u]);
     }
+  };
+  // The weights are asked for before the activations: a launch this short is the two trips to memory, one after
+  // the other or side by side (1024 x 1024: 5.2 -> 4.5 us).
+  fetch(wave_global);
+  typename Codec::template X<R> x;
+  if constexpr (Codec::kStageX) {
+    Codec::template load_x<R>(args, chunk, true, x, GlobalX{args.a, args.k});
+  } else {
+    Codec::template load_x<R>(args, chunk, true, x, 0);
+  }
+  for (uint32_t g0 = wave_global; g0 < groups; g0 += waves_total * U) {
+    if (g0 != wave_global) fetch(g0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       float v[R];
@@ -1610,8 +1616,12 @@ hipError_t launch_gemv_r(const typename Codec::Args& args, float* c, uint32_t n,
       constexpr int U = D > 4 ? 4 : D;
       const uint32_t rows_per_wave = 64u / cpr;
       const uint32_t groups = (n + rows_per_wave - 1) / rows_per_wave;
-      uint32_t grid = (groups + 4u * U - 1) / (4u * U);
       const uint32_t cap = static_cast<uint32_t>(g_num_cus) * 8u;
+      if (groups <= static_cast<uint32_t>(g_num_cus) * 4u) {   // fewer groups than the chip has SIMDs: one a wavefront
+        hipLaunchKernelGGL((gemv_smallk_kernel<Codec, R, 1>), dim3((groups + 3u) / 4u), dim3(256), 0, stream, args, c, n, cpr, ldc);
+        return hipGetLastError();
+      }
+      uint32_t grid = (groups + 4u * U - 1) / (4u * U);
       grid = grid > cap ? cap : (grid == 0 ? 1 : grid);
       hipLaunchKernelGGL((gemv_smallk_kernel<Codec, R, U>), dim3(grid), dim3(256), 0, stream, args, c,
                          n, cpr, ldc);
