@@ -516,13 +516,15 @@ __global__ __launch_bounds__(256) void top_k_short_rows_kernel(const float* __re
 // list that grows past kKeep is cut down by the same rule over its own entries.  At the end every entry
 // counts the entries above it, which is its place.  One workgroup and no scratch memory, so launches on
 // different streams stay independent; one row of 131072 with 8 places takes 27 us, where one pass over
-// the row for each place took 850 us.
+// the row for each place took 850 us.  Where the stream has a scratch block, workgroups share a row: each leaves the
+// largest keys of its columns there and top_k_merge_kernel ranks them (the same row 5 and 5 us).
 constexpr uint32_t kTopKThreads = 1024, kTopKPerTile = 8, kTopKTile = kTopKThreads * kTopKPerTile;
 constexpr uint32_t kTopKKeep = 1024, kTopKList = kTopKKeep + kTopKTile;
 
 __global__ __launch_bounds__(kTopKThreads) void top_k_long_rows_kernel(const float* __restrict__ logits,
                                                                        uint32_t* __restrict__ ids, float* __restrict__ vals,
-                                                                       uint32_t vocab, uint32_t top_k, uint64_t row_base) {
+                                                                       uint32_t vocab, uint32_t top_k, uint64_t row_base,
+                                                                       uint32_t share, uint64_t* __restrict__ keys) {
   __shared__ uint64_t list[kTopKList];
   __shared__ uint64_t wave_top[32];
   __shared__ uint64_t bound_s;
@@ -556,9 +558,11 @@ __global__ __launch_bounds__(kTopKThreads) void top_k_long_rows_kernel(const flo
       next[j] = row[c < vocab ? c : vocab - 1u];
     }
   };
-  load(0);
-  const uint32_t tiles = (vocab + kTopKTile - 1u) / kTopKTile;
-  for (uint32_t t = 0; t < tiles; ++t) {
+  // `share` tiles of the row for each workgroup of grid.y (keys null: all of them, and the places at once)
+  const uint32_t all_tiles = (vocab + kTopKTile - 1u) / kTopKTile, first_tile = blockIdx.y * share;
+  const uint32_t tiles = all_tiles - first_tile < share ? all_tiles : first_tile + share;
+  load(first_tile);
+  for (uint32_t t = first_tile; t < tiles; ++t) {
     uint64_t key[kTopKPerTile];
 #pragma unroll
     for (uint32_t j = 0; j < kTopKPerTile; ++j) {
@@ -566,7 +570,7 @@ __global__ __launch_bounds__(kTopKThreads) void top_k_long_rows_kernel(const flo
       key[j] = c < vocab ? top_k_key(next[j], c) : 0ull;
     }
     if (t + 1u < tiles) load(t + 1u);
-    if (t == 0u) {
+    if (t == first_tile) {
       uint64_t most = 0ull;
 #pragma unroll
       for (uint32_t j = 0; j < kTopKPerTile; ++j) most = key[j] > most ? key[j] : most;
@@ -602,11 +606,33 @@ __global__ __launch_bounds__(kTopKThreads) void top_k_long_rows_kernel(const flo
     const uint64_t mine = list[tid];
     uint32_t above = 0u;
     for (uint32_t i = 0; i < count; ++i) above += list[i] > mine ? 1u : 0u;
-    if (above < top_k) {
+    if (above < top_k && keys != nullptr) {
+      keys[(static_cast<size_t>(blockIdx.x) * gridDim.y + blockIdx.y) * top_k + above] = mine;
+    } else if (above < top_k) {
       const uint32_t c = top_k_column(mine);
       ids[static_cast<size_t>(blockIdx.x) * top_k + above] = c;
       vals[static_cast<size_t>(blockIdx.x) * top_k + above] = row[c];
     }
+  }
+}
+
+// The top_k of a row's shares: every key counts the keys above it, which is its place.
+constexpr uint32_t kTopKShares = 16;
+__global__ __launch_bounds__(512) void top_k_merge_kernel(const uint64_t* __restrict__ keys, const float* __restrict__ logits,
+                                                          uint32_t* __restrict__ ids, float* __restrict__ vals, uint32_t vocab,
+                                                          uint32_t top_k, uint64_t row_base, uint32_t shares) {
+  __shared__ uint64_t list[kTopKShares * 32u];
+  const uint32_t t = threadIdx.x, count = shares * top_k;
+  const uint64_t mine = t < count ? keys[static_cast<size_t>(blockIdx.x) * count + t] : 0ull;
+  if (t < count) list[t] = mine;
+  __syncthreads();
+  if (t >= count) return;
+  uint32_t above = 0u;
+  for (uint32_t i = 0; i < count; ++i) above += list[i] > mine ? 1u : 0u;
+  if (above < top_k) {
+    const uint32_t c = top_k_column(mine);
+    ids[static_cast<size_t>(blockIdx.x) * top_k + above] = c;
+    vals[static_cast<size_t>(blockIdx.x) * top_k + above] = logits[(row_base + blockIdx.x) * vocab + c];
   }
 }
 
@@ -930,8 +956,24 @@ hipError_t launch_moe_gate(const float* vals, const float* x, const float* w, fl
   return hipGetLastError();
 }
 
+// Tiles of a row that a workgroup takes where a row is shared; the last share too holds top_k columns or more.
+static uint32_t top_k_share(uint64_t vocab, uint32_t top_k) {
+  const uint64_t tiles = (vocab + kTopKTile - 1u) / kTopKTile;
+  uint64_t share = (tiles + kTopKShares - 1u) / kTopKShares;
+  while (share < tiles && (vocab - (tiles - 1u) / share * share * kTopKTile) < top_k) ++share;
+  return static_cast<uint32_t>(share);
+}
+
+// Rows are shared where they are few and long (one row of 131072: 27 us, shared 10).
+size_t top_k_rows_scratch_bytes(uint32_t rows, uint64_t vocab, uint32_t top_k) {
+  const uint64_t tiles = (vocab + kTopKTile - 1u) / kTopKTile;
+  if (rows > 16u || tiles < 4u) return 0;
+  const uint64_t share = top_k_share(vocab, top_k), shares = (tiles + share - 1u) / share;
+  return shares < 2u ? 0 : static_cast<size_t>(rows * shares * top_k) * 8u;
+}
+
 hipError_t launch_top_k_rows(const float* logits, uint32_t* ids, float* vals, uint32_t rows,
-                             uint64_t vocab, uint32_t top_k, uint64_t row_base, hipStream_t stream) {
+                             uint64_t vocab, uint32_t top_k, uint64_t row_base, void* scratch, hipStream_t stream) {
   // Up to 512 columns fit the registers of one wavefront; a workgroup of sixteen has a tile of 8192 to
   // itself beyond that.
   const uint32_t v = static_cast<uint32_t>(vocab);
@@ -940,12 +982,18 @@ hipError_t launch_top_k_rows(const float* logits, uint32_t* ids, float* vals, ui
     hipLaunchKernelGGL(top_k_short_rows_kernel<4>, four_rows, dim3(256), 0, stream, logits, ids, vals, rows, v, top_k, row_base);
   } else if (vocab <= 512) {
     hipLaunchKernelGGL(top_k_short_rows_kernel<8>, four_rows, dim3(256), 0, stream, logits, ids, vals, rows, v, top_k, row_base);
+  } else if (scratch != nullptr) {
+    const uint32_t tiles = (v + kTopKTile - 1u) / kTopKTile, share = top_k_share(vocab, top_k), shares = (tiles + share - 1u) / share;
+    uint64_t* keys = static_cast<uint64_t*>(scratch);
+    hipLaunchKernelGGL(top_k_long_rows_kernel, dim3(rows, shares), dim3(kTopKThreads), 0, stream, logits, ids, vals, v, top_k,
+                       row_base, share, keys);
+    hipLaunchKernelGGL(top_k_merge_kernel, dim3(rows), dim3(512), 0, stream, keys, logits, ids, vals, v, top_k, row_base, shares);
   } else {
     constexpr uint32_t kMost = static_cast<uint32_t>(kMaxGridThreads / kTopKThreads) - 1u;   // rows of one launch
     for (uint32_t r = 0; r < rows; r += kMost) {
       const size_t at = static_cast<size_t>(r) * top_k;
       hipLaunchKernelGGL(top_k_long_rows_kernel, dim3(rows - r < kMost ? rows - r : kMost), dim3(kTopKThreads), 0, stream, logits,
-                         ids + at, vals + at, v, top_k, row_base + r);
+                         ids + at, vals + at, v, top_k, row_base + r, (v + kTopKTile - 1u) / kTopKTile, static_cast<uint64_t*>(nullptr));
     }
   }
   return hipGetLastError();

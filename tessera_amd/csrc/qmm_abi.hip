@@ -156,7 +156,7 @@ void* decode_scratch(const LaunchCtx& c) {
   return c.no_alloc ? g_static_scratch[g_device] : g_decode_scratch;
 }
 
-// Scratch of "gemm_fp8", of Q5_K / Q6_K with a few rows and of "attention" with few columns and of "gemm_mxfp4" from 17 rows, whose calls on different streams are independent of
+// Scratch of "gemm_fp8", of Q5_K / Q6_K with a few rows and of "attention" with few columns, of "gemm_mxfp4" from 17 rows and of "top_k_rows" over long rows, whose calls on different streams are independent of
 // one another: see stream_scratch.hpp.  qmm_init reserves the first slab; later ones are allocated under the
 // relaxed capture mode, which permits it while a stream is captured, unless the caller has handed over a workspace
 // (then a launch allocates nothing).
@@ -1317,9 +1317,11 @@ qmm_status run_top_k_rows(const LaunchCtx& c) {
       !c.fits(2, static_cast<u128>(rows) * top_k * 4)) {
     return bad("top_k_rows: buffer too small");
   }
+  const size_t keys = qmm::top_k_rows_scratch_bytes(static_cast<uint32_t>(rows), vocab, static_cast<uint32_t>(top_k));
+  const StreamBlock block(c, keys);
   return map_hip(qmm::launch_top_k_rows(c.ptr<const float>(0), c.ptr<uint32_t>(1), c.ptr<float>(2),
                                         static_cast<uint32_t>(rows), vocab, static_cast<uint32_t>(top_k), base,
-                                        c.stream));
+                                        keys == 0 ? nullptr : block.get(), c.stream));
 }
 
 // "moe_experts_ffn_q4k_rows" (not a reference id): the routed-expert feed-forward of a chunk

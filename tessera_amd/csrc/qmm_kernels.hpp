@@ -224,8 +224,10 @@ hipError_t launch_dequant_mxfp4(const uint8_t* w, float* out, uint64_t n, uint64
                                 hipStream_t stream);
 hipError_t launch_moe_gate(const float* vals, const float* x, const float* w, float* wts, float* sig,
                            uint32_t top_k, uint32_t hidden, hipStream_t stream);
-hipError_t launch_top_k_rows(const float* logits, uint32_t* ids, float* vals, uint32_t rows,
-                             uint64_t vocab, uint32_t top_k, uint64_t row_base, hipStream_t stream);
+// top_k_rows_scratch_bytes: what shared rows' keys take of `scratch`, which may be null (rows are then not shared).
+size_t top_k_rows_scratch_bytes(uint32_t rows, uint64_t vocab, uint32_t top_k);
+hipError_t launch_top_k_rows(const float* logits, uint32_t* ids, float* vals, uint32_t rows, uint64_t vocab, uint32_t top_k,
+                             uint64_t row_base, void* scratch, hipStream_t stream);
 hipError_t launch_moe_scale_add(const float* a, const float* b, const float* f, float* o,
                                 uint64_t n, uint64_t idx, hipStream_t stream);
 
