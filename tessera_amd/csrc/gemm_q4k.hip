@@ -74,6 +74,24 @@ void launch_range(const _Float16* a16, const float* a_scale, const uint8_t* w, f
                      a16, a_scale, w, c, m, n, k, n_begin, n_end);
 }
 
+// silu(A Wg^T) * (A Wu^T) on columns n_begin .. n_end, BN / 2 of them a tile.
+template <int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void q4k_gate_up_kernel(
+    const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const uint8_t* __restrict__ gate, const uint8_t* __restrict__ up,
+    float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end) {
+  const uint32_t tiles_n = (n_end - n_begin + BN / 2 - 1) / (BN / 2);
+  q4k_gemm_tile<BM, BN, WM, WN, true>(a16, a_scale, gate, c, m, n, k, (blockIdx.x / tiles_n) * BM,
+                                      n_begin + (blockIdx.x % tiles_n) * (BN / 2), n_end, up);
+}
+
+template <int BM, int BN, int WM, int WN>
+void launch_pair_range(const _Float16* a16, const float* a_scale, const uint8_t* gate, const uint8_t* up, float* c, uint32_t m,
+                       uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end, hipStream_t stream) {
+  const uint32_t tiles = ((m + BM - 1) / BM) * ((n_end - n_begin + BN / 2 - 1) / (BN / 2));
+  hipLaunchKernelGGL((q4k_gate_up_kernel<BM, BN, WM, WN>), dim3(tiles), dim3(tile_waves<BM, BN, WM, WN>() * 64), 0, stream,
+                     a16, a_scale, gate, up, c, m, n, k, n_begin, n_end);
+}
+
 }  // namespace
 
 void launch_rows_to_f16(const float* src, _Float16* dst, float* scale, uint32_t rows, uint32_t cols, const uint32_t* pos,
@@ -116,6 +134,27 @@ hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* wor
   const uint32_t n_split = main_tn * 256u < n ? main_tn * 256u : n;
   if (n_split > 0) launch_range<256, 256, 128, 64>(a16, a_scale, w, c, m, n, k, 0u, n_split, stream);
   if (n_split < n) launch_range<128, 64, 64, 32>(a16, a_scale, w, c, m, n, k, n_split, n, stream);
+  return hipGetLastError();
+}
+
+// The feed forward's front half in one product: tiles as launch_q4k_gemm's, 128 columns of either matrix each.  2048 rows of
+// 17408 x 5120: 858 us, as two products and silu_mul 940.
+hipError_t launch_q4k_gate_up(const float* a, const uint8_t* gate, const uint8_t* up, float* c, void* workspace, uint32_t m,
+                              uint32_t n, uint32_t k, hipStream_t stream) {
+  _Float16* a16 = static_cast<_Float16*>(workspace);
+  float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
+  launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
+  const uint32_t cus = static_cast<uint32_t>(num_cus());
+  const uint32_t tiles_m = (m + 255u) / 256u, tiles_n = (n + 127u) / 128u, tiles = tiles_m * tiles_n;
+  uint32_t main_tn = tiles_n;
+  if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) {
+    main_tn = (tiles / cus) * cus / tiles_m;
+  } else if (tiles < cus / 2) {
+    main_tn = 0;
+  }
+  const uint32_t n_split = main_tn * 128u < n ? main_tn * 128u : n;
+  if (n_split > 0) launch_pair_range<256, 256, 128, 64>(a16, a_scale, gate, up, c, m, n, k, 0u, n_split, stream);
+  if (n_split < n) launch_pair_range<128, 128, 64, 64>(a16, a_scale, gate, up, c, m, n, k, n_split, n, stream);
   return hipGetLastError();
 }
 

@@ -137,16 +137,23 @@ constexpr int tile_waves() { return (BM / WM) * (BN / WN); }
 // wavefront, against 128 bytes a clock for the whole CU, which four SIMDs running 32-clock MFMAs
 // would need in full); with WN = 64 a fragment read feeds two MFMAs.  The price is that the
 // BM / WM wavefronts that share a column range each decode its weights.
-template <int BM, int BN, int WM, int WN>
+//
+// PAIR: silu(A Wg^T) * (A Wu^T), gate weights `w` and up weights `w_up`.  The tile's columns are BN / 2 of either
+// matrix and a wavefront's two column tiles the same columns of both, so that the two products meet in its registers:
+// no product goes to memory, and the activations are read once.
+template <int BM, int BN, int WM, int WN, bool PAIR = false>
 __device__ __forceinline__ void q4k_gemm_tile(
     const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const uint8_t* __restrict__ w,
-    float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t m0, uint32_t n0, uint32_t n_end) {
+    float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t m0, uint32_t n0, uint32_t n_end,
+    const uint8_t* __restrict__ w_up = nullptr) {
   constexpr int kWaves = tile_waves<BM, BN, WM, WN>();
   constexpr int kWavesN = BN / WN;
   constexpr int kTI = WM / 32, kTJ = WN / 32;      // MFMA tiles per wavefront: rows x columns
   constexpr int kABlk = BM / 16 / kWaves;          // 1 KB activation blocks a wavefront loads per step
   constexpr int kWL = (BN * 9 + 64 * kWaves - 1) / (64 * kWaves);  // 1 KB weight blocks per super-block
   constexpr uint32_t kAStage = BM * 64, kWStage = kWL * kWaves * 1024;
+  constexpr uint32_t kJRows = PAIR ? BN / 2 : 32;  // weight rows from a wavefront's column tile to its next
+  static_assert(!PAIR || (kTJ == 2 && BN * 9 % 128 == 0), "a load block lies in one matrix");
   static_assert(BM % WM == 0 && BN % WN == 0 && WM % 32 == 0 && WN % 32 == 0 && BM % (16 * kWaves) == 0, "tile shape");
   __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kAStage + 2 * kWStage];
 
@@ -159,6 +166,7 @@ __device__ __forceinline__ void q4k_gemm_tile(
       (__attribute__((address_space(3))) uint8_t*)lds));
   const uint8_t* a_tile = reinterpret_cast<const uint8_t*>(a16) + static_cast<size_t>(m0) * k * 2;
   const uint8_t* w_tile = w + static_cast<size_t>(n0) * row_blocks * 144;
+  const uint8_t* up_tile = PAIR ? w_up + static_cast<size_t>(n0) * row_blocks * 144 : nullptr;
 
   // Direct loads.  Activation block L of a step (1 KB, rows 16L..16L+15, four 16-byte chunks
   // a row): lane p fetches row 16L + p/4, chunk (p%4) ^ ((row>>2)&3).  Weight chunk q of a
@@ -176,7 +184,7 @@ __device__ __forceinline__ void q4k_gemm_tile(
   for (int i = 0; i < kWL; ++i) {
     uint32_t q = (wave * kWL + i) * 64u + lane;
     q = q < BN * 9u ? q : BN * 9u - 1u;
-    const uint32_t row = q / 9u, part = q % 9u;
+    const uint32_t row = PAIR ? q / 9u % (BN / 2) : q / 9u, part = q % 9u;
     w_src[i] = (n0 + row < n ? row : n - 1u - n0) * (row_blocks * 144u) + part * 16u;
   }
   auto issue_a = [&](uint32_t stage, uint32_t slice) {      // slice = 32 K values = 64 bytes a row
@@ -185,9 +193,11 @@ __device__ __forceinline__ void q4k_gemm_tile(
     for (int i = 0; i < kABlk; ++i) direct_load16(g, a_src[i], lds_base + stage * kAStage + (wave * kABlk + i) * 1024u);
   };
   auto issue_w = [&](uint32_t stage, uint32_t block) {
-    const uint8_t* g = w_tile + block * 144u;
 #pragma unroll
-    for (int i = 0; i < kWL; ++i) direct_load16(g, w_src[i], lds_base + 4 * kAStage + stage * kWStage + (wave * kWL + i) * 1024u);
+    for (int i = 0; i < kWL; ++i) {
+      const uint8_t* g = (PAIR && (wave * kWL + i) * 128u >= BN * 9u ? up_tile : w_tile) + block * 144u;
+      direct_load16(g, w_src[i], lds_base + 4 * kAStage + stage * kWStage + (wave * kWL + i) * 1024u);
+    }
   };
 
   float16_t acc[kTI][kTJ];
@@ -201,7 +211,7 @@ __device__ __forceinline__ void q4k_gemm_tile(
   // This lane's first weight row inside a raw stage (column tile j is 32 rows further), and its
   // activation fragment offsets: MFMA step t of a slice takes chunk 2kg + t of the row
   // (k = 16kg + 8t + [0,8), the positions decode_subblock gives the step).
-  const uint32_t w_row = (wave_n * WN + l32) * 144u;
+  const uint32_t w_row = (wave_n * (PAIR ? 32u : WN) + l32) * 144u;
   uint32_t a_fr[2];
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt) a_fr[tt] = (wave_m * WM + l32) * 64u + (((kg * 2u + tt) ^ ((l32 >> 2) & 3u)) * 16u);
@@ -221,7 +231,7 @@ __device__ __forceinline__ void q4k_gemm_tile(
     const bool more = blk + 1 < row_blocks;        // uniform
     BlockHead head[kTJ];
 #pragma unroll
-    for (int j = 0; j < kTJ; ++j) head[j] = load_block_head(raw + j * 32 * 144);
+    for (int j = 0; j < kTJ; ++j) head[j] = load_block_head(raw + j * kJRows * 144);
     uint32_t qw[kTJ][4], qs8[kTJ][4];
     unrolled<8>([&](auto step) {
       constexpr int sb = decltype(step)::value;
@@ -231,7 +241,7 @@ __device__ __forceinline__ void q4k_gemm_tile(
 
       half8_t b[kTJ][2];
 #pragma unroll
-      for (int j = 0; j < kTJ; ++j) decode_subblock<sb>(raw + j * 32 * 144, kg, head[j], qw[j], qs8[j], b[j]);
+      for (int j = 0; j < kTJ; ++j) decode_subblock<sb>(raw + j * kJRows * 144, kg, head[j], qw[j], qs8[j], b[j]);
 
       const uint8_t* a_stage = lds + (slice & 3u) * kAStage;
 #pragma unroll
@@ -265,6 +275,18 @@ __device__ __forceinline__ void q4k_gemm_tile(
     float4 sc[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) sc[q] = *reinterpret_cast<const float4*>(a_scale + row0 + q * 8u);
+    if constexpr (PAIR) {
+      const uint32_t col = n0 + wave_n * 32u + l32;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const uint32_t row = row0 + (e >> 2) * 8u + (e & 3u);
+        const float4 s4 = sc[e >> 2];
+        const float rs = (e & 3) == 0 ? s4.x : (e & 3) == 1 ? s4.y : (e & 3) == 2 ? s4.z : s4.w;
+        const float gate = acc[i][0][e] * rs, up = acc[i][1][e] * rs;
+        if (row < m && col < n_end) c[static_cast<size_t>(row) * n + col] = (gate / (1.0f + expf(-gate))) * up;
+      }
+      continue;
+    }
 #pragma unroll
     for (int j = 0; j < kTJ; ++j) {
       const uint32_t col = n0 + wave_n * WN + j * 32u + l32;

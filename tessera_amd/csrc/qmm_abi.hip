@@ -749,6 +749,14 @@ qmm_status run_ffn_gate_up_silu_q4k(const LaunchCtx& c) {
   if (m == 1 && qmm::ffn_gate_up_q4k_supported(k)) {
     return map_hip(qmm::launch_ffn_gate_up_q4k(x, gate, up, out, static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
   }
+  // The tensor tile takes both products at once where it fills its rows.
+  if (m > 64 && m >= g_q4k_tensor_rows.load(std::memory_order_relaxed) && qmm::gemm_q4k_supported(m, k)) {
+    void* ws = nullptr;
+    const qmm_status st = workspace(c, qmm::gemm_q4k_workspace_bytes(m, k), &ws);
+    if (st != QMM_OK) return st;
+    return map_hip(qmm::launch_q4k_gate_up(x, gate, up, out, ws, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
+                                           static_cast<uint32_t>(k), c.stream));
+  }
   const FfnScratch lay = ffn_scratch(m, n, k);
   float* u = nullptr;
   qmm_status st = QMM_OK;

@@ -123,6 +123,9 @@ hipError_t launch_mxfp4_f32_gemm(const float* a, const uint8_t* w, float* c, voi
 // Q4_K prefill GEMM on fp16 MFMA (gemm_q4k.hip).  `workspace` holds m*k fp16 values.
 bool gemm_q4k_supported(uint64_t m, uint64_t k);
 size_t gemm_q4k_workspace_bytes(uint64_t m, uint64_t k);
+// silu(A gate^T) * (A up^T) for more than 64 rows, with gemm_q4k_workspace_bytes(m, k) of workspace.
+hipError_t launch_q4k_gate_up(const float* a, const uint8_t* gate, const uint8_t* up, float* c, void* workspace, uint32_t m,
+                              uint32_t n, uint32_t k, hipStream_t stream);
 hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* workspace, uint32_t m,
                            uint32_t n, uint32_t k, hipStream_t stream);
 
