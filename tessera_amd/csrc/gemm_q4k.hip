@@ -250,21 +250,27 @@ __global__ __launch_bounds__(256) void q5k_to_f16_kernel(const uint8_t* __restri
 }
 
 // C tile = A16 (rows scaled by a_scale) . W16^T, both operands fp16 row-major with row length k.
-template <int BM, int BN>
-__global__ __launch_bounds__(BN * 2) void f16w_gemm_kernel(
+//
+// A wavefront owns WM rows x WN columns.  An operand read from LDS is 1 KB a wavefront against 128 bytes a clock for the
+// CU, and four SIMDs start a matrix instruction of 32 clocks each: 128 x 64 takes six reads to eight instructions, 64 x 96
+// five to six (256 x 32, nine to eight, was bound by them: 160 tiles of 2048 rows x 5120 columns, K = 17408, 500 us).  The
+// reads of a 16-wide K step go between the matrix instructions of the one before.
+template <int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
     const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const _Float16* __restrict__ w16,
     float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end) {
-  constexpr int kWaves = BN / 32, kTI = BM / 32;
-  constexpr int kABlk = BM / 16 / kWaves, kWBlk = BN / 16 / kWaves;   // 1 KB blocks per wavefront and slice
+  constexpr int kWavesN = BN / WN, kWaves = (BM / WM) * kWavesN, kTI = WM / 32, kTJ = WN / 32;
+  constexpr int kABlk = BM / 16 / kWaves, kWBlk = (BN / 16 + kWaves - 1) / kWaves;   // 1 KB blocks per wavefront and slice
   constexpr int kDma = kABlk + kWBlk;
-  constexpr uint32_t kAStage = BM * 64, kWStage = BN * 64, kStage = kAStage + kWStage;
-  static_assert(BM % (16 * kWaves) == 0 && BN % (16 * kWaves) == 0, "tile shape");
+  constexpr uint32_t kAStage = BM * 64, kWStage = kWBlk * kWaves * 1024, kStage = kAStage + kWStage;
+  static_assert(BM % (16 * kWaves) == 0 && BN % 16 == 0 && WM % 32 == 0 && WN % 32 == 0, "tile shape");
   __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kStage];
 
   const uint32_t tiles_n = (n_end - n_begin + BN - 1) / BN;
   const uint32_t m0 = (blockIdx.x / tiles_n) * BM, n0 = n_begin + (blockIdx.x % tiles_n) * BN;
   const uint32_t t = threadIdx.x, lane = t & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t wave_m = wave / kWavesN, wave_n = wave % kWavesN;
   const uint32_t l32 = lane & 31u, kg = lane >> 5;
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
       (__attribute__((address_space(3))) uint8_t*)lds));
@@ -272,7 +278,8 @@ __global__ __launch_bounds__(BN * 2) void f16w_gemm_kernel(
   const uint8_t* w_tile = reinterpret_cast<const uint8_t*>(w16) + static_cast<size_t>(n0) * k * 2;
 
   // Block L of a slice = rows 16L..16L+15, four 16-byte chunks a row: lane p fetches row
-  // 16L + p/4, chunk (p%4) ^ ((row>>2)&3).  Rows past the matrix edge are clamped (never stored).
+  // 16L + p/4, chunk (p%4) ^ ((row>>2)&3).  Rows past the matrix edge are clamped (never stored), and so are
+  // those of blocks past the tile, which where BN / 16 does not divide go to spare LDS.
   uint32_t a_src[kABlk], w_src[kWBlk];
 #pragma unroll
   for (int i = 0; i < kABlk; ++i) {
@@ -281,11 +288,12 @@ __global__ __launch_bounds__(BN * 2) void f16w_gemm_kernel(
   }
 #pragma unroll
   for (int i = 0; i < kWBlk; ++i) {
-    const uint32_t row = 16u * (wave * kWBlk + i) + lane / 4u;
+    const uint32_t row_any = 16u * (wave * kWBlk + i) + lane / 4u, row = row_any < BN ? row_any : BN - 1u;
     w_src[i] = (n0 + row < n ? row : n - 1u - n0) * (k * 2u) + (((lane % 4u) ^ ((row >> 2) & 3u)) * 16u);
   }
-  auto issue = [&](uint32_t stage, uint32_t slice_any) {
-    const uint32_t slice = __builtin_amdgcn_readfirstlane(slice_any);
+  const uint32_t slices = k / 32;
+  auto issue = [&](uint32_t slice_any) {
+    const uint32_t slice = __builtin_amdgcn_readfirstlane(slice_any < slices ? slice_any : slices - 1u), stage = slice_any & 3u;
 #pragma unroll
     for (int i = 0; i < kABlk; ++i)
       direct_load16(a_tile + slice * 64u, a_src[i], lds_base + stage * kStage + (wave * kABlk + i) * 1024u);
@@ -294,52 +302,92 @@ __global__ __launch_bounds__(BN * 2) void f16w_gemm_kernel(
       direct_load16(w_tile + slice * 64u, w_src[i], lds_base + stage * kStage + kAStage + (wave * kWBlk + i) * 1024u);
   };
 
-  float16_t acc[kTI];
+  float16_t acc[kTI][kTJ];
 #pragma unroll
   for (int i = 0; i < kTI; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
-  uint32_t fr[2];   // fragment offset inside a 32-row group: MFMA step tt takes chunk 2tt + kg
+    for (int j = 0; j < kTJ; ++j)
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt) fr[tt] = l32 * 64u + (((tt * 2u + kg) ^ ((l32 >> 2) & 3u)) * 16u);
-
-  const uint32_t slices = k / 32;
-  issue(0, 0);
-  issue(1, slices > 1 ? 1 : 0);
-  issue(2, slices > 2 ? 2 : slices - 1);
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kDma) : "memory");
-  for (uint32_t slice = 0; slice < slices; ++slice) {
-    issue((slice + 3u) & 3u, slice + 3u < slices ? slice + 3u : slices - 1u);
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  uint32_t a_fr[2], w_fr[2];   // fragment offsets: MFMA step tt takes chunk 2tt + kg
+#pragma unroll
+  for (int tt = 0; tt < 2; ++tt) {
+    const uint32_t at = l32 * 64u + (((tt * 2u + kg) ^ ((l32 >> 2) & 3u)) * 16u);
+    a_fr[tt] = wave_m * (WM * 64u) + at, w_fr[tt] = kAStage + wave_n * (WN * 64u) + at;
+  }
+  struct Frag {
+    half8_t a[kTI], b[kTJ];
+  };
+  auto read = [&](uint32_t slice, int tt, Frag& f) {
     const uint8_t* stage = lds + (slice & 3u) * kStage;
-    half8_t b[2];
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) b[tt] = *reinterpret_cast<const half8_t*>(stage + kAStage + wave * 32 * 64 + fr[tt]);
+    for (int j = 0; j < kTJ; ++j) f.b[j] = *reinterpret_cast<const half8_t*>(stage + w_fr[tt] + j * 32 * 64);
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
+    for (int i = 0; i < kTI; ++i) f.a[i] = *reinterpret_cast<const half8_t*>(stage + a_fr[tt] + i * 32 * 64);
+  };
+  // The matrix instructions of `f`, the reads of `g` spread among them.
+  auto multiply_reading = [&](const Frag& f, uint32_t slice, int tt, Frag& g) {
+    read(slice, tt, g);
 #pragma unroll
-      for (int i = 0; i < kTI; ++i) {
-        const half8_t af = *reinterpret_cast<const half8_t*>(stage + fr[tt] + i * 32 * 64);
-        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, b[tt], acc[i], 0, 0, 0);
-      }
+    for (int i = 0; i < kTI; ++i)
+#pragma unroll
+      for (int j = 0; j < kTJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
+    constexpr int kMost = kTI * kTJ > kTI + kTJ ? kTI * kTJ : kTI + kTJ;
+#pragma unroll
+    for (int q = 0; q < kMost; ++q) {
+      if (q < kTI * kTJ) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (q < kTI + kTJ) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
+  };
+
+  issue(0);
+  issue(1);
+  issue(2);
+  issue(3);
+  Frag f0, f1;
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * kDma) : "memory");
+  read(0, 0, f0);
+  for (uint32_t slice = 0; slice < slices; ++slice) {
+    multiply_reading(f0, slice, 1, f1);
+    if constexpr (kWaves == 8) {       // keeps these matrix instructions on this side of the barrier
+#pragma unroll
+      for (int i = 0; i < kTI; ++i)
+#pragma unroll
+        for (int j = 0; j < kTJ; ++j) asm volatile("" : "+v"(acc[i][j]));
+    }
+    // slice + 1 has landed; every wavefront has read all of `slice`, whose stage takes slice + 4
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kDma) : "memory");
+    issue(slice + 4u);
+    multiply_reading(f1, slice + 1u, 0, f0);    // (after the last slice: a stage that nobody needs)
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct load may outlive the workgroup
 
-  const uint32_t col = n0 + wave * 32u + l32;
 #pragma unroll
   for (int i = 0; i < kTI; ++i) {
+    const uint32_t row0 = m0 + wave_m * WM + i * 32u + kg * 4u;
     float4 sc[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) sc[q] = *reinterpret_cast<const float4*>(a_scale + m0 + i * 32u + q * 8u + kg * 4u);
+    for (int q = 0; q < 4; ++q) sc[q] = *reinterpret_cast<const float4*>(a_scale + row0 + q * 8u);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const uint32_t row = m0 + i * 32u + (e >> 2) * 8u + kg * 4u + (e & 3u);
-      const float4 s4 = sc[e >> 2];
-      const float rs = (e & 3) == 0 ? s4.x : (e & 3) == 1 ? s4.y : (e & 3) == 2 ? s4.z : s4.w;
-      if (row < m && col < n_end) c[static_cast<size_t>(row) * n + col] = acc[i][e] * rs;
+    for (int j = 0; j < kTJ; ++j) {
+      const uint32_t col = n0 + wave_n * WN + j * 32u + l32;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const uint32_t row = row0 + (e >> 2) * 8u + (e & 3u);
+        const float4 s4 = sc[e >> 2];
+        const float rs = (e & 3) == 0 ? s4.x : (e & 3) == 1 ? s4.y : (e & 3) == 2 ? s4.z : s4.w;
+        if (row < m && col < n_end) c[static_cast<size_t>(row) * n + col] = acc[i][j][e] * rs;
+      }
     }
   }
+}
+
+template <int BM, int BN, int WM, int WN>
+void launch_f16w_range(const _Float16* a16, const float* a_scale, const _Float16* w16, float* c, uint32_t m, uint32_t n, uint32_t k,
+                       uint32_t n_begin, uint32_t n_end, hipStream_t stream) {
+  const uint32_t tiles = ((m + BM - 1) / BM) * ((n_end - n_begin + BN - 1) / BN);
+  hipLaunchKernelGGL((f16w_gemm_kernel<BM, BN, WM, WN>), dim3(tiles), dim3((BM / WM) * (BN / WN) * 64), 0, stream, a16, a_scale,
+                     w16, c, m, n, k, n_begin, n_end);
 }
 
 }  // namespace
@@ -370,24 +418,25 @@ hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t blo
     return hipErrorInvalidValue;
   }
   launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
-  // whole rounds of 256 x 256 tiles, leftover columns as 128 x 64 tiles (as launch_q4k_gemm)
-  const uint32_t cus = static_cast<uint32_t>(num_cus());
-  const uint32_t tiles_m = (m + 255u) / 256u, tiles_n = (n + 255u) / 256u, tiles = tiles_m * tiles_n;
-  uint32_t main_tn = tiles_n;
-  if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) {
-    main_tn = (tiles / cus) * cus / tiles_m;
-  } else if (tiles < cus / 2) {
-    main_tn = 0;
-  }
-  const uint32_t n_split = main_tn * 256u < n ? main_tn * 256u : n;
-  if (n_split > 0) {
-    hipLaunchKernelGGL((f16w_gemm_kernel<256, 256>), dim3(tiles_m * main_tn), dim3(512), 0, stream, a16, a_scale, w16,
-                       c, m, n, k, 0u, n_split);
-  }
-  if (n_split < n) {
-    const uint32_t t2 = ((m + 127u) / 128u) * ((n - n_split + 63u) / 64u);
-    hipLaunchKernelGGL((f16w_gemm_kernel<128, 64>), dim3(t2), dim3(128), 0, stream, a16, a_scale, w16, c, m, n, k,
-                       n_split, n);
+  // Whole rounds of 256 x 256 tiles, leftover columns as 128 x 64 tiles (as launch_q4k_gemm).  Where the columns fit one
+  // round, the narrowest tile with which they still do: 2048 x 5120 as 216 tiles of 192 columns instead of 160 of 256.
+  const uint32_t cus = static_cast<uint32_t>(num_cus()), tiles_m = (m + 255u) / 256u;
+  auto tiles_of = [&](uint32_t bn) { return tiles_m * ((n + bn - 1u) / bn); };
+  const uint32_t tiles = tiles_of(256u);
+  if (tiles_of(128u) <= cus && tiles_of(128u) > cus / 2) {
+    launch_f16w_range<256, 128, 64, 64>(a16, a_scale, w16, c, m, n, k, 0u, n, stream);
+  } else if (tiles_of(192u) <= cus && tiles_of(192u) > cus / 2) {
+    launch_f16w_range<256, 192, 64, 96>(a16, a_scale, w16, c, m, n, k, 0u, n, stream);
+  } else {
+    uint32_t main_tn = (n + 255u) / 256u;
+    if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) {
+      main_tn = (tiles / cus) * cus / tiles_m;
+    } else if (tiles < cus / 2) {
+      main_tn = 0;
+    }
+    const uint32_t n_split = main_tn * 256u < n ? main_tn * 256u : n;
+    if (n_split > 0) launch_f16w_range<256, 256, 128, 64>(a16, a_scale, w16, c, m, n, k, 0u, n_split, stream);
+    if (n_split < n) launch_f16w_range<128, 64, 64, 32>(a16, a_scale, w16, c, m, n, k, n_split, n, stream);
   }
   return hipGetLastError();
 }
