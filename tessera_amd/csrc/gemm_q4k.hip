@@ -62,8 +62,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void q4k_gemm_kernel(
     const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const uint8_t* __restrict__ w,
     float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end) {
   const uint32_t tiles_n = (n_end - n_begin + BN - 1) / BN;
-  q4k_gemm_tile<BM, BN, WM, WN>(a16, a_scale, w, c, m, n, k, (blockIdx.x / tiles_n) * BM, n_begin + (blockIdx.x % tiles_n) * BN,
-                        n_end);
+  const TileAt at = xcd_tile(blockIdx.x, (m + BM - 1) / BM, tiles_n);
+  q4k_gemm_tile<BM, BN, WM, WN>(a16, a_scale, w, c, m, n, k, at.m * BM, n_begin + at.n * BN, n_end);
 }
 
 template <int BM, int BN, int WM = BM, int WN = 32>
@@ -80,8 +80,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void q4k_gate_up_kernel
     const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const uint8_t* __restrict__ gate, const uint8_t* __restrict__ up,
     float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end) {
   const uint32_t tiles_n = (n_end - n_begin + BN / 2 - 1) / (BN / 2);
-  q4k_gemm_tile<BM, BN, WM, WN, true>(a16, a_scale, gate, c, m, n, k, (blockIdx.x / tiles_n) * BM,
-                                      n_begin + (blockIdx.x % tiles_n) * (BN / 2), n_end, up);
+  const TileAt at = xcd_tile(blockIdx.x, (m + BM - 1) / BM, tiles_n);
+  q4k_gemm_tile<BM, BN, WM, WN, true>(a16, a_scale, gate, c, m, n, k, at.m * BM, n_begin + at.n * (BN / 2), n_end, up);
 }
 
 template <int BM, int BN, int WM, int WN>
@@ -267,7 +267,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
   __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kStage];
 
   const uint32_t tiles_n = (n_end - n_begin + BN - 1) / BN;
-  const uint32_t m0 = (blockIdx.x / tiles_n) * BM, n0 = n_begin + (blockIdx.x % tiles_n) * BN;
+  const TileAt at = xcd_tile(blockIdx.x, (m + BM - 1) / BM, tiles_n);
+  const uint32_t m0 = at.m * BM, n0 = n_begin + at.n * BN;
   const uint32_t t = threadIdx.x, lane = t & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const uint32_t wave_m = wave / kWavesN, wave_n = wave % kWavesN;
@@ -312,8 +313,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
   uint32_t a_fr[2], w_fr[2];   // fragment offsets: MFMA step tt takes chunk 2tt + kg
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt) {
-    const uint32_t at = l32 * 64u + (((tt * 2u + kg) ^ ((l32 >> 2) & 3u)) * 16u);
-    a_fr[tt] = wave_m * (WM * 64u) + at, w_fr[tt] = kAStage + wave_n * (WN * 64u) + at;
+    const uint32_t in = l32 * 64u + (((tt * 2u + kg) ^ ((l32 >> 2) & 3u)) * 16u);
+    a_fr[tt] = wave_m * (WM * 64u) + in, w_fr[tt] = kAStage + wave_n * (WN * 64u) + in;
   }
   struct Frag {
     half8_t a[kTI], b[kTJ];

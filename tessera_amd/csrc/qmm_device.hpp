@@ -147,6 +147,20 @@ __device__ __forceinline__ void direct_load16(const void* base, uint32_t voff, u
                :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
 
+// Tile of workgroup `b` of tiles_m x tiles_n, for kernels whose workgroups walk K side by side.  Workgroups go round the
+// eight XCDs, each with an L2 of its own: an XCD's take neighbours in an order of panels of four row tiles, so that the
+// 32 that run on it at once share four row tiles' and eight column tiles' operands.
+struct TileAt {
+  uint32_t m, n;
+};
+__device__ __forceinline__ TileAt xcd_tile(uint32_t b, uint32_t tiles_m, uint32_t tiles_n) {
+  const uint32_t tiles = tiles_m * tiles_n, x = b % 8u, share = tiles / 8u, rest = tiles % 8u;
+  const uint32_t s = x * share + (x < rest ? x : rest) + b / 8u;
+  const uint32_t panel = s / (4u * tiles_n), in = s - panel * 4u * tiles_n;
+  const uint32_t rows = tiles_m - panel * 4u < 4u ? tiles_m - panel * 4u : 4u;
+  return TileAt{panel * 4u + in % rows, in / rows};
+}
+
 __device__ __forceinline__ uint4 load_u4(const void* p) {
   return *reinterpret_cast<const uint4*>(p);
 }
