@@ -39,6 +39,16 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* g, const flo
   o[i] = (gate / (1.0f + expf(-gate))) * u[i];
 }
 
+// vec_reduce_kernel of two products and silu_mul of the sums, every operation as there.
+__global__ __launch_bounds__(256) void vec_reduce_silu_kernel(const float* __restrict__ gate, const float* __restrict__ up,
+                                                              float* __restrict__ c, uint64_t total, uint64_t split) {
+  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  float g = 0.0f, u = 0.0f;
+  for (uint64_t s = 0; s < split; ++s) g += gate[s * total + i], u += up[s * total + i];
+  c[i] = (g / (1.0f + expf(-g))) * u;
+}
+
 // "round_bf16": every fp32 value rounded in place to bfloat16 precision, nearest even, by the
 // reference's integer arithmetic on the bits (src/backends/rocm/rocm_kernels_basic.cpp:885-899;
 // NaN payloads and infinities go through the same add, as there).
@@ -646,6 +656,11 @@ hipError_t launch_vec_reduce(const float* part, float* c, uint64_t total, uint64
                              hipStream_t stream) {
   hipLaunchKernelGGL(vec_reduce_kernel, grid_for(total, 256), dim3(256), 0, stream, part, c, total,
                      split);
+  return hipGetLastError();
+}
+
+hipError_t launch_vec_reduce_silu(const float* gate, const float* up, float* c, uint64_t total, uint64_t split, hipStream_t stream) {
+  hipLaunchKernelGGL(vec_reduce_silu_kernel, grid_for(total, 256), dim3(256), 0, stream, gate, up, c, total, split);
   return hipGetLastError();
 }
 

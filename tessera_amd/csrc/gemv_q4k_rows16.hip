@@ -65,6 +65,8 @@ struct R16Args {
   const uint8_t* w;        // n rows of k/256 blocks
   float* c;                // m x n, the result
   float* ws;               // [parts][m][n] partial sums of the K parts (unused with one part)
+  const uint8_t* w2;       // a second matrix and its sums, taken by the workgroups of gridDim.z = 1
+  float* ws2;
   uint32_t m, n, k;
   uint32_t tiles_per_wg;
   uint32_t blocks_per_part;
@@ -124,6 +126,8 @@ __global__ __launch_bounds__(768) void q4k_rows16_kernel(R16Args p) {
   const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const uint32_t waves = blockDim.x >> 6;
   const uint32_t nrow = lane & 15u, gq = lane >> 4;        // weight row of the tile, K chunk of a sub-block
+  const uint8_t* w = blockIdx.z == 0u ? p.w : p.w2;
+  float* ws = blockIdx.z == 0u ? p.ws : p.ws2;
   uint32_t nbp = p.blocks_per_part, b0 = blockIdx.y * nbp;   // block columns of this K part
   uint32_t tiles_per_wg = p.tiles_per_wg, tiles_per_sync = p.tiles_per_sync, wg = blockIdx.x;
   uint32_t part_index = blockIdx.y, n_parts = gridDim.y;
@@ -201,7 +205,7 @@ __global__ __launch_bounds__(768) void q4k_rows16_kernel(R16Args p) {
     const uint32_t tl = u / BW, jb = u % BW;
     const uint32_t first_row = row0 + tl * kTile;
     const uint32_t last = p.n - 1u - first_row;             // rows past the matrix: the last row, never stored
-    const uint8_t* base = p.w + static_cast<size_t>(col(jb)) * 144u + static_cast<size_t>(first_row) * row_bytes;
+    const uint8_t* base = w + static_cast<size_t>(col(jb)) * 144u + static_cast<size_t>(first_row) * row_bytes;
     const uint32_t dst = ring_addr + fill_slot * kUnitBytes;
 #pragma unroll
     for (int i = 0; i < kKL; ++i) {
@@ -375,7 +379,7 @@ __global__ __launch_bounds__(768) void q4k_rows16_kernel(R16Args p) {
 
   // ---- tiles.  Every wavefront walks the same tiles, so the barriers match.
   const size_t region = static_cast<size_t>(p.m) * p.n;
-  float* cpart = n_parts == 1u ? p.c : p.ws + part_index * region;
+  float* cpart = n_parts == 1u ? p.c : ws + part_index * region;
   // One tile: its BW units, then the wavefront's partial tile into LDS.  A unit is waited for when
   // RING - 1 later ones are all that may still be under way (stores of the sums count as well and
   // only make the wait longer); its slot is asked for again as soon as its words are in registers.
@@ -565,20 +569,40 @@ hipError_t gemv_q4k_rows16_prepare() {
   return err;
 }
 
+namespace {
+R16Args r16_launch(const R16Plan& pl, const float* a, const uint8_t* w, const uint8_t* w2, float* c, float* ws, uint32_t m, uint32_t n,
+                   uint32_t k, hipStream_t stream) {
+  R16Args args{a, w, c, ws, w2, ws + static_cast<size_t>(pl.parts) * m * n, m, n, k, pl.tiles_per_wg,
+               static_cast<uint32_t>(k / 256) / pl.parts, pl.tiles_per_sync, pl.n_table, {}};
+  for (uint32_t i = 0; i < pl.n_table; ++i) args.part[i] = pl.table[i];
+  const dim3 grid(pl.row_groups, pl.n_table != 0u ? 1u : pl.parts, w2 != nullptr ? 2u : 1u), block(64 * pl.waves);
+  const uint32_t lds = r16_lds_bytes(pl.waves, pl.mt, pl.bw, pl.ring, pl.tiles_per_sync);
+  r16_with_kernel(pl.mt, pl.bw, pl.ring, [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, lds, stream, args); });
+  return args;
+}
+}  // namespace
+
 hipError_t launch_q4k_rows16(const float* a, const uint8_t* w, float* c, void* workspace, uint32_t m, uint32_t n,
                              uint32_t k, hipStream_t stream) {
   R16Plan pl;
   if (!r16_plan(m, n, k, pl)) return hipErrorInvalidValue;
-  R16Args args{a, w, c, static_cast<float*>(workspace), m, n, k, pl.tiles_per_wg, static_cast<uint32_t>(k / 256) / pl.parts,
-               pl.tiles_per_sync, pl.n_table, {}};
-  for (uint32_t i = 0; i < pl.n_table; ++i) args.part[i] = pl.table[i];
-  const dim3 grid(pl.row_groups, pl.n_table != 0u ? 1u : pl.parts), block(64 * pl.waves);
-  const uint32_t lds = r16_lds_bytes(pl.waves, pl.mt, pl.bw, pl.ring, pl.tiles_per_sync);
-  r16_with_kernel(pl.mt, pl.bw, pl.ring, [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, lds, stream, args); });
+  const R16Args args = r16_launch(pl, a, w, nullptr, c, static_cast<float*>(workspace), m, n, k, stream);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (pl.parts > 1) return launch_vec_reduce(args.ws, c, static_cast<uint64_t>(m) * n, pl.parts, stream);
   return hipSuccess;
+}
+
+// Both matrices in one launch, and the sums of their parts where they are multiplied: two launches instead of five
+// (the feed forward of 5 rows of 5120 x 17408: 76 -> 69 us).
+hipError_t launch_q4k_rows16_gate_up(const float* a, const uint8_t* gate, const uint8_t* up, float* c, void* workspace, uint32_t m,
+                                     uint32_t n, uint32_t k, hipStream_t stream) {
+  R16Plan pl;
+  if (!r16_plan(m, n, k, pl) || pl.parts < 2) return hipErrorInvalidValue;
+  const R16Args args = r16_launch(pl, a, gate, up, c, static_cast<float*>(workspace), m, n, k, stream);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return launch_vec_reduce_silu(args.ws, args.ws2, c, static_cast<uint64_t>(m) * n, pl.parts, stream);
 }
 
 }  // namespace qmm

@@ -232,6 +232,11 @@ constexpr uint64_t kQ4KRows16MinRows = 3;      // from here the 16x16x32 kernel,
 constexpr uint64_t kQ4KFewRowsMaxK = 262144;   // its activation operand must fit the decode scratch
 constexpr uint64_t kQ4KRowsI8MaxK = 5120;      // up to here the int8 one-pass kernel leads for two rows
 
+bool q4k_takes_rows16(uint64_t m, uint64_t n, uint64_t k) {
+  return (m >= kQ4KRows16MinRows || (m == 2 && k > 8192)) && m <= 16 && (n * k >= kQ4KFewRowsMinWeights || m >= 5) &&
+         qmm::gemv_q4k_rows16_supported(m, n, k) && qmm::gemv_q4k_rows16_workspace_bytes(m, n, k) <= kDecodeScratchBytes;
+}
+
 qmm_status q4k_matmul(const LaunchCtx& ctx, const float* a, const uint8_t* w, float* c, uint64_t m, uint64_t n,
                       uint64_t k, uint64_t f16_from) {
   const hipStream_t s = ctx.stream;
@@ -266,9 +271,7 @@ qmm_status q4k_matmul(const LaunchCtx& ctx, const float* a, const uint8_t* w, fl
   // resident kernel, 4096 x 14336 15.3 against 18.5; at 8192 and below the resident kernel leads)
   // From five rows on it leads at any size (1024 x 1024, 8 rows: 5.1 against 14.5 us on the
   // multiply-add passes; four rows are level with them below 16 M weights).
-  if ((m >= kQ4KRows16MinRows || (m == 2 && k > 8192)) && m <= 16 && (n * k >= kQ4KFewRowsMinWeights || m >= 5) &&
-      qmm::gemv_q4k_rows16_supported(m, n, k) &&
-      qmm::gemv_q4k_rows16_workspace_bytes(m, n, k) <= kDecodeScratchBytes) {
+  if (q4k_takes_rows16(m, n, k)) {
     void* ws = decode_scratch(ctx);
     if (ws == nullptr) {
       g_last_error = "Q4_K: decode scratch missing";
@@ -756,6 +759,13 @@ qmm_status run_ffn_gate_up_silu_q4k(const LaunchCtx& c) {
     if (st != QMM_OK) return st;
     return map_hip(qmm::launch_q4k_gate_up(x, gate, up, out, ws, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                            static_cast<uint32_t>(k), c.stream));
+  }
+  if (q4k_takes_rows16(m, n, k) && decode_scratch(c) != nullptr) {
+    const size_t parts = qmm::gemv_q4k_rows16_workspace_bytes(m, n, k);     // 0: one part, nothing to add up
+    if (parts != 0 && 2 * parts <= kDecodeScratchBytes) {
+      return map_hip(qmm::launch_q4k_rows16_gate_up(x, gate, up, out, decode_scratch(c), static_cast<uint32_t>(m),
+                                                    static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
+    }
   }
   const FfnScratch lay = ffn_scratch(m, n, k);
   float* u = nullptr;

@@ -159,6 +159,7 @@ hipError_t launch_moe_ffn_q4k(const float* x, const uint8_t* gate, const uint8_t
                               bool accumulate, hipStream_t stream);
 
 // ---- element-wise helpers (elementwise.hip) ---------------------------------
+hipError_t launch_vec_reduce_silu(const float* gate, const float* up, float* c, uint64_t total, uint64_t split, hipStream_t stream);
 hipError_t launch_vec_reduce(const float* part, float* c, uint64_t total, uint64_t split,
                              hipStream_t stream);
 hipError_t launch_fill_f32(float* dst, float value, uint64_t count, hipStream_t stream);
@@ -198,6 +199,9 @@ hipError_t launch_q6k_rows_i8(const float* a, const uint8_t* w, float* c, uint32
                               hipStream_t stream);
 bool gemv_q4k_rows16_supported(uint64_t m, uint64_t n, uint64_t k);
 size_t gemv_q4k_rows16_workspace_bytes(uint64_t m, uint64_t n, uint64_t k);
+// silu(A gate^T) * (A up^T) where the plan has several K parts: twice the workspace.
+hipError_t launch_q4k_rows16_gate_up(const float* a, const uint8_t* gate, const uint8_t* up, float* c, void* workspace, uint32_t m,
+                                     uint32_t n, uint32_t k, hipStream_t stream);
 hipError_t launch_q4k_rows16(const float* a, const uint8_t* w, float* c, void* workspace, uint32_t m, uint32_t n,
                              uint32_t k, hipStream_t stream);
 
