@@ -10,25 +10,47 @@
 namespace qmm {
 namespace {
 
-// One thread per (row, head, pair): (x[j], x[j + pairs]) rotated by pos * theta^(-2j / rope_dim).
+// (x[j], x[j + pairs]) rotated by pos * theta^(-2j / rope_dim), one thread for pair j of HEADS heads of a row.
 // The angle, its cosine and sine are formed in double and rounded to fp32 once, as RopeRef does
 // (src/core/numerics/attention.cpp:11-44); `pos3` non-null selects the multimodal form, where pair
 // j takes the temporal, height or width position of its row (MropeRef, attention.cpp:227-264).
+// That arithmetic is the kernel's time (512 rows of 24 heads of 256: 23 us at a thread a pair, 7.5 at eight heads), so
+// many rows share it among heads; with few there is one head a thread, and the elements are under way meanwhile.
+template <int HEADS>
 __global__ __launch_bounds__(256) void rope_kernel(float* __restrict__ data, const uint64_t* __restrict__ pos3, uint64_t rows,
                                                    uint64_t heads, uint64_t head_dim, uint64_t rope_dim, uint64_t pos_base,
                                                    float theta, uint64_t sec_t, uint64_t sec_h) {
-  const uint64_t pairs = rope_dim / 2;
+  const uint64_t pairs = rope_dim / 2, groups = (heads + HEADS - 1) / HEADS, total = rows * groups * pairs;
   const uint64_t t = static_cast<uint64_t>(blockIdx.x) * 256u + threadIdx.x;
-  if (t >= rows * heads * pairs) return;
-  const uint64_t row = t / (heads * pairs), rem = t % (heads * pairs), head = rem / pairs, j = rem % pairs;
+  if (t >= total) return;
+  uint64_t row, rem, group, j;
+  if (total <= 0xFFFFFFFFull) {        // uniform: 32-bit divisions where they do
+    const uint32_t t32 = static_cast<uint32_t>(t), per_row = static_cast<uint32_t>(groups * pairs), p32 = static_cast<uint32_t>(pairs);
+    row = t32 / per_row, rem = t32 % per_row;
+    group = static_cast<uint32_t>(rem) / p32, j = static_cast<uint32_t>(rem) % p32;
+  } else {
+    row = t / (groups * pairs), rem = t % (groups * pairs), group = rem / pairs, j = rem % pairs;
+  }
+  float* base = data + (row * heads + group * HEADS) * head_dim;
+  const uint64_t left = heads - group * HEADS;
+  const uint32_t here = left < HEADS ? static_cast<uint32_t>(left) : HEADS;
+  float x1[HEADS], x2[HEADS];
+#pragma unroll
+  for (uint32_t h = 0; h < HEADS; ++h) {
+    const float* x = base + (h < here ? h : 0u) * head_dim;
+    x1[h] = x[j], x2[h] = x[j + pairs];
+  }
   uint64_t p = pos_base + row;
   if (pos3 != nullptr) p = pos3[row * 3 + (j < sec_t ? 0 : (j < sec_t + sec_h ? 1 : 2))];
   const double angle = static_cast<double>(p) * pow(static_cast<double>(theta), -2.0 * static_cast<double>(j) / static_cast<double>(rope_dim));
   const float c = static_cast<float>(cos(angle)), s = static_cast<float>(sin(angle));
-  float* base = data + (row * heads + head) * head_dim;
-  const float x1 = base[j], x2 = base[j + pairs];
-  base[j] = x1 * c - x2 * s;
-  base[j + pairs] = x1 * s + x2 * c;
+#pragma unroll
+  for (uint32_t h = 0; h < HEADS; ++h) {
+    if (h >= here) break;
+    float* x = base + h * head_dim;
+    x[j] = fmaf(x1[h], c, -(x2[h] * s));         // written out: the same bits from either instance
+    x[j + pairs] = fmaf(x2[h], c, x1[h] * s);
+  }
 }
 
 __global__ __launch_bounds__(256) void qgate_split_kernel(const float* __restrict__ fused, float* __restrict__ q,
@@ -101,8 +123,13 @@ dim3 blocks_for(uint64_t count) { return dim3(static_cast<uint32_t>((count + 255
 
 hipError_t launch_rope(float* data, const uint64_t* pos3, uint64_t rows, uint64_t heads, uint64_t head_dim, uint64_t rope_dim,
                        uint64_t pos_base, float theta, uint64_t sec_t, uint64_t sec_h, hipStream_t stream) {
-  hipLaunchKernelGGL(rope_kernel, blocks_for(rows * heads * (rope_dim / 2)), dim3(256), 0, stream, data, pos3, rows, heads,
-                     head_dim, rope_dim, pos_base, theta, sec_t, sec_h);
+  const uint64_t pairs = rope_dim / 2;
+  auto go = [&](auto kernel, uint64_t per_thread) {
+    hipLaunchKernelGGL(kernel, blocks_for(rows * ((heads + per_thread - 1) / per_thread) * pairs), dim3(256), 0, stream, data, pos3,
+                       rows, heads, head_dim, rope_dim, pos_base, theta, sec_t, sec_h);
+  };
+  // from a wavefront a SIMD on, heads share
+  rows * heads * pairs >= 65536u ? go(rope_kernel<8>, 8) : go(rope_kernel<1>, 1);
   return hipGetLastError();
 }
 
