@@ -733,6 +733,21 @@ FfnScratch ffn_scratch(uint64_t m, uint64_t n, uint64_t k) {
   return FfnScratch{false, up_off, up_off + up_bytes};
 }
 
+// The tensor tile takes both products at once where it fills its rows; 3..16 rows take both matrices in one launch where K
+// is in parts that fit the decode scratch twice.
+bool ffn_takes_pair_tile(uint64_t m, uint64_t k) {
+  return m > 64 && m >= g_q4k_tensor_rows.load(std::memory_order_relaxed) && qmm::gemm_q4k_supported(m, k);
+}
+bool ffn_takes_pair_rows(uint64_t m, uint64_t n, uint64_t k) {
+  if (!q4k_takes_rows16(m, n, k)) return false;
+  const size_t parts = qmm::gemv_q4k_rows16_workspace_bytes(m, n, k);       // 0: one part, nothing to add up
+  return parts != 0 && 2 * parts <= kDecodeScratchBytes;
+}
+size_t ffn_workspace_bytes(uint64_t m, uint64_t n, uint64_t k) {
+  if (ffn_takes_pair_tile(m, k)) return qmm::gemm_q4k_workspace_bytes(m, k);
+  return ffn_takes_pair_rows(m, n, k) ? 0 : ffn_scratch(m, n, k).workspace_bytes;
+}
+
 // Out = silu(X Gate^T) * (X Up^T), what the reference computes with two "gemm_q4k*" launches
 // and "silu_mul" (src/models/qwen3_5/trunk.cpp:294-304).  One row of a supported k is a single launch that
 // reads the activations once for both matrices; anything else runs the two products through the
@@ -752,20 +767,16 @@ qmm_status run_ffn_gate_up_silu_q4k(const LaunchCtx& c) {
   if (m == 1 && qmm::ffn_gate_up_q4k_supported(k)) {
     return map_hip(qmm::launch_ffn_gate_up_q4k(x, gate, up, out, static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
   }
-  // The tensor tile takes both products at once where it fills its rows.
-  if (m > 64 && m >= g_q4k_tensor_rows.load(std::memory_order_relaxed) && qmm::gemm_q4k_supported(m, k)) {
+  if (ffn_takes_pair_tile(m, k)) {
     void* ws = nullptr;
     const qmm_status st = workspace(c, qmm::gemm_q4k_workspace_bytes(m, k), &ws);
     if (st != QMM_OK) return st;
     return map_hip(qmm::launch_q4k_gate_up(x, gate, up, out, ws, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                            static_cast<uint32_t>(k), c.stream));
   }
-  if (q4k_takes_rows16(m, n, k) && decode_scratch(c) != nullptr) {
-    const size_t parts = qmm::gemv_q4k_rows16_workspace_bytes(m, n, k);     // 0: one part, nothing to add up
-    if (parts != 0 && 2 * parts <= kDecodeScratchBytes) {
-      return map_hip(qmm::launch_q4k_rows16_gate_up(x, gate, up, out, decode_scratch(c), static_cast<uint32_t>(m),
-                                                    static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
-    }
+  if (ffn_takes_pair_rows(m, n, k) && decode_scratch(c) != nullptr) {
+    return map_hip(qmm::launch_q4k_rows16_gate_up(x, gate, up, out, decode_scratch(c), static_cast<uint32_t>(m),
+                                                  static_cast<uint32_t>(n), static_cast<uint32_t>(k), c.stream));
   }
   const FfnScratch lay = ffn_scratch(m, n, k);
   float* u = nullptr;
@@ -1661,7 +1672,7 @@ qmm_status qmm_workspace_bytes(qmm_kernel kernel, const uint64_t* scalars, size_
     if (layout != 0 && m > 1 && k % 256 == 0) *out_bytes = q4k_regime_workspace(m, k, from) + static_cast<size_t>(q4k_bytes(n, k));
   } else if (id == "ffn_gate_up_silu_q4k") {
     const uint64_t m = sc(0), n = sc(1), k = sc(2);
-    if (m >= 2 && n != 0 && k != 0) *out_bytes = ffn_scratch(m, n, k).workspace_bytes;
+    if (m >= 2 && n != 0 && k != 0) *out_bytes = ffn_workspace_bytes(m, n, k);
   } else if (id == "gemm_mxfp4_wmma") {
     const uint64_t m = sc(0), n = sc(1), k = sc(2), wperm = sc(4);
     if (wperm == 1 && !qmm::gemm_mxfp4_a8_wperm_supported(m, n, k)) *out_bytes = static_cast<size_t>(mxfp4_bytes(n, k));
