@@ -556,10 +556,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 //   S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_16x16x32_f16, a lane's weights taken as they stand, as in
 //   attend_row, but with a column a pair and both of its terms in one lane.  Row r of block j of O^T stands for
 //   element VE r + j, so that a lane ends up with runs of a row of the result.
-// Both terms of a weight go into one sum: the second, x - hi as it is, is off by 2^-25 where it is an fp16
-// subnormal, with the largest weight at 2^14 (with values' scales, the largest contribution between 2^9 and 2^15):
-// 2^-34 of the largest at most.  A tile's contribution is summed by itself and added to the running sum, so that
-// rounding there goes with a few terms and not with the number of keys.
+// A tile's contribution, the second terms' sum brought down by 2^-11 and the first terms' added to it, is summed by
+// itself and added to the running sum, so that rounding there goes with a few terms and not with the number of keys.
 // 512 rows of 24 heads of 256 on 2512 fp16 keys of 4: 119 us (432 with a workgroup a row and key head, which read each
 // key for six columns), int8 keys 125 (455).  Vector instructions issue in 51 % of the cycles, the matrix cores are busy
 // in 32 %, LDS in 29 %; a wavefront waits in 39 % of its own, at the tile's barrier and for operands.
@@ -850,7 +848,7 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
       const float x = s[e] * value_up;
       const _Float16 hi = static_cast<_Float16>(x);
       p_hi[e] = hi;
-      p_lo[e] = static_cast<_Float16>(x - static_cast<float>(hi));
+      p_lo[e] = static_cast<_Float16>((x - static_cast<float>(hi)) * 0x1p11f);
     }
     if (__any(corr != 1.0f)) {
 #pragma unroll
@@ -867,7 +865,11 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
 #pragma unroll
       for (int i = 0; i < GROUP; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n & 1][i], p_lo, float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < GROUP; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n & 1][i], p_hi, acc[i], 0, 0, 0);
+      for (int i = 0; i < GROUP; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] *= 0x1p-11f;
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n & 1][i], p_hi, acc[i], 0, 0, 0);
+      }
 #pragma unroll
       for (int i = 0; i < GROUP; ++i) o[n * GROUP + i] += acc[i];
     }

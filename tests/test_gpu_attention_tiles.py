@@ -87,3 +87,47 @@ def test_attention_tiles_special_values(backend, shape, what):
     fine = np.isfinite(want)
     assert np.array_equal(got[~fine & ~np.isnan(want)], want[~fine & ~np.isnan(want)])
     assert np.max(np.abs(got[fine] - want[fine]), initial=0.0) <= 4e-6 * max(1.0, np.max(np.abs(want[fine]), initial=0.0))
+
+
+def softmax_rows(q, k, v, heads, kv_heads, head_dim, q_base):
+    """Causal attention in float64 over keys and values as the cache stands for them."""
+    m, n = q.shape[0], k.shape[0]
+    out = np.empty((m, heads * head_dim))
+    q, k, v = (x.astype(np.float64).reshape(x.shape[0], -1, head_dim) for x in (q, k, v))
+    for h in range(heads):
+        s = q[:, h] @ k[:, h * kv_heads // heads].T / np.sqrt(head_dim)
+        s[np.arange(n)[None, :] > q_base + np.arange(m)[:, None]] = -np.inf
+        w = np.exp(s - s.max(1, keepdims=True))
+        out[:, h * head_dim:(h + 1) * head_dim] = w @ v[:, h * kv_heads // heads] / w.sum(1, keepdims=True)
+    return out
+
+
+@pytest.mark.parametrize("kind", ["f16", "q8"])
+@pytest.mark.parametrize("shape", [(101, 449, 4, 4, 128), (33, 2100, 24, 4, 256), (410, 410, 2, 1, 64)])
+def test_attention_tiles_key_of_nearly_all_weight_and_no_value(backend, kind, shape):
+    """The first key takes all but some e^-20 = 2^-29 of every row's weight and its values are zero, so that the result is
+    made of the small weights alone.  They are off by 2^-50 of the largest over an fp16 cache and by 2^-45 of the largest
+    contribution over a quantized one: 2^-16 of themselves at most; a score of 20 in fp32 moves them by 20 * 2^-24 < 2^-19.
+    The values' signs are random, so a row's sum has its weights' relative error.  (Measured: 1.3e-6.)"""
+    m, n, heads, kv_heads, head_dim = shape
+    g = synth.rng(n + 1)
+    q = g.standard_normal((m, heads, head_dim)).astype(np.float32)
+    q[:, :, 0] = 5.0
+    k, ks = cache(g, kind, n, kv_heads * head_dim)
+    v, vs = cache(g, kind, n, kv_heads * head_dim)
+    k, v = (x.copy() if kind == "f16" else x.reshape(n, -1).view(np.int8).copy() for x in (k, v))
+    by_head = k.reshape(n, kv_heads, head_dim)
+    by_head[:, :, 0] = 0
+    by_head[0] = 0
+    v[0] = 0
+    top = 4.0 * np.sqrt(head_dim)                           # score 20
+    by_head[0, :, 0] = top if kind == "f16" else 127
+    if kind == "q8":
+        ks[0] = top / 127
+    keys, values = (x.astype(np.float64) * (1.0 if s is None else s[:, None].astype(np.float64)) for x, s in ((k, ks), (v, vs)))
+    q = q.reshape(m, heads * head_dim)
+    want = softmax_rows(q, keys, values, heads, kv_heads, head_dim, n - m)
+    got = attend(backend, kind, q, k, v, ks, vs, m, n, heads, kv_heads, head_dim, n - m, 0)
+    rows = slice(1, None) if n == m else slice(None)        # (the first row of a cache that starts with it sees that key alone)
+    err = np.linalg.norm(got[rows] - want[rows]) / np.linalg.norm(want[rows])
+    assert err <= 2.0 ** -16, err
