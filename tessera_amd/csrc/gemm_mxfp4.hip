@@ -28,6 +28,7 @@
 
 #include "qmm_device.hpp"
 #include "qmm_kernels.hpp"
+#include "launch_rules.hpp"
 
 namespace qmm {
 namespace {
@@ -41,33 +42,32 @@ __device__ __forceinline__ void direct_load4(const void* base, uint32_t voff, ui
                :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
 
-// First of the `tiles` x `steps` units of workgroup g of `groups`; without `shared` a tile's units stay together.
-__host__ __device__ inline uint64_t unit_bound(uint32_t g, uint32_t groups, uint32_t tiles, uint32_t steps, bool shared) {
-  return shared ? static_cast<uint64_t>(g) * (static_cast<uint64_t>(tiles) * steps) / groups
-                : static_cast<uint64_t>(g) * tiles / groups * steps;
-}
+// What the activation operand is.  E4M3: codes with a scale a row.  Terms: a sum of E4M3 terms (see split_rows_kernel):
+// a8 holds kMaxTerms planes of m x k codes, term t weighing 2^(-4t); `need` says how many terms each row has.  A
+// tile walks K once per term it needs, all into the same accumulators, the term's weight being
+// the E8M0 scale of the A operand.
+// Shared: terms, a tile taking those it needs one after the other at each step of K (the weights' step then comes
+// from L2).  The (tile, step) units of the product's plan are dealt out evenly, workgroup g taking those from
+// unit_bound(g) on: 453 rows of 17408 columns are 136 tiles of 256 x 256, which took half the chip 247 us; shared by all
+// of it 165 and 20 for the sums, the clock then held down by power, the matrix cores busy in 58 % of the cycles.  A tile
+// that several workgroups share has its sums in `parts`, one block of BM x BN a piece, for split_sums_kernel to add up in
+// their order.
+// Cut: the same where there is no room for `parts`.  A workgroup has whole tiles, each within one of the plan's; it cuts
+// their sums where the plan does and adds the pieces in the same order, in registers: the same bits.
+enum class Rows { E4M3, Terms, Shared, Cut };
 
-// SPLIT: the activation is a sum of E4M3 terms (see split_rows_kernel): a8 holds kMaxTerms
-// planes of m x k codes, term t weighing 2^(-4t); `need` says how many terms each row has.  A
-// tile takes the terms it needs one after the other at each step of K (the weights' step then comes
-// from L2), all into the same accumulators, the term's weight being the E8M0 scale of the A operand.
-// The (tile, step) pairs of the whole product are dealt out evenly, workgroup g taking those from
-// unit_bound(g) on (whole tiles where `parts` is null): 453 rows of 17408 columns are 136 tiles of
-// 256 x 256, which took half the chip 247 us; shared by all of it 165 and 20 for the sums, the clock
-// then held down by power, the matrix cores busy in 58 % of the cycles.  A tile that several workgroups share has its sums in
-// `parts`, one block of BM x BN a piece, for split_sums_kernel to add up in their order.
-//
 // WPERM: the nibble bytes of W are in the reference's 16-row fragment order (PermuteMxFp4ToWmma,
 // src/core/numerics/quant.cpp:926-954: dword (tile t, 16-wide K step s, half h, row r) at
 // ((t * k/16 + s) * 2 + h) * 16 + r; the scales stay row-major).  The 16 rows x 128 K of one
 // direct-load block are still 1 KB of contiguous memory, only transposed inside, so the block is
 // fetched dword by dword (global_load_lds_dword), each lane asking for the dword that belongs at
 // its LDS position: the LDS image, and everything after it, is the row-major one.
-template <int BM, int BN, int WM, int WN, bool SPLIT, bool WPERM = false>
+template <int BM, int BN, int WM, int WN, Rows ROWS, bool WPERM = false>
 __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
     const uint8_t* __restrict__ a8, const float* __restrict__ as, const uint8_t* __restrict__ w,
     float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end,
-    const uint8_t* __restrict__ need, float* __restrict__ parts) {
+    const uint8_t* __restrict__ need, float* __restrict__ parts, SharedTiles plan) {
+  constexpr bool SPLIT = ROWS != Rows::E4M3, SHARED = ROWS == Rows::Shared, CUT = ROWS == Rows::Cut, TERMS_INSIDE = SHARED || CUT;
   constexpr int kWaves = WM * WN;
   static_assert(BM % (32 * WM) == 0 && BN % (32 * WN) == 0 && BN % 64 == 0, "tile shape");
   static_assert((BM / 8) % kWaves == 0 && (BN / 16) % kWaves == 0, "direct-load blocks divide among the wavefronts");
@@ -280,31 +280,30 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   // multiply cursor and simply moves on to the next tile when a tile's K is exhausted, so
   // the first loads and fragment reads of a tile run under the previous tile's epilogue.
   // Past the last tile the cursor reloads a stage nobody reads rather than branching.
-  // SPLIT: tiles follow one another, the first from step `step` on, the last up to step `stop`.
+  // Shared: tiles follow one another, the first from step `step` on, the last up to step `last_stop`.
   uint32_t tile = blockIdx.x, step = 0, last_tile = 0, last_stop = steps, unit_group = 0;
-  if constexpr (SPLIT) {
+  if constexpr (SHARED) {
     // Workgroups go round the eight XCDs: neighbours in the units' order, which read the same rows of A, stay on one.
-    const uint32_t g = gridDim.x % 8u == 0u ? blockIdx.x % 8u * (gridDim.x / 8u) + blockIdx.x / 8u : blockIdx.x;
-    const uint64_t from = unit_bound(g, gridDim.x, tiles, steps, parts != nullptr);
-    const uint64_t to = unit_bound(g + 1u, gridDim.x, tiles, steps, parts != nullptr);
-    unit_group = g;
+    unit_group = gridDim.x % 8u == 0u ? blockIdx.x % 8u * (gridDim.x / 8u) + blockIdx.x / 8u : blockIdx.x;
+    const uint64_t from = unit_bound(unit_group, gridDim.x, tiles, steps), to = unit_bound(unit_group + 1u, gridDim.x, tiles, steps);
     if (from == to) return;
     tile = static_cast<uint32_t>(from / steps), step = static_cast<uint32_t>(from % steps);
     last_tile = static_cast<uint32_t>((to - 1u) / steps), last_stop = static_cast<uint32_t>((to - 1u) % steps) + 1u;
   }
   if (tile >= tiles) return;
-  const uint32_t tile_step = SPLIT ? 1u : gridDim.x;
-  if constexpr (!SPLIT) last_tile = tile + (tiles - 1u - tile) / gridDim.x * gridDim.x;
-  const uint32_t first_tile = tile;
+  const uint32_t tile_step = SHARED ? 1u : gridDim.x;
+  if constexpr (!SHARED) last_tile = tile + (tiles - 1u - tile) / gridDim.x * gridDim.x;
   Source src;
   locate(tile, src);
   uint32_t load_tile = tile, load_step = step, load_term = 0, load_stop = tile == last_tile ? last_stop : steps;
   auto advance_load = [&]() {
-    if (SPLIT && ++load_term < src.terms) return;
-    load_term = 0;
+    if (TERMS_INSIDE && ++load_term < src.terms) return;
+    if (TERMS_INSIDE) load_term = 0;
     if (++load_step == load_stop) {      // uniform
       asm volatile("" ::: "memory");     // keeps this rare block a branch, not a chain of selects
       load_step = 0;
+      if (SPLIT && !TERMS_INSIDE && ++load_term < src.terms) return;
+      load_term = 0;
       load_stop = steps;
       if (load_tile != last_tile) {
         load_tile += tile_step;
@@ -330,52 +329,84 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
+  // One step of K on stage `rd`; `nx` holds the step after it, `ld` the one after that (its
+  // loads were asked for half a step ago).  First half: the matrix instructions of the
+  // step's first K slice, whose operands the previous step read, with the reads of the
+  // second slice in between.  Then every wavefront has read all of `rd` and `nx` has landed
+  // (publish), so `rd` is asked for again with the step three ahead.  Second half: the second
+  // slice, with the reads of the NEXT step's first slice (and its scale words) in between.
+  auto one_step = [&](uint32_t term) {
+    const int sa = 0x7F - 4 * static_cast<int>(term);      // E8M0 of 2^(-4 term), byte 0 is the one used
+#pragma unroll
+    for (int j = 0; j < kTJ; ++j) sv[j] = static_cast<int>(sv_raw[j] >> (kg * 8u));
+    mfmas_reading(f0, std::integral_constant<int, 0>{}, sa, f1, rd, 1);
+    if constexpr (SHARED && kWaves == 8) {
+      // keeps these matrix instructions on this side of the barrier: below it they would hold up the reads
+#pragma unroll
+      for (int i = 0; i < kTI; ++i)
+#pragma unroll
+        for (int j = 0; j < kTJ; ++j) asm volatile("" : "+v"(acc[i][j]));
+    }
+    publish();
+    issue_stage(rd, src, load_step * kKS, load_term);
+    advance_load();
+    mfmas_reading(f1, std::integral_constant<int, 1>{}, sa, f0, nx, 0);
+    read_scales(nx, sv_raw);
+    const uint32_t done = rd;
+    rd = nx;
+    nx = ld;
+    ld = done;
+  };
+
   for (;;) {
-    const uint32_t terms = tile_terms((tile / tiles_n) * BM), from = step, stop = tile == last_tile ? last_stop : steps;
-    for (; step < stop; ++step) {
-      for (uint32_t term = 0; term < terms; ++term) {
-        const int sa = 0x7F - 4 * static_cast<int>(term);    // E8M0 of 2^(-4 term), byte 0 is the one used
-        // One step of K on stage `rd`; `nx` holds the step after it, `ld` the one after that (its
-        // loads were asked for half a step ago).  First half: the matrix instructions of the
-        // step's first K slice, whose operands the previous step read, with the reads of the
-        // second slice in between.  Then every wavefront has read all of `rd` and `nx` has landed
-        // (publish), so `rd` is asked for again with the step three ahead.  Second half: the second
-        // slice, with the reads of the NEXT step's first slice (and its scale words) in between.
-#pragma unroll
-        for (int j = 0; j < kTJ; ++j) sv[j] = static_cast<int>(sv_raw[j] >> (kg * 8u));
-        mfmas_reading(f0, std::integral_constant<int, 0>{}, sa, f1, rd, 1);
-        if constexpr (SPLIT && kWaves == 8) {
-          // keeps these matrix instructions on this side of the barrier: below it they would hold up the reads
-#pragma unroll
-          for (int i = 0; i < kTI; ++i)
-#pragma unroll
-            for (int j = 0; j < kTJ; ++j) asm volatile("" : "+v"(acc[i][j]));
+    const uint32_t m0 = (tile / tiles_n) * BM, n0 = n_begin + (tile % tiles_n) * BN;
+    const uint32_t terms = tile_terms(m0), from = step, stop = tile == last_tile ? last_stop : steps;
+    if constexpr (CUT) {
+      float16_t total[kTI][kTJ] = {};
+      const uint64_t first = static_cast<uint64_t>(m0 / plan.rows * ((n + 255u) / 256u) + n0 / 256u) * steps;
+      uint32_t owner = unit_owner(first, plan, steps);
+      while (step < steps) {
+        const uint64_t cut = unit_bound(++owner, plan.groups, plan.tiles, steps) - first;
+        const uint32_t end = cut < steps ? static_cast<uint32_t>(cut) : steps;
+        const bool one_piece = step == 0u && end == steps;
+        for (; step < end; ++step) {
+          for (uint32_t term = 0; term < terms; ++term) one_step(term);
         }
-        publish();
-        issue_stage(rd, src, load_step * kKS, load_term);
-        advance_load();
-        mfmas_reading(f1, std::integral_constant<int, 1>{}, sa, f0, nx, 0);
-        read_scales(nx, sv_raw);
-        const uint32_t done = rd;
-        rd = nx;
-        nx = ld;
-        ld = done;
+        if (one_piece) break;
+#pragma unroll
+        for (int i = 0; i < kTI; ++i)
+#pragma unroll
+          for (int j = 0; j < kTJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              total[i][j][e] += acc[i][j][e];
+              acc[i][j][e] = step == steps ? total[i][j][e] : 0.0f;
+            }
+      }
+    } else if constexpr (SHARED) {
+      for (; step < stop; ++step) {
+        for (uint32_t term = 0; term < terms; ++term) one_step(term);
+      }
+    } else {
+      for (uint32_t term = 0; term < terms; ++term) {
+        for (uint32_t cur = 0; cur < steps; ++cur) one_step(term);
       }
     }
 
     // Epilogue: lane holds column l32 and rows (e/4)*8 + kg*4 + e%4 of each 32 x 32 tile.
-    const uint32_t m0 = (tile / tiles_n) * BM, n0 = n_begin + (tile % tiles_n) * BN;
-    const bool whole = !SPLIT || (from == 0u && stop == steps);
+    const bool whole = !SHARED || (from == 0u && stop == steps);
+    uint32_t lane_row = wm * (BM / WM) + kg * 4u, lane_col = wn * (BN / WN) + l32;
+    asm volatile("" : "+v"(lane_row), "+v"(lane_col));     // what follows from them is formed here, not held over the steps
     if (!whole) {
-      float* block = parts + static_cast<size_t>(2u * unit_group + (tile == first_tile ? 0u : 1u)) * (BM * BN);
+      float* block = parts + static_cast<size_t>(unit_group + tile) * (BM * BN);
 #pragma unroll
       for (int i = 0; i < kTI; ++i) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const uint32_t row = wm * (BM / WM) + i * 32u + (e >> 2) * 8u + kg * 4u + (e & 3u);
+          const uint32_t row = lane_row + i * 32u + (e >> 2) * 8u + (e & 3u);
 #pragma unroll
           for (int j = 0; j < kTJ; ++j) {
-            if (m0 + row < m) block[row * BN + wn * (BN / WN) + j * 32u + l32] = acc[i][j][e];
+            if (m0 + row < m) block[row * BN + lane_col + j * 32u] = acc[i][j][e];
           }
         }
       }
@@ -384,11 +415,11 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
     for (int i = 0; whole && i < kTI; ++i) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const uint32_t row = m0 + wm * (BM / WM) + i * 32u + (e >> 2) * 8u + kg * 4u + (e & 3u);
+        const uint32_t row = m0 + lane_row + i * 32u + (e >> 2) * 8u + (e & 3u);
         const float scale = as[row < m ? row : m - 1u];
 #pragma unroll
         for (int j = 0; j < kTJ; ++j) {
-          const uint32_t col = n0 + wn * (BN / WN) + j * 32u + l32;
+          const uint32_t col = n0 + lane_col + j * 32u;
           if (row < m && col < n_end) c[static_cast<size_t>(row) * n + col] = acc[i][j][e] * scale;
         }
       }
@@ -412,25 +443,18 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
 template <int BM, int BN>
 __global__ __launch_bounds__(BN) void split_sums_kernel(const float* __restrict__ parts, const float* __restrict__ as,
                                                         float* __restrict__ c, uint32_t m, uint32_t n, uint32_t steps,
-                                                        uint32_t tiles, uint32_t groups) {
+                                                        SharedTiles plan) {
   const uint32_t tile = blockIdx.x / (BM / 16), tiles_n = (n + BN - 1) / BN;
   const uint32_t m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BN;
   const uint32_t r0 = blockIdx.x % (BM / 16) * 16u + threadIdx.x / (BN / 4), col = threadIdx.x % (BN / 4) * 4u;
   const uint64_t v0 = static_cast<uint64_t>(tile) * steps, v1 = v0 + steps;
-  // the workgroup that holds unit v: the last whose bound is not above it
-  auto owner = [&](uint64_t v) {
-    uint32_t g = static_cast<uint32_t>(v * groups / (static_cast<uint64_t>(tiles) * steps));
-    while (g + 1u < groups && unit_bound(g + 1u, groups, tiles, steps, true) <= v) ++g;
-    return g;
-  };
-  const uint32_t first = owner(v0), last = owner(v1 - 1u);
+  const uint32_t first = unit_owner(v0, plan, steps), last = unit_owner(v1 - 1u, plan, steps);
   if (first == last) return;
   float4_t sum[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) sum[r] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
   for (uint32_t g = first; g <= last; ++g) {
-    const bool second = unit_bound(g, groups, tiles, steps, true) < v0;     // the group came from an earlier tile
-    const float* block = parts + static_cast<size_t>(2u * g + (second ? 1u : 0u)) * (BM * BN) + r0 * BN + col;
+    const float* block = parts + static_cast<size_t>(g + tile) * (BM * BN) + r0 * BN + col;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       if (m0 + r0 + 4u * r < m) sum[r] += *reinterpret_cast<const float4_t*>(block + 4u * r * BN);
@@ -1133,11 +1157,11 @@ void launch_range(const uint8_t* a8, const float* as, const uint8_t* w, float* c
   const uint32_t grid = tiles < max_groups ? tiles : max_groups;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * WM * WN), 0, stream, a8, as, w, c, m, n, k, n_begin, n_end, need,
-                       static_cast<float*>(nullptr));
+                       static_cast<float*>(nullptr), SharedTiles{});
   };
-  if (wperm) go(mxfp4_a8_gemm_kernel<BM, BN, WM, WN, false, true>);
-  else if (need != nullptr) go(mxfp4_a8_gemm_kernel<BM, BN, WM, WN, true>);
-  else go(mxfp4_a8_gemm_kernel<BM, BN, WM, WN, false>);
+  if (wperm) go(mxfp4_a8_gemm_kernel<BM, BN, WM, WN, Rows::E4M3, true>);
+  else if (need != nullptr) go(mxfp4_a8_gemm_kernel<BM, BN, WM, WN, Rows::Terms>);
+  else go(mxfp4_a8_gemm_kernel<BM, BN, WM, WN, Rows::E4M3>);
 }
 
 // Tiled launch of C = diag(as) . A8 . deq(W)^T; `need` non-null selects the split-activation form.
@@ -1157,30 +1181,22 @@ void launch_tiles(const uint8_t* a8, const float* as, const uint8_t* w, float* c
   if (n_split < n) launch_range<128, 64, 2, 2>(a8, as, w, c, m, n, k, n_split, n, 2u * cus, need, wperm, stream);
 }
 
-// ---- the split form with shared tiles: BM rows a tile (the padding it takes decides), 256 columns ----
-uint32_t split_tile_rows(uint64_t m) {
-  return m <= 64 ? 64u : (m + 127) / 128 * 128 < (m + 255) / 256 * 256 ? 128u : 256u;
-}
-uint32_t split_tiles(uint64_t m, uint64_t n) {
-  const uint32_t rows = split_tile_rows(m);
-  return static_cast<uint32_t>((m + rows - 1) / rows * ((n + 255) / 256));
-}
-// Workgroups that share the tiles' units, at least four units each: as many as the chip holds.
-uint32_t split_groups(uint64_t m, uint64_t n, uint64_t k) {
-  const uint64_t room = static_cast<uint64_t>(num_cus()) * (split_tile_rows(m) == 64u ? 2u : 1u);
-  const uint64_t most = split_tiles(m, n) * (k / kKS) / 4u;
-  return static_cast<uint32_t>(room < most ? room : most);
+template <int BM, int WM, int WN>
+void launch_shared(const uint8_t* a8, const float* as, const uint8_t* w, float* c, uint32_t m, uint32_t n, uint32_t k,
+                   const uint8_t* need, float* parts, const SharedTiles& plan, hipStream_t stream) {
+  constexpr int BN = 256;
+  hipLaunchKernelGGL((mxfp4_a8_gemm_kernel<BM, BN, WM, WN, Rows::Shared>), dim3(plan.groups), dim3(64 * WM * WN), 0, stream, a8,
+                     as, w, c, m, n, k, 0u, n, need, parts, plan);
+  hipLaunchKernelGGL((split_sums_kernel<BM, BN>), dim3(plan.tiles * (BM / 16)), dim3(BN), 0, stream, parts, as, c, m, n, k / kKS,
+                     plan);
 }
 
-template <int BM, int WM, int WN>
-void launch_split(const uint8_t* a8, const float* as, const uint8_t* w, float* c, uint32_t m, uint32_t n, uint32_t k,
-                  const uint8_t* need, float* parts, hipStream_t stream) {
-  constexpr int BN = 256;
-  const uint32_t tiles = split_tiles(m, n), groups = split_groups(m, n, k);
-  hipLaunchKernelGGL((mxfp4_a8_gemm_kernel<BM, BN, WM, WN, true>), dim3(groups), dim3(64 * WM * WN), 0, stream, a8, as, w, c,
-                     m, n, k, 0u, n, need, parts);
-  hipLaunchKernelGGL((split_sums_kernel<BM, BN>), dim3(tiles * (BM / 16)), dim3(BN), 0, stream, parts, as, c, m, n, k / kKS,
-                     tiles, groups);
+// Without room for the pieces: 128 x 64 tiles, each within one of the plan's (one of 64 rows is all of them).
+void launch_cut(const uint8_t* a8, const float* as, const uint8_t* w, float* c, uint32_t m, uint32_t n, uint32_t k,
+                const uint8_t* need, const SharedTiles& plan, hipStream_t stream) {
+  const uint32_t tiles = (m + 127u) / 128u * ((n + 63u) / 64u), most = 2u * static_cast<uint32_t>(num_cus());
+  hipLaunchKernelGGL((mxfp4_a8_gemm_kernel<128, 64, 2, 2, Rows::Cut>), dim3(tiles < most ? tiles : most), dim3(256), 0, stream, a8,
+                     as, w, c, m, n, k, 0u, n, need, static_cast<float*>(nullptr), plan);
 }
 
 }  // namespace
@@ -1261,14 +1277,8 @@ size_t gemm_mxfp4_f32_workspace_bytes(uint64_t m, uint64_t k) {
   return static_cast<size_t>(kMaxTerms) * m * k + ((m * 4 + 255) / 256) * 256 + ((m + 255) / 256) * 256;
 }
 
-// Tiles are shared where whole ones leave much of the chip idle for long.  Sides measured (us, whole or small tiles /
-// shared): 17 rows of 6144 x 5120 58 / 41, 100 rows 69 / 53, 453 rows 123 / 105, 1000 rows (96 tiles) 188 / 151, 30 rows of
-// 5120 x 17408 171 / 95, 60 of 2000 x 2048 31 / 28; but 2048 of 6144 x 5120 (192 tiles) 254 / 262, 1500 of 4000 x 1792 (14
-// steps) 73 / 83, 20 of 520 x 1024 19 / 21: the blocks cost a launch and twice their bytes.
 size_t gemm_mxfp4_f32_parts_bytes(uint64_t m, uint64_t n, uint64_t k) {
-  const uint64_t cus = static_cast<uint64_t>(num_cus());
-  if (m > 256 * cus || n > 256 * cus || k / kKS < 16 || split_tiles(m, n) * 8u > cus * 5u) return 0;
-  return static_cast<size_t>(split_groups(m, n, k)) * 2 * split_tile_rows(m) * 256 * 4;
+  return shared_tiles_bytes(shared_tiles(m, n, k / kKS, static_cast<uint64_t>(num_cus())));
 }
 
 hipError_t launch_mxfp4_f32_gemm(const float* a, const uint8_t* w, float* c, void* workspace, float* parts, uint32_t m,
@@ -1277,10 +1287,12 @@ hipError_t launch_mxfp4_f32_gemm(const float* a, const uint8_t* w, float* c, voi
   float* as = reinterpret_cast<float*>(planes + static_cast<size_t>(kMaxTerms) * m * k);
   uint8_t* need = reinterpret_cast<uint8_t*>(as) + ((static_cast<size_t>(m) * 4 + 255) / 256) * 256;
   launch_split_rows(a, planes, as, need, m, k, stream);
-  if (parts == nullptr) launch_tiles(planes, as, w, c, m, n, k, need, false, stream);
-  else if (split_tile_rows(m) == 64u) launch_split<64, 1, 8>(planes, as, w, c, m, n, k, need, parts, stream);
-  else if (split_tile_rows(m) == 128u) launch_split<128, 2, 4>(planes, as, w, c, m, n, k, need, parts, stream);
-  else launch_split<256, 4, 2>(planes, as, w, c, m, n, k, need, parts, stream);
+  const SharedTiles plan = shared_tiles(m, n, k / kKS, static_cast<uint64_t>(num_cus()));
+  if (plan.groups == 0u) launch_tiles(planes, as, w, c, m, n, k, need, false, stream);
+  else if (parts == nullptr) launch_cut(planes, as, w, c, m, n, k, need, plan, stream);
+  else if (plan.rows == 64u) launch_shared<64, 1, 8>(planes, as, w, c, m, n, k, need, parts, plan, stream);
+  else if (plan.rows == 128u) launch_shared<128, 2, 4>(planes, as, w, c, m, n, k, need, parts, plan, stream);
+  else launch_shared<256, 4, 2>(planes, as, w, c, m, n, k, need, parts, plan, stream);
   return hipGetLastError();
 }
 

@@ -1,0 +1,43 @@
+// Rules that choose a launch's shape from a call's sizes.  Host logic only; no HIP calls.  (A constexpr function is
+// device code's as well.)
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+namespace qmm {
+
+// ---- MXFP4, 17 fp32 rows and more: tiles whose steps of K workgroups share --------------------------------------
+// Tiles of `rows` x 256, `tiles` of them; the (tile, step) units go to `groups` workgroups.  groups 0: not shared.
+struct SharedTiles {
+  uint32_t rows = 0, tiles = 0, groups = 0;
+};
+// First of the units of workgroup g.
+constexpr uint64_t unit_bound(uint32_t g, uint32_t groups, uint32_t tiles, uint32_t steps) {
+  return static_cast<uint64_t>(g) * (static_cast<uint64_t>(tiles) * steps) / groups;
+}
+// The workgroup that holds unit v: the last whose bound is not above it.
+constexpr uint32_t unit_owner(uint64_t v, const SharedTiles& plan, uint32_t steps) {
+  uint32_t g = static_cast<uint32_t>(v * plan.groups / (static_cast<uint64_t>(plan.tiles) * steps));
+  while (g + 1u < plan.groups && unit_bound(g + 1u, plan.groups, plan.tiles, steps) <= v) ++g;
+  return g;
+}
+// The piece of tile t that workgroup g holds is block g + t: along the units one of the two grows from piece to piece.
+constexpr size_t shared_tiles_bytes(const SharedTiles& plan) {
+  return plan.groups == 0u ? 0 : (static_cast<size_t>(plan.groups) + plan.tiles - 1u) * plan.rows * 256u * 4u;
+}
+// Rows a tile: the padding it takes decides.  Workgroups: as many as the chip holds, at least four units each.
+// Tiles are shared where whole ones leave much of the chip idle for long.  Sides measured (us, whole or small tiles /
+// shared): 17 rows of 6144 x 5120 58 / 41, 100 rows 69 / 53, 453 rows 123 / 105, 1000 rows (96 tiles) 188 / 151, 30 rows of
+// 5120 x 17408 171 / 95, 60 of 2000 x 2048 31 / 28; but 2048 of 6144 x 5120 (192 tiles) 254 / 262, 1500 of 4000 x 1792 (14
+// steps) 73 / 83, 20 of 520 x 1024 19 / 21: the blocks cost a launch and twice their bytes.
+constexpr SharedTiles shared_tiles(uint64_t m, uint64_t n, uint64_t steps, uint64_t cus) {
+  if (m > 256 * cus || n > 256 * cus || steps < 16) return {};
+  const uint64_t rows = m <= 64 ? 64 : (m + 127) / 128 * 128 < (m + 255) / 256 * 256 ? 128 : 256;
+  const uint64_t tiles = (m + rows - 1) / rows * ((n + 255) / 256);
+  if (tiles * 8 > cus * 5) return {};
+  const uint64_t room = cus * (rows == 64 ? 2 : 1), most = tiles * steps / 4;
+  return {static_cast<uint32_t>(rows), static_cast<uint32_t>(tiles), static_cast<uint32_t>(room < most ? room : most)};
+}
+
+}  // namespace qmm

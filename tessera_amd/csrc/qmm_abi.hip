@@ -103,8 +103,13 @@ static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 constexpr int kMaxDevices = 64;
 void* g_static_scratch[kMaxDevices] = {};
 
-qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out) {
+// `bytes` of scratch, and `*more` bytes behind them where they can be had (0 is left in it where not: such a call does
+// without).
+qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out, size_t* more = nullptr) {
+  size_t none = 0;
+  size_t& extra = more != nullptr ? *more : none;
   if (c.no_alloc) {
+    if (bytes + extra > kStaticScratchBytes) extra = 0;
     if (bytes > kStaticScratchBytes) {
       g_last_error = "qmm_launch_static: this launch needs " + std::to_string(bytes) +
                      " bytes of scratch, the static scratch holds " + std::to_string(kStaticScratchBytes);
@@ -115,6 +120,7 @@ qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out) {
   }
   std::lock_guard<std::mutex> lock(g_workspace_mutex);
   if (g_user_workspace != nullptr) {
+    if (bytes + extra > g_user_workspace_bytes) extra = 0;
     if (bytes > g_user_workspace_bytes) {
       g_last_error = "qmm_launch: this launch needs " + std::to_string(bytes) + " bytes of workspace, the one set with "
                      "qmm_set_workspace holds " + std::to_string(g_user_workspace_bytes);
@@ -123,27 +129,36 @@ qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out) {
     *out = g_user_workspace;
     return QMM_OK;
   }
-  if (bytes > g_workspace_bytes) {
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c.stream, &capturing) != hipSuccess) (void)hipGetLastError();
-    if (capturing != hipStreamCaptureStatusNone) {
-      g_last_error = "qmm_launch: this launch needs " + std::to_string(bytes) + " bytes of workspace and the library's holds " +
-                     std::to_string(g_workspace_bytes) + "; it cannot grow while the stream is being captured (hand one over "
-                     "with qmm_set_workspace, or make one eager call of this size first)";
-      return QMM_INVALID_ARGUMENT;
-    }
+  auto grow = [](size_t need) {
     // at least double, so that the retired blocks together stay below the live one
-    size_t want = (bytes + (size_t{1} << 24) - 1) & ~((size_t{1} << 24) - 1);
+    size_t want = (need + (size_t{1} << 24) - 1) & ~((size_t{1} << 24) - 1);
     if (want < 2 * g_workspace_bytes) want = 2 * g_workspace_bytes;
     void* fresh = nullptr;
     const hipError_t e = hipMalloc(&fresh, want);
     if (e != hipSuccess) {
       (void)hipGetLastError();
-      return map_hip(e);
+      return e;
     }
     if (g_workspace != nullptr) g_retired_workspaces.push_back(g_workspace);
     g_workspace = fresh;
     g_workspace_bytes = want;
+    return e;
+  };
+  if (bytes + extra > g_workspace_bytes) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c.stream, &capturing) != hipSuccess) (void)hipGetLastError();
+    const bool fixed = capturing != hipStreamCaptureStatusNone;
+    if (fixed || (extra != 0 && grow(bytes + extra) != hipSuccess)) extra = 0;
+    if (bytes > g_workspace_bytes) {
+      if (fixed) {
+        g_last_error = "qmm_launch: this launch needs " + std::to_string(bytes) + " bytes of workspace and the library's holds " +
+                       std::to_string(g_workspace_bytes) + "; it cannot grow while the stream is being captured (hand one over "
+                       "with qmm_set_workspace, or make one eager call of this size first)";
+        return QMM_INVALID_ARGUMENT;
+      }
+      const hipError_t e = grow(bytes);
+      if (e != hipSuccess) return map_hip(e);
+    }
   }
   *out = g_workspace;
   return QMM_OK;
@@ -156,7 +171,7 @@ void* decode_scratch(const LaunchCtx& c) {
   return c.no_alloc ? g_static_scratch[g_device] : g_decode_scratch;
 }
 
-// Scratch of "gemm_fp8", of Q5_K / Q6_K with a few rows and of "attention" with few columns, of "gemm_mxfp4" from 17 rows and of "top_k_rows" over long rows, whose calls on different streams are independent of
+// Scratch of "gemm_fp8", of Q5_K / Q6_K with a few rows and of "attention" with few columns and of "top_k_rows" over long rows, whose calls on different streams are independent of
 // one another: see stream_scratch.hpp.  qmm_init reserves the first slab; later ones are allocated under the
 // relaxed capture mode, which permits it while a stream is captured, unless the caller has handed over a workspace
 // (then a launch allocates nothing).
@@ -969,14 +984,12 @@ qmm_status run_gemm_mxfp4(const LaunchCtx& c) {
   // scale) and the fp32 rows as a short sum of E4M3 terms (gemm_mxfp4.hip).
   if (m >= kMxfp4GemmMinRows && m <= 0xFFFFFFFFull && n <= 0xFFFFFFFFull && qmm::gemm_mxfp4_f32_supported(m, k)) {
     void* ws = nullptr;
-    const size_t ws_bytes = (qmm::gemm_mxfp4_f32_workspace_bytes(m, k) + 255) / 256 * 256;
-    const qmm_status st = workspace(c, qmm::gemm_mxfp4_f32_workspace_bytes(m, k), &ws);
+    // The shared tiles' pieces lie behind the rows' terms; without room for them the result's bits are the same.
+    const size_t terms = qmm::gemm_mxfp4_f32_workspace_bytes(m, k);           // a multiple of 256
+    size_t pieces = qmm::gemm_mxfp4_f32_parts_bytes(m, n, k);
+    const qmm_status st = workspace(c, terms, &ws, &pieces);
     if (st != QMM_OK) return st;
-    // The shared tiles' blocks: the stream's scratch block, or what the static array has left behind the workspace.
-    const size_t parts_bytes = qmm::gemm_mxfp4_f32_parts_bytes(m, n, k);
-    const StreamBlock block(c, c.no_alloc && parts_bytes != 0 ? ws_bytes + parts_bytes : parts_bytes);
-    float* parts = parts_bytes == 0 ? nullptr : static_cast<float*>(block.get());
-    if (parts != nullptr && c.no_alloc) parts += ws_bytes / 4;
+    float* parts = pieces == 0 ? nullptr : reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + terms);
     return map_hip(qmm::launch_mxfp4_f32_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), c.ptr<float>(2), ws, parts,
                                               static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                               static_cast<uint32_t>(k), c.stream));
@@ -1677,8 +1690,10 @@ qmm_status qmm_workspace_bytes(qmm_kernel kernel, const uint64_t* scalars, size_
     const uint64_t m = sc(0), n = sc(1), k = sc(2), wperm = sc(4);
     if (wperm == 1 && !qmm::gemm_mxfp4_a8_wperm_supported(m, n, k)) *out_bytes = static_cast<size_t>(mxfp4_bytes(n, k));
   } else if (id == "gemm_mxfp4" || id == "gemm_mxfp4_batched") {
-    const uint64_t m = sc(0), k = sc(2);
-    if (m >= kMxfp4GemmMinRows && qmm::gemm_mxfp4_f32_supported(m, k)) *out_bytes = qmm::gemm_mxfp4_f32_workspace_bytes(m, k);
+    const uint64_t m = sc(0), n = sc(1), k = sc(2);
+    if (m >= kMxfp4GemmMinRows && qmm::gemm_mxfp4_f32_supported(m, k)) {
+      *out_bytes = qmm::gemm_mxfp4_f32_workspace_bytes(m, k) + qmm::gemm_mxfp4_f32_parts_bytes(m, n, k);
+    }
   } else if (starts("gemm_q5k") || starts("gemm_q6k")) {
     const uint64_t m = sc(0), n = sc(1), k = sc(2);
     if (m >= kQ4KGemmMinRows && qmm::gemm_kquant_f16_supported(m, n, k)) *out_bytes = qmm::gemm_kquant_f16_workspace_bytes(m, n, k);

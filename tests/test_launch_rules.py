@@ -1,0 +1,63 @@
+"""The rules that choose a launch's shape (tessera_amd/csrc/launch_rules.hpp): host logic without HIP, run here as a small
+C++ program over the sizes the ids take."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+HEAD = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#include "launch_rules.hpp"
+using namespace qmm;
+#define CHECK(x, ...) do { if (!(x)) { std::printf("line %d: %s (", __LINE__, #x); std::printf(__VA_ARGS__); std::printf(")\n"); std::exit(1); } } while (0)
+"""
+
+
+def run_program(tmp_path, body):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not found")
+    src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
+    src.write_text(HEAD + "int main() {\n" + body + "\n}\n")
+    subprocess.run(["g++", "-std=c++20", "-O1", "-Wall", "-Wextra", "-I" + os.path.join(ROOT, "tessera_amd", "csrc"), "-o", str(exe),
+                    str(src)], check=True, timeout=120)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout
+    return out.stdout
+
+
+def test_shared_mxfp4_tiles_cover_every_step_once(tmp_path):
+    """Every (tile, step) unit has one owner, its bounds say so, and the pieces of cut tiles have blocks of their own."""
+    run_program(tmp_path, r"""
+  const uint64_t ms[] = {17, 64, 65, 128, 129, 256, 257, 300, 453, 640, 1000, 1300, 2048};
+  const uint64_t ns[] = {1, 256, 257, 1000, 2306, 5120, 6144, 17408, 40000};
+  const uint64_t ks[] = {8, 16, 17, 31, 32, 40, 53, 136};
+  int shared = 0;
+  for (uint64_t cus : {8, 60, 256}) for (uint64_t m : ms) for (uint64_t n : ns) for (uint64_t k : ks) {
+    const SharedTiles plan = shared_tiles(m, n, k, cus);
+    if (plan.groups == 0) { CHECK(shared_tiles_bytes(plan) == 0, "not shared"); continue; }
+    ++shared;
+    const uint32_t steps = static_cast<uint32_t>(k);
+    const uint64_t units = uint64_t{plan.tiles} * steps;
+    CHECK(plan.tiles == (m + plan.rows - 1) / plan.rows * ((n + 255) / 256), "%u rows", plan.rows);
+    CHECK(units >= uint64_t{4} * plan.groups, "%u groups", plan.groups);
+    const size_t blocks = shared_tiles_bytes(plan) / (size_t{plan.rows} * 1024);
+    std::vector<bool> taken(blocks, false);
+    CHECK(unit_bound(0, plan.groups, plan.tiles, steps) == 0 && unit_bound(plan.groups, plan.groups, plan.tiles, steps) == units, "ends");
+    for (uint32_t g = 0; g < plan.groups; ++g) {
+      const uint64_t from = unit_bound(g, plan.groups, plan.tiles, steps), to = unit_bound(g + 1, plan.groups, plan.tiles, steps);
+      CHECK(from < to, "group %u", g);
+      for (uint64_t v : {from, (from + to) / 2, to - 1}) CHECK(unit_owner(v, plan, steps) == g, "unit %zu", static_cast<size_t>(v));
+      for (uint64_t t = from / steps; t <= (to - 1) / steps; ++t) {
+        if (t * steps >= from && (t + 1) * steps <= to) continue;      // the whole tile
+        CHECK(g + t < blocks && !taken[g + t], "group %u tile %zu", g, static_cast<size_t>(t));
+        taken[g + t] = true;
+      }
+    }
+  }
+  CHECK(shared > 300, "%d", shared);
+""")
