@@ -27,15 +27,21 @@ constexpr size_t shared_tiles_bytes(const SharedTiles& plan) {
   return plan.groups == 0u ? 0 : (static_cast<size_t>(plan.groups) + plan.tiles - 1u) * plan.rows * 256u * 4u;
 }
 // Rows a tile: the padding it takes decides.  Workgroups: as many as the chip holds, at least four units each.
-// Tiles are shared where whole ones leave much of the chip idle for long.  Sides measured (us, whole or small tiles /
-// shared): 17 rows of 6144 x 5120 58 / 41, 100 rows 69 / 53, 453 rows 123 / 105, 1000 rows (96 tiles) 188 / 151, 30 rows of
-// 5120 x 17408 171 / 95, 60 of 2000 x 2048 31 / 28; but 2048 of 6144 x 5120 (192 tiles) 254 / 262, 1500 of 4000 x 1792 (14
-// steps) 73 / 83, 20 of 520 x 1024 19 / 21: the blocks cost a launch and twice their bytes.
+// Tiles are shared where whole ones, small (128 x 64) or 256 x 256, leave much of the chip idle for long.  Sides measured
+// (us, whole / shared): 17 rows of 6144 x 5120 57 / 42, 100 rows 69 / 54, 453 rows of 17408 x 5120 238 / 190, 1024 of 5120 x
+// 17408 591 / 349, 640 of 4096 x 2048 55 / 48; but 2048 of 6144 x 5120 (192 tiles) 254 / 262, 1500 of 4000 x 1792 (14 steps)
+// 73 / 83, 20 of 520 x 1024 19 / 21: the pieces cost a launch and twice their bytes, 64 MB of 256-row tiles where the chip
+// is full of them.  With few steps that is more than small tiles lose which fill a round of a workgroup a CU, or of two:
+// 256 rows of 2048 x 2048 34 / 45, 128 of 8192 x 2048 (128 small tiles) 33 / 38, but of 1024 x 2048 (16) 33 / 32, 512 of 8192
+// x 2048 (512) 58 / 60, 512 of 4096 x 4096 (32 steps, 256 small tiles) 61 / 66, but 256 (128) 59 / 53.
 constexpr SharedTiles shared_tiles(uint64_t m, uint64_t n, uint64_t steps, uint64_t cus) {
   if (m > 256 * cus || n > 256 * cus || steps < 16) return {};
   const uint64_t rows = m <= 64 ? 64 : (m + 127) / 128 * 128 < (m + 255) / 256 * 256 ? 128 : 256;
-  const uint64_t tiles = (m + rows - 1) / rows * ((n + 255) / 256);
+  const uint64_t tiles = (m + rows - 1) / rows * ((n + 255) / 256), small = (m + 127) / 128 * ((n + 63) / 64);
   if (tiles * 8 > cus * 5) return {};
+  if (steps < 32 && rows == 128 && small <= cus && small * 8 > cus) return {};
+  if (steps < 32 && rows == 256 && small <= 2 * cus) return {};
+  if (steps < 40 && small * 8 >= cus * 7 && small <= cus) return {};
   const uint64_t room = cus * (rows == 64 ? 2 : 1), most = tiles * steps / 4;
   return {static_cast<uint32_t>(rows), static_cast<uint32_t>(tiles), static_cast<uint32_t>(room < most ? room : most)};
 }

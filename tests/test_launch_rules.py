@@ -61,3 +61,22 @@ def test_shared_mxfp4_tiles_cover_every_step_once(tmp_path):
   }
   CHECK(shared > 300, "%d", shared);
 """)
+
+
+def test_mxfp4_test_cases_are_shared(tmp_path):
+    import test_gpu_mxfp4_shared_tiles as cases
+    checks = "\n".join(f"  CHECK((shared_tiles({m}, {n}, {k // 128}, 256).groups != 0) == {wanted}, \"{m} x {n} x {k}\");"
+                       for group, wanted in ((cases.WHOLE, "false"), (cases.SHARED, "true")) for m, n, k in group)
+    run_program(tmp_path, checks)
+
+
+def test_mxfp4_small_tiles_that_fill_the_chip_stay_whole(tmp_path):
+    """Few steps of K and a round of small tiles: sharing cost a third more (measured beside the rule)."""
+    run_program(tmp_path, r"""
+  for (uint64_t m : {129, 192, 256, 385, 512, 1024, 2048}) CHECK(shared_tiles(m, 1024, 16, 256).groups == 0, "%zu", static_cast<size_t>(m));
+  for (uint64_t m : {129, 256, 400, 512, 1024}) CHECK(shared_tiles(m, 2048, 16, 256).groups == 0, "%zu", static_cast<size_t>(m));
+  for (uint64_t m : {65, 128, 200, 256, 512}) CHECK(shared_tiles(m, 8192, 16, 256).groups == 0, "%zu", static_cast<size_t>(m));
+  CHECK(shared_tiles(512, 4096, 32, 256).groups == 0, "a full round of small tiles");
+  CHECK(shared_tiles(256, 4096, 32, 256).groups != 0, "half a round");
+  CHECK(shared_tiles(453, 17408, 40, 256).groups == 256 && shared_tiles(17, 6144, 40, 256).groups != 0, "sharing leads");
+""")
