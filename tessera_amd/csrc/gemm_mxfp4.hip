@@ -43,11 +43,11 @@ __device__ __forceinline__ void direct_load4(const void* base, uint32_t voff, ui
 }
 
 // What the activation operand is.  E4M3: codes with a scale a row.  Terms: a sum of E4M3 terms (see split_rows_kernel):
-// a8 holds kMaxTerms planes of m x k codes, term t weighing 2^(-4t); `need` says how many terms each row has.  A
-// tile walks K once per term it needs, all into the same accumulators, the term's weight being
-// the E8M0 scale of the A operand.
-// Shared: terms, a tile taking those it needs one after the other at each step of K (the weights' step then comes
-// from L2).  The (tile, step) units of the product's plan are dealt out evenly, workgroup g taking those from
+// a8 holds kMaxTerms planes of m x k codes, term t weighing 2^(-4t); `need` says how many terms each row has.  A tile takes
+// those it needs one after the other at each step of K (the weights' step then comes from L2), all into the same
+// accumulators, the term's weight being the E8M0 scale of the A operand: 300 rows of 17408 x 5120 215 us, walking K once
+// per term 237, 800 of 6144 x 5120 178 / 183, 256 of 4096 x 2048 36 / 34.
+// Shared: likewise, and the (tile, step) units of the product's plan are dealt out evenly, workgroup g taking those from
 // unit_bound(g) on: 453 rows of 17408 columns are 136 tiles of 256 x 256, which took half the chip 247 us; shared by all
 // of it 165 and 20 for the sums, the clock then held down by power, the matrix cores busy in 58 % of the cycles.  A tile
 // that several workgroups share has its sums in `parts`, one block of BM x BN a piece, for split_sums_kernel to add up in
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
     const uint8_t* __restrict__ a8, const float* __restrict__ as, const uint8_t* __restrict__ w,
     float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end,
     const uint8_t* __restrict__ need, float* __restrict__ parts, SharedTiles plan) {
-  constexpr bool SPLIT = ROWS != Rows::E4M3, SHARED = ROWS == Rows::Shared, CUT = ROWS == Rows::Cut, TERMS_INSIDE = SHARED || CUT;
+  constexpr bool SPLIT = ROWS != Rows::E4M3, SHARED = ROWS == Rows::Shared, CUT = ROWS == Rows::Cut;
   constexpr int kWaves = WM * WN;
   static_assert(BM % (32 * WM) == 0 && BN % (32 * WN) == 0 && BN % 64 == 0, "tile shape");
   static_assert((BM / 8) % kWaves == 0 && (BN / 16) % kWaves == 0, "direct-load blocks divide among the wavefronts");
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   struct Source {
     const uint8_t *a, *b, *s;           // tile origins (wave-uniform)
     uint32_t a_off[kABlk], b_off[kBBlk][kBLoads], s_off;
-    uint32_t terms;                     // passes over K (SPLIT)
+    uint32_t terms;                     // of the tile's rows (SPLIT)
   };
   const size_t plane = static_cast<size_t>(m) * k;
   // Terms the rows m0 .. m0 + BM - 1 need: the largest of their `need` bytes (wave-uniform).
@@ -297,13 +297,11 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   locate(tile, src);
   uint32_t load_tile = tile, load_step = step, load_term = 0, load_stop = tile == last_tile ? last_stop : steps;
   auto advance_load = [&]() {
-    if (TERMS_INSIDE && ++load_term < src.terms) return;
-    if (TERMS_INSIDE) load_term = 0;
+    if (SPLIT && ++load_term < src.terms) return;
+    load_term = 0;
     if (++load_step == load_stop) {      // uniform
       asm volatile("" ::: "memory");     // keeps this rare block a branch, not a chain of selects
       load_step = 0;
-      if (SPLIT && !TERMS_INSIDE && ++load_term < src.terms) return;
-      load_term = 0;
       load_stop = steps;
       if (load_tile != last_tile) {
         load_tile += tile_step;
@@ -340,7 +338,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
 #pragma unroll
     for (int j = 0; j < kTJ; ++j) sv[j] = static_cast<int>(sv_raw[j] >> (kg * 8u));
     mfmas_reading(f0, std::integral_constant<int, 0>{}, sa, f1, rd, 1);
-    if constexpr (SHARED && kWaves == 8) {
+    if constexpr (SPLIT && kWaves == 8) {
       // keeps these matrix instructions on this side of the barrier: below it they would hold up the reads
 #pragma unroll
       for (int i = 0; i < kTI; ++i)
@@ -383,13 +381,9 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
               acc[i][j][e] = step == steps ? total[i][j][e] : 0.0f;
             }
       }
-    } else if constexpr (SHARED) {
+    } else {
       for (; step < stop; ++step) {
         for (uint32_t term = 0; term < terms; ++term) one_step(term);
-      }
-    } else {
-      for (uint32_t term = 0; term < terms; ++term) {
-        for (uint32_t cur = 0; cur < steps; ++cur) one_step(term);
       }
     }
 
