@@ -31,6 +31,7 @@
 
 #include "q4k_tile.hpp"
 #include "qmm_kernels.hpp"
+#include "launch_rules.hpp"
 
 namespace qmm {
 namespace {
@@ -164,21 +165,14 @@ hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* wor
   return hipGetLastError();
 }
 
-// The feed forward's front half in one product: tiles as launch_q4k_gemm's, 128 columns of either matrix each.  2048 rows of
+// The feed forward's front half in one product: tiles of 128 columns of either matrix (gate_up_large_tiles).  2048 rows of
 // 17408 x 5120: 858 us, as two products and silu_mul 940.
 hipError_t launch_q4k_gate_up(const float* a, const uint8_t* gate, const uint8_t* up, float* c, void* workspace, uint32_t m,
                               uint32_t n, uint32_t k, hipStream_t stream) {
   _Float16* a16 = static_cast<_Float16*>(workspace);
   float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
   launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
-  const uint32_t cus = static_cast<uint32_t>(num_cus());
-  const uint32_t tiles_m = (m + 255u) / 256u, tiles_n = (n + 127u) / 128u, tiles = tiles_m * tiles_n;
-  uint32_t main_tn = tiles_n;
-  if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) {
-    main_tn = (tiles / cus) * cus / tiles_m;
-  } else if (tiles < cus / 2) {
-    main_tn = 0;
-  }
+  const uint32_t main_tn = gate_up_large_tiles(m, n, static_cast<uint32_t>(num_cus()));
   const uint32_t n_split = main_tn * 128u < n ? main_tn * 128u : n;
   if (n_split > 0) launch_pair_range<256, 256, 128, 64>(a16, a_scale, gate, up, c, m, n, k, 0u, n_split, stream);
   if (n_split < n) launch_pair_range<128, 128, 64, 64>(a16, a_scale, gate, up, c, m, n, k, n_split, n, stream);

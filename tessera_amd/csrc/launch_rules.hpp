@@ -46,4 +46,17 @@ constexpr SharedTiles shared_tiles(uint64_t m, uint64_t n, uint64_t steps, uint6
   return {static_cast<uint32_t>(rows), static_cast<uint32_t>(tiles), static_cast<uint32_t>(room < most ? room : most)};
 }
 
+// ---- "ffn_gate_up_silu_q4k", more than 64 rows ----------------------------------------------------------------------
+// Tiles of 256 rows and 128 columns of either matrix, from column 0 on; what they leave goes to tiles of 128 rows and 64.
+// As in the single product, whole rounds of a tile a CU, and none where they fill less than half the chip.  Nor with 128
+// rows or fewer, half of each tile being padding (us, small tiles / 256-row tiles, in brackets as two products: 17408 x 5120
+// 103 / 138 (117)), nor with 257 to 384, half of the second ones, unless they fill three quarters of a round or all of it: 300
+// rows of 17408 x 5120 (136 tiles) 209 / 233 (287), of 8192 x 4096 (64) 88 / 113 (107), of 12288 x 2048 (192) 74 / 70.
+constexpr uint32_t gate_up_large_tiles(uint32_t m, uint32_t n, uint32_t cus) {
+  const uint32_t tiles_m = (m + 255u) / 256u, tiles_n = (n + 127u) / 128u, tiles = tiles_m * tiles_n;
+  if (m <= 128u || (m > 256u && m <= 384u && (tiles * 4u < cus * 3u || tiles > cus))) return 0;
+  if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) return tiles / cus * cus / tiles_m;
+  return tiles < cus / 2 ? 0 : tiles_n;
+}
+
 }  // namespace qmm

@@ -80,3 +80,19 @@ def test_mxfp4_small_tiles_that_fill_the_chip_stay_whole(tmp_path):
   CHECK(shared_tiles(256, 4096, 32, 256).groups != 0, "half a round");
   CHECK(shared_tiles(453, 17408, 40, 256).groups == 256 && shared_tiles(17, 6144, 40, 256).groups != 0, "sharing leads");
 """)
+
+
+def test_gate_up_rows_that_would_be_padding_take_small_tiles(tmp_path):
+    """65 to 128 rows leave half of a 256-row tile empty, 257 to 384 half of the second."""
+    run_program(tmp_path, r"""
+  for (uint32_t n : {3072u, 8192u, 16384u, 17408u, 24576u, 40000u}) {
+    for (uint32_t m : {65u, 100u, 128u}) CHECK(gate_up_large_tiles(m, n, 256) == 0, "%u x %u", m, n);
+  }
+  for (uint32_t n : {3072u, 8192u, 10240u, 17408u, 24576u}) for (uint32_t m : {257u, 300u, 384u}) CHECK(gate_up_large_tiles(m, n, 256) == 0, "%u x %u", m, n);
+  CHECK(gate_up_large_tiles(300, 12288, 256) == 96, "three quarters of a round");
+  CHECK(gate_up_large_tiles(129, 17408, 256) == 136 && gate_up_large_tiles(512, 17408, 256) == 128, "full rows");
+  CHECK(gate_up_large_tiles(2048, 17408, 256) == 128 && gate_up_large_tiles(700, 17408, 256) == 136, "whole rounds");
+  for (uint32_t m = 65; m < 3000; m += 7) for (uint32_t n : {1u, 100u, 5000u, 17408u, 60000u}) {
+    CHECK(gate_up_large_tiles(m, n, 256) <= (n + 127) / 128, "%u x %u", m, n);
+  }
+""")
