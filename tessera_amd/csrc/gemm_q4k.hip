@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void q5k_to_f16_kernel(const uint8_t* __restri
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
     const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const _Float16* __restrict__ w16,
-    float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end) {
+    float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end, bool as_decoded) {
   constexpr int kWavesN = BN / WN, kWaves = (BM / WM) * kWavesN, kTI = WM / 32, kTJ = WN / 32;
   constexpr int kABlk = BM / 16 / kWaves, kWBlk = (BN / 16 + kWaves - 1) / kWaves;   // 1 KB blocks per wavefront and slice
   constexpr int kDma = kABlk + kWBlk;
@@ -288,7 +288,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
   __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kStage];
 
   const uint32_t tiles_n = (n_end - n_begin + BN - 1) / BN;
-  const TileAt at = xcd_tile(blockIdx.x, (m + BM - 1) / BM, tiles_n);
+  const TileAt at = as_decoded ? TileAt{blockIdx.x / tiles_n, blockIdx.x % tiles_n} : xcd_tile(blockIdx.x, (m + BM - 1) / BM, tiles_n);
   const uint32_t m0 = at.m * BM, n0 = n_begin + at.n * BN;
   const uint32_t t = threadIdx.x, lane = t & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -409,7 +409,7 @@ void launch_f16w_range(const _Float16* a16, const float* a_scale, const _Float16
                        uint32_t n_begin, uint32_t n_end, hipStream_t stream) {
   const uint32_t tiles = ((m + BM - 1) / BM) * ((n_end - n_begin + BN - 1) / BN);
   hipLaunchKernelGGL((f16w_gemm_kernel<BM, BN, WM, WN>), dim3(tiles), dim3((BM / WM) * (BN / WN) * 64), 0, stream, a16, a_scale,
-                     w16, c, m, n, k, n_begin, n_end);
+                     w16, c, m, n, k, n_begin, n_end, f16w_tiles_as_decoded(m, n, k, static_cast<uint32_t>(num_cus()), BM == 128));
 }
 
 }  // namespace
@@ -440,26 +440,16 @@ hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t blo
     return hipErrorInvalidValue;
   }
   launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
-  // Whole rounds of 256 x 256 tiles, leftover columns as 128 x 64 tiles (as launch_q4k_gemm).  Where the columns fit one
-  // round, the narrowest tile with which they still do: 2048 x 5120 as 216 tiles of 192 columns instead of 160 of 256.
-  const uint32_t cus = static_cast<uint32_t>(num_cus()), tiles_m = (m + 255u) / 256u;
-  auto tiles_of = [&](uint32_t bn) { return tiles_m * ((n + bn - 1u) / bn); };
-  const uint32_t tiles = tiles_of(256u);
-  if (tiles_of(128u) <= cus && tiles_of(128u) > cus / 2) {
-    launch_f16w_range<256, 128, 64, 64>(a16, a_scale, w16, c, m, n, k, 0u, n, stream);
-  } else if (tiles_of(192u) <= cus && tiles_of(192u) > cus / 2) {
-    launch_f16w_range<256, 192, 64, 96>(a16, a_scale, w16, c, m, n, k, 0u, n, stream);
-  } else {
-    uint32_t main_tn = (n + 255u) / 256u;
-    if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) {
-      main_tn = (tiles / cus) * cus / tiles_m;
-    } else if (tiles < cus / 2) {
-      main_tn = 0;
+  const F16wTiles tiles = f16w_tiles(m, n, k, static_cast<uint32_t>(num_cus()));
+  const uint32_t n_split = tiles.large * tiles.columns < n ? tiles.large * tiles.columns : n;
+  if (n_split > 0) {
+    switch (tiles.columns) {
+      case 128: launch_f16w_range<256, 128, 64, 64>(a16, a_scale, w16, c, m, n, k, 0u, n_split, stream); break;
+      case 192: launch_f16w_range<256, 192, 64, 96>(a16, a_scale, w16, c, m, n, k, 0u, n_split, stream); break;
+      default: launch_f16w_range<256, 256, 128, 64>(a16, a_scale, w16, c, m, n, k, 0u, n_split, stream); break;
     }
-    const uint32_t n_split = main_tn * 256u < n ? main_tn * 256u : n;
-    if (n_split > 0) launch_f16w_range<256, 256, 128, 64>(a16, a_scale, w16, c, m, n, k, 0u, n_split, stream);
-    if (n_split < n) launch_f16w_range<128, 64, 64, 32>(a16, a_scale, w16, c, m, n, k, n_split, n, stream);
   }
+  if (n_split < n) launch_f16w_range<128, 64, 64, 32>(a16, a_scale, w16, c, m, n, k, n_split, n, stream);
   return hipGetLastError();
 }
 

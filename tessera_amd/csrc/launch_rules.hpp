@@ -59,4 +59,37 @@ constexpr uint32_t gate_up_large_tiles(uint32_t m, uint32_t n, uint32_t cus) {
   return tiles < cus / 2 ? 0 : tiles_n;
 }
 
+// ---- Q5_K and Q6_K from 17 rows: fp16 weights, decoded by the launch before ----------------------------------------------
+// `large` tiles of 256 rows and `columns` columns, from column 0 on, for each 256 rows; the columns they leave go to tiles of
+// 128 x 64.  Whole rounds of 256 columns, a tile a CU, and none where they fill less than half the chip.  Where the columns
+// fit one round of narrower ones, the narrowest with which they still do: 2048 x 5120 as 216 tiles of 192 columns instead of
+// 160 of 256 (515 -> 455 us at K = 17408).  But not with 64 rows or fewer, nor with 128 and a short K, which leave three
+// quarters or half of those tiles empty (us, small tiles / 256 x 128): 64 rows of 24576 x 1024 30 / 39, of 32000 x 2048 58 / 68,
+// 128 rows 34 / 40, 64 / 69; of 17408 x 5120 and 20000 x 5120 64 rows 97 / 95, 132 / 131, 128 rows 114 / 104, 143 / 135.
+struct F16wTiles {
+  uint32_t large, columns;
+};
+constexpr F16wTiles f16w_tiles(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
+  const uint32_t tiles_m = (m + 255u) / 256u;
+  if (m > 128u || (m > 64u && k >= 4096u)) {
+    for (uint32_t columns : {128u, 192u}) {
+      const uint32_t tiles_n = (n + columns - 1u) / columns;
+      if (tiles_m * tiles_n <= cus && tiles_m * tiles_n > cus / 2) return {tiles_n, columns};
+    }
+  }
+  const uint32_t tiles_n = (n + 255u) / 256u, tiles = tiles_m * tiles_n;
+  if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) return {tiles / cus * cus / tiles_m, 256u};
+  return {tiles < cus / 2 ? 0u : tiles_n, 256u};
+}
+// The order of the tiles.  Workgroups go round the XCDs, in the launch that decodes as here, so that along the columns an XCD
+// finds part of the weights that it has written itself in its L2; an XCD's share of neighbouring tiles (xcd_tile) instead
+// reads them once for several row tiles.  The first leads with one row tile, with up to three where the weights are small, and
+// where small tiles are few (us, along / shares): 100 rows of 16384 x 1024 27 / 33, 256 rows 33 / 39, 300 of 6144 x 5120 70 /
+// 84, 512 of 5120 x 17408 (320 small tiles) 286 / 324, 700 of 3072 x 1024 (288) 24 / 29; 256 rows of 17408 x 5120 161 / 151, of
+// 12288 x 4096 (384) 78 / 76, 512 of 6144 x 5120 (384) 84 / 80.
+constexpr bool f16w_tiles_as_decoded(uint32_t m, uint32_t n, uint32_t k, uint32_t cus, bool small) {
+  return m <= 128u || (m <= 384u && static_cast<uint64_t>(n) * k <= (uint64_t{32} << 20)) ||
+         (small && static_cast<uint64_t>((m + 127u) / 128u) * ((n + 63u) / 64u) * 4u <= cus * 5u);
+}
+
 }  // namespace qmm

@@ -96,3 +96,19 @@ def test_gate_up_rows_that_would_be_padding_take_small_tiles(tmp_path):
     CHECK(gate_up_large_tiles(m, n, 256) <= (n + 127) / 128, "%u x %u", m, n);
   }
 """)
+
+
+def test_decoded_weights_rows_that_would_be_padding_take_small_tiles(tmp_path):
+    """64 rows and fewer, and up to 128 with a short K, stay off 256-row tiles; the tiles cover the columns."""
+    run_program(tmp_path, r"""
+  for (uint32_t n : {16500u, 20000u, 24576u, 32000u}) for (uint32_t k : {256u, 1024u, 2048u, 5120u}) {
+    for (uint32_t m : {17u, 64u}) CHECK(f16w_tiles(m, n, k, 256).large == 0, "%u x %u x %u", m, n, k);
+    CHECK((f16w_tiles(128, n, k, 256).large == 0) == (k < 4096), "128 x %u x %u", n, k);
+    CHECK(f16w_tiles(256, n, k, 256).large != 0, "256 x %u x %u", n, k);
+  }
+  for (uint32_t m = 17; m < 3000; m += 5) for (uint32_t n : {1u, 100u, 5000u, 17408u, 60000u}) {
+    const F16wTiles t = f16w_tiles(m, n, 5120, 256);
+    CHECK(t.large <= (n + t.columns - 1) / t.columns && (t.columns == 256 || t.large == (n + t.columns - 1) / t.columns), "%u x %u", m, n);
+  }
+  CHECK(f16w_tiles(2048, 5120, 17408, 256).columns == 192 && f16w_tiles(2048, 5120, 17408, 256).large == 27, "one round of 192");
+""")
