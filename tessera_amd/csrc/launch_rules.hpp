@@ -92,4 +92,11 @@ constexpr bool f16w_tiles_as_decoded(uint32_t m, uint32_t n, uint32_t k, uint32_
          (small && static_cast<uint64_t>((m + 127u) / 128u) * ((n + 63u) / 64u) * 4u <= cus * 5u);
 }
 
+// ---- "rope", "mrope" -------------------------------------------------------------------------------------------------
+// Heads that share a thread's angle: eight from a wavefront a SIMD on (512 rows of 24 heads of 256 23 -> 7.5 us), of one head
+// none, which would be read eight times (8193 rows of 64 5.7 / 6.2 us).
+constexpr uint32_t rope_heads_a_thread(uint64_t rows, uint64_t heads, uint64_t pairs) {
+  return heads > 1 && rows * heads * pairs >= 65536 ? 8 : 1;
+}
+
 }  // namespace qmm

@@ -6,6 +6,7 @@
 
 #include "qmm_device.hpp"
 #include "qmm_kernels.hpp"
+#include "launch_rules.hpp"
 
 namespace qmm {
 namespace {
@@ -128,8 +129,7 @@ hipError_t launch_rope(float* data, const uint64_t* pos3, uint64_t rows, uint64_
     hipLaunchKernelGGL(kernel, blocks_for(rows * ((heads + per_thread - 1) / per_thread) * pairs), dim3(256), 0, stream, data, pos3,
                        rows, heads, head_dim, rope_dim, pos_base, theta, sec_t, sec_h);
   };
-  // from a wavefront a SIMD on, heads share
-  rows * heads * pairs >= 65536u ? go(rope_kernel<8>, 8) : go(rope_kernel<1>, 1);
+  rope_heads_a_thread(rows, heads, pairs) == 8u ? go(rope_kernel<8>, 8) : go(rope_kernel<1>, 1);
   return hipGetLastError();
 }
 

@@ -112,3 +112,9 @@ def test_decoded_weights_rows_that_would_be_padding_take_small_tiles(tmp_path):
   }
   CHECK(f16w_tiles(2048, 5120, 17408, 256).columns == 192 && f16w_tiles(2048, 5120, 17408, 256).large == 27, "one round of 192");
 """)
+
+
+def test_rope_of_one_head_shares_nothing(tmp_path):
+    run_program(tmp_path, r"""
+  CHECK(rope_heads_a_thread(1u << 20, 1, 128) == 1 && rope_heads_a_thread(512, 2, 128) == 8 && rope_heads_a_thread(1, 24, 128) == 1, "heads");
+""")
