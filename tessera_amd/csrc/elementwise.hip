@@ -4,6 +4,7 @@
 
 #include "qmm_device.hpp"
 #include "qmm_kernels.hpp"
+#include "launch_rules.hpp"
 
 namespace qmm {
 namespace {
@@ -866,21 +867,14 @@ hipError_t launch_quantize_fp8(float* data, float* scale, uint64_t rows, uint64_
   return hipGetLastError();
 }
 
-// Workgroups per row of the pack kernel: while the rows alone cannot fill the chip, one per 1024 columns, at
-// most 16, of 1024 threads where the row is long (4 rows of 17408 and of 5120: 4.2 us, with 256 threads 6.7); one otherwise.
+// PackShape says how many workgroups share a row and how many threads they have.
 template <bool kBf16>
 static hipError_t quantize_pack(const void* in, uint8_t* out, float* scale, uint64_t rows, uint64_t cols, hipStream_t stream) {
-  const dim3 whole(static_cast<uint32_t>(rows));
-  if (rows >= 256) {
-    hipLaunchKernelGGL((quantize_fp8_pack_kernel<kBf16, 256>), whole, dim3(256), 0, stream, in, out, scale, cols);
-  } else if (cols <= 2048) {
-    hipLaunchKernelGGL((quantize_fp8_pack_kernel<kBf16, 256>), dim3(whole.x, static_cast<uint32_t>((cols + 1023) / 1024)), dim3(256),
-                       0, stream, in, out, scale, cols);
-  } else {
-    const uint64_t share = (cols + 4095) / 4096;
-    hipLaunchKernelGGL((quantize_fp8_pack_kernel<kBf16, 1024>), dim3(whole.x, static_cast<uint32_t>(share < 16 ? share : 16)),
-                       dim3(1024), 0, stream, in, out, scale, cols);
-  }
+  const PackShape shape = pack_shape(rows, cols);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(rows), shape.per_row), dim3(shape.threads), 0, stream, in, out, scale, cols);
+  };
+  shape.threads == 1024u ? go(quantize_fp8_pack_kernel<kBf16, 1024>) : go(quantize_fp8_pack_kernel<kBf16, 256>);
   return hipGetLastError();
 }
 

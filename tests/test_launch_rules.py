@@ -118,3 +118,16 @@ def test_rope_of_one_head_shares_nothing(tmp_path):
     run_program(tmp_path, r"""
   CHECK(rope_heads_a_thread(1u << 20, 1, 128) == 1 && rope_heads_a_thread(512, 2, 128) == 8 && rope_heads_a_thread(1, 24, 128) == 1, "heads");
 """)
+
+
+def test_quantized_rows_are_covered(tmp_path):
+    """Every thread of a row has work, sixteen workgroups at most; rows of up to 6144 columns stay with 256 threads."""
+    run_program(tmp_path, r"""
+  for (uint64_t rows : {1, 4, 64, 200, 255, 256, 5000}) for (uint64_t cols : {4, 1024, 1028, 5120, 6144, 6148, 8192, 17408, 1 << 20}) {
+    const PackShape s = pack_shape(rows, cols);
+    CHECK(s.per_row >= 1 && s.per_row <= 16 && (s.per_row == 1 || (s.per_row - 1) * s.threads * 4 < cols), "%zu x %zu", static_cast<size_t>(rows), static_cast<size_t>(cols));
+    CHECK(cols > 6144 || s.threads == 256, "%zu x %zu", static_cast<size_t>(rows), static_cast<size_t>(cols));
+    CHECK(rows < 256 || (s.per_row == 1 && s.threads == 256), "%zu rows", static_cast<size_t>(rows));
+  }
+  CHECK(pack_shape(4, 17408).threads == 256 && pack_shape(4, 17408).per_row == 16 && pack_shape(64, 17408).threads == 1024, "long rows");
+""")
