@@ -15,6 +15,7 @@
 
 #include "qmm_device.hpp"
 #include "qmm_kernels.hpp"
+#include "launch_rules.hpp"
 
 namespace qmm {
 namespace {
@@ -1042,23 +1043,23 @@ __global__ __launch_bounds__(256) void attention_any_kernel(AttentionArgs a) {
 }
 
 // out[row][head] = sum_s w_s pacc_s / sum_s w_s psum_s with w_s = exp(pmax_s - max_s pmax_s)
-// (src/backends/rocm/rocm_kernels_basic.cpp:664-690).  One workgroup of sixteen wavefronts per (row, head), V
-// consecutive elements a lane, the parts dealt to the wavefronts.  Latency is all there is to it: a wavefront asks for
-// four parts' sums before it knows their weights, which its lanes form for 64 parts at once.  24 rows of 256 over 64
-// parts: 5.9 us (four wavefronts, a weight formed by every lane for each part: 12.7).
-constexpr int kCombineWaves = 16;
-template <int V>
-__global__ __launch_bounds__(kCombineWaves * 64) void attention_combine_kernel(const float* __restrict__ pacc, const float* __restrict__ pmax,
-                                                                const float* __restrict__ psum, float* __restrict__ out,
-                                                                uint32_t head_dim, uint32_t split) {
-  __shared__ float num[kCombineWaves][64 * V + 1], den_s;
+// (src/backends/rocm/rocm_kernels_basic.cpp:664-690).  One workgroup of WAVES wavefronts per (row, head), V
+// consecutive elements a lane, the parts dealt to the wavefronts.  With few rows latency is all there is to it: a wavefront
+// asks for four parts' sums before it knows their weights, which its lanes form for all of a round's parts at once.  24 rows
+// of 256 over 64 parts: 5.9 us (four wavefronts, a weight formed by every lane for each part: 12.7).
+template <int V, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attention_combine_kernel(const float* __restrict__ pacc, const float* __restrict__ pmax,
+                                                                       const float* __restrict__ psum, float* __restrict__ out,
+                                                                       uint32_t head_dim, uint32_t split) {
+  constexpr uint32_t kRound = 4 * WAVES;                           // parts taken at once
+  __shared__ float num[WAVES][64 * V + 1], den_s;
   const uint64_t at = blockIdx.x, base = at * split;
   const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), e0 = lane * V;
   float held[4][V];
-  auto fetch = [&](uint32_t s0) {      // parts s0 + wave + 16 i
+  auto fetch = [&](uint32_t s0) {      // parts s0 + wave + WAVES i
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
-      const uint32_t s = s0 + wave + kCombineWaves * i;
+      const uint32_t s = s0 + wave + WAVES * i;
 #pragma unroll
       for (int c = 0; c < V; ++c) held[i][c] = s < split && e0 + c < head_dim ? pacc[(base + s) * head_dim + e0 + c] : 0.0f;
     }
@@ -1070,23 +1071,31 @@ __global__ __launch_bounds__(kCombineWaves * 64) void attention_combine_kernel(c
   for (uint32_t s = lane + 64u; s < split; s += 64u) top = fmaxf(top, pmax[base + s]);
   top = wave_max(top);
   float n[V] = {}, d = 0.0f;
-  for (uint32_t s0 = 0; s0 < split; s0 += 64u) {
+  for (uint32_t s0 = 0; s0 < split; s0 += kRound) {
     if (s0 != 0u) {
       fetch(s0);
       first_max = s0 + lane < split ? pmax[base + s0 + lane] : -1e30f;
       first_sum = s0 + lane < split ? psum[base + s0 + lane] : 0.0f;
     }
-    const float w = s0 + lane < split ? expf(first_max - top) : 0.0f;
-    d = fmaf(w, first_sum, d);
+    const bool here = lane < kRound && s0 + lane < split;
+    const float w = here ? expf(first_max - top) : 0.0f;
+    d = fmaf(w, here ? first_sum : 0.0f, d);
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
-      if (s0 + wave + kCombineWaves * i >= split) break;               // wave-uniform: nothing enters for a part that is not there
-      const float part_w = bit_cast<float>(__builtin_amdgcn_readlane(bit_cast<int>(w), wave + kCombineWaves * i));
+      if (s0 + wave + WAVES * i >= split) break;                       // wave-uniform: nothing enters for a part that is not there
+      const float part_w = bit_cast<float>(__builtin_amdgcn_readlane(bit_cast<int>(w), wave + WAVES * i));
 #pragma unroll
       for (int c = 0; c < V; ++c) n[c] = fmaf(part_w, held[i][c], n[c]);
     }
   }
   d = wave_sum(d);
+  if constexpr (WAVES == 1) {
+#pragma unroll
+    for (int c = 0; c < V; ++c) {
+      if (e0 + c < head_dim) out[at * head_dim + e0 + c] = n[c] / d;
+    }
+    return;
+  }
 #pragma unroll
   for (int c = 0; c < V; ++c) num[wave][e0 + c] = n[c];
   if (threadIdx.x == 0) den_s = d;
@@ -1095,7 +1104,8 @@ __global__ __launch_bounds__(kCombineWaves * 64) void attention_combine_kernel(c
     float sum[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      sum[q] = (num[4 * q][threadIdx.x] + num[4 * q + 1][threadIdx.x]) + (num[4 * q + 2][threadIdx.x] + num[4 * q + 3][threadIdx.x]);
+      if constexpr (WAVES < 16) sum[q] = num[q % WAVES][threadIdx.x];
+      else sum[q] = (num[4 * q][threadIdx.x] + num[4 * q + 1][threadIdx.x]) + (num[4 * q + 2][threadIdx.x] + num[4 * q + 3][threadIdx.x]);
     }
     out[at * head_dim + threadIdx.x] = ((sum[0] + sum[1]) + (sum[2] + sum[3])) / den_s;
   }
@@ -1235,11 +1245,19 @@ hipError_t launch_attention_split(const float* q, const void* k, const void* v, 
 
 hipError_t launch_attention_combine(const float* pacc, const float* pmax, const float* psum, float* out, uint64_t m,
                                     uint64_t heads, uint64_t head_dim, uint64_t split, hipStream_t stream) {
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(m * heads)), dim3(kCombineWaves * 64), 0, stream, pacc, pmax, psum, out,
-                       static_cast<uint32_t>(head_dim), static_cast<uint32_t>(split));
+  auto go = [&](auto waves) {
+    constexpr int W = decltype(waves)::value;
+    auto with = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(m * heads)), dim3(W * 64), 0, stream, pacc, pmax, psum, out,
+                         static_cast<uint32_t>(head_dim), static_cast<uint32_t>(split));
+    };
+    head_dim <= 64 ? with(attention_combine_kernel<1, W>) : head_dim <= 128 ? with(attention_combine_kernel<2, W>) : with(attention_combine_kernel<4, W>);
   };
-  head_dim <= 64 ? go(attention_combine_kernel<1>) : head_dim <= 128 ? go(attention_combine_kernel<2>) : go(attention_combine_kernel<4>);
+  switch (combine_waves(m * heads, head_dim, split)) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    default: go(std::integral_constant<int, 16>{}); break;
+  }
   return hipGetLastError();
 }
 

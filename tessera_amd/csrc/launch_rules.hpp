@@ -114,4 +114,14 @@ constexpr PackShape pack_shape(uint64_t rows, uint64_t cols) {
   return {static_cast<uint32_t>(share < 16 ? share : 16), threads};
 }
 
+// ---- "attention_combine" ---------------------------------------------------------------------------------------------
+// Wavefronts of a (row, head): sixteen where there are few and many parts, four where the rows fill the chip by themselves or
+// sixteen parts are all that there are, one where its four are and that does not make a lane's run long with few rows (us, 1 /
+// 4 / 16 wavefronts: 24 rows of 256 over 4 parts 3.3 / 2.9 / 3.2, over 64 15 / 6.9 / 6.0; 12288 rows of 64 over 2 parts 5.4 / 10 / 39,
+// of 256 over 8 26 / 25 / 55).
+constexpr uint32_t combine_waves(uint64_t rows, uint64_t head_dim, uint64_t parts) {
+  if (parts <= 4 && (rows >= 1024 || head_dim <= 64 || parts == 1)) return 1;
+  return parts <= 16 || rows > 256 ? 4 : 16;
+}
+
 }  // namespace qmm

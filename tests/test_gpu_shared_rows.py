@@ -55,3 +55,27 @@ def test_attention_combine_parts(backend, split, head_dim):
     size = np.einsum("rs,rsd->rd", w, np.abs(acc).astype(np.float64)) / den
     # rounding of a weight (2^-22: expf and its argument) and of sums of no more than split / 16 + 20 terms
     assert np.all(np.abs(got - num / den) <= size * (2.0 ** -21 + (split / 16 + 20) * 2.0 ** -24))
+
+
+# one, four and sixteen wavefronts a row; more rows than a launch has threads for with sixteen each
+@pytest.mark.parametrize("rows,heads,head_dim,parts", [
+    (1500, 3, 64, 2), (2, 4, 256, 4), (700, 4, 256, 3), (5, 2, 130, 1), (3, 5, 100, 9), (300, 1, 256, 20), (4, 6, 36, 17), (1, 2, 64, 33),
+    (65537, 64, 2, 1), (65537, 64, 1, 6)])
+def test_attention_combine_rows_and_parts(backend, rows, heads, head_dim, parts):
+    """Against the merge in float64; weights of some parts vanish and some parts are empty (0, -1e30, 0)."""
+    g = synth.rng(rows + parts)
+    count = rows * heads
+    acc = g.standard_normal((count, parts, head_dim)).astype(np.float32)
+    most = (g.standard_normal((count, parts)) * 20).astype(np.float32)
+    total = (1 + g.random((count, parts))).astype(np.float32)
+    if parts > 2:
+        acc[::3, 1], most[::3, 1], total[::3, 1] = 0.0, -1e30, 0.0
+    bufs = [backend.Upload(x) for x in (acc, most, total)]
+    out = backend.AllocateBuffer(4 * count * head_dim)
+    run(backend, "attention_combine", [*bufs, out], [rows, heads, head_dim, parts], grid=(count, 1, 1))
+    backend.Synchronize()
+    got = backend.CopyD2H(out, dtype=np.float32).reshape(count, head_dim)
+    w = np.exp(most.astype(np.float64) - most.max(1, keepdims=True))
+    want = np.einsum("rp,rpd->rd", w, acc) / np.sum(w * total, axis=1, keepdims=True)
+    # an exponential of a difference of up to 100 in fp32 (2^-17), the largest terms' alone: 2^-22; sums of parts terms
+    assert np.max(np.abs(got - want)) <= (parts + 8) * 2.0 ** -23 * max(1.0, np.max(np.abs(want)))

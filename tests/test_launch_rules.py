@@ -131,3 +131,16 @@ def test_quantized_rows_are_covered(tmp_path):
   }
   CHECK(pack_shape(4, 17408).threads == 256 && pack_shape(4, 17408).per_row == 16 && pack_shape(64, 17408).threads == 1024, "long rows");
 """)
+
+
+def test_combine_stays_within_a_launch(tmp_path):
+    """Rows that four wavefronts each have threads for (2^32 of them) are never given sixteen; a lane's parts are few."""
+    run_program(tmp_path, r"""
+  for (uint64_t parts = 1; parts <= 100; ++parts) for (uint64_t d : {1, 64, 65, 256}) for (uint64_t rows : {1, 24, 256, 257, 1024, 1 << 22, (1 << 24) - 1}) {
+    const uint32_t waves = combine_waves(rows, d, parts);
+    CHECK(waves == 1 || waves == 4 || waves == 16, "%u", waves);
+    CHECK(rows * waves * 64 < (uint64_t{1} << 32), "%zu rows", static_cast<size_t>(rows));
+    CHECK(waves > 1 || parts <= 4, "%zu parts", static_cast<size_t>(parts));
+  }
+  CHECK(combine_waves(24, 256, 64) == 16 && combine_waves(24, 256, 4) == 4 && combine_waves(12288, 256, 2) == 1, "waves");
+""")
