@@ -212,13 +212,12 @@ __device__ __forceinline__ void empty_part(const AttentionArgs& a, uint64_t row,
 }
 
 // Heads head0 .. head0 + here - 1 (at most rows_heads, all of key head kv) of query row `row` over keys start .. last:
-// part s_part of the row, or all of it.
-template <KvKind KV, int DP, int NW>
+// part s_part of the row, or all of it.  KEYS: keys a tile, 16 where the registers of 32 are not to be had.
+template <KvKind KV, int DP, int NW, int KEYS = KV == KvKind::F32 ? 16 : 32>
 __device__ __forceinline__ void attend_row(const AttentionArgs& a, uint64_t row, uint32_t kv, uint32_t head0, uint32_t here,
                                            uint64_t start, uint64_t last, uint64_t s_part, RowsShared<KV, DP, NW>& merge) {
   constexpr bool F32 = KV == KvKind::F32, QUANT = kv_quantized(KV);
   constexpr int BITS = kv_bits(KV);
-  constexpr int KEYS = F32 ? 16 : 32;                              // keys a tile
   constexpr int CE = F32 ? 4 : 128 / BITS < DP / 4 ? 128 / BITS : DP / 4;   // elements of a key a lane loads at once
   constexpr int RUNS = DP / (4 * CE);                              // such loads a key row
   constexpr int STEPS = F32 ? DP / 4 : DP / 32;                    // matrix instructions over head_dim
@@ -464,12 +463,11 @@ __device__ __forceinline__ void attend_row(const AttentionArgs& a, uint64_t row,
     } else {
       half8_t p;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) p[e] = term_of(s[e]);
+      for (int e = 0; e < 8; ++e) p[e] = e < 4 * HALVES ? term_of(s[e % (4 * HALVES)]) : static_cast<_Float16>(0.0f);
 #pragma unroll
       for (int j = 0; j < VE; ++j) {
-        const uint4 w = {value_pair<KV>(vr[0], vr[1], j), value_pair<KV>(vr[2], vr[3], j),
-                         value_pair<KV>(vr[4 % (4 * HALVES)], vr[5 % (4 * HALVES)], j),
-                         value_pair<KV>(vr[6 % (4 * HALVES)], vr[7 % (4 * HALVES)], j)};
+        uint4 w = {value_pair<KV>(vr[0], vr[1], j), value_pair<KV>(vr[2], vr[3], j), 0u, 0u};
+        if constexpr (HALVES == 2) w.z = value_pair<KV>(vr[4], vr[5], j), w.w = value_pair<KV>(vr[6], vr[7], j);
         o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bit_cast<half8_t>(w), p, o[j], 0, 0, 0);
       }
     }
@@ -597,14 +595,27 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
   const uint32_t D = a.head_dim, group = a.heads / a.kv_heads;
   const uint32_t split = a.part.split == 0 ? 1u : static_cast<uint32_t>(a.part.split), units = gridDim.x / a.kv_heads;
   const uint32_t kv = blockIdx.x % a.kv_heads, unit = units - 1u - blockIdx.x / a.kv_heads, s_part = unit % split;
-  const uint64_t columns = a.rows * group;
-  const uint64_t c0 = static_cast<uint64_t>(unit / split) * 64;    // the longest first
-  const uint64_t c_end = c0 + 64 < columns ? c0 + 64 : columns;
-  const uint64_t col_any = c0 + col_group * 16 + r, col = col_any < c_end ? col_any : c_end - 1;
-  const uint64_t row = col / group;
-  const uint32_t head = kv * group + static_cast<uint32_t>(col % group);
+  const uint32_t columns = static_cast<uint32_t>(a.rows * group);  // fewer than 2^29, as a grid has fewer than 2^32 threads
+  const uint32_t c0 = unit / split * 64u;                          // the longest first
+  const uint32_t c_end = c0 + 64u < columns ? c0 + 64u : columns;
+  // A value the compiler takes for a new one: at head size 256, where the registers are just enough, what is needed
+  // only now and then or after the walk over the keys is formed from the thread's number again, not held.
+  auto again = [](uint32_t v) {
+    if constexpr (DP == 256) asm volatile("" : "+v"(v));
+    return v;
+  };
+  // This lane's column of the workgroup's, past the last one the last.
+  struct Column {
+    uint64_t row;
+    uint32_t head;
+  };
+  auto column = [&]() {
+    const uint32_t at = c0 + col_group * 16u + (again(t) & 15u), col = at < c_end ? at : c_end - 1u;
+    return Column{col / group, kv * group + col % group};
+  };
+  const Column mine = column();
   uint64_t first_key, last_key;
-  key_range(a, row, first_key, last_key);
+  key_range(a, mine.row, first_key, last_key);
   const uint32_t start = static_cast<uint32_t>(first_key), last = static_cast<uint32_t>(last_key);
   key_range(a, c0 / group, first_key, last_key);
   uint32_t wg_start = static_cast<uint32_t>(first_key);
@@ -614,10 +625,10 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
   const uint32_t last_row_start = static_cast<uint32_t>(first_key);
   // Calls f(row, first head, heads) for the workgroup's columns, rows_heads of a row at most at a time.
   auto for_rows = [&](auto f) {
-    for (uint64_t c = c0; c < c_end;) {
-      const uint32_t h = static_cast<uint32_t>(c % group);
+    for (uint32_t c = c0; c < c_end;) {
+      const uint32_t h = c % group;
       uint32_t here = group - h < rows_heads<KV>() ? group - h : rows_heads<KV>();
-      if (here > c_end - c) here = static_cast<uint32_t>(c_end - c);
+      if (here > c_end - c) here = c_end - c;
       f(c / group, kv * group + h, here);
       c += here;
     }
@@ -637,12 +648,22 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
   const uint8_t* vb = static_cast<const uint8_t*>(a.v) + static_cast<uint64_t>(kv) * D * BITS / 8;
   uint32_t kr[KLOADS][KW], vr[4][VW];
   float sr = 0.0f;
-  // Values: elements RE v_run.., keys 4 v_four.. of the tile; lanes l and l + 16 write the halves of a chunk.
-  const uint32_t v_run = (lane & 15u) * 2u + (lane >> 5), v_four = half * 8u + (lane >> 4 & 1u) * 4u + col_group;
-  const uint32_t k_key = t / CHUNKS, k_chunk = t % CHUNKS;         // keys k_key + (512 / CHUNKS) i
-  // Elements past head_dim are read as the row's first: the queries are 0 there, of the result they are not stored.
-  const uint32_t k_elem = k_chunk * 8u < D ? k_chunk * BITS : 0u, v_elem = v_run * RE < D ? v_run * RE * BITS / 8 : 0u;
-  const uint32_t k_off = k_key * static_cast<uint32_t>(stride) + k_elem, v_off = v_four * 4u * static_cast<uint32_t>(stride) + v_elem;
+  // This thread's share of a tile's loads: chunk k_chunk of keys k_key + (512 / CHUNKS) i, elements RE v_run.. of keys
+  // 4 v_four.. (lanes l and l + 16 write the halves of a chunk).  Elements past head_dim are read as the row's first: the
+  // queries are 0 there, of the result they are not stored.
+  struct Share {
+    uint32_t k_key, k_chunk, v_run, v_four, k_elem, v_elem;
+  };
+  auto share_of = [&](uint32_t thread) {
+    Share s;
+    s.k_key = thread / CHUNKS, s.k_chunk = thread % CHUNKS;
+    s.v_run = (thread & 15u) * 2u + (thread >> 5 & 1u), s.v_four = half * 8u + (thread >> 4 & 1u) * 4u + col_group;
+    s.k_elem = s.k_chunk * 8u < D ? s.k_chunk * BITS : 0u, s.v_elem = s.v_run * RE < D ? s.v_run * RE * BITS / 8 : 0u;
+    return s;
+  };
+  const Share own_share = share_of(t);
+  const uint32_t stride32 = static_cast<uint32_t>(stride);
+  const uint32_t k_off = own_share.k_key * stride32 + own_share.k_elem, v_off = own_share.v_four * 4u * stride32 + own_share.v_elem;
   auto fetch = [&](uint32_t j0) {
     const uint32_t left = wg_last - j0;
     const uint8_t *k_tile = kb + j0 * stride, *v_tile = vb + j0 * stride;
@@ -653,15 +674,16 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
       for (int e = 0; e < 4; ++e) load_run<RE * BITS / 8>(v_tile + e * stride + v_off, vr[e]);
     } else {
       // The last tile: keys past the range's end are read as its last one; no column sees them.
+      const Share late = share_of(again(t));
 #pragma unroll
       for (int i = 0; i < KLOADS; ++i) {
-        const uint32_t key = k_key + i * (512u / CHUNKS);
-        load_run<BITS>(k_tile + (key < left ? key : left) * stride + k_elem, kr[i]);
+        const uint32_t key = late.k_key + i * (512u / CHUNKS);
+        load_run<BITS>(k_tile + (key < left ? key : left) * stride32 + late.k_elem, kr[i]);
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint32_t key = v_four * 4u + e;
-        load_run<RE * BITS / 8>(v_tile + (key < left ? key : left) * stride + v_elem, vr[e]);
+        const uint32_t key = late.v_four * 4u + e;
+        load_run<RE * BITS / 8>(v_tile + (key < left ? key : left) * stride32 + late.v_elem, vr[e]);
       }
     }
     if constexpr (QUANT) {
@@ -677,13 +699,13 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
     uint8_t* keys = sh.stage[b];
 #pragma unroll
     for (int i = 0; i < KLOADS; ++i) {
-      const uint32_t key = k_key + i * (512u / CHUNKS);
-      *reinterpret_cast<half8_t*>(keys + key * (DP * 2u) + ((k_chunk ^ key_swizzle(key)) * 16u)) = key_operand<KV>(kr[i]);
+      const uint32_t key = own_share.k_key + i * (512u / CHUNKS);
+      *reinterpret_cast<half8_t*>(keys + key * (DP * 2u) + ((own_share.k_chunk ^ key_swizzle(key)) * 16u)) = key_operand<KV>(kr[i]);
     }
     // Row r of block j of a half's values: four chunks of sixteen bytes, chunk c of keys 4c.. and 16 + 4c.. at
     // c ^ r % 4; the rows in the order 0, 4, 8, 12, 1, .., which with that puts sixteen lanes on sixteen bank groups.
-    const uint32_t vrow = v_run >> 1, four = v_four & 7u;
-    uint8_t* values = keys + Shared::kKeyBytes + half * (DP * 64u) + (v_run & 1u) * (RE * 1024u) + value_place(vrow, four & 3u) + (four >> 2) * 8u;
+    const uint32_t vrow = own_share.v_run >> 1, four = own_share.v_four & 7u;
+    uint8_t* values = keys + Shared::kKeyBytes + half * (DP * 64u) + (own_share.v_run & 1u) * (RE * 1024u) + value_place(vrow, four & 3u) + (four >> 2) * 8u;
 #pragma unroll
     for (int j = 0; j < RE; ++j) {
       *reinterpret_cast<uint2*>(values + j * 1024u) = uint2{value_pair<KV>(vr[0], vr[1], j), value_pair<KV>(vr[2], vr[3], j)};
@@ -703,7 +725,7 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
   half8_t q_hi[STEPS], q_lo[STEPS];
   float score_scale = kLog2E / sqrtf(static_cast<float>(D));
   {
-    const float* qp = a.q + ((a.row_base + row) * a.heads + head) * D;
+    const float* qp = a.q + ((a.row_base + mine.row) * a.heads + mine.head) * D;
     float raw[STEPS][8], most = 0.0f;
 #pragma unroll
     for (int i = 0; i < STEPS; ++i) {
@@ -879,10 +901,11 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
 
   // Merge of the two halves' sums under the larger maximum; the lanes' shares of the sum of weights first.
   run_sum = groups_sum(run_sum);
-  float* other = reinterpret_cast<float*>(sh.stage[0]) + col_group * (VE * 256u) + lane;
-  const uint32_t at = col_group * 16u + r;
+  const uint32_t late = again(t), late_g = late >> 4 & 3u;
+  float* other = reinterpret_cast<float*>(sh.stage[0]) + col_group * (VE * 256u) + (late & 63u);
+  const uint32_t at = col_group * 16u + (late & 15u);
   if (half == 1u) {
-    if (g == 0u) sh.most[at] = run_max, sh.sum[at] = run_sum, sh.up[at] = value_up;
+    if (late_g == 0u) sh.most[at] = run_max, sh.sum[at] = run_sum, sh.up[at] = value_up;
 #pragma unroll
     for (int j = 0; j < VE; ++j)
 #pragma unroll
@@ -905,7 +928,7 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
       }
     }
     if (!finite) sh.special = 1u;
-    if (g == 0u) sh.most[at] = most, sh.sum[at] = total;
+    if (late_g == 0u) sh.most[at] = most, sh.sum[at] = total;
   }
   __syncthreads();
   // (the results only now: `out` may be q's memory, which attend_row reads)
@@ -921,25 +944,26 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
         }
       }
       __syncthreads();
-      attend_row<KV, DP, 8>(a, i, kv, head0, here, row_start, row_last, s_part, lds.rows);
+      attend_row<KV, DP, 8, DP == 256 ? 16 : 32>(a, i, kv, head0, here, row_start, row_last, s_part, lds.rows);
     });
     return;
   }
-  if (col_any >= c_end) return;
+  if (c0 + at >= c_end) return;
+  const Column own = column();
   const float total = sh.sum[at];
-  float* out = a.out + ((a.row_base + row) * a.heads + head) * D;
+  float* out = a.out + ((a.row_base + own.row) * a.heads + own.head) * D;
   float factor = 1.0f;
   if (split > 1u) {
-    const uint64_t part = (row * a.heads + head) * split + s_part;
+    const uint64_t part = (own.row * a.heads + own.head) * split + s_part;
     out = a.part.pacc + part * D;
     // The part's largest score in natural units is rounded; the sums move by what that took from it.
     const float most = sh.most[at], natural = score_scale * kLn2, largest = most * natural;
     factor = most == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(fmaf(most, natural, -largest) * kLog2E);
-    if (g == 0u && half == 0u) a.part.pmax[part] = fmaxf(largest, -1e30f), a.part.psum[part] = total * factor;
+    if (late_g == 0u && half == 0u) a.part.pmax[part] = fmaxf(largest, -1e30f), a.part.psum[part] = total * factor;
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const uint32_t e = half * 2u + i, d = (g * 4u + e) * VE;
+    const uint32_t e = half * 2u + i, d = (late_g * 4u + e) * VE;
 #pragma unroll
     for (int j = 0; j < VE; j += 4) {
       float x[4];

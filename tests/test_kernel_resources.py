@@ -20,7 +20,7 @@ NO_SCRATCH = {
     "gemv_kquant_rows.hip": ["kquant_rows_kernel", "kquant_rows_stream_kernel"],
     "gemm_fp8.hip": ["fp8_gemm_kernel"],
     "gemm_mxfp4.hip": ["mxfp4_a8_gemm_kernel"],
-    "attention.hip": ["attention_rows_kernel"],
+    "attention.hip": ["attention_rows_kernel", "attention_tile_kernel"],
     "gemv_q4k_i8.hip": ["q4k_i8_gemv_kernel"],
 }
 
