@@ -1168,13 +1168,12 @@ bool runs_fit(uint32_t head_dim) {
   return head_dim % run == 0 && head_dim % (padded / 16) == 0;
 }
 
-uint64_t tile_units(uint64_t m, uint64_t heads, uint64_t kv_heads) { return (m * (heads / kv_heads) + 63) / 64 * kv_heads; }
-
 // `a.part.split` parts of the keys (0: one, into `a.out`) for each 64 (row, head) pairs.
 template <KvKind KV>
 hipError_t launch_tiles(const AttentionArgs& a, hipStream_t stream) {
   const uint64_t split = a.part.split == 0 ? 1 : a.part.split;
-  const dim3 grid(static_cast<uint32_t>(tile_units(a.rows, a.heads, a.kv_heads) * split));
+  const AttentionCall call{a.rows, a.n, a.heads, a.kv_heads, a.head_dim, 0, false};
+  const dim3 grid(static_cast<uint32_t>(attention_pairs64(call) * split));
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, a); };
   a.head_dim <= 64 ? go(attention_tile_kernel<KV, 64>) : a.head_dim <= 128 ? go(attention_tile_kernel<KV, 128>) : go(attention_tile_kernel<KV, 256>);
   return hipGetLastError();
@@ -1217,24 +1216,15 @@ uint64_t attention_parts(uint32_t kind, uint64_t m, uint64_t n, uint64_t heads, 
   const uint32_t dim = static_cast<uint32_t>(head_dim);
   if (!with_kind(kind, [&](auto tag) { return runs_fit<decltype(tag)::value>(dim); })) return 0;
   if (kv_heads * head_dim * 2 >= (1u << 25)) return 0;             // a tile's rows lie within 2^31 bytes
-  // Sides measured (us, rows' kernel / this one): in parts 17 rows of 24 heads of 256 on 2000 fp16 keys 47 / 30, 40 rows of
-  // 32 of 128 on 2000 int8 keys 53 / 24, but 64 rows of 24 of 256 on 300 keys 17 / 27, 100 rows of 8 of 64 on 500 keys
-  // 10 / 13: the line lies at some 24 M elements of keys met.  In one part: 300 rows of 8 heads of 128 with keys of their own
-  // 152 / 40, 256 rows of 16 of 64 on 100 keys 17 / 12, 100 rows of 8 of 64 on 500 keys 10 / 16.
-  const uint64_t units = tile_units(m, heads, kv_heads), cus = static_cast<uint64_t>(num_cus());
-  if (units >= kMaxGridThreads / 512u) return 0;
   uint64_t keys = causal && q_base + m < n ? q_base + m : n;
   if (causal && window != 0 && window < keys) keys = window;
-  uint64_t parts = cus / units < keys / 256 ? cus / units : keys / 256;
-  if (parts > most_parts) parts = most_parts;
-  while (parts > 1 && attention_parts_bytes(m, heads, head_dim, parts) > kAttentionPartsMost) --parts;
-  const uint64_t row_units = m * kv_heads * ((heads / kv_heads + 7) / 8);   // workgroups of the rows' kernel
-  if (parts > 1 && row_units * padded_head(dim) >= (24u << 20) / keys) return parts;
-  return row_units >= 400 ? 1 : 0;
+  const AttentionCall call{m, keys, heads, kv_heads, head_dim, padded_head(dim), kind != 1};
+  if (attention_pairs64(call) >= kMaxGridThreads / 512u) return 0;
+  return attention_rule(call, static_cast<uint64_t>(num_cus()), most_parts, kAttentionPartsMost);
 }
 
 size_t attention_parts_bytes(uint64_t m, uint64_t heads, uint64_t head_dim, uint64_t parts) {
-  return parts < 2 ? 0 : static_cast<size_t>(m * heads * parts * (head_dim + 2) * 4);
+  return attention_parts_size(m, heads, head_dim, parts);
 }
 
 // kind: 0 fp32, 1 fp16 keys and values; 2 int8, 3 4-bit, 4 E4M3 codes with one scale per key row (always causal).

@@ -4,6 +4,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 
 namespace qmm {
 
@@ -112,6 +113,55 @@ constexpr PackShape pack_shape(uint64_t rows, uint64_t cols) {
   const uint32_t threads = cols <= 6144 || rows * cols <= (uint64_t{1} << 19) ? 256 : 1024;
   const uint64_t share = (cols + threads * 4 - 1) / (threads * 4);
   return {static_cast<uint32_t>(share < 16 ? share : 16), threads};
+}
+
+// ---- "attention" with many query rows -------------------------------------------------------------------------------
+// How a call over an fp16 or a quantized cache runs: 0, the rows' kernel, a workgroup for up to eight heads of a row and
+// key head; else the kernel that shares 64 keys at a time among 64 (row, head) pairs, in so many parts of the keys.  `keys`:
+// how many a row sees at most; `padded`: the head size, 64, 128 or 256.
+//
+// The shorter of the estimated times, in us: a fixed part, then for the rows' kernel what a round of a workgroup a CU takes
+// by its keys (four wavefronts up to 160 keys, eight beyond), for the other what 64 keys take, and for its parts the
+// second launch and the sums' way through memory.  Fitted to 1716 calls (17 to 512 rows, 17 to 2512 keys, 2 to 32 heads over
+// 1 to 8 key heads of 64, 96, 128 and 256, fp16 and int8), which they meet within 4 % on average: one call of them
+// takes the longer way by more than 5 %.  Rows' kernel / one part / parts: 64 rows of 24 heads over 4 of 256 on 564 keys 21 / 34 /
+// 29, on 2064 48 / 95 / 42; 512 rows of 16 over 4 of 64 on 512 27 / 14 / 39; 64 of 8 over 8 of 128 on 64 7 / 10; 300 of 24
+// over 4 of 256 on 2300 285 / 105.
+struct AttentionCall {
+  uint64_t rows, keys, heads, kv_heads, head_dim, padded;
+  bool quantized;
+};
+constexpr uint64_t attention_pairs64(const AttentionCall& a) { return (a.rows * (a.heads / a.kv_heads) + 63) / 64 * a.kv_heads; }
+// Bytes of `parts` parts: a sum of head_dim, the largest score and the sum of weights for each.
+constexpr size_t attention_parts_size(uint64_t rows, uint64_t heads, uint64_t head_dim, uint64_t parts) {
+  return parts < 2 ? 0 : static_cast<size_t>(rows * heads * parts * (head_dim + 2) * 4);
+}
+constexpr uint64_t attention_rule(const AttentionCall& a, uint64_t cus, uint64_t most_parts, size_t most_bytes) {
+  const uint64_t units = attention_pairs64(a), tiles = (a.keys + 63) / 64;
+  const uint64_t row_units = a.rows * a.kv_heads * ((a.heads / a.kv_heads + 7) / 8);
+  uint64_t parts = cus / units < a.keys / 256 ? cus / units : a.keys / 256;
+  if (parts > most_parts) parts = most_parts;
+  while (parts > 1 && attention_parts_size(a.rows, a.heads, a.head_dim, parts) > most_bytes) --parts;
+
+  const int size = a.padded == 64 ? 0 : a.padded == 128 ? 1 : 2;
+  constexpr double kRowFixed[2][3] = {{5.2, 5.5, 5.3}, {5.3, 4.1, 5.3}}, kRowRound[2][3] = {{0.3, 0.65, 3.4}, {0.5, 3.1, 3.4}};
+  constexpr double kRowKey[2][3] = {{0.0047, 0.0102, 0.0194}, {0.005, 0.0083, 0.0194}};
+  constexpr double kTileFixed[3] = {6.1, 8.1, 12.8}, kTile[3] = {1.0, 1.32, 2.31}, kPartsMegabyte[3] = {1.07, 0.85, 0.79};
+  constexpr double kPartsFixed = 2.5;
+  const int wide = a.keys > 160 ? 1 : 0;
+  const uint64_t row_rounds = (row_units + cus - 1) / cus, rounds = (units + cus - 1) / cus;
+  const double key_us = kRowKey[wide][size] * (a.quantized ? 1.12 : 1.0);
+  const double row_us = kRowFixed[wide][size] + (a.quantized ? 0.6 : 0.0) +
+                        static_cast<double>(row_rounds) * (kRowRound[wide][size] + key_us * static_cast<double>(a.keys));
+  const double tile = kTile[size] * (a.quantized ? 1.25 : 1.0);
+  const double one_us = kTileFixed[size] + tile * static_cast<double>(rounds * tiles);
+  if (parts > 1) {
+    const uint64_t part_tiles = ((a.keys + parts - 1) / parts + 63) / 64;
+    const double parts_us = kTileFixed[size] + kPartsFixed + tile * static_cast<double>(part_tiles) +
+                            kPartsMegabyte[size] * static_cast<double>(a.rows * a.heads * parts * a.head_dim * 4) * 1e-6;
+    if (parts_us <= one_us && parts_us < 0.98 * row_us) return parts;
+  }
+  return one_us < 0.98 * row_us ? 1 : 0;
 }
 
 // ---- "attention_combine" ---------------------------------------------------------------------------------------------

@@ -9,13 +9,20 @@ from test_gpu_attention import KINDS, attend, cache, expected
 
 pytestmark = pytest.mark.gpu
 
-CASES = [
+# too little work for it: the rows' kernels
+FEW = [
+    (410, 410, 2, 1, 64, 0, 0), (101, 449, 4, 4, 128, 348, 0), (203, 300, 6, 2, 256, 97, 70), (137, 140, 9, 3, 96, 3, 0),
+    (401, 200, 1, 1, 64, 100, 0),
+]
+ONE_PART = [
     # m, n, heads, kv_heads, head_dim, q_base, window
-    (410, 410, 2, 1, 64, 0, 0),          # 820 pairs: the last workgroup has 52
-    (101, 449, 4, 4, 128, 348, 0),       # a pair a row; one key more than seven tiles
-    (203, 300, 6, 2, 256, 97, 70),       # a window shorter than two tiles
-    (137, 140, 9, 3, 96, 3, 0),          # padded to 128; rows across workgroups
-    (401, 200, 1, 1, 64, 100, 0),        # rows past the last key
+    (410, 410, 8, 4, 64, 0, 0),          # 820 pairs a key head: the last workgroup has 52
+    (101, 449, 16, 16, 128, 348, 0),     # a pair a row; one key more than seven tiles
+    (203, 300, 24, 8, 256, 97, 70),      # a window shorter than two tiles
+    (137, 140, 27, 9, 96, 3, 0),         # padded to 128; rows across workgroups
+    (401, 200, 4, 4, 64, 100, 0),        # rows past the last key
+]
+PARTS = [
     (33, 2100, 24, 4, 256, 2067, 0),     # parts of the keys
     (40, 1100, 8, 8, 128, 1060, 0),
     (70, 1300, 8, 8, 64, 1230, 820),     # parts of which early rows see none of the last, late rows little of the first
@@ -24,7 +31,7 @@ CASES = [
 
 
 @pytest.mark.parametrize("kind", ["f16", "q8", "q4", "fp8"])
-@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("case", FEW + ONE_PART + PARTS)
 def test_attention_tiles(backend, kind, case):
     m, n, heads, kv_heads, head_dim, q_base, window = case
     g = synth.rng(n + head_dim + KINDS[kind])
@@ -39,8 +46,12 @@ def test_attention_tiles(backend, kind, case):
     assert np.all(got[:2] == 7.0) and np.all(got[2 + m:] == 7.0)
 
 
-def test_attention_tiles_not_causal(backend):
-    m, n, heads, kv_heads, head_dim = 101, 203, 4, 4, 128
+SPECIAL = [(101, 449, 16, 16, 128), (33, 2100, 24, 4, 256), (410, 410, 8, 4, 64)]
+
+
+@pytest.mark.parametrize("heads", [4, 16])
+def test_attention_tiles_not_causal(backend, heads):
+    m, n, kv_heads, head_dim = 101, 203, heads, 128
     g = synth.rng(5)
     q = g.standard_normal((m, heads * head_dim)).astype(np.float32)
     k, v = (cache(g, "f16", n, kv_heads * head_dim)[0] for _ in range(2))
@@ -49,7 +60,7 @@ def test_attention_tiles_not_causal(backend):
     assert np.max(np.abs(got - want)) <= 2e-6 * max(1.0, np.max(np.abs(want)))
 
 
-@pytest.mark.parametrize("shape", [(101, 449, 4, 4, 128), (33, 2100, 24, 4, 256), (410, 410, 2, 1, 64)])
+@pytest.mark.parametrize("shape", [*SPECIAL, (101, 449, 4, 4, 128), (410, 410, 2, 1, 64)])
 @pytest.mark.parametrize("what", ["key", "key-", "value", "value nan", "query", "key scale", "value scale", "zeros"])
 def test_attention_tiles_special_values(backend, shape, what):
     m, n, heads, kv_heads, head_dim = shape
@@ -103,7 +114,7 @@ def softmax_rows(q, k, v, heads, kv_heads, head_dim, q_base):
 
 
 @pytest.mark.parametrize("kind", ["f16", "q8"])
-@pytest.mark.parametrize("shape", [(101, 449, 4, 4, 128), (33, 2100, 24, 4, 256), (410, 410, 2, 1, 64)])
+@pytest.mark.parametrize("shape", SPECIAL)
 def test_attention_tiles_key_of_nearly_all_weight_and_no_value(backend, kind, shape):
     """The first key takes all but some e^-20 = 2^-29 of every row's weight and its values are zero, so that the result is
     made of the small weights alone.  They are off by 2^-50 of the largest over an fp16 cache and by 2^-45 of the largest

@@ -144,3 +144,30 @@ def test_combine_stays_within_a_launch(tmp_path):
   }
   CHECK(combine_waves(24, 256, 64) == 16 && combine_waves(24, 256, 4) == 4 && combine_waves(12288, 256, 2) == 1, "waves");
 """)
+
+
+def attention_call(m, n, heads, kv_heads, head_dim, q_base, window, quantized):
+    keys = min(n, q_base + m)
+    keys = min(keys, window) if window else keys
+    padded = 64 if head_dim <= 64 else 128 if head_dim <= 128 else 256
+    return f"attention_rule(AttentionCall{{{m}, {keys}, {heads}, {kv_heads}, {head_dim}, {padded}, {quantized}}}, 256, 64, 16u << 20)"
+
+
+def test_attention_test_cases_take_the_kernel_they_are_for(tmp_path):
+    import test_gpu_attention_tiles as cases
+    special = [(m, n, heads, kv_heads, head_dim, n - m, 0) for m, n, heads, kv_heads, head_dim in cases.SPECIAL]
+    run_program(tmp_path, "\n".join(
+        f"  CHECK({attention_call(*case, quantized)} {wanted}, \"{case}\");"
+        for group, wanted in ((cases.FEW, "== 0"), (cases.ONE_PART, "== 1"), (cases.PARTS, "> 1"), (special, "!= 0"))
+        for case in group for quantized in ("false", "true")))
+
+
+def test_attention_with_too_little_work_stays_with_the_rows_kernel(tmp_path):
+    """Calls that lost by a half or more in the other kernel (measured; us in the rows' kernel / in the other)."""
+    calls = [(64, 564, 24, 4, 256, 500, 0),      # 21 / 34
+             (100, 600, 12, 2, 256, 500, 0),     # 21 / 34
+             (128, 1128, 16, 2, 128, 1000, 0),   # 18 / 27
+             (64, 64, 8, 8, 128, 0, 0),          # 7 / 10
+             (512, 512, 2, 1, 64, 0, 0)]         # 10 / 14
+    leads = [(512, 2512, 24, 4, 256, 2000, 0), (17, 8017, 24, 4, 256, 8000, 0), (200, 200, 24, 4, 256, 0, 0), (512, 512, 16, 4, 64, 0, 0)]
+    run_program(tmp_path, "\n".join(f"  CHECK({attention_call(*c, 'false')} {want}, \"{c}\");" for group, want in ((calls, "== 0"), (leads, "!= 0")) for c in group))
