@@ -17,8 +17,8 @@
  *     tessera::StatusCode (include/tessera/types.hpp:36-48);
  *   - no exceptions cross the boundary;
  *   - device memory: qmm_alloc allocates what the caller asks for; qmm_init allocates the 16 MB
- *     scratch of the decode-sized kernels once and reserves 256 MB for the blocks below; prefill-sized launches (Q4_K/Q5_K/Q6_K from 17
- *     rows, the grouped routed-expert ids) need a workspace, which is the caller's when one was
+ *     scratch of the decode-sized kernels once and reserves 256 + 64 MB for the blocks below; prefill-sized launches
+ *     (Q4_K/Q5_K/Q6_K and MXFP4 with fp32 rows from 17 rows, the grouped routed-expert ids) need a workspace, which is the caller's when one was
  *     set with qmm_set_workspace and otherwise a library-owned block that qmm_launch grows on
  *     demand with hipMalloc.  A block that a launch has used is never freed (growth allocates a
  *     new one of at least twice the size and keeps the old until the process ends, so a launch
@@ -27,14 +27,16 @@
  *     qmm_launch_static never allocates.
  *   - streams: launches that use the decode scratch or the workspace share it, so the caller orders
  *     them (one stream, or events).  Every other launch is independent of launches on other streams;
- *     "gemm_fp8" from 17 rows and "gemm_q5k*" / "gemm_q6k*" with 2..16 rows, which also hand
- *     intermediate results from one kernel to the next, keep them in blocks of their own: 16 MB for
- *     the eager launches of each stream (128 MB more where a "gemm_fp8" call does not fit), and what
- *     they need for each capture and stream that records them.  Blocks come out of the 256 MB that qmm_init reserves, then out of slabs of 128 MB, 2 GB in
- *     all; while a caller's workspace is set no slab is allocated.  They are not given back (a graph may
+ *     those which also hand intermediate results from one kernel to the next keep them in blocks of
+ *     their own, 16 MB for the eager launches of each stream and what they need for each capture and
+ *     stream that records them: "gemm_fp8" from 17 rows (128 MB more where a call does not fit) and
+ *     "gemm_q5k*" / "gemm_q6k*" with 2..16 rows out of the 256 MB that qmm_init reserves, then out of slabs of
+ *     128 MB, 2 GB in all; "attention", "attention_q8", "_q4" and "_fp8" from 17 rows and "top_k_rows" over long
+ *     rows out of 64 MB, then slabs of 64 MB, 512 MB in all.  While a caller's workspace is set no slab is
+ *     allocated.  The blocks are not given back (a graph may
  *     still use them), and a stream handle's block passes to the next stream with that handle: let a
  *     stream's launches finish before it is destroyed.  A launch that gets no block, or is made on
- *     hipStreamPerThread, runs kernels that need none (slower; sums in another order).
+ *     hipStreamPerThread, runs kernels that need none (slower; sums in another order, "top_k_rows" the same results).
  */
 #ifndef TESSERA_QMM_H_
 #define TESSERA_QMM_H_

@@ -171,15 +171,19 @@ void* decode_scratch(const LaunchCtx& c) {
   return c.no_alloc ? g_static_scratch[g_device] : g_decode_scratch;
 }
 
-// Scratch of "gemm_fp8", of Q5_K / Q6_K with a few rows and of "attention" with few columns and of "top_k_rows" over long rows, whose calls on different streams are independent of
+// Scratch of "gemm_fp8" and of Q5_K / Q6_K with a few rows, whose calls on different streams are independent of
 // one another: see stream_scratch.hpp.  qmm_init reserves the first slab; later ones are allocated under the
 // relaxed capture mode, which permits it while a stream is captured, unless the caller has handed over a workspace
 // (then a launch allocates nothing).
 qmm::StreamScratch g_stream_scratch;
+// That of "attention" in parts of its keys and of "top_k_rows" over long rows, likewise, but apart from the first: these
+// calls are as correct without it and lose less, and a program that records them again and again uses theirs up.
+constexpr qmm::ScratchLimits kPartsLimits{size_t{16} << 20, size_t{16} << 20, size_t{64} << 10, size_t{64} << 20, size_t{64} << 20, size_t{512} << 20};
+qmm::StreamScratch g_parts_scratch(kPartsLimits);
 
 class StreamBlock {
  public:
-  StreamBlock(const LaunchCtx& c, size_t bytes) {
+  StreamBlock(const LaunchCtx& c, size_t bytes, qmm::StreamScratch& pool = g_stream_scratch) {
     if (c.no_alloc) {
       ptr_ = bytes <= kStaticScratchBytes ? g_static_scratch[g_device] : nullptr;
       return;
@@ -192,7 +196,7 @@ class StreamBlock {
       status = hipStreamCaptureStatusNone;
     }
     if (status == hipStreamCaptureStatusInvalidated) return;
-    block_ = g_stream_scratch.find(status == hipStreamCaptureStatusActive ? id + 1 : 0, c.stream, bytes, grow);
+    block_ = pool.find(status == hipStreamCaptureStatusActive ? id + 1 : 0, c.stream, bytes, grow);
     if (block_ == nullptr) return;
     block_->busy.lock();
     ptr_ = block_->ptr;
@@ -227,7 +231,7 @@ class StreamBlock {
   qmm::ScratchBlock* block_ = nullptr;
   void* ptr_ = nullptr;
 };
-static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock && qmm::kAttentionPartsMost <= qmm::StreamScratch::kSmallBlock);
+static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock && qmm::kAttentionPartsMost <= kPartsLimits.small);
 
 // Q4_K regimes by activation rows.  One row and small matrices: the VALU GEMV.  2..16 rows of a
 // matrix with at least kQ4KFewRowsMinWeights weights: the exact few-row MFMA kernels (weights read
@@ -520,7 +524,7 @@ qmm_status attend(const LaunchCtx& c, uint32_t kind, const float* k_scale, const
   auto plan = [&](uint64_t most) { return qmm::attention_parts(kind, m, n, heads, kv_heads, head_dim, q_base, window, causal, out, most); };
   const uint64_t parts = plan(64);
   if (parts > 1) {
-    const StreamBlock block(c, qmm::attention_parts_bytes(m, heads, head_dim, parts));
+    const StreamBlock block(c, qmm::attention_parts_bytes(m, heads, head_dim, parts), g_parts_scratch);
     if (block.get() != nullptr) return go(parts, block.get());
     return go(plan(1), nullptr);
   }
@@ -1360,7 +1364,7 @@ qmm_status run_top_k_rows(const LaunchCtx& c) {
     return bad("top_k_rows: buffer too small");
   }
   const size_t keys = qmm::top_k_rows_scratch_bytes(static_cast<uint32_t>(rows), vocab, static_cast<uint32_t>(top_k));
-  const StreamBlock block(c, keys);
+  const StreamBlock block(c, keys, g_parts_scratch);
   return map_hip(qmm::launch_top_k_rows(c.ptr<const float>(0), c.ptr<uint32_t>(1), c.ptr<float>(2),
                                         static_cast<uint32_t>(rows), vocab, static_cast<uint32_t>(top_k), base,
                                         keys == 0 ? nullptr : block.get(), c.stream));
@@ -1538,7 +1542,9 @@ qmm_status qmm_init(int device) {
       return map_hip(e);
     }
   }
-  (void)g_stream_scratch.reserve(StreamBlock::grow);   // (without it the ids that use it run kernels that need none)
+  // (without them the ids that use them run kernels that need none)
+  (void)g_stream_scratch.reserve(StreamBlock::grow);
+  (void)g_parts_scratch.reserve(StreamBlock::grow);
   return QMM_OK;
 }
 

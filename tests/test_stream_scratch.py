@@ -82,6 +82,17 @@ int main() {
     last = x.second;
   }
   std::printf("%zu blocks\n", all.size());
+  // limits of its own: another pool with small blocks, used up by captures, and what is given out still found
+  static StreamScratch small({MB, MB, 64 << 10, 4 * MB, 4 * MB, 8 * MB});
+  taken = 0;
+  CHECK(small.reserve(grow) && taken == 4 * MB && small.find(0, stream(1), MB + 1, grow) == nullptr);
+  ScratchBlock* eager = small.find(0, stream(1), 100, grow);
+  ScratchBlock* first = small.find(1, stream(1), 100, grow);
+  CHECK(eager && eager->bytes == MB && first && first->bytes == 64 << 10);
+  size_t given = 0;
+  for (uint64_t i = 2; i < 1000; ++i) given += small.find(i, stream(1), 100, grow) != nullptr;
+  CHECK(given == (7 * MB) / (64 << 10) - 1 && taken == 8 * MB);
+  CHECK(small.find(1, stream(1), 64 << 10, grow) == first && small.find(0, stream(1), MB, grow) == eager);
 }
 """
 
