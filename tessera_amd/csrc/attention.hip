@@ -557,9 +557,10 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 //   element VE r + j, so that a lane ends up with runs of a row of the result.
 // A tile's contribution, the second terms' sum brought down by 2^-11 and the first terms' added to it, is summed by
 // itself and added to the running sum, so that rounding there goes with a few terms and not with the number of keys.
-// 512 rows of 24 heads of 256 on 2512 fp16 keys of 4: 119 us (432 with a workgroup a row and key head, which read each
-// key for six columns), int8 keys 125 (455).  Vector instructions issue in 51 % of the cycles, the matrix cores are busy
-// in 32 %, LDS in 29 %; a wavefront waits in 39 % of its own, at the tile's barrier and for operands.
+// 512 rows of 24 heads of 256 on 2512 fp16 keys of 4: 121 us among other calls (432 with a workgroup a row and key head,
+// which read each key for six columns), back to back 107 (417), int8 keys 121 (439).  Vector instructions issue in 60 % of
+// the cycles, the matrix cores are busy in 32 %, LDS in 29 %; a wavefront waits in 34 % of its own, at the tile's barrier
+// and for operands.
 // Infinities and NaN are not kept apart here.  Whatever meets one ends with a sum that is not finite, or sets
 // `special`; the workgroup's columns are then done again with attend_row.
 template <int DP>

@@ -49,9 +49,9 @@ __device__ __forceinline__ void direct_load4(const void* base, uint32_t voff, ui
 // per term 237, 800 of 6144 x 5120 178 / 183, 256 of 4096 x 2048 36 / 34.
 // Shared: likewise, and the (tile, step) units of the product's plan are dealt out evenly, workgroup g taking those from
 // unit_bound(g) on: 453 rows of 17408 columns are 136 tiles of 256 x 256, which took half the chip 247 us; shared by all
-// of it 165 and 20 for the sums, the clock then held down by power, the matrix cores busy in 58 % of the cycles.  A tile
-// that several workgroups share has its sums in `parts`, one block of BM x BN a piece, for split_sums_kernel to add up in
-// their order.
+// of it 176 (155 to 199 with the clock, held down by power) and 17 to 24 for the sums, the matrix cores busy in 65 % of
+// the cycles.  A tile that several workgroups share has its sums in `parts`, one block of BM x BN a piece, for
+// split_sums_kernel to add up in their order.
 // Cut: the same where there is no room for `parts`.  A workgroup has whole tiles, each within one of the plan's; it cuts
 // their sums where the plan does and adds the pieces in the same order, in registers: the same bits.
 enum class Rows { E4M3, Terms, Shared, Cut };

@@ -115,7 +115,7 @@ size_t gemm_fp8_f16_scratch_bytes(uint64_t m, uint64_t n, uint64_t k, size_t lim
 hipError_t launch_fp8_f16_gemm(const float* a, const uint8_t* w, const float* w_scale, float* c, void* scratch, size_t limit,
                                uint32_t m, uint32_t n, uint32_t k, hipStream_t stream);
 size_t gemm_mxfp4_f32_workspace_bytes(uint64_t m, uint64_t k);
-// gemm_mxfp4_f32_parts_bytes: of `parts`, which may be null (tiles are then not shared among workgroups); 0: not used.
+// gemm_mxfp4_f32_parts_bytes: of `parts`; 0: not used.  Without them (null) no workgroups share a tile; the same bits.
 size_t gemm_mxfp4_f32_parts_bytes(uint64_t m, uint64_t n, uint64_t k);
 hipError_t launch_mxfp4_f32_gemm(const float* a, const uint8_t* w, float* c, void* workspace, float* parts, uint32_t m,
                                  uint32_t n, uint32_t k, hipStream_t stream);
