@@ -132,39 +132,6 @@ bool gemm_q4k_supported(uint64_t m, uint64_t k) { return k % 256 == 0 && k <= (1
 // fp16 copy of A, then one scale per row padded by a tile of rows (the epilogue reads scales in fours).
 size_t gemm_q4k_workspace_bytes(uint64_t m, uint64_t k) { return static_cast<size_t>(m) * k * 2 + (static_cast<size_t>(m) + 256) * 4; }
 
-// The bulk of C goes to 256 x 256 tiles, whole rounds of one tile per CU; columns left over
-// when the tile count is not a multiple of the CU count are cut into 128 x 64 tiles that
-// spread over every CU instead of keeping a few CUs busy for a whole extra round.
-hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* workspace, uint32_t m,
-                           uint32_t n, uint32_t k, hipStream_t stream) {
-  _Float16* a16 = static_cast<_Float16*>(workspace);
-  float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
-  launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
-  const uint32_t cus = static_cast<uint32_t>(num_cus());
-  const uint32_t tiles_m = (m + 255u) / 256u, tiles_n = (n + 255u) / 256u;
-  const uint32_t tiles = tiles_m * tiles_n;
-  uint32_t main_tn = tiles_n;
-  if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) {
-    main_tn = (tiles / cus) * cus / tiles_m;
-  } else if (tiles < cus / 2) {
-    main_tn = 0;
-  }
-  if (m <= 64) {
-    // A short stack of rows is bound by the weight stream: narrow tiles (one wavefront, 32
-    // columns) give every CU several workgroups' worth of super-blocks in flight.
-    if (m <= 32) {
-      launch_range<32, 32>(a16, a_scale, w, c, m, n, k, 0u, n, stream);
-    } else {
-      launch_range<64, 32>(a16, a_scale, w, c, m, n, k, 0u, n, stream);
-    }
-    return hipGetLastError();
-  }
-  const uint32_t n_split = main_tn * 256u < n ? main_tn * 256u : n;
-  if (n_split > 0) launch_range<256, 256, 128, 64>(a16, a_scale, w, c, m, n, k, 0u, n_split, stream);
-  if (n_split < n) launch_range<128, 64, 64, 32>(a16, a_scale, w, c, m, n, k, n_split, n, stream);
-  return hipGetLastError();
-}
-
 // The feed forward's front half in one product: tiles of 128 columns of either matrix (gate_up_large_tiles).  2048 rows of
 // 17408 x 5120: 858 us, as two products and silu_mul 940.
 hipError_t launch_q4k_gate_up(const float* a, const uint8_t* gate, const uint8_t* up, float* c, void* workspace, uint32_t m,
@@ -276,10 +243,13 @@ __global__ __launch_bounds__(256) void q5k_to_f16_kernel(const uint8_t* __restri
 // CU, and four SIMDs start a matrix instruction of 32 clocks each: 128 x 64 takes six reads to eight instructions, 64 x 96
 // five to six (256 x 32, nine to eight, was bound by them: 160 tiles of 2048 rows x 5120 columns, K = 17408, 500 us).  The
 // reads of a 16-wide K step go between the matrix instructions of the one before.
+//
+// The sums of one tile at (m0, n0) over `slices` 32-wide slices of K from slice0 on; no direct load is in flight when it
+// returns.
 template <int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
-    const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const _Float16* __restrict__ w16,
-    float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end, bool as_decoded) {
+__device__ __forceinline__ void f16w_tile_sums(TileSums<WM, WN>& acc, const _Float16* __restrict__ a16, const _Float16* __restrict__ w16,
+                                               uint32_t m, uint32_t n, uint32_t k, uint32_t m0, uint32_t n0, uint32_t slice0,
+                                               uint32_t slices) {
   constexpr int kWavesN = BN / WN, kWaves = (BM / WM) * kWavesN, kTI = WM / 32, kTJ = WN / 32;
   constexpr int kABlk = BM / 16 / kWaves, kWBlk = (BN / 16 + kWaves - 1) / kWaves;   // 1 KB blocks per wavefront and slice
   constexpr int kDma = kABlk + kWBlk;
@@ -287,17 +257,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
   static_assert(BM % (16 * kWaves) == 0 && BN % 16 == 0 && WM % 32 == 0 && WN % 32 == 0, "tile shape");
   __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kStage];
 
-  const uint32_t tiles_n = (n_end - n_begin + BN - 1) / BN;
-  const TileAt at = as_decoded ? TileAt{blockIdx.x / tiles_n, blockIdx.x % tiles_n} : xcd_tile(blockIdx.x, (m + BM - 1) / BM, tiles_n);
-  const uint32_t m0 = at.m * BM, n0 = n_begin + at.n * BN;
   const uint32_t t = threadIdx.x, lane = t & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const uint32_t wave_m = wave / kWavesN, wave_n = wave % kWavesN;
   const uint32_t l32 = lane & 31u, kg = lane >> 5;
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
       (__attribute__((address_space(3))) uint8_t*)lds));
-  const uint8_t* a_tile = reinterpret_cast<const uint8_t*>(a16) + static_cast<size_t>(m0) * k * 2;
-  const uint8_t* w_tile = reinterpret_cast<const uint8_t*>(w16) + static_cast<size_t>(n0) * k * 2;
+  const uint8_t* a_tile = reinterpret_cast<const uint8_t*>(a16) + static_cast<size_t>(m0) * k * 2 + slice0 * 64u;
+  const uint8_t* w_tile = reinterpret_cast<const uint8_t*>(w16) + static_cast<size_t>(n0) * k * 2 + slice0 * 64u;
 
   // Block L of a slice = rows 16L..16L+15, four 16-byte chunks a row: lane p fetches row
   // 16L + p/4, chunk (p%4) ^ ((row>>2)&3).  Rows past the matrix edge are clamped (never stored), and so are
@@ -313,7 +280,6 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
     const uint32_t row_any = 16u * (wave * kWBlk + i) + lane / 4u, row = row_any < BN ? row_any : BN - 1u;
     w_src[i] = (n0 + row < n ? row : n - 1u - n0) * (k * 2u) + (((lane % 4u) ^ ((row >> 2) & 3u)) * 16u);
   }
-  const uint32_t slices = k / 32;
   auto issue = [&](uint32_t slice_any) {
     const uint32_t slice = __builtin_amdgcn_readfirstlane(slice_any < slices ? slice_any : slices - 1u), stage = slice_any & 3u;
 #pragma unroll
@@ -324,7 +290,6 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
       direct_load16(w_tile + slice * 64u, w_src[i], lds_base + stage * kStage + kAStage + (wave * kWBlk + i) * 1024u);
   };
 
-  float16_t acc[kTI][kTJ];
 #pragma unroll
   for (int i = 0; i < kTI; ++i)
 #pragma unroll
@@ -383,25 +348,18 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
     multiply_reading(f1, slice + 1u, 0, f0);    // (after the last slice: a stage that nobody needs)
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct load may outlive the workgroup
+}
 
-#pragma unroll
-  for (int i = 0; i < kTI; ++i) {
-    const uint32_t row0 = m0 + wave_m * WM + i * 32u + kg * 4u;
-    float4 sc[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) sc[q] = *reinterpret_cast<const float4*>(a_scale + row0 + q * 8u);
-#pragma unroll
-    for (int j = 0; j < kTJ; ++j) {
-      const uint32_t col = n0 + wave_n * WN + j * 32u + l32;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const uint32_t row = row0 + (e >> 2) * 8u + (e & 3u);
-        const float4 s4 = sc[e >> 2];
-        const float rs = (e & 3) == 0 ? s4.x : (e & 3) == 1 ? s4.y : (e & 3) == 2 ? s4.z : s4.w;
-        if (row < m && col < n_end) c[static_cast<size_t>(row) * n + col] = acc[i][j][e] * rs;
-      }
-    }
-  }
+template <int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void f16w_gemm_kernel(
+    const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const _Float16* __restrict__ w16,
+    float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end, bool as_decoded) {
+  const uint32_t tiles_n = (n_end - n_begin + BN - 1) / BN;
+  const TileAt at = as_decoded ? TileAt{blockIdx.x / tiles_n, blockIdx.x % tiles_n} : xcd_tile(blockIdx.x, (m + BM - 1) / BM, tiles_n);
+  const uint32_t m0 = at.m * BM, n0 = n_begin + at.n * BN;
+  TileSums<WM, WN> acc;
+  f16w_tile_sums<BM, BN, WM, WN>(acc, a16, w16, m, n, k, m0, n0, 0u, k / 32u);
+  q4k_tile_store<BM, BN, WM, WN>(acc, a_scale, c, m, n, m0, n0, n_end);
 }
 
 template <int BM, int BN, int WM, int WN>
@@ -412,7 +370,174 @@ void launch_f16w_range(const _Float16* a16, const float* a_scale, const _Float16
                      w16, c, m, n, k, n_begin, n_end, f16w_tiles_as_decoded(m, n, k, static_cast<uint32_t>(num_cus()), BM == 128));
 }
 
+// ---- tiles whose steps of K workgroups share --------------------------------------------------------------------------
+// A (tile, super-block) unit is 256 of K.  The tiles' units, tile after tile down the columns, are dealt out evenly:
+// workgroup g takes those from unit_bound(g) on.  A tile that several share has its sums in `parts`, block g + t for
+// workgroup g's piece of tile t, each in the order in which the registers lie (a float4 of a lane is four rows of a
+// column), for piece_sums_kernel to add up in the workgroups' order.  512 rows of 1024 x 5120: Q4_K 44 -> 26 us (the tiles
+// 37 -> 14, the sums 5), Q6_K 46 -> 30; of 6144 x 5120 Q4_K 66 -> 60.
+// CUT: no room for `parts`, but the same bits.  A workgroup has a whole tile (within one of the plan's, of as many rows) and adds
+// its pieces in registers, in that order: the same bits.
+struct Q4KWeights {
+  using Type = uint8_t;
+  static constexpr int kCutWN = 64;
+  template <int BM, int BN, int WM, int WN>
+  static __device__ __forceinline__ void sums(TileSums<WM, WN>& acc, const _Float16* a16, const Type* w, uint32_t m, uint32_t n,
+                                              uint32_t k, uint32_t m0, uint32_t n0, uint32_t from, uint32_t to) {
+    q4k_tile_sums<BM, BN, 2 * WM, WN, false, 2>(acc, a16, w, m, n, k, m0, n0, from, to - from);
+  }
+};
+struct F16Weights {
+  using Type = _Float16;
+  static constexpr int kCutWN = 32;
+  template <int BM, int BN, int WM, int WN>
+  static __device__ __forceinline__ void sums(TileSums<WM, WN>& acc, const _Float16* a16, const Type* w, uint32_t m, uint32_t n,
+                                              uint32_t k, uint32_t m0, uint32_t n0, uint32_t from, uint32_t to) {
+    f16w_tile_sums<BM, BN, WM, WN>(acc, a16, w, m, n, k, m0, n0, from * 8u, (to - from) * 8u);
+  }
+};
+
+template <class W, int BM, int BN, int WM, int WN, bool CUT>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, CUT ? 1 : 2) void shared_tiles_kernel(
+    const _Float16* __restrict__ a16, const float* __restrict__ a_scale, const typename W::Type* __restrict__ w,
+    float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, float* __restrict__ parts, SharedTiles plan) {
+  constexpr int kTI = WM / 32, kTJ = WN / 32;
+  const uint32_t steps = k / 256u, tiles_m = (m + BM - 1) / BM;
+  TileSums<WM, WN> acc;
+  if constexpr (CUT) {
+    const uint32_t m0 = blockIdx.x % tiles_m * BM, n0 = blockIdx.x / tiles_m * BN;
+    const uint64_t first = static_cast<uint64_t>(n0 / plan.columns * tiles_m + m0 / plan.rows) * steps;
+    uint32_t owner = unit_owner(first, plan, steps), from = 0;
+    TileSums<WM, WN> total = {};
+    while (from < steps) {
+      const uint64_t cut = unit_bound(++owner, plan.groups, plan.tiles, steps) - first;
+      const uint32_t to = cut < steps ? static_cast<uint32_t>(cut) : steps;
+      W::template sums<BM, BN, WM, WN>(acc, a16, w, m, n, k, m0, n0, from, to);
+      const bool whole = from == 0u && to == steps;
+#pragma unroll
+      for (int i = 0; i < kTI; ++i)
+#pragma unroll
+        for (int j = 0; j < kTJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) total[i][j][e] = whole ? acc[i][j][e] : total[i][j][e] + acc[i][j][e];
+      from = to;
+      if (from < steps) __syncthreads();      // every wavefront has read the last slice
+    }
+    q4k_tile_store<BM, BN, WM, WN>(total, a_scale, c, m, n, m0, n0, n);
+  } else {
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Workgroups go round the eight XCDs: neighbours in the units' order, which read the same weights, stay on one.
+    const uint32_t group = gridDim.x % 8u == 0u ? blockIdx.x % 8u * (gridDim.x / 8u) + blockIdx.x / 8u : blockIdx.x;
+    uint64_t v = unit_bound(group, plan.groups, plan.tiles, steps);
+    const uint64_t end = unit_bound(group + 1u, plan.groups, plan.tiles, steps);
+    while (v < end) {
+      const uint32_t tile = static_cast<uint32_t>(v / steps), from = static_cast<uint32_t>(v % steps);
+      const uint32_t to = end - v < steps - from ? from + static_cast<uint32_t>(end - v) : steps;
+      const uint32_t m0 = tile % tiles_m * BM, n0 = tile / tiles_m * BN;
+      W::template sums<BM, BN, WM, WN>(acc, a16, w, m, n, k, m0, n0, from, to);
+      if (from == 0u && to == steps) {
+        q4k_tile_store<BM, BN, WM, WN>(acc, a_scale, c, m, n, m0, n0, n);
+      } else {
+        float4_t* block = reinterpret_cast<float4_t*>(parts + static_cast<size_t>(group + tile) * (BM * BN));
+#pragma unroll
+        for (int i = 0; i < kTI; ++i) {
+          if (m0 + (wave / (BN / WN)) * WM + i * 32u >= m) continue;
+#pragma unroll
+          for (int j = 0; j < kTJ; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              block[(((wave * kTI + i) * kTJ + j) * 4u + q) * 64u + lane] =
+                  float4_t{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        }
+      }
+      v += to - from;
+      if (v < end) __syncthreads();           // every wavefront has read the last slice
+    }
+  }
+}
+
+// Adds the pieces of the tiles that several workgroups shared and scales: a workgroup a 32 x 32 matrix tile, a float4 a thread.
+template <int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256) void piece_sums_kernel(const float* __restrict__ parts, const float* __restrict__ a_scale,
+                                                         float* __restrict__ c, uint32_t m, uint32_t n, uint32_t steps,
+                                                         SharedTiles plan) {
+  constexpr uint32_t kTI = WM / 32, kTJ = WN / 32, kPer = BM * BN / 1024;
+  const uint32_t tile = blockIdx.x / kPer, at = blockIdx.x % kPer, tiles_m = (m + BM - 1) / BM;
+  const uint64_t v0 = static_cast<uint64_t>(tile) * steps, v1 = v0 + steps;
+  const uint32_t first = unit_owner(v0, plan, steps), last = unit_owner(v1 - 1u, plan, steps);
+  const uint32_t wave = at / (kTI * kTJ), i = at / kTJ % kTI, j = at % kTJ, lane = threadIdx.x & 63u;
+  const uint32_t row0 = tile % tiles_m * BM + wave / (BN / WN) * WM + i * 32u;
+  if (first == last || row0 >= m) return;
+  const float4_t* block = reinterpret_cast<const float4_t*>(parts + static_cast<size_t>(first + tile) * (BM * BN)) + at * 256u + threadIdx.x;
+  float4_t sum = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  for (uint32_t g = first; g <= last; ++g, block += BM * BN / 4) sum += *block;
+  const uint32_t col = tile / tiles_m * BN + wave % (BN / WN) * WN + j * 32u + (lane & 31u);
+  const uint32_t row = row0 + (threadIdx.x >> 6) * 8u + (lane >> 5) * 4u;
+  if (col >= n) return;
+#pragma unroll
+  for (uint32_t e = 0; e < 4; ++e) {
+    if (row + e < m) c[static_cast<size_t>(row + e) * n + col] = sum[e] * a_scale[row + e];
+  }
+}
+
+template <class W>
+hipError_t launch_shared(const _Float16* a16, const float* a_scale, const typename W::Type* w, float* c, float* parts, uint32_t m,
+                         uint32_t n, uint32_t k, const SharedTiles& plan, hipStream_t stream) {
+  if (parts == nullptr) {
+    constexpr int WN = W::kCutWN;
+    hipLaunchKernelGGL((shared_tiles_kernel<W, 128, 64, 64, WN, true>), dim3((m + 127u) / 128u * ((n + 63u) / 64u)),
+                       dim3(2 * 64 / WN * 64), 0, stream, a16, a_scale, w, c, m, n, k, parts, plan);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((shared_tiles_kernel<W, 128, 128, 64, 64, false>), dim3(plan.groups), dim3(256), 0, stream, a16, a_scale, w, c, m,
+                     n, k, parts, plan);
+  hipLaunchKernelGGL((piece_sums_kernel<128, 128, 64, 64>), dim3(plan.tiles * 16u), dim3(256), 0, stream, parts, a_scale, c, m, n,
+                     k / 256u, plan);
+  return hipGetLastError();
+}
+
 }  // namespace
+
+// The bulk of C goes to 256 x 256 tiles, whole rounds of one tile per CU; columns left over
+// when the tile count is not a multiple of the CU count are cut into 128 x 64 tiles that
+// spread over every CU instead of keeping a few CUs busy for a whole extra round.
+hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* workspace, const SharedPieces& pieces, uint32_t m,
+                           uint32_t n, uint32_t k, hipStream_t stream) {
+  _Float16* a16 = static_cast<_Float16*>(workspace);
+  float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
+  launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
+  const uint32_t cus = static_cast<uint32_t>(num_cus());
+  const SharedTiles plan = shared_f16_tiles(m, n, k / 256u, cus, true);
+  if (plan.groups != 0u && (pieces.at != nullptr || pieces.cut)) {
+    return launch_shared<Q4KWeights>(a16, a_scale, w, c, pieces.at, m, n, k, plan, stream);
+  }
+  const uint32_t tiles_m = (m + 255u) / 256u, tiles_n = (n + 255u) / 256u;
+  const uint32_t tiles = tiles_m * tiles_n;
+  uint32_t main_tn = tiles_n;
+  if (tiles > cus && tiles % cus != 0 && tiles % cus <= cus / 2) {
+    main_tn = (tiles / cus) * cus / tiles_m;
+  } else if (tiles < cus / 2) {
+    main_tn = 0;
+  }
+  if (m <= 64) {
+    // A short stack of rows is bound by the weight stream: narrow tiles (one wavefront, 32
+    // columns) give every CU several workgroups' worth of super-blocks in flight.
+    if (m <= 32) {
+      launch_range<32, 32>(a16, a_scale, w, c, m, n, k, 0u, n, stream);
+    } else {
+      launch_range<64, 32>(a16, a_scale, w, c, m, n, k, 0u, n, stream);
+    }
+    return hipGetLastError();
+  }
+  const uint32_t n_split = main_tn * 256u < n ? main_tn * 256u : n;
+  if (n_split > 0) launch_range<256, 256, 128, 64>(a16, a_scale, w, c, m, n, k, 0u, n_split, stream);
+  if (n_split < n) launch_range<128, 64, 64, 32>(a16, a_scale, w, c, m, n, k, n_split, n, stream);
+  return hipGetLastError();
+}
+
+size_t gemm_f16_parts_bytes(uint64_t m, uint64_t n, uint64_t k, bool q4k) {
+  return shared_tiles_bytes(shared_f16_tiles(m, n, k / 256, static_cast<uint64_t>(num_cus()), q4k));
+}
 
 bool gemm_kquant_f16_supported(uint64_t m, uint64_t n, uint64_t k) {
   return k % 256 == 0 && k <= (1u << 20) && m * k < (1ull << 31) && n * k < (1ull << 31);
@@ -425,7 +550,7 @@ size_t gemm_kquant_f16_workspace_bytes(uint64_t m, uint64_t n, uint64_t k) {
 
 // block_bytes selects the format: 176 = Q5_K, 210 = Q6_K.
 hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t block_bytes, float* c, void* workspace,
-                                  uint32_t m, uint32_t n, uint32_t k, hipStream_t stream) {
+                                  const SharedPieces& pieces, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream) {
   _Float16* a16 = static_cast<_Float16*>(workspace);
   float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
   _Float16* w16 = reinterpret_cast<_Float16*>(a_scale + m + 256);
@@ -440,6 +565,10 @@ hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t blo
     return hipErrorInvalidValue;
   }
   launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
+  const SharedTiles plan = shared_f16_tiles(m, n, k / 256u, static_cast<uint64_t>(num_cus()), false);
+  if (plan.groups != 0u && (pieces.at != nullptr || pieces.cut)) {
+    return launch_shared<F16Weights>(a16, a_scale, w16, c, pieces.at, m, n, k, plan, stream);
+  }
   const F16wTiles tiles = f16w_tiles(m, n, k, static_cast<uint32_t>(num_cus()));
   const uint32_t n_split = tiles.large * tiles.columns < n ? tiles.large * tiles.columns : n;
   if (n_split > 0) {

@@ -9,9 +9,9 @@
 namespace qmm {
 
 // ---- MXFP4, 17 fp32 rows and more: tiles whose steps of K workgroups share --------------------------------------
-// Tiles of `rows` x 256, `tiles` of them; the (tile, step) units go to `groups` workgroups.  groups 0: not shared.
+// Tiles of `rows` x `columns`, `tiles` of them; the (tile, step) units go to `groups` workgroups.  groups 0: not shared.
 struct SharedTiles {
-  uint32_t rows = 0, tiles = 0, groups = 0;
+  uint32_t rows = 0, tiles = 0, groups = 0, columns = 256;
 };
 // First of the units of workgroup g.
 constexpr uint64_t unit_bound(uint32_t g, uint32_t groups, uint32_t tiles, uint32_t steps) {
@@ -25,7 +25,7 @@ constexpr uint32_t unit_owner(uint64_t v, const SharedTiles& plan, uint32_t step
 }
 // The piece of tile t that workgroup g holds is block g + t: along the units one of the two grows from piece to piece.
 constexpr size_t shared_tiles_bytes(const SharedTiles& plan) {
-  return plan.groups == 0u ? 0 : (static_cast<size_t>(plan.groups) + plan.tiles - 1u) * plan.rows * 256u * 4u;
+  return plan.groups == 0u ? 0 : (static_cast<size_t>(plan.groups) + plan.tiles - 1u) * plan.rows * plan.columns * 4u;
 }
 // Rows a tile: the padding it takes decides.  Workgroups: as many as the chip holds, at least four units each.
 // Tiles are shared where whole ones, small (128 x 64) or 256 x 256, leave much of the chip idle for long.  Sides measured
@@ -45,6 +45,27 @@ constexpr SharedTiles shared_tiles(uint64_t m, uint64_t n, uint64_t steps, uint6
   if (steps < 40 && small * 8 >= cus * 7 && small <= cus) return {};
   const uint64_t room = cus * (rows == 64 ? 2 : 1), most = tiles * steps / 4;
   return {static_cast<uint32_t>(rows), static_cast<uint32_t>(tiles), static_cast<uint32_t>(room < most ? room : most)};
+}
+
+// ---- Q4_K from 64 rows, Q5_K and Q6_K from 17: tiles whose super-blocks workgroups share --------------------------------
+// Tiles of 128 x 128 whose (tile, super-block) units go to one workgroup a CU, at least two units each.  Whole tiles of
+// 128 x 64 leave most CUs idle while a few walk all of K: 512 rows of 1024 x 5120 are 64 of them.  The pieces cost a launch
+// and twice their bytes, so that with few super-blocks, or tiles that fill the chip, whole ones lead; `small` counts those.
+// Sides measured (us, whole / shared).  Q4_K, rows x n x k: 100 x 512 x 2048 (8 small) 19.6 / 14.5, 100 x 6144 x 2048 (96) 21.2 /
+// 22.9; 512 x 2048 x 3072 (128) 31 / 25, 200 x 6144 x 3072 (192) 29 / 32; 512 x 1024 x 5120 (64) 44 / 26, 512 x 6144 x 5120 (384)
+// 69 / 56, 2048 x 6144 x 5120 (1536) 183 / 220; 256 x 5120 x 17408 (160) 126 / 84, 1024 (640) 316 / 267, 2048 (1280) 452 / 492.
+// Q5_K and Q6_K, whose whole tiles need no decode and go up to 256 x 256: 100 x 512 x 2048 (8) 22 / 19, 24 x 6144 x 2048 (96) 28 /
+// 33; 200 x 2048 x 3072 (64) 33 / 28, 24 x 4096 x 3072 (64) 32 / 33, 384 x 4096 x 3072 (192) 36 / 38; 512 x 1024 x 5120 (64) 46 / 29,
+// 512 x 6144 x 5120 (384) 80 / 79, 200 x 6144 x 5120 (192) 57 / 59; 512 x 3072 x 8192 (192) 66 / 75.
+constexpr SharedTiles shared_f16_tiles(uint64_t m, uint64_t n, uint64_t steps, uint64_t cus, bool q4k) {
+  if (m > 256 * cus || n > 256 * cus || steps < 8) return {};
+  const uint64_t tiles = (m + 127) / 128 * ((n + 127) / 128), small = (m + 127) / 128 * ((n + 63) / 64);
+  uint64_t most = 0;       // small tiles, eighths of the CUs
+  if (q4k) most = steps < 12 ? 2 : steps < 16 ? 4 : steps < 20 ? 8 : 20;
+  else most = (steps < 12 ? 2 : steps < 16 ? 4 : steps < 20 ? 6 : 8) / (m <= 32 && steps < 20 ? 2 : 1);
+  if (small * (q4k ? 8 : 16) > cus * most) return {};
+  const uint64_t units = tiles * steps / 2;
+  return {128, static_cast<uint32_t>(tiles), static_cast<uint32_t>(cus < units ? cus : units), 128};
 }
 
 // ---- "ffn_gate_up_silu_q4k", more than 64 rows ----------------------------------------------------------------------

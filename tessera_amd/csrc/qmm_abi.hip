@@ -103,6 +103,8 @@ static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 constexpr int kMaxDevices = 64;
 void* g_static_scratch[kMaxDevices] = {};
 
+constexpr size_t round256(size_t bytes) { return (bytes + 255) & ~size_t{255}; }
+
 // `bytes` of scratch, and `*more` bytes behind them where they can be had (0 is left in it where not: such a call does
 // without).
 qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out, size_t* more = nullptr) {
@@ -233,6 +235,31 @@ class StreamBlock {
 };
 static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock && qmm::kAttentionPartsMost <= kPartsLimits.small);
 
+// The workspace of a product whose tiles workgroups may share (`operands` bytes) and room for the tiles' pieces: a stream's
+// block, apart from the other families' for their sake; for qmm_launch_static what the static array has behind the
+// operands and behind `taken`.  Without room the tiles stay whole; without room in the static array their sums are cut and
+// added as the pieces are, so that the bits are qmm_launch's.
+constexpr qmm::ScratchLimits kTilesLimits{size_t{16} << 20, size_t{40} << 20, size_t{512} << 10, size_t{128} << 20, size_t{128} << 20, size_t{1} << 30};
+qmm::StreamScratch g_tiles_scratch(kTilesLimits);
+
+class PiecesRoom {
+ public:
+  PiecesRoom(const LaunchCtx& c, size_t operands, size_t taken, size_t pieces, void** ws)
+      : at_(round256(operands > taken ? operands : taken)), more_(c.no_alloc && pieces != 0 ? at_ - operands + pieces : 0),
+        status_(workspace(c, operands, ws, &more_)), block_(c, c.no_alloc || status_ != QMM_OK ? 0 : pieces, g_tiles_scratch) {
+    if (c.no_alloc) pieces_ = {more_ == 0 ? nullptr : reinterpret_cast<float*>(static_cast<uint8_t*>(*ws) + at_), true};
+    else pieces_ = {static_cast<float*>(block_.get()), false};
+  }
+  qmm_status status() const { return status_; }
+  qmm::SharedPieces pieces() const { return pieces_; }
+
+ private:
+  size_t at_, more_;
+  qmm_status status_;
+  StreamBlock block_;
+  qmm::SharedPieces pieces_{};
+};
+
 // Q4_K regimes by activation rows.  One row and small matrices: the VALU GEMV.  2..16 rows of a
 // matrix with at least kQ4KFewRowsMinWeights weights: the exact few-row MFMA kernels (weights read
 // once).  The tiled fp16 MFMA GEMM, whose operands are rounded to fp16 as in the reference's
@@ -256,20 +283,21 @@ bool q4k_takes_rows16(uint64_t m, uint64_t n, uint64_t k) {
          qmm::gemv_q4k_rows16_supported(m, n, k) && qmm::gemv_q4k_rows16_workspace_bytes(m, n, k) <= kDecodeScratchBytes;
 }
 
+// `taken`: bytes at the workspace's start that the caller keeps something in, past what the tiles take there.
 qmm_status q4k_matmul(const LaunchCtx& ctx, const float* a, const uint8_t* w, float* c, uint64_t m, uint64_t n,
-                      uint64_t k, uint64_t f16_from) {
+                      uint64_t k, uint64_t f16_from, size_t taken) {
   const hipStream_t s = ctx.stream;
   if (m >= f16_from && qmm::gemm_q4k_supported(m, k)) {
     void* ws = nullptr;
-    const qmm_status st = workspace(ctx, qmm::gemm_q4k_workspace_bytes(m, k), &ws);
-    if (st != QMM_OK) return st;
-    return map_hip(qmm::launch_q4k_gemm(a, w, c, ws, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
+    const PiecesRoom room(ctx, qmm::gemm_q4k_workspace_bytes(m, k), taken, qmm::gemm_f16_parts_bytes(m, n, k, true), &ws);
+    if (room.status() != QMM_OK) return room.status();
+    return map_hip(qmm::launch_q4k_gemm(a, w, c, ws, room.pieces(), static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                         static_cast<uint32_t>(k), s));
   }
   if (m > 16 && (n * k >= kQ4KFewRowsMinWeights || qmm::gemv_q4k_rows16_supported(16, n, k))) {
     // exact, sixteen rows at a time (each chunk takes the regime of its own row count)
     for (uint64_t r = 0; r < m; r += 16) {
-      const qmm_status st = q4k_matmul(ctx, a + r * k, w, c + r * n, m - r < 16 ? m - r : 16, n, k, f16_from);
+      const qmm_status st = q4k_matmul(ctx, a + r * k, w, c + r * n, m - r < 16 ? m - r : 16, n, k, f16_from, taken);
       if (st != QMM_OK) return st;
     }
     return QMM_OK;
@@ -318,8 +346,8 @@ qmm_status q4k_matmul(const LaunchCtx& ctx, const float* a, const uint8_t* w, fl
                                       static_cast<uint32_t>(k), s));
 }
 qmm_status q4k_matmul(const LaunchCtx& ctx, const float* a, const uint8_t* w, float* c, uint64_t m, uint64_t n,
-                      uint64_t k) {
-  return q4k_matmul(ctx, a, w, c, m, n, k, g_q4k_tensor_rows.load(std::memory_order_relaxed));
+                      uint64_t k, size_t taken) {
+  return q4k_matmul(ctx, a, w, c, m, n, k, g_q4k_tensor_rows.load(std::memory_order_relaxed), taken);
 }
 
 // Weights handed over as the load-time row-group copy (`layout` = its rows per group; 0 = GGUF order):
@@ -334,7 +362,7 @@ size_t q4k_regime_workspace(uint64_t m, uint64_t k, uint64_t f16_from) {
 }
 qmm_status q4k_matmul_layout(const LaunchCtx& ctx, const float* a, const uint8_t* w, float* c, uint64_t m, uint64_t n,
                              uint64_t k, uint64_t f16_from, uint64_t layout) {
-  if (layout == 0) return q4k_matmul(ctx, a, w, c, m, n, k, f16_from);
+  if (layout == 0) return q4k_matmul(ctx, a, w, c, m, n, k, f16_from, 0);
   if (m == 1) {
     return map_hip(qmm::launch_q4k_i8_gemv(a, w, c, static_cast<uint32_t>(n), static_cast<uint32_t>(k),
                                            static_cast<uint32_t>(layout), ctx.stream));
@@ -347,7 +375,7 @@ qmm_status q4k_matmul_layout(const LaunchCtx& ctx, const float* a, const uint8_t
   st = map_hip(qmm::launch_q4k_rowgroup(w, gguf, static_cast<uint32_t>(n), static_cast<uint32_t>(k),
                                         static_cast<uint32_t>(layout), true, ctx.stream));
   if (st != QMM_OK) return st;
-  return q4k_matmul(ctx, a, gguf, c, m, n, k, f16_from);
+  return q4k_matmul(ctx, a, gguf, c, m, n, k, f16_from, front + static_cast<size_t>(q4k_bytes(n, k)));
 }
 
 // "gemm_q4k", "gemm_q4k_row", "gemm_q4k_batched", "gemm_q4k_wmma": buffers A, W, C;
@@ -808,8 +836,8 @@ qmm_status run_ffn_gate_up_silu_q4k(const LaunchCtx& c) {
     if (st != QMM_OK) return st;
     u = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + lay.up_off);
   }
-  st = q4k_matmul(c, x, gate, out, m, n, k);
-  if (st == QMM_OK) st = q4k_matmul(c, x, up, u, m, n, k);
+  st = q4k_matmul(c, x, gate, out, m, n, k, lay.workspace_bytes);
+  if (st == QMM_OK) st = q4k_matmul(c, x, up, u, m, n, k, lay.workspace_bytes);
   if (st == QMM_OK) st = map_hip(qmm::launch_silu_mul(out, u, out, m * n, c.stream));
   return st;
 }
@@ -830,10 +858,11 @@ qmm_status run_dequant_q4k(const LaunchCtx& c) {
 qmm_status kquant_prefill(const LaunchCtx& c, uint32_t block_bytes, uint64_t m, uint64_t n, uint64_t k,
                           uint64_t split) {
   void* ws = nullptr;
-  qmm_status st = workspace(c, qmm::gemm_kquant_f16_workspace_bytes(m, n, k), &ws);
+  const PiecesRoom room(c, qmm::gemm_kquant_f16_workspace_bytes(m, n, k), 0, qmm::gemm_f16_parts_bytes(m, n, k, false), &ws);
+  qmm_status st = room.status();
   if (st != QMM_OK) return st;
   float* out = c.ptr<float>(2);
-  st = map_hip(qmm::launch_kquant_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), block_bytes, out, ws,
+  st = map_hip(qmm::launch_kquant_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), block_bytes, out, ws, room.pieces(),
                                            static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                            static_cast<uint32_t>(k), c.stream));
   if (st == QMM_OK && split > 1) st = map_hip(qmm::launch_fill_f32(out + m * n, 0.0f, (split - 1) * m * n, c.stream));
@@ -1545,6 +1574,7 @@ qmm_status qmm_init(int device) {
   // (without them the ids that use them run kernels that need none)
   (void)g_stream_scratch.reserve(StreamBlock::grow);
   (void)g_parts_scratch.reserve(StreamBlock::grow);
+  (void)g_tiles_scratch.reserve(StreamBlock::grow);
   return QMM_OK;
 }
 

@@ -1,0 +1,104 @@
+"""Q4_K from 64 rows and Q5_K, Q6_K from 17 where workgroups share a tile's super-blocks: row and column counts around the
+128 x 128 tiles and the 32 x 32 matrix tiles, super-blocks dealt out in pieces of two and of many, tiles with one owner
+beside shared ones.  Against the float64 product of the two fp16 operands; and the same bits through the entry point
+that allocates nothing, with and without room for the pieces, with a caller's workspace, and recorded."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tessera_amd import KernelLaunch, synth
+from test_gpu_gemm_q4k import ACC_TOL, f16_operands_product
+from util import rms_err, same_bits
+
+pytestmark = pytest.mark.gpu
+
+WEIGHTS = {"q4k": synth.q4k_weights, "q5k": synth.q5k_weights, "q6k": synth.q6k_weights}
+NAMES = {"q4k": "gemm_q4k_wmma", "q5k": "gemm_q5k_batched", "q6k": "gemm_q6k_batched"}
+# rows, columns, K; all shared with 256 CUs (tests/test_launch_rules.py)
+SHARED = [(64, 40, 2048), (65, 127, 2048), (127, 129, 2304), (129, 257, 2048), (257, 384, 3072), (300, 1030, 5120), (100, 33, 17408)]
+# Q5_K's decode rounds a multiply-add once, the oracle a product and a difference: where the two lie on either side of an fp16
+# midpoint a weight differs by a unit in the last place, which moves a result by up to 5 * 2^-11 * 2 rms(w) against an rms of
+# sqrt(k) rms(w): 7e-5 at K = 5120 (1.1e-4 at 2048), and hardly more than one such weight meets a large activation.
+TOL = {"q4k": ACC_TOL, "q5k": ACC_TOL + 2 * 1.1e-4, "q6k": ACC_TOL}
+SHARED_FEW = [(17, 256, 2048), (33, 130, 2304)]
+
+
+def product(a, kind, w, m, n, k):
+    if kind == "q4k":
+        return f16_operands_product(a, w, m, n, k)
+    deq = (oracle.dequantize_q5k if kind == "q5k" else oracle.dequantize_q6k)(w).reshape(n, k)
+    amax = np.max(np.abs(a), axis=1)
+    s = np.exp2(np.floor(np.log2(amax)) - 10.0).astype(np.float32)
+    a16 = (a / s[:, None]).astype(np.float16).astype(np.float64) * s[:, None].astype(np.float64)
+    return a16 @ deq.astype(np.float16).astype(np.float64).T
+
+
+class Product:
+    def __init__(self, backend, kind, m, n, k, seed=1):
+        g = synth.rng(seed + m + n + k)
+        self.backend, self.shape, self.kind = backend, (m, n), kind
+        self.w, self.a = WEIGHTS[kind](g, n, k), g.standard_normal((m, k)).astype(np.float32)
+        self.c = backend.AllocateBuffer(4 * m * n)
+        self.kernel, self.scalars = backend.LoadKernel(NAMES[kind]), [m, n, k]
+        self.launch = KernelLaunch(grid_x=1, buffers=[backend.Upload(self.a), backend.Upload(self.w), self.c], scalars=self.scalars)
+
+    def clear(self):
+        self.backend.CopyH2D(self.c, np.full(self.shape, np.nan, np.float32))
+
+    def bits(self):
+        self.backend.Synchronize()
+        return self.backend.CopyD2H(self.c, dtype=np.float32).reshape(self.shape)
+
+    def result(self, **kw):
+        self.clear()
+        self.backend.LaunchKernel(self.kernel, self.launch, **kw)
+        return self.bits()
+
+
+@pytest.mark.parametrize("kind,m,n,k", [(kind, *s) for kind in WEIGHTS for s in SHARED] + [(kind, *s) for kind in ("q5k", "q6k") for s in SHARED_FEW])
+def test_shared_tiles(backend, kind, m, n, k):
+    p = Product(backend, kind, m, n, k)
+    got = p.result()
+    assert rms_err(got, product(p.a, kind, p.w, m, n, k)) <= TOL[kind]
+    assert same_bits(p.result(), got) and same_bits(p.result(no_alloc=True), got)
+
+
+# (the pieces of the last of each kind do not fit the static array behind the operands)
+@pytest.mark.parametrize("kind,m,n,k", [("q4k", 300, 1030, 5120), ("q4k", 1000, 2040, 5120), ("q6k", 100, 1030, 5120), ("q6k", 300, 1400, 5120)])
+def test_same_bits_wherever_there_is_scratch(backend, kind, m, n, k):
+    p = Product(backend, kind, m, n, k)
+    want = p.result()
+    assert np.all(np.isfinite(want)) and same_bits(p.result(no_alloc=True), want)
+    need = backend.WorkspaceBytes(p.kernel, p.scalars)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    backend.SetWorkspace(backend.WrapBuffer(ws.data_ptr(), need))
+    try:
+        assert same_bits(p.result(), want)
+    finally:
+        backend.SetWorkspace(None)
+
+
+def test_recorded(backend):
+    """Two products recorded together, replayed with eager work of other sizes between the replays."""
+    calls = [Product(backend, "q4k", 300, 1030, 5120), Product(backend, "q6k", 100, 1030, 5120)]
+    other = Product(backend, "q4k", 129, 257, 2048, 9)
+    want, want_other = [p.result() for p in calls], other.result()
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            backend.SetStream(torch.cuda.current_stream().cuda_stream)
+            for p in calls:
+                backend.LaunchKernel(p.kernel, p.launch)
+        backend.SetStream(torch.cuda.current_stream().cuda_stream)
+        for _ in range(3):
+            for p in calls:
+                p.clear()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(same_bits(p.bits(), w) for p, w in zip(calls, want))
+            assert same_bits(other.result(), want_other)
+    finally:
+        backend.SetStream(0)

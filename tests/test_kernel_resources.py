@@ -20,6 +20,7 @@ NO_SCRATCH = {
     "gemv_kquant_rows.hip": ["kquant_rows_kernel", "kquant_rows_stream_kernel"],
     "gemm_fp8.hip": ["fp8_gemm_kernel"],
     "gemm_mxfp4.hip": ["mxfp4_a8_gemm_kernel"],
+    "gemm_q4k.hip": ["q4k_gemm_kernel", "q4k_gate_up_kernel", "f16w_gemm_kernel", "shared_tiles_kernel"],
     "attention.hip": ["attention_rows_kernel", "attention_tile_kernel"],
     "gemv_q4k_i8.hip": ["q4k_i8_gemv_kernel"],
 }

@@ -63,6 +63,47 @@ def test_shared_mxfp4_tiles_cover_every_step_once(tmp_path):
 """)
 
 
+def test_shared_f16_tiles_cover_every_super_block_once(tmp_path):
+    """As above for the K-quants' 128 x 128 tiles: at least two units a workgroup, and the pieces fit a stream's block."""
+    run_program(tmp_path, r"""
+  const uint64_t ms[] = {17, 32, 33, 64, 100, 128, 129, 300, 512, 1000, 2048};
+  const uint64_t ns[] = {1, 64, 65, 128, 129, 1000, 2306, 5120, 6144, 20000};
+  const uint64_t ks[] = {4, 8, 9, 11, 12, 16, 20, 21, 32, 68, 300};
+  int shared = 0;
+  for (uint64_t cus : {60, 256}) for (bool q4k : {false, true}) for (uint64_t m : ms) for (uint64_t n : ns) for (uint64_t k : ks) {
+    const SharedTiles plan = shared_f16_tiles(m, n, k, cus, q4k);
+    if (plan.groups == 0) { CHECK(shared_tiles_bytes(plan) == 0, "not shared"); continue; }
+    ++shared;
+    const uint32_t steps = static_cast<uint32_t>(k);
+    const uint64_t units = uint64_t{plan.tiles} * steps;
+    CHECK(plan.rows == 128 && plan.columns == 128 && plan.tiles == (m + 127) / 128 * ((n + 127) / 128), "%u tiles", plan.tiles);
+    CHECK(units >= uint64_t{2} * plan.groups && plan.groups <= cus, "%u groups", plan.groups);
+    CHECK(shared_tiles_bytes(plan) <= (size_t{40} << 20), "%zu bytes", shared_tiles_bytes(plan));
+    std::vector<bool> taken(shared_tiles_bytes(plan) / 65536, false);
+    CHECK(unit_bound(0, plan.groups, plan.tiles, steps) == 0 && unit_bound(plan.groups, plan.groups, plan.tiles, steps) == units, "ends");
+    for (uint32_t g = 0; g < plan.groups; ++g) {
+      const uint64_t from = unit_bound(g, plan.groups, plan.tiles, steps), to = unit_bound(g + 1, plan.groups, plan.tiles, steps);
+      CHECK(from < to, "group %u", g);
+      for (uint64_t v : {from, (from + to) / 2, to - 1}) CHECK(unit_owner(v, plan, steps) == g, "unit %zu", static_cast<size_t>(v));
+      for (uint64_t t = from / steps; t <= (to - 1) / steps; ++t) {
+        if (t * steps >= from && (t + 1) * steps <= to) continue;      // the whole tile
+        CHECK(g + t < taken.size() && !taken[g + t], "group %u tile %zu", g, static_cast<size_t>(t));
+        taken[g + t] = true;
+      }
+    }
+  }
+  CHECK(shared > 300, "%d", shared);
+""")
+
+
+def test_shared_f16_test_cases_are_shared(tmp_path):
+    import test_gpu_shared_f16_tiles as cases
+    checks = [f"  CHECK(shared_f16_tiles({m}, {n}, {k // 256}, 256, {q}).groups != 0, \"{m} x {n} x {k}\");"
+              for m, n, k in cases.SHARED for q in ("true", "false")]
+    checks += [f"  CHECK(shared_f16_tiles({m}, {n}, {k // 256}, 256, false).groups != 0, \"{m} x {n} x {k}\");" for m, n, k in cases.SHARED_FEW]
+    run_program(tmp_path, "\n".join(checks))
+
+
 def test_mxfp4_test_cases_are_shared(tmp_path):
     import test_gpu_mxfp4_shared_tiles as cases
     checks = "\n".join(f"  CHECK((shared_tiles({m}, {n}, {k // 128}, 256).groups != 0) == {wanted}, \"{m} x {n} x {k}\");"
