@@ -47,7 +47,7 @@ def ffn(backend, x, gate, up, m, n, k):
     return backend.CopyD2H(do, dtype=np.float32).reshape(m, n)
 
 
-# one row: the fused launch for 4096 <= k <= 24576 (even and odd row counts, ragged last group,
+# one row: the fused launch for k <= 24576 (even and odd row counts, ragged last group,
 # a row count below one group), the composed path for the other k
 ONE_ROW = [(512, 4096), (1027, 5120), (3, 5120), (1, 4096), (130, 8192), (67, 17408), (40, 24576),
            (96, 2048), (33, 256), (9, 32768)]
@@ -85,6 +85,23 @@ def test_several_rows_match_oracle(backend, m, n, k):
     run(backend, "gemm_q4k", [dx, dg, og], [m, n, k])
     run(backend, "gemm_q4k", [dx, du, ou], [m, n, k])
     run(backend, "silu_mul", [og, ou, og], [m * n])
+    backend.Synchronize()
+    assert same_bits(got.reshape(-1), backend.CopyD2H(og, dtype=np.float32))
+
+
+# rows of 8, 16 and 32 lanes (whole rows a wavefront; one group and several a wavefront), and of other lengths below 64
+@pytest.mark.parametrize("n,k", [(1, 256), (33, 256), (17, 512), (1023, 512), (3, 1024), (3072, 1024), (20001, 1024), (9, 2048), (512, 2048),
+                                 (9001, 2048), (5, 768), (700, 1280), (129, 2304), (67, 3840)])
+def test_one_short_row_is_the_products_and_silu(backend, n, k):
+    """Below k = 4096 the fused launch makes each product as the single one does: the same bits."""
+    g = synth.rng(740 + n + k)
+    gate, up, x = synth.q4k_weights(g, n, k), synth.q4k_weights(g, n, k), synth.activations_f32(g, 1, k)
+    got = ffn(backend, x, gate, up, 1, n, k)
+    dx, dg, du = backend.Upload(x), backend.Upload(gate), backend.Upload(up)
+    og, ou = backend.AllocateBuffer(4 * n), backend.AllocateBuffer(4 * n)
+    run(backend, "gemm_q4k", [dx, dg, og], [1, n, k])
+    run(backend, "gemm_q4k", [dx, du, ou], [1, n, k])
+    run(backend, "silu_mul", [og, ou, og], [n])
     backend.Synchronize()
     assert same_bits(got.reshape(-1), backend.CopyD2H(og, dtype=np.float32))
 
