@@ -23,9 +23,13 @@
 // converts the codes of its columns once per stage and uses them against both terms of all its rows.  Whatever
 // part of the chip one round of tiles leaves idle is filled by splitting K (fp8_plan); the partial sums are added
 // in part order by a last launch: no atomics, the same bits every time.  What bounds it: at 300 x 6144 x 5120 the
-// matrix cores are busy 37 % of the product's cycles, vector instructions issue in 30 % and a wavefront waits in
-// 23 %, and with one wavefront a SIMD none of these overlap; a short stack of rows is bound by the weight stream.
+// matrix cores are busy 41 % of the product's cycles, vector instructions issue in 21 %, and a wavefront, alone on its SIMD,
+// waits in 24 % (direct loads, barrier) and for issue in 30 %; neither a deeper ring (five stages) nor a tile that reads
+// less LDS changes it.  A short stack of rows is bound by the weight stream.  Half a step's operands are read and
+// converted between the matrix instructions of the half before: 57.2 -> 54.0 us with the rows' conversion.
 // 300 x 6144 x 5120: 1108 -> 56 us against 75 four-row passes of the multiply-add kernel; 17 rows 68 -> 16 us.
+
+#include <type_traits>
 
 #include "q4k_tile.hpp"
 #include "qmm_kernels.hpp"
@@ -176,62 +180,112 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_kernel(const _Float16* __rest
 #pragma unroll
   for (uint32_t h = 0; h < 2; ++h) w_fr[h] = kWBase + (wave_n * WN + l32) * 64u + (((2u * h + kg) ^ ((l32 >> 2) & 3u)) * 16u);
 
+  // The operands of half a step.
+  struct Frag {
+    half8_t b[kTJ][2], hi[kTI][2], lo[kTI][2];
+  };
+  uint4 codes[kTJ];
+  auto read = [&](const uint8_t* stage, int h, Frag& f) {
 #pragma unroll
-  for (int i = 0; i < STAGES - 1; ++i) issue(i, static_cast<uint32_t>(i) < count ? i : count - 1u);
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * kDma) : "memory");
-  uint32_t rd = 0, fill = STAGES - 1;
-  for (uint32_t step = 0; step < count; ++step) {
-    issue(fill, step + (STAGES - 1) < count ? step + (STAGES - 1) : count - 1u);
-    const uint8_t* stage = lds + rd * kStage;
+    for (int j = 0; j < kTJ; ++j) codes[j] = *reinterpret_cast<const uint4*>(stage + w_fr[h] + j * 32 * 64);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      half8_t b[kTJ][2];
+    for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int j = 0; j < kTJ; ++j) {
-        const uint4 q = *reinterpret_cast<const uint4*>(stage + w_fr[h] + j * 32 * 64);
-        const uint32_t words[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const half2_t p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(words[2 * tt + i], 1.0f, false);
-            const half2_t p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(words[2 * tt + i], 1.0f, true);
-            b[j][tt][4 * i] = p0[0], b[j][tt][4 * i + 1] = p0[1], b[j][tt][4 * i + 2] = p1[0], b[j][tt][4 * i + 3] = p1[1];
-          }
+      for (int i = 0; i < kTI; ++i) {
+        const uint8_t* at = stage + a_fr[2 * h + tt] + i * 32 * 128;
+        f.hi[i][tt] = *reinterpret_cast<const half8_t*>(at);
+        f.lo[i][tt] = *reinterpret_cast<const half8_t*>(at + kTermStage);
       }
+  };
+  auto convert = [&](int tt, Frag& f) {
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
+    for (int j = 0; j < kTJ; ++j) {
+      const uint32_t words[2] = {tt == 0 ? codes[j].x : codes[j].z, tt == 0 ? codes[j].y : codes[j].w};
 #pragma unroll
-        for (int i = 0; i < kTI; ++i) {
-          const uint8_t* at = stage + a_fr[2 * h + tt] + i * 32 * 128;
-          const half8_t hi = *reinterpret_cast<const half8_t*>(at);
-          const half8_t lo = *reinterpret_cast<const half8_t*>(at + kTermStage);
-#pragma unroll
-          for (int j = 0; j < kTJ; ++j) {
-            run[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b[j][tt], run[i][j], 0, 0, 0);
-            low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, b[j][tt], low[i][j], 0, 0, 0);
-          }
-        }
+      for (int i = 0; i < 2; ++i) {
+        const half2_t p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(words[i], 1.0f, false);
+        const half2_t p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(words[i], 1.0f, true);
+        f.b[j][tt][4 * i] = p0[0], f.b[j][tt][4 * i + 1] = p0[1], f.b[j][tt][4 * i + 2] = p1[0], f.b[j][tt][4 * i + 3] = p1[1];
+      }
+      asm volatile("" : "+v"(f.b[j][tt]));      // here, not where it is used
     }
-    if (step % kRunSteps == kRunSteps - 1u) {
+  };
+  // Half a step: the matrix instructions of `f`, and the operands `g` of the next half made meanwhile.  With a wavefront a
+  // SIMD nothing hides what waits, so the order is fixed: reads, half of the matrix instructions, and the conversions
+  // between the others; no two in a row into the same sums.  With `first` the second term's instructions go first, and
+  // under them the run that has ended is added.
+  auto half_step = [&](const Frag& f, const uint8_t* stage, int h, Frag& g, auto first) {
+    constexpr bool FIRST = decltype(first)::value;
+    read(stage, h, g);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int tt = FIRST ? q & 1 : q >> 1;
+      const bool second_term = FIRST ? q < 2 : (q & 1) == 0;
+      if (q >= 2) {
+        convert(q - 2, g);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int i = 0; i < kTI; ++i)
 #pragma unroll
-        for (int j = 0; j < kTJ; ++j)
+        for (int j = 0; j < kTJ; ++j) {
+          if (second_term) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.lo[i][tt], f.b[j][tt], low[i][j], 0, 0, 0);
+          else run[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.hi[i][tt], f.b[j][tt], run[i][j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (FIRST && q < 2) {
+            constexpr int kEach = 8;      // of the 16 sums of each matrix tile, twice as many instructions as tiles
 #pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] += run[i][j][e], run[i][j][e] = 0.0f;
-      if (step % kAccSteps == kAccSteps - 1u) {
-#pragma unroll
-        for (int i = 0; i < kTI; ++i)
-#pragma unroll
-          for (int j = 0; j < kTJ; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) total[i][j][e] += acc[i][j][e], acc[i][j][e] = 0.0f;
-      }
+            for (int e = 0; e < kEach; ++e) {
+              const int at = q * kEach + e;
+              acc[i][j][at] += run[i][j][at], run[i][j][at] = 0.0f;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
     }
+  };
+
+#pragma unroll
+  for (int i = 0; i < STAGES; ++i) issue(i, static_cast<uint32_t>(i) < count ? i : count - 1u);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 1) * kDma) : "memory");
+  uint32_t rd = 0, step = 0;
+  Frag f0, f1;
+  read(lds, 0, f0);
+  convert(0, f0);
+  convert(1, f0);
+  // Between a step's halves every wavefront has read all of its stage, which is asked for again, and the next stage has
+  // landed.  (After the last step: operands of a stage that nobody needs.)
+  auto one_step = [&](auto first) {
+    half_step(f0, lds + rd * kStage, 1, f1, first);
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * kDma) : "memory");
-    fill = rd;
+    issue(rd, step + STAGES < count ? step + STAGES : count - 1u);
     rd = rd + 1u == STAGES ? 0u : rd + 1u;
+    half_step(f1, lds + rd * kStage, 0, f0, std::false_type{});
+    return ++step == count;
+  };
+  auto add_acc = [&]() {
+#pragma unroll
+    for (int i = 0; i < kTI; ++i)
+#pragma unroll
+      for (int j = 0; j < kTJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) total[i][j][e] += acc[i][j][e], acc[i][j][e] = 0.0f;
+  };
+  static_assert(kRunSteps == 2, "the loop's steps");
+  for (;;) {
+    if (one_step(std::true_type{})) break;
+    if (step % kAccSteps == 1u && step != 1u) add_acc();
+    if (one_step(std::false_type{})) break;
+  }
+  if (count % kRunSteps == 0u) {      // the last run, as the step after it would have
+#pragma unroll
+    for (int i = 0; i < kTI; ++i)
+#pragma unroll
+      for (int j = 0; j < kTJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] += run[i][j][e], run[i][j][e] = 0.0f;
+    if (count % kAccSteps == 0u) add_acc();
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct load may outlive the workgroup
 
