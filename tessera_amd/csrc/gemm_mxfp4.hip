@@ -68,13 +68,17 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
     float* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t n_begin, uint32_t n_end,
     const uint8_t* __restrict__ need, float* __restrict__ parts, SharedTiles plan) {
   constexpr bool SPLIT = ROWS != Rows::E4M3, SHARED = ROWS == Rows::Shared, CUT = ROWS == Rows::Cut;
+  // KEEP: a step's weights are brought and read with its first term and stay in registers for the others.  100 rows of
+  // 6144 x 5120 52 -> 47 us, 33 rows of 5120 x 5120 40 -> 35, 300 of 6144 x 2048 46 -> 42; but tiles of 256 rows have no
+  // registers left for both halves of a step (453 rows of 5120 x 17408 201 / 214, 1024 of 5120 x 4096 107 / 117).
+  constexpr bool KEEP = SPLIT && BM < 256;
   constexpr int kWaves = WM * WN;
   static_assert(BM % (32 * WM) == 0 && BN % (32 * WN) == 0 && BN % 64 == 0, "tile shape");
   static_assert((BM / 8) % kWaves == 0 && (BN / 16) % kWaves == 0, "direct-load blocks divide among the wavefronts");
   constexpr int kTI = BM / WM / 32, kTJ = BN / WN / 32;      // MFMA tiles per wavefront
   constexpr int kABlk = BM / 8 / kWaves, kBBlk = BN / 16 / kWaves;  // 1 KB direct-load blocks per wavefront
   constexpr int kBLoads = WPERM ? 4 : 1;                     // load instructions per weight block
-  constexpr int kDma = kABlk + kBBlk * kBLoads + 1;          // direct loads a wavefront issues per stage
+  constexpr int kDma = kABlk + kBBlk * kBLoads + 1;          // direct loads a wavefront issues per stage (KEEP: of a first term)
   constexpr uint32_t kBBase = BM * kKS, kSBase = kBBase + BN * kKS / 2;
   constexpr uint32_t kStage = kSBase + BN * 4;
   __shared__ __attribute__((aligned(16))) uint8_t lds[3 * kStage];
@@ -114,14 +118,16 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   };
   auto locate = [&](uint32_t tile, Source& src) {
     const uint32_t m0 = (tile / tiles_n) * BM, n0 = n_begin + (tile % tiles_n) * BN;
+    uint32_t in = lane;
+    asm volatile("" : "+v"(in));         // what follows from it is formed here, not held over the steps
     src.terms = tile_terms(m0);
     src.a = a8 + static_cast<size_t>(m0) * k;
     src.b = w + static_cast<size_t>(n0) * row_bytes;        // also the origin of 16-row tile n0 / 16 in fragment order
     src.s = w + static_cast<size_t>(n) * row_bytes + static_cast<size_t>(n0) * row_blocks;
 #pragma unroll
     for (int i = 0; i < kABlk; ++i) {
-      const uint32_t row = 8u * (wave * kABlk + i) + lane / 8u;
-      const uint32_t chunk = (lane % 8u) ^ ((row >> 1) & 7u);
+      const uint32_t row = 8u * (wave * kABlk + i) + in / 8u;
+      const uint32_t chunk = (in % 8u) ^ ((row >> 1) & 7u);
       src.a_off[i] = (m0 + row < m ? row : m - 1u - m0) * k + chunk * 16u;
     }
 #pragma unroll
@@ -133,17 +139,17 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
         const uint32_t blk_in = n0 + 16u * blk < n ? blk : (n - 1u - n0) / 16u;    // n is a multiple of 16
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const uint32_t d = j * 64u + lane, row = d / 16u, pos = (d % 16u) / 4u;
+          const uint32_t d = j * 64u + in, row = d / 16u, pos = (d % 16u) / 4u;
           const uint32_t wd = 4u * (pos ^ ((row >> 2) & 3u)) + d % 4u;
           src.b_off[i][j] = blk_in * 16u * row_bytes + (wd * 16u + row) * 4u;
         }
       } else {
-        const uint32_t row = 16u * (wave * kBBlk + i) + lane / 4u;
-        const uint32_t chunk = (lane % 4u) ^ ((row >> 2) & 3u);
+        const uint32_t row = 16u * (wave * kBBlk + i) + in / 4u;
+        const uint32_t chunk = (in % 4u) ^ ((row >> 2) & 3u);
         src.b_off[i][0] = (n0 + row < n ? row : n - 1u - n0) * row_bytes + chunk * 16u;
       }
     }
-    const uint32_t row = 64u * (wave % (BN / 64)) + lane;
+    const uint32_t row = 64u * (wave % (BN / 64)) + in;
     src.s_off = (n0 + row < n ? row : n - 1u - n0) * row_blocks;
   };
   auto issue_stage = [&](uint32_t stage_off, const Source& src, uint32_t k0, uint32_t term) {
@@ -153,6 +159,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
     const uint8_t* gs = src.s + k0 / 32;
 #pragma unroll
     for (int i = 0; i < kABlk; ++i) direct_load16(ga, src.a_off[i], stage + (wave * kABlk + i) * 1024u);
+    if (KEEP && term != 0u) return;      // the first term's weights are still in registers
 #pragma unroll
     for (int i = 0; i < kBBlk; ++i) {
       if constexpr (WPERM) {
@@ -171,7 +178,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   // 4*ks + 2 + kg of its row; the 4-bit B operand is k = 32*kg + [0,32), chunk 2*ks + kg.
   struct Frag {
     int8v_t a[kTI];
-    uint4 b[kTJ];
+    int4v_t b[kTJ];
   };
   uint32_t a_fr[2][2], b_fr[2];
   {
@@ -199,7 +206,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
     }
 #pragma unroll
     for (int j = 0; j < kTJ; ++j) {
-      f.b[j] = *reinterpret_cast<const uint4*>(stage + b_fr[ks] + j * 32 * 64);
+      f.b[j] = *reinterpret_cast<const int4v_t*>(stage + b_fr[ks] + j * 32 * 64);
     }
   };
   // Scale words of this lane's weight rows; block 2*ks + kg sits at byte 2*ks once lanes of
@@ -215,8 +222,13 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   // but the youngest stage's; loads complete in issue order, and stores issued in between
   // only make the wait longer), and for its LDS reads of the stage about to be overwritten,
   // before the barrier.
+  bool young_weights = true;      // the youngest stage's loads bring weights
   auto publish = [&]() {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kDma) : "memory");
+    if (!KEEP || young_weights) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kDma) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kABlk) : "memory");
+    }
   };
 
   const uint32_t steps = k / kKS;
@@ -233,18 +245,24 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   // first).  Worth 2-3 % at M = 2048 (0.2036 -> 0.1992 ms at 17408 x 5120); the matrix cores stay busy
   // 52 % of the cycles either way, the wavefronts spending 43 % of theirs in the step's wait for the
   // direct loads and the barrier behind it.
-  auto mfmas_reading = [&](const Frag& f, auto ks_c, int sa, Frag& g, uint32_t g_stage, int g_ks) {
+  // Without `weights` the other fragment's weights stay those it has: a step's terms share them.
+  auto mfmas_reading = [&](const Frag& f, auto ks_c, int sa, Frag& g, uint32_t g_stage, int g_ks, auto weights) {
     constexpr int ks = decltype(ks_c)::value;
-    constexpr int kReads = 2 * kTI + kTJ, kMfmas = kTI * kTJ;
+    constexpr int kReads = 2 * kTI + (decltype(weights)::value ? kTJ : 0), kMfmas = kTI * kTJ;
     const uint8_t* stage = lds + g_stage;
     uint4 lo[kTI], hi[kTI];
+    int4v_t own[kTJ];
+#pragma unroll
+    for (int j = 0; j < kTJ; ++j) {
+      own[j] = f.b[j];
+      if constexpr (KEEP) asm volatile("" : "+v"(own[j]));      // widened at each use: held over the terms, the empty half would be too
+    }
     const int a_scale = SPLIT ? sa : 0x7F7F7F7F;
 #pragma unroll
     for (int q = 0; q < (kReads > kMfmas ? kReads : kMfmas); ++q) {
       if (q < kMfmas) {
         const int j = q / kTI, i = q % kTI;
-        const int8v_t bf = int8v_t{static_cast<int>(f.b[j].x), static_cast<int>(f.b[j].y),
-                                   static_cast<int>(f.b[j].z), static_cast<int>(f.b[j].w), 0, 0, 0, 0};
+        const int8v_t bf = __builtin_shufflevector(own[j], int4v_t{0, 0, 0, 0}, 0, 1, 2, 3, 4, 5, 6, 7);
         // A: E4M3 (cbsz 0) with unit scale (E8M0 127), or the term's weight; B: E2M1 (blgp 4)
         // with the block scale.
         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.a[i], bf, acc[i][j], 0, 4, 0, a_scale, ks == 0 ? 0 : 2,
@@ -258,7 +276,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
           else lo[i] = v;
         } else {
           const int j = q - 2 * kTI;
-          g.b[j] = *reinterpret_cast<const uint4*>(stage + b_fr[g_ks] + j * 32 * 64);
+          g.b[j] = *reinterpret_cast<const int4v_t*>(stage + b_fr[g_ks] + j * 32 * 64);
         }
       }
     }
@@ -314,10 +332,11 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   advance_load();
   issue_stage(kStage, src, load_step * kKS, load_term);
   advance_load();
+  young_weights = load_term == 0u;
   issue_stage(2 * kStage, src, load_step * kKS, load_term);
   advance_load();
-  // the first stage has landed when only the two younger ones may be outstanding
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * kDma) : "memory");
+  // the first stage has landed when only the two younger ones may be outstanding (KEEP: at least their rows)
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(KEEP ? 2 * kABlk : 2 * kDma) : "memory");
   read_scales(rd, sv_raw);
   read_frags(rd, 0, f0);
 #pragma unroll
@@ -333,11 +352,14 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
   // second slice in between.  Then every wavefront has read all of `rd` and `nx` has landed
   // (publish), so `rd` is asked for again with the step three ahead.  Second half: the second
   // slice, with the reads of the NEXT step's first slice (and its scale words) in between.
-  auto one_step = [&](uint32_t term) {
+  // KEEP: a step's weights are read with its `first` term, the first half of the next step's with the `last`.
+  auto one_step = [&](uint32_t term, auto first, auto last) {
     const int sa = 0x7F - 4 * static_cast<int>(term);      // E8M0 of 2^(-4 term), byte 0 is the one used
+    if constexpr (decltype(first)::value) {
 #pragma unroll
-    for (int j = 0; j < kTJ; ++j) sv[j] = static_cast<int>(sv_raw[j] >> (kg * 8u));
-    mfmas_reading(f0, std::integral_constant<int, 0>{}, sa, f1, rd, 1);
+      for (int j = 0; j < kTJ; ++j) sv[j] = static_cast<int>(sv_raw[j] >> (kg * 8u));
+    }
+    mfmas_reading(f0, std::integral_constant<int, 0>{}, sa, f1, rd, 1, first);
     if constexpr (SPLIT && kWaves == 8) {
       // keeps these matrix instructions on this side of the barrier: below it they would hold up the reads
 #pragma unroll
@@ -346,14 +368,32 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
         for (int j = 0; j < kTJ; ++j) asm volatile("" : "+v"(acc[i][j]));
     }
     publish();
+    young_weights = load_term == 0u;
     issue_stage(rd, src, load_step * kKS, load_term);
     advance_load();
-    mfmas_reading(f1, std::integral_constant<int, 1>{}, sa, f0, nx, 0);
-    read_scales(nx, sv_raw);
+    mfmas_reading(f1, std::integral_constant<int, 1>{}, sa, f0, nx, 0, last);
+    if constexpr (decltype(last)::value) read_scales(nx, sv_raw);
     const uint32_t done = rd;
     rd = nx;
     nx = ld;
     ld = done;
+  };
+  // Steps step .. end - 1 of a tile in `terms` terms each.
+  auto walk = [&](uint32_t end, uint32_t terms) {
+    constexpr std::true_type yes;
+    constexpr std::false_type no;
+    if constexpr (KEEP) {
+      if (terms > 1u) {
+        for (; step < end; ++step) {
+          one_step(0u, yes, no);
+          for (uint32_t term = 1u; term + 1u < terms; ++term) one_step(term, no, no);
+          one_step(terms - 1u, no, yes);
+        }
+      }
+    }
+    for (; step < end; ++step) {
+      for (uint32_t term = 0; term < (KEEP ? 1u : terms); ++term) one_step(term, yes, yes);
+    }
   };
 
   for (;;) {
@@ -367,9 +407,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
         const uint64_t cut = unit_bound(++owner, plan.groups, plan.tiles, steps) - first;
         const uint32_t end = cut < steps ? static_cast<uint32_t>(cut) : steps;
         const bool one_piece = step == 0u && end == steps;
-        for (; step < end; ++step) {
-          for (uint32_t term = 0; term < terms; ++term) one_step(term);
-        }
+        walk(end, terms);
         if (one_piece) break;
 #pragma unroll
         for (int i = 0; i < kTI; ++i)
@@ -382,9 +420,7 @@ __global__ __launch_bounds__(64 * WM * WN) void mxfp4_a8_gemm_kernel(
             }
       }
     } else {
-      for (; step < stop; ++step) {
-        for (uint32_t term = 0; term < terms; ++term) one_step(term);
-      }
+      walk(stop, terms);
     }
 
     // Epilogue: lane holds column l32 and rows (e/4)*8 + kg*4 + e%4 of each 32 x 32 tile.
