@@ -280,10 +280,21 @@ __device__ __forceinline__ void attend_row(const AttentionArgs& a, uint64_t row,
   const uint32_t column_head = F32 ? r : r / 2u;
   const bool second = !F32 && (r & 1u) != 0u;                      // this lane's column is a second term
   const float term_down = second ? 0x1p-11f : 1.0f;
-  // Two terms of x, this lane's: hi, or 2^11 (x - hi).
-  auto term_of = [&](float x) {
-    const _Float16 hi = static_cast<_Float16>(x);
-    return second ? static_cast<_Float16>((x - static_cast<float>(hi)) * 0x1p11f) : hi;
+  // Of the two terms of x and of y this lane's: hi, or 2^11 (x - hi).  (x and y are kept apart from their conversions, which
+  // make two numbers at once: a multiply-add that rounds to fp16 takes the vector unit twice a conversion's time.  Not where
+  // the registers are just enough, KEYS = 16.)
+  auto terms_of = [&](float x, float y) {
+    constexpr bool APART = F32 || KEYS == 32;
+    if constexpr (APART) asm("" : "+v"(x), "+v"(y));
+    const half2_t hi = {static_cast<_Float16>(x), static_cast<_Float16>(y)};
+    if constexpr (!APART) {
+      return half2_t{second ? static_cast<_Float16>((x - static_cast<float>(hi[0])) * 0x1p11f) : hi[0],
+                     second ? static_cast<_Float16>((y - static_cast<float>(hi[1])) * 0x1p11f) : hi[1]};
+    }
+    float low_x = (x - static_cast<float>(hi[0])) * 0x1p11f, low_y = (y - static_cast<float>(hi[1])) * 0x1p11f;
+    asm("" : "+v"(low_x), "+v"(low_y));
+    const half2_t lo = {static_cast<_Float16>(low_x), static_cast<_Float16>(low_y)};
+    return bit_cast<half2_t>(second ? bit_cast<uint32_t>(lo) : bit_cast<uint32_t>(hi));
   };
   const float* qp = a.q + ((a.row_base + row) * a.heads + head0 + (column_head < here ? column_head : here - 1u)) * D;
   float qf[F32 ? STEPS : 1];
@@ -316,8 +327,9 @@ __device__ __forceinline__ void attend_row(const AttentionArgs& a, uint64_t row,
 #pragma unroll
     for (int i = 0; i < STEPS; ++i) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        qh[i][e] = term_of(raw[i][kq_dim<KV>(e)] * up);
+      for (int e = 0; e < 8; e += 2) {
+        const half2_t pair = terms_of(raw[i][kq_dim<KV>(e)] * up, raw[i][kq_dim<KV>(e + 1)] * up);
+        qh[i][e] = pair[0], qh[i][e + 1] = pair[1];
       }
     }
   }
@@ -463,7 +475,10 @@ __device__ __forceinline__ void attend_row(const AttentionArgs& a, uint64_t row,
     } else {
       half8_t p;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) p[e] = e < 4 * HALVES ? term_of(s[e % (4 * HALVES)]) : static_cast<_Float16>(0.0f);
+      for (int e = 0; e < 8; e += 2) {
+        const half2_t pair = e < 4 * HALVES ? terms_of(s[e % (4 * HALVES)], s[(e + 1) % (4 * HALVES)]) : half2_t{};
+        p[e] = pair[0], p[e + 1] = pair[1];
+      }
 #pragma unroll
       for (int j = 0; j < VE; ++j) {
         uint4 w = {value_pair<KV>(vr[0], vr[1], j), value_pair<KV>(vr[2], vr[3], j), 0u, 0u};
@@ -1165,17 +1180,23 @@ hipError_t launch_rows(const AttentionArgs& a, uint64_t m, hipStream_t stream) {
   const uint64_t split = a.part.split == 0 ? 1 : a.part.split;
   const uint64_t workgroups = m * a.kv_heads * blocks * split;
   const dim3 grid(static_cast<uint32_t>(workgroups));
-  // Four wavefronts a workgroup take 128 keys at once; where a workgroup has more to do and the
-  // registers and the size of a grid allow it, eight.
+  // Four wavefronts a workgroup take 128 keys at once; where a workgroup has more to do and the registers and the size of a
+  // grid allow it, eight; with no more workgroups than CUs, five take the 129 to 160 keys that parts of 128 come to where they
+  // do not divide the keys, and spare the second time round (us, four / five: int8, 1200 keys in 9 parts, 4 key heads of 128 8.6 /
+  // 7.9, 9301 in 64, 4 of 64 6.7 / 6.2; but two workgroups a CU, 9301 keys, 8 of 128 12.4 / 15.6).
+  const uint64_t each = (a.n + split - 1) / split;
   const bool wide = a.n / split > 160 && workgroups < kMaxGridThreads / 512u;
+  const bool five = each > 128 && each <= 160 && workgroups <= static_cast<uint64_t>(num_cus());
   auto go = [&](auto kernel, uint32_t waves) { hipLaunchKernelGGL(kernel, grid, dim3(waves * 64u), 0, stream, a); };
-  if (a.head_dim <= 64) {
-    wide ? go(attention_rows_kernel<KV, 64, 8>, 8) : go(attention_rows_kernel<KV, 64, 4>, 4);
-  } else if (a.head_dim <= 128) {
-    wide ? go(attention_rows_kernel<KV, 128, 8>, 8) : go(attention_rows_kernel<KV, 128, 4>, 4);
-  } else {
-    go(attention_rows_kernel<KV, 256, 4>, 4);
-  }
+  auto pick = [&](auto dim) {
+    constexpr int DP = decltype(dim)::value;
+    if (DP < 256 && five) go(attention_rows_kernel<KV, DP, DP < 256 ? 5 : 4>, 5);
+    else if (DP < 256 && wide) go(attention_rows_kernel<KV, DP, DP < 256 ? 8 : 4>, 8);
+    else go(attention_rows_kernel<KV, DP, 4>, 4);
+  };
+  if (a.head_dim <= 64) pick(std::integral_constant<int, 64>{});
+  else if (a.head_dim <= 128) pick(std::integral_constant<int, 128>{});
+  else pick(std::integral_constant<int, 256>{});
   return hipGetLastError();
 }
 
