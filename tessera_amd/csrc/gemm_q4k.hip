@@ -42,12 +42,10 @@ namespace {
 // NV > 0: the row is held in registers between its maximum and its conversion (cols <= 2048 NV) and read once: 2048 rows
 // of 17408 63 -> 46 us; 0: read twice.
 template <int NV>
-__global__ __launch_bounds__(256) void rows_to_f16_kernel(const float* __restrict__ src, _Float16* __restrict__ dst,
-                                                          float* __restrict__ scale, uint32_t cols,
-                                                          const uint32_t* __restrict__ pos, uint32_t top_k) {
+__device__ __forceinline__ void row_to_f16(const float* __restrict__ src, _Float16* __restrict__ dst, float* __restrict__ scale,
+                                           uint32_t cols, uint32_t drow, uint32_t srow) {
   __shared__ float red[4];
-  const uint32_t p = blockIdx.x, groups = cols / 8u;
-  const uint32_t drow = pos != nullptr ? pos[p] : p, srow = pos != nullptr ? p / top_k : p;
+  const uint32_t groups = cols / 8u;
   const float4* in = reinterpret_cast<const float4*>(src + static_cast<size_t>(srow) * cols);
   float amax = 0.0f;
   auto scan = [&](const float4& v) {
@@ -78,6 +76,21 @@ __global__ __launch_bounds__(256) void rows_to_f16_kernel(const float* __restric
     for (uint32_t g = threadIdx.x; g < groups; g += 256u) out[g] = to_f16_group(in[2 * g], in[2 * g + 1], inv);
   }
   if (threadIdx.x == 0) scale[drow] = s;
+}
+template <int NV>
+__global__ __launch_bounds__(256) void rows_to_f16_kernel(const float* __restrict__ src, _Float16* __restrict__ dst,
+                                                          float* __restrict__ scale, uint32_t cols,
+                                                          const uint32_t* __restrict__ pos, uint32_t top_k) {
+  const uint32_t p = blockIdx.x;
+  row_to_f16<NV>(src, dst, scale, cols, pos != nullptr ? pos[p] : p, pos != nullptr ? p / top_k : p);
+}
+// How much of a row of `cols` a thread holds.
+template <class F>
+void with_row_registers(uint32_t cols, F&& f) {
+  if (cols <= 2048u) f(std::integral_constant<int, 1>{});
+  else if (cols <= 6144u) f(std::integral_constant<int, 3>{});
+  else if (cols <= 18432u) f(std::integral_constant<int, 9>{});
+  else f(std::integral_constant<int, 0>{});
 }
 
 
@@ -120,11 +133,9 @@ void launch_pair_range(const _Float16* a16, const float* a_scale, const uint8_t*
 
 void launch_rows_to_f16(const float* src, _Float16* dst, float* scale, uint32_t rows, uint32_t cols, const uint32_t* pos,
                         uint32_t top_k, hipStream_t stream) {
-  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, stream, src, dst, scale, cols, pos, top_k); };
-  if (cols <= 2048u) go(rows_to_f16_kernel<1>);
-  else if (cols <= 6144u) go(rows_to_f16_kernel<3>);
-  else if (cols <= 18432u) go(rows_to_f16_kernel<9>);
-  else go(rows_to_f16_kernel<0>);
+  with_row_registers(cols, [&](auto nv) {
+    hipLaunchKernelGGL(rows_to_f16_kernel<decltype(nv)::value>, dim3(rows), dim3(256), 0, stream, src, dst, scale, cols, pos, top_k);
+  });
 }
 
 bool gemm_q4k_supported(uint64_t m, uint64_t k) { return k % 256 == 0 && k <= (1u << 20) && m * k < (1ull << 31); }
@@ -173,9 +184,7 @@ __device__ __forceinline__ uint64_t load8_a2(const uint8_t* p) {   // eight byte
 
 // One thread per (block, half n, eight lanes l = 8o..8o+7): 32 values, four 16-byte stores
 // (src/core/numerics/quant.cpp:421-450).
-__global__ __launch_bounds__(256) void q6k_to_f16_kernel(const uint8_t* __restrict__ w, _Float16* __restrict__ out,
-                                                         uint64_t nitems) {
-  const uint64_t t = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void q6k_to_f16(const uint8_t* __restrict__ w, _Float16* __restrict__ out, uint64_t nitems, uint64_t t) {
   if (t >= nitems) return;
   const uint64_t blk = t >> 3;
   const uint32_t n = static_cast<uint32_t>(t >> 2) & 1u, o = static_cast<uint32_t>(t) & 3u, is = o >> 1;
@@ -200,9 +209,7 @@ __global__ __launch_bounds__(256) void q6k_to_f16_kernel(const uint8_t* __restri
 
 // One thread per (block, group g, eight lanes): 16 values, two 16-byte stores
 // (src/core/numerics/quant.cpp:388-419).
-__global__ __launch_bounds__(256) void q5k_to_f16_kernel(const uint8_t* __restrict__ w, _Float16* __restrict__ out,
-                                                         uint64_t nitems) {
-  const uint64_t t = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void q5k_to_f16(const uint8_t* __restrict__ w, _Float16* __restrict__ out, uint64_t nitems, uint64_t t) {
   if (t >= nitems) return;
   const uint64_t blk = t >> 4;
   const uint32_t g = static_cast<uint32_t>(t >> 2) & 3u, o = static_cast<uint32_t>(t) & 3u;
@@ -235,6 +242,22 @@ __global__ __launch_bounds__(256) void q5k_to_f16_kernel(const uint8_t* __restri
   }
   store_perm8(out + blk * 256 + g * 64 + o * 8, v0);
   store_perm8(out + blk * 256 + g * 64 + 32 + o * 8, v1);
+}
+
+// Both operands in one launch: workgroups below `rows` convert a row of A each, the others the weights.  Two launches one
+// after the other cost a start and an end more: the product as a whole Q6_K 512 x 1024 x 5120 30.0 -> 27.8 us,
+// 100 x 5120 x 5120 41.1 -> 38.4, 64 x 5120 x 17408 100 -> 93, Q5_K 200 x 2048 x 3072 31.9 -> 28.3.
+template <int BITS, int NV>
+__global__ __launch_bounds__(256) void operands_to_f16_kernel(const float* __restrict__ a, _Float16* __restrict__ a16,
+                                                              float* __restrict__ a_scale, uint32_t rows, uint32_t cols,
+                                                              const uint8_t* __restrict__ w, _Float16* __restrict__ w16, uint64_t nitems) {
+  if (blockIdx.x < rows) {        // workgroup-uniform
+    row_to_f16<NV>(a, a16, a_scale, cols, blockIdx.x, blockIdx.x);
+    return;
+  }
+  const uint64_t t = static_cast<uint64_t>(blockIdx.x - rows) * 256u + threadIdx.x;
+  if constexpr (BITS == 6) q6k_to_f16(w, w16, nitems, t);
+  else q5k_to_f16(w, w16, nitems, t);
 }
 
 // C tile = A16 (rows scaled by a_scale) . W16^T, both operands fp16 row-major with row length k.
@@ -555,16 +578,24 @@ hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t blo
   float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
   _Float16* w16 = reinterpret_cast<_Float16*>(a_scale + m + 256);
   const uint64_t blocks = static_cast<uint64_t>(n) * (k / 256);
-  if (block_bytes == 210) {
-    hipLaunchKernelGGL(q6k_to_f16_kernel, dim3(static_cast<uint32_t>((blocks * 8 + 255) / 256)), dim3(256), 0, stream,
-                       w, w16, blocks * 8);
-  } else if (block_bytes == 176) {
-    hipLaunchKernelGGL(q5k_to_f16_kernel, dim3(static_cast<uint32_t>((blocks * 16 + 255) / 256)), dim3(256), 0, stream,
-                       w, w16, blocks * 16);
-  } else {
-    return hipErrorInvalidValue;
-  }
-  launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
+  if (block_bytes != 210 && block_bytes != 176) return hipErrorInvalidValue;
+  const uint64_t items = blocks * (block_bytes == 210 ? 8 : 16), weight_groups = (items + 255) / 256;
+  with_row_registers(k, [&](auto nv) {
+    constexpr int NV = decltype(nv)::value;
+    auto go = [&](uint32_t rows, uint64_t groups) {
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups)), dim3(256), 0, stream, a, a16, a_scale, rows, k, w, w16, items);
+      };
+      if (block_bytes == 210) launch(operands_to_f16_kernel<6, NV>);
+      else launch(operands_to_f16_kernel<5, NV>);
+    };
+    if (m + weight_groups < kMaxGridThreads / 256u) {
+      go(m, m + weight_groups);
+    } else {                      // more than a launch can have
+      go(m, m);
+      go(0u, weight_groups);
+    }
+  });
   const SharedTiles plan = shared_f16_tiles(m, n, k / 256u, static_cast<uint64_t>(num_cus()), false);
   if (plan.groups != 0u && (pieces.at != nullptr || pieces.cut)) {
     return launch_shared<F16Weights>(a16, a_scale, w16, c, pieces.at, m, n, k, plan, stream);
