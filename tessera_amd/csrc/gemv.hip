@@ -1912,8 +1912,8 @@ hipError_t launch_q4k_gemv_split(const float* a, const uint8_t* w, float* c, uin
   return launch_gemv_r<Q4KSliceCodec, 1, 768, 2, 12>(args, c, n, slice, n, stream, split);
 }
 
-// silu(G x) * (U x) for one activation row, one launch: a row of 64 to 384 chunks of 64 weights
-// (two slot rows of it must fit a 768-thread workgroup and a wavefront may span two rows at most).
+// silu(G x) * (U x) for one activation row, one launch: a row of at most 384 chunks of 64 weights (two slot rows of it must
+// fit a 768-thread workgroup).  Rows below 64 chunks take the kernels that gemm_q4k takes for them, and have its bits.
 bool ffn_gate_up_q4k_supported(uint64_t k) { return k % 256 == 0 && k >= 256 && k <= 24576; }
 
 hipError_t launch_ffn_gate_up_q4k(const float* x, const uint8_t* gate, const uint8_t* up, float* out,
