@@ -1048,24 +1048,11 @@ uint32_t stream_rows_per_workgroup(uint32_t n) {
 // rowmax * 2^-(12+4T) at the least); what lies below is dropped.  `need` = terms the row's
 // widest significand asks for: 2 for bf16-valued rows, 3 up to 12 bits, else 4 (16 bits kept).
 // A non-finite element becomes the E4M3 NaN, which spoils its row of C.
-__device__ __forceinline__ uint32_t e4m3_cut(float x, float& val) {        // |x| < 256
-  const uint32_t b = bit_cast<uint32_t>(x), sign = (b >> 24) & 0x80u;
-  if (fabsf(x) >= 0x1p-6f) {
-    const uint32_t tb = b & 0xFFF00000u;                                  // sign, exponent, three mantissa bits
-    val = bit_cast<float>(tb);
-    return sign | ((((tb >> 23) & 0xFFu) - 120u) << 3) | ((tb >> 20) & 7u);
-  }
-  const uint32_t q = static_cast<uint32_t>(fabsf(x) * 512.0f);           // the subnormal grid, 2^-9
-  val = copysignf(static_cast<float>(q) * 0x1p-9f, x);
-  return sign | q;
-}
-__device__ __forceinline__ uint32_t e4m3_near(float x) {                  // |x| < 256, to nearest
-  const uint32_t b = bit_cast<uint32_t>(x), sign = (b >> 24) & 0x80u, mag = b & 0x7FFFFFFFu;
-  if (fabsf(x) >= 0x1p-6f) {
-    const uint32_t r = mag + 0x7FFFFu + ((mag >> 20) & 1u);               // carry may reach the exponent (256 = 0x78)
-    return sign | ((r >> 20) - (120u << 3));
-  }
-  return sign | static_cast<uint32_t>(rintf(fabsf(x) * 512.0f));         // 8 = 2^-6, the first normal code
+// |x| < 256 cut to an E4M3 number; below the first normal one, 2^-6, to the grid of 2^-9.  (A cut value's code is then the
+// hardware's conversion, which is exact on it and to nearest, ties to even, for the last term.)
+__device__ __forceinline__ float e4m3_cut(float x) {
+  const float normal = bit_cast<float>(bit_cast<uint32_t>(x) & 0xFFF00000u);   // sign, exponent, three mantissa bits
+  return fabsf(x) >= 0x1p-6f ? normal : truncf(x * 512.0f) * 0x1p-9f;
 }
 
 // NV > 0: a thread keeps its NV 16-byte pieces of the row in registers between the two passes (the
@@ -1079,7 +1066,8 @@ __global__ __launch_bounds__(1024) void split_rows_kernel(const float* __restric
   const uint32_t row = blockIdx.x, t = threadIdx.x, stride = blockDim.x * 4u, waves = blockDim.x >> 6;
   const float* ar = a + static_cast<size_t>(row) * k;
   float amax = 0.0f;
-  uint32_t low = 0;
+  constexpr uint32_t kNotFinite = 0x80000000u;
+  uint32_t low = 0;                        // the mantissas' bits, and whether an element is not finite
   uint4 held[NV > 0 ? NV : 1];
   auto scan = [&](const uint4 v) {
     const uint32_t b[4] = {v.x, v.y, v.z, v.w};
@@ -1088,7 +1076,9 @@ __global__ __launch_bounds__(1024) void split_rows_kernel(const float* __restric
       const uint32_t mag = b[e] & 0x7FFFFFFFu;
       if (mag < 0x7F800000u) {
         amax = fmaxf(amax, bit_cast<float>(mag));
-        if (mag != 0) low |= mag & 0x7FFFFFu;
+        low |= mag & 0x7FFFFFu;
+      } else {
+        low |= kNotFinite;
       }
     }
   };
@@ -1118,6 +1108,7 @@ __global__ __launch_bounds__(1024) void split_rows_kernel(const float* __restric
   e = amax == 0.0f ? 7 : (e < -112 ? -112 : e);
   const float s0 = bit_cast<float>(static_cast<uint32_t>(e - 7 + 127) << 23);
   const float inv = bit_cast<float>(static_cast<uint32_t>(7 - e + 127) << 23);
+  const bool special = __builtin_amdgcn_readfirstlane(low & kNotFinite) != 0u;
   if (t == 0) {
     as[row] = s0;
     const uint32_t bits = 24u - static_cast<uint32_t>(__builtin_ctz(low | 0x800000u));
@@ -1127,22 +1118,29 @@ __global__ __launch_bounds__(1024) void split_rows_kernel(const float* __restric
   uint8_t* out = planes + static_cast<size_t>(row) * k;
   auto emit = [&](const uint4 v, uint32_t i) {
     const uint32_t b[4] = {v.x, v.y, v.z, v.w};
-    uint32_t code[kMaxTerms] = {0, 0, 0, 0};
+    float r[4];
+    uint32_t nan = 0;
 #pragma unroll
-    for (int el = 0; el < 4; ++el) {
-      if ((b[el] & 0x7FFFFFFFu) >= 0x7F800000u) {
-        code[0] |= 0x7Fu << (8 * el);
-        continue;
-      }
-      float r = bit_cast<float>(b[el]) * inv;
+    for (int el = 0; el < 4; ++el) r[el] = bit_cast<float>(b[el]) * inv;
+    if (special) {
 #pragma unroll
-      for (int term = 0; term < kMaxTerms - 1; ++term) {
-        float val;
-        code[term] |= e4m3_cut(r, val) << (8 * el);
-        r = (r - val) * 16.0f;
+      for (int el = 0; el < 4; ++el) {
+        if ((b[el] & 0x7FFFFFFFu) >= 0x7F800000u) r[el] = 0.0f, nan |= 0x7Fu << (8 * el);
       }
-      code[kMaxTerms - 1] |= e4m3_near(r) << (8 * el);
     }
+    uint32_t code[kMaxTerms];
+#pragma unroll
+    for (int term = 0; term < kMaxTerms; ++term) {
+      float val[4];
+#pragma unroll
+      for (int el = 0; el < 4; ++el) {
+        val[el] = term < kMaxTerms - 1 ? e4m3_cut(r[el]) : r[el];
+        r[el] = (r[el] - val[el]) * 16.0f;
+      }
+      const int pair = __builtin_amdgcn_cvt_pk_fp8_f32(val[0], val[1], 0, false);
+      code[term] = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(val[2], val[3], pair, true));
+    }
+    code[0] |= nan;
 #pragma unroll
     for (int term = 0; term < kMaxTerms; ++term) *reinterpret_cast<uint32_t*>(out + term * plane + i) = code[term];
   };
@@ -1157,12 +1155,16 @@ __global__ __launch_bounds__(1024) void split_rows_kernel(const float* __restric
   }
 }
 
-// A few rows: 1024 threads a row and the row kept in registers, so that the launch is one trip to
-// memory and back (the split of 4 rows of 5120: 8.6 -> 4.7 us); many rows: 256 threads a row, several rows a CU.
+// The row kept in registers, so that the launch is one trip to memory and back.  A few rows: 1024 threads a row, several
+// wavefronts a SIMD (the split of 4 rows of 5120: 8.6 -> 4.7 us).  Many: four or fewer pieces a thread where 1024 threads hold
+// the row so, and no more threads than that takes.  us with 256 threads that read the row twice / as it is here: 453 rows of
+// 17408 21.4 / 18.6, 256 of 16384 19.8 / 13.0, 65 of 17408 14.8 / 9.5, 453 of 5120 9.9 / 9.3, 2048 of 17408 75 / 64; 256 threads
+// up to K = 8192 and 512 up to 16384 were 0 to 1.0 us slower.  Cutting by mask and truncation with the hardware's conversion, in
+// place of codes put together bit by bit under a branch, gave as much again: with those 30.7 (453 of 17408), 12.6 (of 5120).
 void launch_split_rows(const float* a, uint8_t* planes, float* as, uint8_t* need, uint32_t m, uint32_t k,
                        hipStream_t stream) {
-  if (m <= 64u && k <= 4096u * 8u) {
-    const uint32_t threads = k >= 4096u ? 1024u : 256u;
+  if (k <= 4096u * 8u) {
+    const uint32_t threads = m <= 64u ? (k >= 4096u ? 1024u : 256u) : k <= 4096u ? 256u : k <= 8192u ? 512u : 1024u;
     const uint32_t nv = (k + threads * 4u - 1u) / (threads * 4u);
     if (nv <= 1u) hipLaunchKernelGGL(split_rows_kernel<1>, dim3(m), dim3(threads), 0, stream, a, planes, as, need, m, k);
     else if (nv == 2u) hipLaunchKernelGGL(split_rows_kernel<2>, dim3(m), dim3(threads), 0, stream, a, planes, as, need, m, k);
