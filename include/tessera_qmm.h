@@ -196,7 +196,9 @@ size_t qmm_static_scratch_bytes(void);
  * qmm_workspace_bytes returns what a launch of `kernel` with these scalars needs (0 for
  * decode-sized launches and ids without scratch; for the grouped routed-expert ids an upper bound
  * over the expert count; for "gemm_mxfp4" from 17 rows with what it only makes use of: it runs, slower and
- * with the same bits, in the 4 m k + 2 * 256 * ceil(m / 64) bytes of the rows' terms).  qmm_set_workspace hands the library a device block of that size
+ * with the same bits, in the 4 m k + 2 * 256 * ceil(m / 64) bytes of the rows' terms; a Q4_K, Q5_K or Q6_K product
+ * with few tiles makes use of 64 KB more for each 128 x 128 tile and 16 MB, and runs slower, with the same bits,
+ * without).  qmm_set_workspace hands the library a device block of that size
  * (256-byte aligned) to use for every later qmm_launch on any stream, in stream order, until it
  * is replaced or cleared with (NULL, 0); while one is set, qmm_launch allocates nothing and a
  * launch that needs more returns InvalidArgument.  The caller must not free or replace the

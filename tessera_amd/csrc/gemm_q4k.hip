@@ -524,16 +524,14 @@ hipError_t launch_shared(const _Float16* a16, const float* a_scale, const typena
 // The bulk of C goes to 256 x 256 tiles, whole rounds of one tile per CU; columns left over
 // when the tile count is not a multiple of the CU count are cut into 128 x 64 tiles that
 // spread over every CU instead of keeping a few CUs busy for a whole extra round.
-hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* workspace, const SharedPieces& pieces, uint32_t m,
+hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* workspace, float* parts, uint32_t m,
                            uint32_t n, uint32_t k, hipStream_t stream) {
   _Float16* a16 = static_cast<_Float16*>(workspace);
   float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
   launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
   const uint32_t cus = static_cast<uint32_t>(num_cus());
   const SharedTiles plan = shared_f16_tiles(m, n, k / 256u, cus, true);
-  if (plan.groups != 0u && (pieces.at != nullptr || pieces.cut)) {
-    return launch_shared<Q4KWeights>(a16, a_scale, w, c, pieces.at, m, n, k, plan, stream);
-  }
+  if (plan.groups != 0u) return launch_shared<Q4KWeights>(a16, a_scale, w, c, parts, m, n, k, plan, stream);
   const uint32_t tiles_m = (m + 255u) / 256u, tiles_n = (n + 255u) / 256u;
   const uint32_t tiles = tiles_m * tiles_n;
   uint32_t main_tn = tiles_n;
@@ -573,7 +571,7 @@ size_t gemm_kquant_f16_workspace_bytes(uint64_t m, uint64_t n, uint64_t k) {
 
 // block_bytes selects the format: 176 = Q5_K, 210 = Q6_K.
 hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t block_bytes, float* c, void* workspace,
-                                  const SharedPieces& pieces, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream) {
+                                  float* parts, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream) {
   _Float16* a16 = static_cast<_Float16*>(workspace);
   float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
   _Float16* w16 = reinterpret_cast<_Float16*>(a_scale + m + 256);
@@ -597,9 +595,7 @@ hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t blo
     }
   });
   const SharedTiles plan = shared_f16_tiles(m, n, k / 256u, static_cast<uint64_t>(num_cus()), false);
-  if (plan.groups != 0u && (pieces.at != nullptr || pieces.cut)) {
-    return launch_shared<F16Weights>(a16, a_scale, w16, c, pieces.at, m, n, k, plan, stream);
-  }
+  if (plan.groups != 0u) return launch_shared<F16Weights>(a16, a_scale, w16, c, parts, m, n, k, plan, stream);
   const F16wTiles tiles = f16w_tiles(m, n, k, static_cast<uint32_t>(num_cus()));
   const uint32_t n_split = tiles.large * tiles.columns < n ? tiles.large * tiles.columns : n;
   if (n_split > 0) {

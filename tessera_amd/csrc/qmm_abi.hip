@@ -235,30 +235,16 @@ class StreamBlock {
 };
 static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock && qmm::kAttentionPartsMost <= kPartsLimits.small);
 
-// The workspace of a product whose tiles workgroups may share (`operands` bytes) and room for the tiles' pieces: a stream's
-// block, apart from the other families' for their sake; for qmm_launch_static what the static array has behind the
-// operands and behind `taken`.  Without room the tiles stay whole; without room in the static array their sums are cut and
-// added as the pieces are, so that the bits are qmm_launch's.
-constexpr qmm::ScratchLimits kTilesLimits{size_t{16} << 20, size_t{40} << 20, size_t{512} << 10, size_t{128} << 20, size_t{128} << 20, size_t{1} << 30};
-qmm::StreamScratch g_tiles_scratch(kTilesLimits);
-
-class PiecesRoom {
- public:
-  PiecesRoom(const LaunchCtx& c, size_t operands, size_t taken, size_t pieces, void** ws)
-      : at_(round256(operands > taken ? operands : taken)), more_(c.no_alloc && pieces != 0 ? at_ - operands + pieces : 0),
-        status_(workspace(c, operands, ws, &more_)), block_(c, c.no_alloc || status_ != QMM_OK ? 0 : pieces, g_tiles_scratch) {
-    if (c.no_alloc) pieces_ = {more_ == 0 ? nullptr : reinterpret_cast<float*>(static_cast<uint8_t*>(*ws) + at_), true};
-    else pieces_ = {static_cast<float*>(block_.get()), false};
-  }
-  qmm_status status() const { return status_; }
-  qmm::SharedPieces pieces() const { return pieces_; }
-
- private:
-  size_t at_, more_;
-  qmm_status status_;
-  StreamBlock block_;
-  qmm::SharedPieces pieces_{};
-};
+// The workspace of a product whose tiles workgroups may share: its `operands` bytes, and behind them and behind `taken` room
+// for the tiles' pieces, which the caller orders as it does the operands.  Without room (the array or the caller's block is too
+// small, or the library's cannot grow) *parts is null: the sums are then cut and added as the pieces are, the same bits.
+qmm_status product_workspace(const LaunchCtx& c, size_t operands, size_t taken, size_t pieces, void** ws, float** parts) {
+  const size_t at = round256(operands > taken ? operands : taken);
+  size_t more = pieces == 0 ? 0 : at - operands + pieces;
+  const qmm_status st = workspace(c, operands, ws, &more);
+  *parts = st != QMM_OK || more == 0 ? nullptr : reinterpret_cast<float*>(static_cast<uint8_t*>(*ws) + at);
+  return st;
+}
 
 // Q4_K regimes by activation rows.  One row and small matrices: the VALU GEMV.  2..16 rows of a
 // matrix with at least kQ4KFewRowsMinWeights weights: the exact few-row MFMA kernels (weights read
@@ -289,9 +275,10 @@ qmm_status q4k_matmul(const LaunchCtx& ctx, const float* a, const uint8_t* w, fl
   const hipStream_t s = ctx.stream;
   if (m >= f16_from && qmm::gemm_q4k_supported(m, k)) {
     void* ws = nullptr;
-    const PiecesRoom room(ctx, qmm::gemm_q4k_workspace_bytes(m, k), taken, qmm::gemm_f16_parts_bytes(m, n, k, true), &ws);
-    if (room.status() != QMM_OK) return room.status();
-    return map_hip(qmm::launch_q4k_gemm(a, w, c, ws, room.pieces(), static_cast<uint32_t>(m), static_cast<uint32_t>(n),
+    float* parts = nullptr;
+    const qmm_status st = product_workspace(ctx, qmm::gemm_q4k_workspace_bytes(m, k), taken, qmm::gemm_f16_parts_bytes(m, n, k, true), &ws, &parts);
+    if (st != QMM_OK) return st;
+    return map_hip(qmm::launch_q4k_gemm(a, w, c, ws, parts, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                         static_cast<uint32_t>(k), s));
   }
   if (m > 16 && (n * k >= kQ4KFewRowsMinWeights || qmm::gemv_q4k_rows16_supported(16, n, k))) {
@@ -858,11 +845,11 @@ qmm_status run_dequant_q4k(const LaunchCtx& c) {
 qmm_status kquant_prefill(const LaunchCtx& c, uint32_t block_bytes, uint64_t m, uint64_t n, uint64_t k,
                           uint64_t split) {
   void* ws = nullptr;
-  const PiecesRoom room(c, qmm::gemm_kquant_f16_workspace_bytes(m, n, k), 0, qmm::gemm_f16_parts_bytes(m, n, k, false), &ws);
-  qmm_status st = room.status();
+  float* parts = nullptr;
+  qmm_status st = product_workspace(c, qmm::gemm_kquant_f16_workspace_bytes(m, n, k), 0, qmm::gemm_f16_parts_bytes(m, n, k, false), &ws, &parts);
   if (st != QMM_OK) return st;
   float* out = c.ptr<float>(2);
-  st = map_hip(qmm::launch_kquant_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), block_bytes, out, ws, room.pieces(),
+  st = map_hip(qmm::launch_kquant_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), block_bytes, out, ws, parts,
                                            static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                            static_cast<uint32_t>(k), c.stream));
   if (st == QMM_OK && split > 1) st = map_hip(qmm::launch_fill_f32(out + m * n, 0.0f, (split - 1) * m * n, c.stream));
@@ -1574,7 +1561,6 @@ qmm_status qmm_init(int device) {
   // (without them the ids that use them run kernels that need none)
   (void)g_stream_scratch.reserve(StreamBlock::grow);
   (void)g_parts_scratch.reserve(StreamBlock::grow);
-  (void)g_tiles_scratch.reserve(StreamBlock::grow);
   return QMM_OK;
 }
 

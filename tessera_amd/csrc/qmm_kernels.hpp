@@ -126,14 +126,10 @@ size_t gemm_q4k_workspace_bytes(uint64_t m, uint64_t k);
 // silu(A gate^T) * (A up^T) for more than 64 rows, with gemm_q4k_workspace_bytes(m, k) of workspace.
 hipError_t launch_q4k_gate_up(const float* a, const uint8_t* gate, const uint8_t* up, float* c, void* workspace, uint32_t m,
                               uint32_t n, uint32_t k, hipStream_t stream);
-// Room for the pieces of tiles that workgroups share; without it the tiles are whole, or with `cut` whole with the shared
-// ones' bits.  And the bytes it takes (q4k, or Q5_K and Q6_K).
-struct SharedPieces {
-  float* at = nullptr;
-  bool cut = false;
-};
+// `parts`: room for the pieces of tiles that workgroups share, gemm_f16_parts_bytes of it (q4k, or Q5_K and Q6_K); null: such
+// tiles are whole, with the same bits.
 size_t gemm_f16_parts_bytes(uint64_t m, uint64_t n, uint64_t k, bool q4k);
-hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* workspace, const SharedPieces& pieces, uint32_t m,
+hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* workspace, float* parts, uint32_t m,
                            uint32_t n, uint32_t k, hipStream_t stream);
 
 // Q5_K (block_bytes 176) and Q6_K (210) prefill: weights decoded once to fp16 in the workspace,
@@ -141,7 +137,7 @@ hipError_t launch_q4k_gemm(const float* a, const uint8_t* w, float* c, void* wor
 bool gemm_kquant_f16_supported(uint64_t m, uint64_t n, uint64_t k);
 size_t gemm_kquant_f16_workspace_bytes(uint64_t m, uint64_t n, uint64_t k);
 hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t block_bytes, float* c, void* workspace,
-                                  const SharedPieces& pieces, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream);
+                                  float* parts, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream);
 
 // Routed experts for a chunk of tokens, grouped by expert (moe_q4k.hip): out[t] (+)= sum over
 // the token's top_k experts of wts * down_e(silu(gate_e x) * up_e x), as grouped MFMA GEMMs.

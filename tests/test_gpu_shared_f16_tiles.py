@@ -1,7 +1,7 @@
 """Q4_K from 64 rows and Q5_K, Q6_K from 17 where workgroups share a tile's super-blocks: row and column counts around the
 128 x 128 tiles and the 32 x 32 matrix tiles, super-blocks dealt out in pieces of two and of many, tiles with one owner
-beside shared ones.  Against the float64 product of the two fp16 operands; and the same bits through the entry point
-that allocates nothing, with and without room for the pieces, with a caller's workspace, and recorded."""
+beside shared ones.  Against the float64 product of the two fp16 operands; and the same bits wherever the pieces lie or find
+no room: through the entry point that allocates nothing, with a caller's workspace, on each thread's own stream, and recorded."""
 import numpy as np
 import pytest
 import torch
@@ -9,7 +9,7 @@ import torch
 import oracle
 from tessera_amd import KernelLaunch, synth
 from test_gpu_gemm_q4k import ACC_TOL, f16_operands_product
-from util import rms_err, same_bits
+from util import rms_err, run, same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -71,12 +71,57 @@ def test_same_bits_wherever_there_is_scratch(backend, kind, m, n, k):
     want = p.result()
     assert np.all(np.isfinite(want)) and same_bits(p.result(no_alloc=True), want)
     need = backend.WorkspaceBytes(p.kernel, p.scalars)
-    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
-    backend.SetWorkspace(backend.WrapBuffer(ws.data_ptr(), need))
+    room = need + (64 << 20)                                # more than any plan's pieces
+    ws = torch.empty(room, dtype=torch.uint8, device="cuda")
     try:
-        assert same_bits(p.result(), want)
+        for size in (need, need + (1 << 20), room):         # no room for the pieces, too little, enough
+            backend.SetWorkspace(backend.WrapBuffer(ws.data_ptr(), size))
+            assert same_bits(p.result(), want), size
     finally:
         backend.SetWorkspace(None)
+
+
+@pytest.mark.parametrize("kind,m,n,k", [("q4k", 300, 1030, 5120), ("q5k", 100, 1030, 5120), ("q6k", 100, 1030, 5120)])
+def test_same_bits_on_each_threads_own_stream(backend, kind, m, n, k):
+    p = Product(backend, kind, m, n, k)
+    want = p.result()
+    try:
+        backend.SetStream(2)                                # hipStreamPerThread
+        assert same_bits(p.result(), want)
+    finally:
+        backend.SetStream(0)
+
+
+def test_feed_forward_keeps_its_products_apart(backend):
+    """64 rows: gate and up as two products in one workspace, the pieces behind the up product's result."""
+    m, n, k = 64, 1030, 5120
+    g = synth.rng(31)
+    gate, up, x = synth.q4k_weights(g, n, k), synth.q4k_weights(g, n, k), g.standard_normal((m, k)).astype(np.float32)
+    bufs = [backend.Upload(x), backend.Upload(gate), backend.Upload(up), backend.AllocateBuffer(4 * m * n)]
+    kernel = backend.LoadKernel("ffn_gate_up_silu_q4k")
+    launch = KernelLaunch(grid_x=1, buffers=bufs, scalars=[m, n, k])
+
+    def result(**kw):
+        backend.CopyH2D(bufs[3], np.full((m, n), np.nan, np.float32))
+        backend.LaunchKernel(kernel, launch, **kw)
+        backend.Synchronize()
+        return backend.CopyD2H(bufs[3], dtype=np.float32).reshape(m, n)
+    products = [backend.AllocateBuffer(4 * m * n) for _ in range(2)]
+    for weights, out in zip(bufs[1:3], products):
+        run(backend, "gemm_q4k_wmma", [bufs[0], weights, out], [m, n, k])
+    run(backend, "silu_mul", [*products, bufs[3]], [m * n])
+    backend.Synchronize()
+    want = backend.CopyD2H(bufs[3], dtype=np.float32).reshape(m, n)
+    assert np.all(np.isfinite(want)) and same_bits(result(), want)
+    need = backend.WorkspaceBytes(kernel, [m, n, k])
+    ws = torch.empty(need + (64 << 20), dtype=torch.uint8, device="cuda")
+    try:
+        for size in (need, need + (64 << 20)):
+            backend.SetWorkspace(backend.WrapBuffer(ws.data_ptr(), size))
+            assert same_bits(result(), want), size
+    finally:
+        backend.SetWorkspace(None)
+    assert same_bits(result(no_alloc=True), want)
 
 
 def test_recorded(backend):
