@@ -47,23 +47,40 @@ constexpr SharedTiles shared_tiles(uint64_t m, uint64_t n, uint64_t steps, uint6
   return {static_cast<uint32_t>(rows), static_cast<uint32_t>(tiles), static_cast<uint32_t>(room < most ? room : most)};
 }
 
-// ---- Q4_K from 64 rows, Q5_K and Q6_K from 17: tiles whose super-blocks workgroups share --------------------------------
+// ---- Q4_K, Q5_K and Q6_K on the tensor tile: tiles whose super-blocks workgroups share -----------------------------------
 // Tiles of 128 x 128 whose (tile, super-block) units go to one workgroup a CU, at least two units each.  Whole tiles of
 // 128 x 64 leave most CUs idle while a few walk all of K: 512 rows of 1024 x 5120 are 64 of them.  The pieces cost a launch
-// and twice their bytes, so that with few super-blocks, or tiles that fill the chip, whole ones lead; `small` counts those.
-// Sides measured (us, whole / shared).  Q4_K, rows x n x k: 100 x 512 x 2048 (8 small) 19.6 / 14.5, 100 x 6144 x 2048 (96) 21.2 /
-// 22.9; 512 x 2048 x 3072 (128) 31 / 25, 200 x 6144 x 3072 (192) 29 / 32; 512 x 1024 x 5120 (64) 44 / 26, 512 x 6144 x 5120 (384)
-// 69 / 56, 2048 x 6144 x 5120 (1536) 183 / 220; 256 x 5120 x 17408 (160) 126 / 84, 1024 (640) 316 / 267, 2048 (1280) 452 / 492.
+// and twice their bytes, so that with few super-blocks, or tiles that fill the chip, whole ones lead; `small` counts those, and
+// the limits are sixteenths of the CUs.
+// Q4_K, sides measured (us, whole / shared; rows x n x k, in brackets the small tiles).  `even`: every workgroup has as many
+// units; otherwise some take two tiles' pieces, which counts where a tile has few.  100 x 4096 x 2048 (64) 20.9 / 19.5, x 2304 22.6 /
+// 23.6, x 2816 25.7 / 25.3; 100 x 5696 x 3072 (89) 27.4 / 27.6, x 6912 (108) 27.5 / 29.2, x 8192 (128, even) 27.4 / 26.3; 128 x 13888 x
+// 4352 (217) 37 / 40, 256 x 8192 x 4096 (256, even) 38 / 36; 512 x 1024 x 5120 (64) 44 / 26, 512 x 6144 x 5120 (384) 64 / 59, 2048 x
+// 6144 x 5120 (1536) 183 / 220; 256 x 5120 x 17408 (160) 126 / 84, 1024 (640) 316 / 267, 2048 (1280) 452 / 492.  Four row tiles and
+// more whose small tiles fill two a CU: 500 x 7168 x 6144 (448) 76 / 82, but 256 x 14336 (448) 76 / 72, 500 x 8704 (544) 115 / 87.
+// Up to 64 rows whole tiles are of 32 columns and 32 or 64 rows, with no padding, and start to take longer with more than a round of
+// them: 17 rows of 2048 x 2048 (32) 14.6 / 15.1, 5120 x 3072 (80) 18.9 / 17.9, 6144 x 3072 (96) 18.9 / 20.7, 8192 x 5120 (128) 27.8 / 23.7,
+// 10240 x 5120 (160) 29 / 30, 17408 x 5120 (272) 29.5 / 40, 12288 x 8192 (192) 43 / 41, 5120 x 17408 (80) 82 / 40; 64 rows of 4096 x
+// 2048 (64) 18.7 / 16.8, 6144 x 3072 (96) 24.7 / 23.3, 7168 x 3072 (112) 24.8 / 25.5, 12288 x 4096 (192) 32 / 30.5, 14336 x 4096 (224) 32.4 /
+// 32.7, 16384 x 5120 (256) 38 / 36, 20480 x 5120 (320) 39 / 46.
+constexpr uint64_t shared_q4k_limit(uint64_t m, uint64_t steps, bool even) {
+  if (m <= 32) return steps < 10 ? 0 : steps < 12 ? 2 : steps < 16 ? 4 : steps < 18 ? 6 : steps < 24 ? 8 : steps < 32 ? 10 : steps < 48 ? 12 : 14;
+  if (steps < 12) return steps == 9 ? 3 : 4;
+  if (m <= 64) return steps < 16 ? 6 : steps < 20 ? 12 : 16;
+  if (steps < 16) return steps == 12 && !even ? 5 : 8;
+  return steps < 18 && !even ? 12 : steps < 20 ? 16 : 40;
+}
 // Q5_K and Q6_K, whose whole tiles need no decode and go up to 256 x 256: 100 x 512 x 2048 (8) 22 / 19, 24 x 6144 x 2048 (96) 28 /
-// 33; 200 x 2048 x 3072 (64) 33 / 28, 24 x 4096 x 3072 (64) 32 / 33, 384 x 4096 x 3072 (192) 36 / 38; 512 x 1024 x 5120 (64) 46 / 29,
+// 33; 200 x 2048 x 3072 (64) 33 / 28, 24 x 4096 x 3072 (64) 32 / 33, 384 x 4096 x 3072 (192) 36 / 38; 512 x 1024 x 5120 (64) 46 / 28,
 // 512 x 6144 x 5120 (384) 80 / 79, 200 x 6144 x 5120 (192) 57 / 59; 512 x 3072 x 8192 (192) 66 / 75.
+constexpr uint64_t shared_kquant_limit(uint64_t m, uint64_t steps) {
+  return (steps < 12 ? 2 : steps < 16 ? 4 : steps < 20 ? 6 : 8) / (m <= 32 && steps < 20 ? 2 : 1);
+}
 constexpr SharedTiles shared_f16_tiles(uint64_t m, uint64_t n, uint64_t steps, uint64_t cus, bool q4k) {
   if (m > 256 * cus || n > 256 * cus || steps < 8) return {};
   const uint64_t tiles = (m + 127) / 128 * ((n + 127) / 128), small = (m + 127) / 128 * ((n + 63) / 64);
-  uint64_t most = 0;       // small tiles, eighths of the CUs
-  if (q4k) most = steps < 12 ? 2 : steps < 16 ? 4 : steps < 20 ? 8 : 20;
-  else most = (steps < 12 ? 2 : steps < 16 ? 4 : steps < 20 ? 6 : 8) / (m <= 32 && steps < 20 ? 2 : 1);
-  if (small * (q4k ? 8 : 16) > cus * most) return {};
+  if (small * 16 > cus * (q4k ? shared_q4k_limit(m, steps, tiles * steps % cus == 0) : shared_kquant_limit(m, steps))) return {};
+  if (q4k && m > 384 && steps < 48 && small * 2 > cus * 3 && small <= 2 * cus) return {};
   const uint64_t units = tiles * steps / 2;
   return {128, static_cast<uint32_t>(tiles), static_cast<uint32_t>(cus < units ? cus : units), 128};
 }

@@ -1,4 +1,4 @@
-"""Q4_K from 64 rows and Q5_K, Q6_K from 17 where workgroups share a tile's super-blocks: row and column counts around the
+"""Q4_K, Q5_K and Q6_K products on the tensor tile where workgroups share a tile's super-blocks: row and column counts around the
 128 x 128 tiles and the 32 x 32 matrix tiles, super-blocks dealt out in pieces of two and of many, tiles with one owner
 beside shared ones.  Against the float64 product of the two fp16 operands; and the same bits wherever the pieces lie or find
 no room: through the entry point that allocates nothing, with a caller's workspace, on each thread's own stream, and recorded."""
@@ -21,7 +21,8 @@ SHARED = [(64, 40, 2048), (65, 127, 2048), (127, 129, 2304), (129, 257, 2048), (
 # midpoint a weight differs by a unit in the last place, which moves a result by up to 5 * 2^-11 * 2 rms(w) against an rms of
 # sqrt(k) rms(w): 7e-5 at K = 5120 (1.1e-4 at 2048), and hardly more than one such weight meets a large activation.
 TOL = {"q4k": ACC_TOL, "q5k": ACC_TOL + 2 * 1.1e-4, "q6k": ACC_TOL}
-SHARED_FEW = [(17, 256, 2048), (33, 130, 2304)]
+SHARED_FEW = {"q4k": [(17, 256, 2560), (32, 130, 5120), (33, 130, 2304), (63, 700, 5120)], "q5k": [(17, 256, 2048), (33, 130, 2304)],
+              "q6k": [(17, 256, 2048), (33, 130, 2304)]}
 
 
 def product(a, kind, w, m, n, k):
@@ -56,7 +57,7 @@ class Product:
         return self.bits()
 
 
-@pytest.mark.parametrize("kind,m,n,k", [(kind, *s) for kind in WEIGHTS for s in SHARED] + [(kind, *s) for kind in ("q5k", "q6k") for s in SHARED_FEW])
+@pytest.mark.parametrize("kind,m,n,k", [(kind, *s) for kind in WEIGHTS for s in SHARED] + [(kind, *s) for kind in WEIGHTS for s in SHARED_FEW[kind]])
 def test_shared_tiles(backend, kind, m, n, k):
     p = Product(backend, kind, m, n, k)
     got = p.result()
