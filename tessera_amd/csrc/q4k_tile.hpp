@@ -126,6 +126,26 @@ __device__ __forceinline__ half8_t decode_step(const uint32_t (&qw)[4], int tt, 
   return decode_eight<HI>(qw[2 * tt], qw[2 * tt + 1], sm);
 }
 
+// Both steps of sub-block SB; an odd one decodes the bytes its even predecessor loaded, so `qw` (the words) and `qs8` (the
+// same shifted down one byte, for bytes 1 and 3) are carried from that call.
+template <int SB>
+__device__ __forceinline__ void decode_subblock(const uint8_t* raw, uint32_t kg, const BlockHead& h, uint32_t (&qw)[4],
+                                                uint32_t (&qs8)[4], half8_t (&b)[2]) {
+  constexpr int kHi = SB & 1;
+  const ScaleMin sm = scale_min_f32<SB>(h.sbytes, h.d, h.ndmin);
+  if (kHi == 0) {
+    load_nibbles<SB>(raw, kg, qw);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) qs8[x] = qw[x] >> 8;
+  }
+#pragma unroll
+  for (int tt = 0; tt < 2; ++tt) {
+    const half2_t p0 = decode_pair<kHi>(qw[2 * tt], sm.dsc, sm.ndmm), p1 = decode_pair<kHi>(qs8[2 * tt], sm.dsc, sm.ndmm);
+    const half2_t p2 = decode_pair<kHi>(qw[2 * tt + 1], sm.dsc, sm.ndmm), p3 = decode_pair<kHi>(qs8[2 * tt + 1], sm.dsc, sm.ndmm);
+    b[tt] = half8_t{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+  }
+}
+
 // Wavefronts of a BM x BN tile whose wavefronts each own WM rows x WN columns.
 template <int BM, int BN, int WM, int WN>
 constexpr int tile_waves() { return (BM / WM) * (BN / WN); }
@@ -226,10 +246,16 @@ __device__ __forceinline__ void q4k_tile_sums(TileSums<WM / KSETS, WN>& out, con
 
   const uint32_t slices = blocks * 8u;
 
-  // One half of a slice's matrix instructions (one step of the slice) go with the making of the next half's operands:
+  // AHEAD: one half of a slice's matrix instructions (one step of the slice) go with the making of the next half's operands:
   // activation fragments read from LDS, weights decoded.  A wavefront issues in order, so what lies between two matrix
   // instructions runs under the first of them.  2048 rows of 2 x 17408 x 5120 with silu 775 -> 765 us, the matrix cores
-  // being held down by power.
+  // being held down by power.  Otherwise a slice's operands are made in the slice: where a half has few matrix instructions to
+  // put the making between and a CU holds several workgroups, they hide what waits, the start and the end are shorter, and
+  // the compiler keeps most of the decode's multiply-adds in fp32 and converts two numbers at once, which takes less of the
+  // vector unit than multiply-adds that round to fp16.  Ahead it took longer by: 17 rows of 17408 x 1536 3 %, 100 rows of 17408 x
+  // 1280 7, gate and up of 128 rows of 8192 x 4096 4 (53.6 / 51.5 us), 256 rows with two of 16 experts of 2048 x 4096 7 (171 / 160);
+  // but 33 to 64 rows, one wavefront of two matrix tiles, 2 % less.
+  constexpr bool AHEAD = KSETS == 2 || kTI * kTJ >= 8 || (kWaves == 1 && kTI == 2);
   half8_t a0[kTI], a1[kTI], b0[kTJ], b1[kTJ];
   BlockHead head[kTJ];
   ScaleMin sm[kTJ];
@@ -264,6 +290,52 @@ __device__ __forceinline__ void q4k_tile_sums(TileSums<WM / KSETS, WN>& out, con
       __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
     });
   };
+
+  if constexpr (!AHEAD) {
+    // Prologue: first super-block and three activation slices in flight, then the first of each is waited for.
+    issue_w(0, 0);
+    issue_a(0, 0);
+    issue_a(1, 1);
+    issue_a(2, 2);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kABlk) : "memory");
+    for (uint32_t blk = 0; blk < blocks; ++blk) {
+      const uint8_t* raw = lds + 4 * kAStage + (blk & 1u) * kWStage + w_row;
+      const bool more = blk + 1 < blocks;        // uniform
+      BlockHead head[kTJ];
+      uint32_t qw[kTJ][4], qs8[kTJ][4];
+#pragma unroll
+      for (int j = 0; j < kTJ; ++j) head[j] = load_block_head(raw + j * kJRows * 144);
+      unrolled<8>([&](auto step) {
+        constexpr int sb = decltype(step)::value;
+        const uint32_t slice = blk * 8u + sb;
+        if (sb == 0 && more) issue_w((blk + 1u) & 1u, blk + 1u);
+        issue_a((slice + 3u) & 3u, slice + 3u < slices ? slice + 3u : slices - 1u);
+        half8_t b[kTJ][2];
+#pragma unroll
+        for (int j = 0; j < kTJ; ++j) decode_subblock<sb>(raw + j * kJRows * 144, kg, head[j], qw[j], qs8[j], b[j]);
+        const uint8_t* a_stage = lds + (slice & 3u) * kAStage;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+#pragma unroll
+          for (int i = 0; i < kTI; ++i) {
+            const half8_t af = *reinterpret_cast<const half8_t*>(a_stage + a_fr[tt] + i * 32 * 64);
+#pragma unroll
+            for (int j = 0; j < kTJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, b[j][tt], acc[i][j], 0, 0, 0);
+          }
+        }
+        // Publish slice + 1: every direct load older than the two youngest activation slices (and, in the two steps after a
+        // weight refill was issued, older than that refill) has landed; this wavefront's LDS reads of the stage about to be
+        // refilled are done.
+        if (sb <= 1 && more) {
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kABlk + kWL) : "memory");
+        } else {
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kABlk) : "memory");
+        }
+      });
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct load may outlive the workgroup
+    return;
+  }
 
   // Prologue: two super-blocks and four activation slices in flight, then the first of each is waited for.
   issue_w(0, 0);
