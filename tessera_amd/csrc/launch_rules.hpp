@@ -53,7 +53,8 @@ constexpr SharedTiles shared_tiles(uint64_t m, uint64_t n, uint64_t steps, uint6
 // and twice their bytes, so that with few super-blocks, or tiles that fill the chip, whole ones lead; `small` counts those, and
 // the limits are sixteenths of the CUs.
 // Q4_K, sides measured (us, whole / shared; rows x n x k, in brackets the small tiles).  `even`: every workgroup has as many
-// units; otherwise some take two tiles' pieces, which counts where a tile has few.  100 x 4096 x 2048 (64) 20.9 / 19.5, x 2304 22.6 /
+// units; otherwise some take two tiles' pieces, which counts where a tile has few; with several row tiles sharing leads
+// all the same (500 x 1728 x 3072 (108) 30.6 / 28.9, 1000 x 1728 x 4096 (216) 40.8 / 39.1).  100 x 4096 x 2048 (64) 20.9 / 19.5, x 2304 22.6 /
 // 23.6, x 2816 25.7 / 25.3; 100 x 5696 x 3072 (89) 27.4 / 27.6, x 6912 (108) 27.5 / 29.2, x 8192 (128, even) 27.4 / 26.3; 128 x 13888 x
 // 4352 (217) 37 / 40, 256 x 8192 x 4096 (256, even) 38 / 36; 512 x 1024 x 5120 (64) 44 / 26, 512 x 6144 x 5120 (384) 64 / 59, 2048 x
 // 6144 x 5120 (1536) 183 / 220; 256 x 5120 x 17408 (160) 126 / 84, 1024 (640) 316 / 267, 2048 (1280) 452 / 492.  Four row tiles and
@@ -67,8 +68,8 @@ constexpr uint64_t shared_q4k_limit(uint64_t m, uint64_t steps, bool even) {
   if (m <= 32) return steps < 10 ? 0 : steps < 12 ? 2 : steps < 16 ? 4 : steps < 18 ? 6 : steps < 24 ? 8 : steps < 32 ? 10 : steps < 48 ? 12 : 14;
   if (steps < 12) return steps == 9 ? 3 : 4;
   if (m <= 64) return steps < 16 ? 6 : steps < 20 ? 12 : 16;
-  if (steps < 16) return steps == 12 && !even ? 5 : 8;
-  return steps < 18 && !even ? 12 : steps < 20 ? 16 : 40;
+  if (steps < 16) return steps == 12 && m <= 256 && !even ? 5 : 8;
+  return steps < 18 && m <= 384 && !even ? 12 : steps < 20 ? 16 : 40;
 }
 // Q5_K and Q6_K, whose whole tiles need no decode and go up to 256 x 256: 100 x 512 x 2048 (8) 22 / 19, 24 x 6144 x 2048 (96) 28 /
 // 33; 200 x 2048 x 3072 (64) 33 / 28, 24 x 4096 x 3072 (64) 32 / 33, 384 x 4096 x 3072 (192) 36 / 38; 512 x 1024 x 5120 (64) 46 / 28,

@@ -113,7 +113,7 @@ def test_q4k_tiles_stay_whole_where_sharing_takes_longer(tmp_path):
     {17, 17408, 5120, false}, {32, 24576, 5120, false}, {17, 8192, 5120, true}, {17, 5120, 17408, true}, {32, 20480, 17408, false},
     {33, 4096, 2048, true}, {64, 7168, 3072, false}, {64, 14336, 4096, false}, {33, 40960, 5120, false}, {64, 17408, 5120, false},
     {64, 8192, 5120, true}, {64, 1024, 17408, true}, {100, 4096, 2304, false}, {100, 4096, 2048, true}, {100, 6912, 3072, false},
-    {100, 8192, 3072, true}, {128, 13888, 4352, false}, {500, 7168, 6144, false}, {1000, 3584, 5120, false}, {500, 8704, 6144, true},
+    {100, 8192, 3072, true}, {128, 13888, 4352, false}, {500, 1728, 3072, true}, {1000, 1728, 4096, true}, {500, 7168, 6144, false}, {1000, 3584, 5120, false}, {500, 8704, 6144, true},
     {512, 6144, 5120, true}, {512, 5120, 6144, true}, {512, 1024, 5120, true}, {256, 14336, 6144, true}};
   for (const auto& r : rows) CHECK((shared_f16_tiles(r.m, r.n, r.k / 256, 256, true).groups != 0) == r.shared, "%zu x %zu x %zu", size_t(r.m), size_t(r.n), size_t(r.k));
 """)
