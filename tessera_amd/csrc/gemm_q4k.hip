@@ -244,20 +244,41 @@ __device__ __forceinline__ void q5k_to_f16(const uint8_t* __restrict__ w, _Float
   store_perm8(out + blk * 256 + g * 64 + 32 + o * 8, v1);
 }
 
-// Both operands in one launch: workgroups below `rows` convert a row of A each, the others the weights.  Two launches one
+// Both operands in one launch: `rows` workgroups from `row0` on convert a row of A each, the others the weights.  Two launches one
 // after the other cost a start and an end more: the product as a whole Q6_K 512 x 1024 x 5120 30.0 -> 27.8 us,
 // 100 x 5120 x 5120 41.1 -> 38.4, 64 x 5120 x 17408 100 -> 93, Q5_K 200 x 2048 x 3072 31.9 -> 28.3.
 template <int BITS, int NV>
 __global__ __launch_bounds__(256) void operands_to_f16_kernel(const float* __restrict__ a, _Float16* __restrict__ a16,
-                                                              float* __restrict__ a_scale, uint32_t rows, uint32_t cols,
+                                                              float* __restrict__ a_scale, uint32_t rows, uint32_t row0, uint32_t cols,
                                                               const uint8_t* __restrict__ w, _Float16* __restrict__ w16, uint64_t nitems) {
-  if (blockIdx.x < rows) {        // workgroup-uniform
-    row_to_f16<NV>(a, a16, a_scale, cols, blockIdx.x, blockIdx.x);
+  const uint32_t row = blockIdx.x - row0;
+  if (row < rows) {        // workgroup-uniform
+    row_to_f16<NV>(a, a16, a_scale, cols, row, row);
     return;
   }
-  const uint64_t t = static_cast<uint64_t>(blockIdx.x - rows) * 256u + threadIdx.x;
+  const uint64_t t = static_cast<uint64_t>(blockIdx.x < row0 ? blockIdx.x : blockIdx.x - rows) * 256u + threadIdx.x;
   if constexpr (BITS == 6) q6k_to_f16(w, w16, nitems, t);
   else q5k_to_f16(w, w16, nitems, t);
+}
+
+// How the two go (kquant_operands in launch_rules.hpp).
+template <int BITS>
+void launch_operands_to_f16(const float* a, _Float16* a16, float* a_scale, uint32_t m, uint32_t k, const uint8_t* w, _Float16* w16,
+                            uint64_t blocks, hipStream_t stream) {
+  const uint64_t items = blocks * (BITS == 6 ? 8 : 16);
+  const uint32_t groups = static_cast<uint32_t>((items + 255) / 256);     // below 2^20, as m is below 2^23 (gemm_kquant_f16_supported)
+  auto go = [&](auto kernel, uint32_t rows, uint32_t row0) {
+    hipLaunchKernelGGL(kernel, dim3(rows + groups), dim3(256), 0, stream, a, a16, a_scale, rows, row0, k, w, w16, items);
+  };
+  const KquantOperands how = kquant_operands(m, k, BITS);
+  if (how == KquantOperands::Apart) {
+    go(operands_to_f16_kernel<BITS, 0>, 0u, 0u);
+    launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
+  } else if (how == KquantOperands::RowsTwice) {
+    go(operands_to_f16_kernel<BITS, 0>, m, 0u);
+  } else {
+    with_row_registers(k, [&](auto nv) { go(operands_to_f16_kernel<BITS, decltype(nv)::value>, m, how == KquantOperands::RowsLast ? groups : 0u); });
+  }
 }
 
 // C tile = A16 (rows scaled by a_scale) . W16^T, both operands fp16 row-major with row length k.
@@ -577,23 +598,8 @@ hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t blo
   _Float16* w16 = reinterpret_cast<_Float16*>(a_scale + m + 256);
   const uint64_t blocks = static_cast<uint64_t>(n) * (k / 256);
   if (block_bytes != 210 && block_bytes != 176) return hipErrorInvalidValue;
-  const uint64_t items = blocks * (block_bytes == 210 ? 8 : 16), weight_groups = (items + 255) / 256;
-  with_row_registers(k, [&](auto nv) {
-    constexpr int NV = decltype(nv)::value;
-    auto go = [&](uint32_t rows, uint64_t groups) {
-      auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups)), dim3(256), 0, stream, a, a16, a_scale, rows, k, w, w16, items);
-      };
-      if (block_bytes == 210) launch(operands_to_f16_kernel<6, NV>);
-      else launch(operands_to_f16_kernel<5, NV>);
-    };
-    if (m + weight_groups < kMaxGridThreads / 256u) {
-      go(m, m + weight_groups);
-    } else {                      // more than a launch can have
-      go(m, m);
-      go(0u, weight_groups);
-    }
-  });
+  if (block_bytes == 210) launch_operands_to_f16<6>(a, a16, a_scale, m, k, w, w16, blocks, stream);
+  else launch_operands_to_f16<5>(a, a16, a_scale, m, k, w, w16, blocks, stream);
   const SharedTiles plan = shared_f16_tiles(m, n, k / 256u, static_cast<uint64_t>(num_cus()), false);
   if (plan.groups != 0u) return launch_shared<F16Weights>(a16, a_scale, w16, c, parts, m, n, k, plan, stream);
   const F16wTiles tiles = f16w_tiles(m, n, k, static_cast<uint32_t>(num_cus()));
