@@ -575,8 +575,10 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 // 512 rows of 24 heads of 256 on 2512 fp16 keys of 4: 121 us among other calls (432 with a workgroup a row and key head,
 // which read each key for six columns), back to back 107 (417), int8 keys 121 (439).  Vector instructions issue in 60 % of
 // the cycles, the matrix cores are busy in 32 %, LDS in 29 %; a wavefront waits in 34 % of its own, at the tile's barrier
-// and for operands.  With the values' operands read two groups ahead, the second terms' matrix instructions one, and the
-// running sums scaled by the multiply-add that adds to them, back to back 112.7 -> 110.7 us, int8 124.4 -> 120.6.
+// and for operands.  STAGGERED: the values' operands are read two groups ahead, the second terms' matrix instructions go one, and
+// the running sums are scaled by the multiply-add that adds to them: 512 rows on 2512 keys back to back, 24 heads of 256 106.9 ->
+// 103.4 us, int8 119.9 -> 116.0, 24 of 128 int8 77.3 -> 74.0.  fp16 keys of heads of 128 (65 to 128) keep a group after the other:
+// 24 heads 60.7 us, staggered 63.6.
 // Infinities and NaN are not kept apart here.  Whatever meets one ends with a sum that is not finite, or sets
 // `special`; the workgroup's columns are then done again with attend_row.
 template <int DP>
@@ -825,7 +827,9 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
     }
     if (wg_last - j0 >= 64u) stash(b ^ 1u);
     if (wg_last - j0 >= 128u) fetch(j0 + 128u);
-    constexpr int BLOCKS = DP == 256 ? 1 : 2, GROUPS = VE / BLOCKS, AHEAD = 2;   // blocks of O^T at once, reads ahead
+    // The values' operands: groups of BLOCKS blocks of O^T, read AHEAD groups before their matrix instructions.
+    constexpr bool STAGGERED = QUANT || DP != 128;
+    constexpr int BLOCKS = !STAGGERED ? GROUP : DP == 256 ? 1 : 2, GROUPS = VE / BLOCKS, AHEAD = STAGGERED ? 2 : 1;
     half8_t vf[AHEAD + 1][BLOCKS];
     auto read_values = [&](int n) {
 #pragma unroll
@@ -883,54 +887,93 @@ __global__ __launch_bounds__(512, 2) void attention_tile_kernel(AttentionArgs a)
         }
       }
     }
-    // (x is kept apart from its conversions: a multiply that rounds to fp16 takes the vector unit twice a conversion's time)
+    // APART: x and the rests are kept apart from their conversions (a multiply that rounds to fp16 takes the vector unit twice a
+    // conversion's time).  It leads for fp16 keys of heads of 64 and 256, elsewhere the compiler's own choice does (us, 512 rows on
+    // 2512 keys, apart / not: fp16, 24 heads of 256 103.4 / 105.7, 16 of 64 30.9 / 31.3; int8, 32 of 64 56.3 / 54.7, 24 of 128 75.4 / 74.0).
+    constexpr bool APART = !QUANT && STAGGERED;
     half8_t p_hi, p_lo;
+    if constexpr (APART) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float x = s[e] * value_up;
-      asm("" : "+v"(x));
-      s[e] = x;
-      p_hi[e] = static_cast<_Float16>(x);
+      for (int e = 0; e < 8; ++e) {
+        float x = s[e] * value_up;
+        asm("" : "+v"(x));
+        s[e] = x;
+        p_hi[e] = static_cast<_Float16>(x);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float x = (s[e] - static_cast<float>(p_hi[e])) * 0x1p11f;
+        asm("" : "+v"(x));
+        p_lo[e] = static_cast<_Float16>(x);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = s[e] * value_up;
+        const _Float16 hi = static_cast<_Float16>(x);
+        p_hi[e] = hi;
+        p_lo[e] = static_cast<_Float16>((x - static_cast<float>(hi)) * 0x1p11f);
+      }
     }
+    if constexpr (STAGGERED) {
+      // Group n of the operands: its second terms' sums with the first terms' of the group before and the running sums of
+      // the one before that, so that no instruction waits for the matrix instruction that has just been issued.
+      float4_t low[2][BLOCKS], own[2][BLOCKS];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float x = (s[e] - static_cast<float>(p_hi[e])) * 0x1p11f;
-      asm("" : "+v"(x));
-      p_lo[e] = static_cast<_Float16>(x);
-    }
-    // Group n of the operands: its second terms' sums with the first terms' of the group before and the running sums of
-    // the one before that, so that no instruction waits for the matrix instruction that has just been issued.
-    float4_t low[2][BLOCKS], own[2][BLOCKS];
-#pragma unroll
-    for (int n = 1; n < AHEAD && n < GROUPS; ++n) read_values(n);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int n = 0; n < GROUPS + 2; ++n) {
-      if (n < GROUPS) {
-#pragma unroll
-        for (int i = 0; i < BLOCKS; ++i) {
-          low[n & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n % (AHEAD + 1)][i], p_lo, float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-        }
-      }
-      if (n >= 1 && n - 1 < GROUPS) {
-#pragma unroll
-        for (int i = 0; i < BLOCKS; ++i) {
-          float4_t x = low[(n - 1) & 1][i];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x[e] *= 0x1p-11f;
-          own[(n - 1) & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[(n - 1) % (AHEAD + 1)][i], p_hi, x, 0, 0, 0);
-        }
-      }
-      if (n >= 2) {
-#pragma unroll
-        for (int i = 0; i < BLOCKS; ++i) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[(n - 2) * BLOCKS + i][e] = fmaf(o[(n - 2) * BLOCKS + i][e], corr, own[n & 1][i][e]);
-          asm volatile("" ::"v"(own[n & 1][i]));      // still held: the multiply-add writes o in place, not here
-        }
-      }
-      if (n + AHEAD < GROUPS) read_values(n + AHEAD);      // where group n - 1 was
+      for (int n = 1; n < AHEAD && n < GROUPS; ++n) read_values(n);
       __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < GROUPS + 2; ++n) {
+        if (n < GROUPS) {
+#pragma unroll
+          for (int i = 0; i < BLOCKS; ++i) {
+            low[n & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n % (AHEAD + 1)][i], p_lo, float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+          }
+        }
+        if (n >= 1 && n - 1 < GROUPS) {
+#pragma unroll
+          for (int i = 0; i < BLOCKS; ++i) {
+            float4_t x = low[(n - 1) & 1][i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] *= 0x1p-11f;
+            own[(n - 1) & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[(n - 1) % (AHEAD + 1)][i], p_hi, x, 0, 0, 0);
+          }
+        }
+        if (n >= 2) {
+#pragma unroll
+          for (int i = 0; i < BLOCKS; ++i) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[(n - 2) * BLOCKS + i][e] = fmaf(o[(n - 2) * BLOCKS + i][e], corr, own[n & 1][i][e]);
+            asm volatile("" ::"v"(own[n & 1][i]));      // still held: the multiply-add writes o in place, not here
+          }
+        }
+        if (n + AHEAD < GROUPS) read_values(n + AHEAD);      // where group n - 1 was
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      if (__any(corr != 1.0f)) {
+#pragma unroll
+        for (int j = 0; j < VE; ++j) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[j][e] *= corr;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < GROUPS; ++n) {
+        if (n + 1 < GROUPS) read_values(n + 1);
+        float4_t acc[BLOCKS];
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n & 1][i], p_lo, float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][e] *= 0x1p-11f;
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[n & 1][i], p_hi, acc[i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i) o[n * BLOCKS + i] += acc[i];
+      }
     }
     __syncthreads();
   }
