@@ -1225,11 +1225,13 @@ hipError_t launch_rows(const AttentionArgs& a, uint64_t m, hipStream_t stream) {
   const dim3 grid(static_cast<uint32_t>(workgroups));
   // Four wavefronts a workgroup take 128 keys at once; where a workgroup has more to do and the registers and the size of a
   // grid allow it, eight; with no more workgroups than CUs, five take the 129 to 160 keys that parts of 128 come to where they
-  // do not divide the keys, and spare the second time round (us, four / five: int8, 1200 keys in 9 parts, 4 key heads of 128 8.6 /
-  // 7.9, 9301 in 64, 4 of 64 6.7 / 6.2; but two workgroups a CU, 9301 keys, 8 of 128 12.4 / 15.6).
+  // do not divide the keys, and spare a time round (us, four / five: int8, 1200 keys in 9 parts, 4 key heads of 128 8.6 /
+  // 7.9, 9301 in 64, 4 of 64 6.7 / 6.2; but two workgroups a CU, 9301 keys, 8 of 128 12.4 / 15.6).  Over an fp32 cache, whose wavefronts
+  // take 16 keys at a time, up to 144: from there on all five go round twice (24 heads over 8 of 128, 140 keys 9.7 / 9.0, 160 9.7 /
+  // 10.4; 9301 keys in 64 parts of 146, 8 heads over 1 of 128 11.0 / 11.5).
   const uint64_t each = (a.n + split - 1) / split;
   const bool wide = a.n / split > 160 && workgroups < kMaxGridThreads / 512u;
-  const bool five = each > 128 && each <= 160 && workgroups <= static_cast<uint64_t>(num_cus());
+  const bool five = each > 128 && each <= (KV == KvKind::F32 ? 144 : 160) && workgroups <= static_cast<uint64_t>(num_cus());
   auto go = [&](auto kernel, uint32_t waves) { hipLaunchKernelGGL(kernel, grid, dim3(waves * 64u), 0, stream, a); };
   auto pick = [&](auto dim) {
     constexpr int DP = decltype(dim)::value;
