@@ -274,9 +274,9 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_kernel(const _Float16* __rest
   };
   static_assert(kRunSteps == 2, "the loop's steps");
   for (;;) {
-    if (one_step(std::true_type{})) break;
+    const bool last = one_step(std::true_type{});
     if (step % kAccSteps == 1u && step != 1u) add_acc();
-    if (one_step(std::false_type{})) break;
+    if (last || one_step(std::false_type{})) break;
   }
   if (count % kRunSteps == 0u) {      // the last run, as the step after it would have
 #pragma unroll

@@ -121,3 +121,16 @@ def test_elements_far_below_the_row_s_largest(backend, m, n, k, binades):
     codes[:, largest] = 0
     codes = codes.reshape(-1)
     assert within(fp8_gemm(backend, a, codes, scales, m, n, k), *exact(a, codes, scales, n, k), k)
+
+
+@pytest.mark.parametrize("steps", [2, 14, 16, 30, 32, 48])
+def test_a_step_of_zeros_changes_nothing(backend, steps):
+    """Sums are kept in runs of 2 and of 16 steps of K, and a run that has ended goes on to the next sum also where one more
+    step is left: 64 more zeros a row have the bits of the product without them.  (300 x 6144: one part of K.)"""
+    m, n, k = 300, 6144, steps * 64
+    g = synth.rng(6300 + steps)
+    codes, scales = synth.fp8_weights(g, n, k + 64)
+    a = synth.activations_f32(g, m, k)
+    short = fp8_gemm(backend, a, np.ascontiguousarray(codes.reshape(n, k + 64)[:, :k]).reshape(-1), scales, m, n, k)
+    long = fp8_gemm(backend, np.concatenate([a, np.zeros((m, 64), np.float32)], 1), codes, scales, m, n, k + 64)
+    assert np.array_equal(short, long)
