@@ -178,6 +178,7 @@ __device__ __forceinline__ void q4k_tile_sums(TileSums<WM / KSETS, WN>& out, con
   constexpr uint32_t kJRows = PAIR ? BN / 2 : 32;  // weight rows from a wavefront's column tile to its next
   static_assert(!PAIR || (kTJ == 2 && BN * 9 % 128 == 0), "a load block lies in one matrix");
   static_assert(KSETS == 1 || (KSETS == 2 && WM == BM && kTI % 2 == 0 && !PAIR), "two sets share a tile of one row of wavefronts");
+  static_assert(KSETS == 1 || (kTJ == 2 && (kWavesN & (kWavesN - 1)) == 0), "two sets: one decode in each half of a slice, partners a bit apart");
   static_assert(BM % WM == 0 && BN % WN == 0 && WM % 32 == 0 && WN % 32 == 0 && BM % (16 * kWaves) == 0, "tile shape");
   __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kAStage + 2 * kWStage];
 
