@@ -106,10 +106,11 @@ void* g_static_scratch[kMaxDevices] = {};
 constexpr size_t round256(size_t bytes) { return (bytes + 255) & ~size_t{255}; }
 
 // `bytes` of scratch, and `*more` bytes behind them where they can be had (0 is left in it where not: such a call does
-// without).
-qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out, size_t* more = nullptr) {
-  size_t none = 0;
+// without); `*holds`: what there is in all.
+qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out, size_t* more = nullptr, size_t* holds = nullptr) {
+  size_t none = 0, unused = 0;
   size_t& extra = more != nullptr ? *more : none;
+  size_t& all = holds != nullptr ? *holds : unused;
   if (c.no_alloc) {
     if (bytes + extra > kStaticScratchBytes) extra = 0;
     if (bytes > kStaticScratchBytes) {
@@ -118,6 +119,7 @@ qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out, size_t* more 
       return QMM_INVALID_ARGUMENT;
     }
     *out = g_static_scratch[g_device];
+    all = kStaticScratchBytes;
     return QMM_OK;
   }
   std::lock_guard<std::mutex> lock(g_workspace_mutex);
@@ -129,6 +131,7 @@ qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out, size_t* more 
       return QMM_INVALID_ARGUMENT;
     }
     *out = g_user_workspace;
+    all = g_user_workspace_bytes;
     return QMM_OK;
   }
   auto grow = [](size_t need) {
@@ -163,6 +166,7 @@ qmm_status workspace(const LaunchCtx& c, size_t bytes, void** out, size_t* more 
     }
   }
   *out = g_workspace;
+  all = g_workspace_bytes;
   return QMM_OK;
 }
 
@@ -236,13 +240,13 @@ class StreamBlock {
 static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock && qmm::kAttentionPartsMost <= kPartsLimits.small);
 
 // The workspace of a product whose tiles workgroups may share: its `operands` bytes, and behind them and behind `taken` room
-// for the tiles' pieces, which the caller orders as it does the operands.  Without room (the array or the caller's block is too
-// small, or the library's cannot grow) *parts is null: the sums are then cut and added as the pieces are, the same bits.
+// for the tiles' pieces, which the caller orders as it does the operands.  They lie at the workspace's end, away from where other
+// products write their operands (a decode to fp16 over them took 8.9 us instead of 7.0).  Without room (the array or the caller's
+// block is too small, or the library's cannot grow) *parts is null: the sums are then cut and added as the pieces are, the same bits.
 qmm_status product_workspace(const LaunchCtx& c, size_t operands, size_t taken, size_t pieces, void** ws, float** parts) {
-  const size_t at = round256(operands > taken ? operands : taken);
-  size_t more = pieces == 0 ? 0 : at - operands + pieces;
-  const qmm_status st = workspace(c, operands, ws, &more);
-  *parts = st != QMM_OK || more == 0 ? nullptr : reinterpret_cast<float*>(static_cast<uint8_t*>(*ws) + at);
+  size_t more = pieces == 0 ? 0 : round256(operands > taken ? operands : taken) - operands + pieces, holds = 0;
+  const qmm_status st = workspace(c, operands, ws, &more, &holds);
+  *parts = st != QMM_OK || more == 0 ? nullptr : reinterpret_cast<float*>(static_cast<uint8_t*>(*ws) + (holds - pieces) / 256 * 256);
   return st;
 }
 
