@@ -212,7 +212,7 @@ qmm_status qmm_set_workspace(void* device_ptr, size_t bytes);
  * src/core/decode_internal.hpp:1428, used at src/models/qwen3_5/project.cpp:307) and keeps fp32
  * activations below (src/models/qwen3_5/project.cpp:307-322), so by default a result carries the fp16 operand
  * rounding exactly where the reference's does; 17..63 rows then run sixteen at a time through the
- * exact kernels (about 28 us per 16 rows of a 17408 x 5120 matrix, against 35..46 us for the
+ * exact kernels (about 28 us per 16 rows of a 17408 x 5120 matrix, against 29..39 us for the
  * tile).  A caller that prefers the tile's speed there sets a lower count, at least 17 (up to 16
  * rows, the speculative-verify batch, always stay exact); a higher count keeps more rows on the
  * exact kernels, sixteen at a time; 0 restores the default.

@@ -573,8 +573,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_rows_kernel(AttentionArg
 // A tile's contribution, the second terms' sum brought down by 2^-11 and the first terms' added to it, is summed by
 // itself and added to the running sum, so that rounding there goes with a few terms and not with the number of keys.
 // 512 rows of 24 heads of 256 on 2512 fp16 keys of 4: 121 us among other calls (432 with a workgroup a row and key head,
-// which read each key for six columns), back to back 107 (417), int8 keys 121 (439).  Vector instructions issue in 60 % of
-// the cycles, the matrix cores are busy in 32 %, LDS in 29 %; a wavefront waits in 34 % of its own, at the tile's barrier
+// which read each key for six columns), back to back 107 (417), int8 keys 121 (439).  Vector instructions issue in 56 % of
+// the cycles, the matrix cores are busy in 34 %, LDS in 30 %; a wavefront waits in 37 % of its own, at the tile's barrier
 // and for operands.  STAGGERED: the values' operands are read two groups ahead, the second terms' matrix instructions go one, and
 // the running sums are scaled by the multiply-add that adds to them: 512 rows on 2512 keys back to back, 24 heads of 256 106.9 ->
 // 103.4 us, int8 119.9 -> 116.0, 24 of 128 int8 77.3 -> 74.0.  fp16 keys of heads of 128 (65 to 128) keep a group after the other:

@@ -23,8 +23,8 @@
 // converts the codes of its columns once per stage and uses them against both terms of all its rows.  Whatever
 // part of the chip one round of tiles leaves idle is filled by splitting K (fp8_plan); the partial sums are added
 // in part order by a last launch: no atomics, the same bits every time.  What bounds it: at 300 x 6144 x 5120 the
-// matrix cores are busy 41 % of the product's cycles, vector instructions issue in 21 %, and a wavefront, alone on its SIMD,
-// waits in 24 % (direct loads, barrier) and for issue in 30 %; neither a deeper ring (five stages) nor a tile that reads
+// matrix cores are busy 41 % of the product's cycles, vector instructions issue in 27 %, and a wavefront, alone on its SIMD,
+// waits in 25 % (direct loads, barrier) and for issue in 29 %; neither a deeper ring (five stages) nor a tile that reads
 // less LDS changes it.  A short stack of rows is bound by the weight stream.  Half a step's operands are read and
 // converted between the matrix instructions of the half before: 57.2 -> 54.0 us with the rows' conversion.
 // 300 x 6144 x 5120: 1108 -> 56 us against 75 four-row passes of the multiply-add kernel; 17 rows 68 -> 16 us.
@@ -337,8 +337,9 @@ struct Fp8Plan {
 };
 
 // Row tile and K parts with the smallest estimate of the launch: the workgroups of the fullest CU one after
-// another (two on a CU take as long as one after the other: 0.36 us a 64-wide step of 32 rows, 0.58 of 64, measured
-// with 1 to 4 a CU), then the launch that adds the parts and the traffic of their sums.
+// another (two on a CU take as long as one after the other), then the launch that adds the parts and the traffic of their
+// sums.  A 64-wide step of 32 rows counts as 0.36 us, of 64 rows 0.58, as measured with 1 to 4 a CU when a step's operands were made
+// in the step; as they are made now a step takes 0.33 and 0.51, two on a CU 0.97 of 64 rows, the same in proportion.
 // 17 x 6144 x 5120: one part 33, five 16 us; 300 x 512 x 5120: 54 and, with eight, 21 us.  A part keeps at least
 // four steps, and the parts' sums fit `room` bytes.  (Tiles of 128 rows were no faster up to 1024 rows and leave no
 // registers for the sums.)

@@ -139,7 +139,8 @@ constexpr F16wTiles f16w_tiles(uint32_t m, uint32_t n, uint32_t k, uint32_t cus)
   return {tiles < cus / 2 ? 0u : tiles_n, 256u};
 }
 // The order of the tiles.  Workgroups go round the XCDs, in the launch that decodes as here, so that along the columns an XCD
-// finds part of the weights that it has written itself in its L2; an XCD's share of neighbouring tiles (xcd_tile) instead
+// finds part of the weights that it has written itself in its L2 (also with the rows' workgroups before the weights', whose count
+// is the shift: 100, 101 and 103 rows of 16384 x 1024 25 us each, shares 32); an XCD's share of neighbouring tiles (xcd_tile) instead
 // reads them once for several row tiles.  The first leads with one row tile, with up to three where the weights are small, and
 // where small tiles are few (us, along / shares): 100 rows of 16384 x 1024 27 / 33, 256 rows 33 / 39, 300 of 6144 x 5120 70 /
 // 84, 512 of 5120 x 17408 (320 small tiles) 286 / 324, 700 of 3072 x 1024 (288) 24 / 29; 256 rows of 17408 x 5120 161 / 151, of
@@ -177,7 +178,8 @@ constexpr PackShape pack_shape(uint64_t rows, uint64_t cols) {
 // how many a row sees at most; `padded`: the head size, 64, 128 or 256.
 //
 // The shorter of the estimated times, in us: a fixed part, then for the rows' kernel what a round of a workgroup a CU takes
-// by its keys (four wavefronts up to 160 keys, eight beyond), for the other what 64 keys take, and for its parts the
+// by its keys (four wavefronts up to 160 keys, eight beyond; where five take 129 to 160 keys they are up to a tenth faster than
+// the estimate, and of 306 such calls none takes the longer way by more than 3 %), for the other what 64 keys take, and for its parts the
 // second launch and the sums' way through memory.  Fitted to 1716 calls (17 to 512 rows, 17 to 2512 keys, 2 to 32 heads over
 // 1 to 8 key heads of 64, 96, 128 and 256, fp16 and int8), which they meet within 4 % on average: one call of them
 // takes the longer way by more than 5 %.  Rows' kernel / one part / parts: 64 rows of 24 heads over 4 of 256 on 564 keys 21 / 34 /
