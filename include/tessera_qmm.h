@@ -32,11 +32,14 @@
  *     stream that records them: "gemm_fp8" from 17 rows (128 MB more where a call does not fit) and
  *     "gemm_q5k*" / "gemm_q6k*" with 2..16 rows out of the 256 MB that qmm_init reserves, then out of slabs of
  *     128 MB, 2 GB in all; "attention", "attention_q8", "_q4" and "_fp8" from 17 rows and "top_k_rows" over long
- *     rows out of 64 MB, then slabs of 64 MB, 512 MB in all.  While a caller's workspace is set no slab is
- *     allocated.  The blocks are not given back (a graph may
+ *     rows out of 64 MB, then slabs of 64 MB, 512 MB in all.  Products of Q4_K, Q5_K and Q6_K with few tiles whose
+ *     workspace has no room for what they hand on (a caller's of just the operands, a capture before the library's
+ *     has grown) likewise, 16 to 40 MB out of slabs of 128 MB, 1 GB in all; qmm_set_workspace reserves the first.
+ *     While a caller's workspace is set no slab is allocated.  The blocks are not given back (a graph may
  *     still use them), and a stream handle's block passes to the next stream with that handle: let a
  *     stream's launches finish before it is destroyed.  A launch that gets no block, or is made on
- *     hipStreamPerThread, runs kernels that need none (slower; sums in another order, "top_k_rows" the same results).
+ *     hipStreamPerThread, runs kernels that need none (slower; "top_k_rows" and the products of Q4_K, Q5_K and Q6_K with
+ *     the same bits, the others with sums in another order).
  */
 #ifndef TESSERA_QMM_H_
 #define TESSERA_QMM_H_
@@ -195,10 +198,10 @@ size_t qmm_static_scratch_bytes(void);
  * (src/models/qwen3_5/project.cpp:127-155,198-206: gemv_part, wmma_a, wmma_as, wmma_part).
  * qmm_workspace_bytes returns what a launch of `kernel` with these scalars needs (0 for
  * decode-sized launches and ids without scratch; for the grouped routed-expert ids an upper bound
- * over the expert count; for "gemm_mxfp4" from 17 rows with what it only makes use of: it runs, slower and
- * with the same bits, in the 4 m k + 2 * 256 * ceil(m / 64) bytes of the rows' terms; a Q4_K, Q5_K or Q6_K product
- * with few tiles makes use of 64 KB more for each 128 x 128 tile and 16 MB, and runs slower, with the same bits,
- * without).  qmm_set_workspace hands the library a device block of that size
+ * over the expert count; for "gemm_mxfp4", "gemm_q5k*" and "gemm_q6k*" from 17 rows with what they only make use of: they
+ * run, slower and with the same bits, in the 4 m k + 2 * 256 * ceil(m / 64) bytes of the rows' terms, in the 2 (m + n) k +
+ * 4 (m + 256) bytes of the fp16 operands.  A Q4_K product's are what it needs; where it has few tiles it makes use of 64 KB
+ * more for each 128 x 128 tile and 16 MB, likewise, or else of a block of the stream's).  qmm_set_workspace hands the library a device block of that size
  * (256-byte aligned) to use for every later qmm_launch on any stream, in stream order, until it
  * is replaced or cleared with (NULL, 0); while one is set, qmm_launch allocates nothing and a
  * launch that needs more returns InvalidArgument.  The caller must not free or replace the

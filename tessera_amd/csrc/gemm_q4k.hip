@@ -421,8 +421,8 @@ void launch_f16w_range(const _Float16* a16, const float* a_scale, const _Float16
 // column), for piece_sums_kernel to add up in the workgroups' order.  512 rows of 1024 x 5120: Q4_K 44 -> 26 us (the tiles
 // 37 -> 14, the sums 5), Q6_K 46 -> 28; of 6144 x 5120 Q4_K 64 -> 59.
 // CUT: no room for `parts`, but the same bits.  A workgroup has a whole tile (within one of the plan's, of as many rows) and adds
-// its pieces in registers, in that order.  us, tiles that are not cut / cut / with room: Q4_K 1000 x 2040 x 5120 48 / 56 / 43, 1024 x
-// 5120 x 5120 103 / 115 / 95, 512 x 6144 x 5120 64 / 61 / 59, Q6_K 512 x 1024 x 5120 46 / 51 / 28.
+// its pieces in registers, in that order.  us, tiles that are not cut / cut / with room: Q4_K 64 x 1024 x 5120 37 / 71 / 18, 1000 x
+// 2040 x 5120 48 / 56 / 43, 1024 x 5120 x 5120 103 / 112 / 95, 512 x 6144 x 5120 64 / 63 / 59, Q6_K 512 x 1024 x 5120 46 / 51 / 28.
 struct Q4KWeights {
   using Type = uint8_t;
   static constexpr int kCutWN = 64;

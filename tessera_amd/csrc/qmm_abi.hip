@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -239,16 +240,33 @@ class StreamBlock {
 };
 static_assert(kDecodeScratchBytes <= qmm::StreamScratch::kSmallBlock && qmm::kAttentionPartsMost <= kPartsLimits.small);
 
-// The workspace of a product whose tiles workgroups may share: its `operands` bytes, and behind them and behind `taken` room
-// for the tiles' pieces, which the caller orders as it does the operands.  They lie at the workspace's end, away from where other
-// products write their operands (a decode to fp16 over them took 8.9 us instead of 7.0).  Without room (the array or the caller's
-// block is too small, or the library's cannot grow) *parts is null: the sums are then cut and added as the pieces are, the same bits.
-qmm_status product_workspace(const LaunchCtx& c, size_t operands, size_t taken, size_t pieces, void** ws, float** parts) {
-  size_t more = pieces == 0 ? 0 : round256(operands > taken ? operands : taken) - operands + pieces, holds = 0;
-  const qmm_status st = workspace(c, operands, ws, &more, &holds);
-  *parts = st != QMM_OK || more == 0 ? nullptr : reinterpret_cast<float*>(static_cast<uint8_t*>(*ws) + (holds - pieces) / 256 * 256);
-  return st;
-}
+// The workspace of a product whose tiles workgroups may share (`operands` bytes) and room for the tiles' pieces.  They lie
+// behind the operands and behind `taken`, at the workspace's end, away from where other products write their operands (a decode to
+// fp16 over them took 8.9 us instead of 7.0), and the caller orders them as it does those.  Where that has no room, which is a
+// caller's workspace of just the operands or a capture before the library's has grown, they take a block of the stream's (64
+// rows of 1024 x 5120 Q4_K 18 us, cut 71), of slabs of their own, the first of which qmm_set_workspace reserves.  Without that too
+// (and in qmm_launch_static) the sums are cut and added as the pieces are: the same bits everywhere.
+constexpr qmm::ScratchLimits kPiecesLimits{size_t{16} << 20, size_t{40} << 20, size_t{512} << 10, size_t{128} << 20, size_t{128} << 20, size_t{1} << 30};
+qmm::StreamScratch g_pieces_scratch(kPiecesLimits);
+
+class ProductRoom {
+ public:
+  ProductRoom(const LaunchCtx& c, size_t operands, size_t taken, size_t pieces) {
+    size_t more = pieces == 0 ? 0 : round256(operands > taken ? operands : taken) - operands + pieces, holds = 0;
+    status_ = workspace(c, operands, &workspace_, &more, &holds);
+    if (status_ != QMM_OK || pieces == 0) return;
+    if (more != 0) pieces_ = static_cast<uint8_t*>(workspace_) + (holds - pieces) / 256 * 256;
+    else if (!c.no_alloc) pieces_ = block_.emplace(c, pieces, g_pieces_scratch).get();
+  }
+  qmm_status status() const { return status_; }
+  void* operands() const { return workspace_; }
+  float* pieces() const { return static_cast<float*>(pieces_); }      // null: no room
+
+ private:
+  qmm_status status_;
+  void *workspace_ = nullptr, *pieces_ = nullptr;
+  std::optional<StreamBlock> block_;      // held to the call's last launch
+};
 
 // Q4_K regimes by activation rows.  One row and small matrices: the VALU GEMV.  2..16 rows of a
 // matrix with at least kQ4KFewRowsMinWeights weights: the exact few-row MFMA kernels (weights read
@@ -278,11 +296,9 @@ qmm_status q4k_matmul(const LaunchCtx& ctx, const float* a, const uint8_t* w, fl
                       uint64_t k, uint64_t f16_from, size_t taken) {
   const hipStream_t s = ctx.stream;
   if (m >= f16_from && qmm::gemm_q4k_supported(m, k)) {
-    void* ws = nullptr;
-    float* parts = nullptr;
-    const qmm_status st = product_workspace(ctx, qmm::gemm_q4k_workspace_bytes(m, k), taken, qmm::gemm_f16_parts_bytes(m, n, k, true), &ws, &parts);
-    if (st != QMM_OK) return st;
-    return map_hip(qmm::launch_q4k_gemm(a, w, c, ws, parts, static_cast<uint32_t>(m), static_cast<uint32_t>(n),
+    const ProductRoom room(ctx, qmm::gemm_q4k_workspace_bytes(m, k), taken, qmm::gemm_f16_parts_bytes(m, n, k, true));
+    if (room.status() != QMM_OK) return room.status();
+    return map_hip(qmm::launch_q4k_gemm(a, w, c, room.operands(), room.pieces(), static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                         static_cast<uint32_t>(k), s));
   }
   if (m > 16 && (n * k >= kQ4KFewRowsMinWeights || qmm::gemv_q4k_rows16_supported(16, n, k))) {
@@ -848,12 +864,11 @@ qmm_status run_dequant_q4k(const LaunchCtx& c) {
 // workspace, then the dense fp16 MFMA GEMM.
 qmm_status kquant_prefill(const LaunchCtx& c, uint32_t block_bytes, uint64_t m, uint64_t n, uint64_t k,
                           uint64_t split) {
-  void* ws = nullptr;
-  float* parts = nullptr;
-  qmm_status st = product_workspace(c, qmm::gemm_kquant_f16_workspace_bytes(m, n, k), 0, qmm::gemm_f16_parts_bytes(m, n, k, false), &ws, &parts);
+  const ProductRoom room(c, qmm::gemm_kquant_f16_workspace_bytes(m, n, k), 0, qmm::gemm_f16_parts_bytes(m, n, k, false));
+  qmm_status st = room.status();
   if (st != QMM_OK) return st;
   float* out = c.ptr<float>(2);
-  st = map_hip(qmm::launch_kquant_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), block_bytes, out, ws, parts,
+  st = map_hip(qmm::launch_kquant_f16_gemm(c.ptr<const float>(0), c.ptr<const uint8_t>(1), block_bytes, out, room.operands(), room.pieces(),
                                            static_cast<uint32_t>(m), static_cast<uint32_t>(n),
                                            static_cast<uint32_t>(k), c.stream));
   if (st == QMM_OK && split > 1) st = map_hip(qmm::launch_fill_f32(out + m * n, 0.0f, (split - 1) * m * n, c.stream));
@@ -1722,7 +1737,10 @@ qmm_status qmm_workspace_bytes(qmm_kernel kernel, const uint64_t* scalars, size_
     }
   } else if (starts("gemm_q5k") || starts("gemm_q6k")) {
     const uint64_t m = sc(0), n = sc(1), k = sc(2);
-    if (m >= kQ4KGemmMinRows && qmm::gemm_kquant_f16_supported(m, n, k)) *out_bytes = qmm::gemm_kquant_f16_workspace_bytes(m, n, k);
+    if (m >= kQ4KGemmMinRows && qmm::gemm_kquant_f16_supported(m, n, k)) {
+      const size_t operands = qmm::gemm_kquant_f16_workspace_bytes(m, n, k), pieces = qmm::gemm_f16_parts_bytes(m, n, k, false);
+      *out_bytes = pieces == 0 ? operands : round256(operands) + pieces;
+    }
   } else if (id == "moe_experts_gate_up_q4k_rows" || id == "moe_experts_down_q4k_rows") {
     const uint64_t hidden = sc(0), inter = sc(1), top_k = sc(2), rows = sc(5);
     if (rows >= kMoeGroupedMinRows) *out_bytes = qmm::moe_ffn_q4k_workspace_bytes(rows * top_k, hidden, inter, 1024);
@@ -1745,6 +1763,8 @@ uint32_t qmm_q4k_tensor_rows(void) { return static_cast<uint32_t>(g_q4k_tensor_r
 qmm_status qmm_set_workspace(void* device_ptr, size_t bytes) {
   if ((device_ptr == nullptr) != (bytes == 0)) return bad("qmm_set_workspace: pointer and size must both be set or both be zero");
   if (reinterpret_cast<uintptr_t>(device_ptr) % 256 != 0) return bad("qmm_set_workspace: the workspace must be 256-byte aligned");
+  // (a launch may allocate nothing from here on, so that what its pieces may lack room for is got now)
+  if (device_ptr != nullptr && g_device >= 0 && hipSetDevice(g_device) == hipSuccess) (void)g_pieces_scratch.reserve(StreamBlock::grow);
   std::lock_guard<std::mutex> lock(g_workspace_mutex);
   g_user_workspace = device_ptr;
   g_user_workspace_bytes = bytes;

@@ -72,10 +72,12 @@ def test_same_bits_wherever_there_is_scratch(backend, kind, m, n, k):
     want = p.result()
     assert np.all(np.isfinite(want)) and same_bits(p.result(no_alloc=True), want)
     need = backend.WorkspaceBytes(p.kernel, p.scalars)
+    operands = 2 * m * k + 4 * (m + 256) + (0 if kind == "q4k" else 2 * n * k)
+    assert need == operands if kind == "q4k" else need > operands
     room = need + (64 << 20)                                # more than any plan's pieces
     ws = torch.empty(room, dtype=torch.uint8, device="cuda")
     try:
-        for size in (need, need + (1 << 20), room):         # no room for the pieces, too little, enough
+        for size in (operands, operands + (1 << 20), need, room):         # the pieces in a block of the stream's, twice; in the workspace
             backend.SetWorkspace(backend.WrapBuffer(ws.data_ptr(), size))
             assert same_bits(p.result(), want), size
     finally:
@@ -84,12 +86,18 @@ def test_same_bits_wherever_there_is_scratch(backend, kind, m, n, k):
 
 @pytest.mark.parametrize("kind,m,n,k", [("q4k", 300, 1030, 5120), ("q5k", 100, 1030, 5120), ("q6k", 100, 1030, 5120)])
 def test_same_bits_on_each_threads_own_stream(backend, kind, m, n, k):
+    """hipStreamPerThread has no block: with a caller's workspace of just the operands there is no room anywhere."""
     p = Product(backend, kind, m, n, k)
     want = p.result()
+    operands = 2 * m * k + 4 * (m + 256) + (0 if kind == "q4k" else 2 * n * k)
+    ws = torch.empty(operands, dtype=torch.uint8, device="cuda")
     try:
-        backend.SetStream(2)                                # hipStreamPerThread
+        backend.SetStream(2)
+        assert same_bits(p.result(), want)
+        backend.SetWorkspace(backend.WrapBuffer(ws.data_ptr(), operands))
         assert same_bits(p.result(), want)
     finally:
+        backend.SetWorkspace(None)
         backend.SetStream(0)
 
 
@@ -125,14 +133,19 @@ def test_feed_forward_keeps_its_products_apart(backend):
     assert same_bits(result(no_alloc=True), want)
 
 
-def test_recorded(backend):
-    """Two products recorded together, replayed with eager work of other sizes between the replays."""
+@pytest.mark.parametrize("tight", [False, True])
+def test_recorded(backend, tight):
+    """Two products recorded together, replayed with eager work of other sizes between the replays; with the library's workspace
+    and with a caller's that holds no more than the operands."""
     calls = [Product(backend, "q4k", 300, 1030, 5120), Product(backend, "q6k", 100, 1030, 5120)]
     other = Product(backend, "q4k", 129, 257, 2048, 9)
     want, want_other = [p.result() for p in calls], other.result()
     stream = torch.cuda.Stream()
     graph = torch.cuda.CUDAGraph()
+    ws = torch.empty(2 * 100 * 5120 + 4 * 356 + 2 * 1030 * 5120, dtype=torch.uint8, device="cuda")     # the second product's
     try:
+        if tight:
+            backend.SetWorkspace(backend.WrapBuffer(ws.data_ptr(), ws.numel()))
         with torch.cuda.graph(graph, stream=stream):
             backend.SetStream(torch.cuda.current_stream().cuda_stream)
             for p in calls:
@@ -147,4 +160,5 @@ def test_recorded(backend):
             assert all(same_bits(p.bits(), w) for p, w in zip(calls, want))
             assert same_bits(other.result(), want_other)
     finally:
+        backend.SetWorkspace(None)
         backend.SetStream(0)

@@ -64,7 +64,7 @@ def test_shared_mxfp4_tiles_cover_every_step_once(tmp_path):
 
 
 def test_shared_f16_tiles_cover_every_super_block_once(tmp_path):
-    """As above for the K-quants' 128 x 128 tiles: at least two units a workgroup, and the pieces fit a stream's block."""
+    """As above for the K-quants' 128 x 128 tiles: at least two units a workgroup, and less than 40 MB of pieces."""
     run_program(tmp_path, r"""
   const uint64_t ms[] = {17, 32, 33, 64, 100, 128, 129, 300, 512, 1000, 2048};
   const uint64_t ns[] = {1, 64, 65, 128, 129, 1000, 2306, 5120, 6144, 20000};
