@@ -263,14 +263,14 @@ __global__ __launch_bounds__(256) void operands_to_f16_kernel(const float* __res
 
 // How the two go (kquant_operands in launch_rules.hpp).
 template <int BITS>
-void launch_operands_to_f16(const float* a, _Float16* a16, float* a_scale, uint32_t m, uint32_t k, const uint8_t* w, _Float16* w16,
-                            uint64_t blocks, hipStream_t stream) {
-  const uint64_t items = blocks * (BITS == 6 ? 8 : 16);
+void launch_operands_to_f16(const float* a, _Float16* a16, float* a_scale, uint32_t m, uint32_t n, uint32_t k, const uint8_t* w,
+                            _Float16* w16, hipStream_t stream) {
+  const uint64_t items = static_cast<uint64_t>(n) * (k / 256u) * (BITS == 6 ? 8 : 16);
   const uint32_t groups = static_cast<uint32_t>((items + 255) / 256);     // below 2^20, as m is below 2^23 (gemm_kquant_f16_supported)
   auto go = [&](auto kernel, uint32_t rows, uint32_t row0) {
     hipLaunchKernelGGL(kernel, dim3(rows + groups), dim3(256), 0, stream, a, a16, a_scale, rows, row0, k, w, w16, items);
   };
-  const KquantOperands how = kquant_operands(m, k, BITS);
+  const KquantOperands how = kquant_operands(m, n, k, BITS);
   if (how == KquantOperands::Apart) {
     go(operands_to_f16_kernel<BITS, 0>, 0u, 0u);
     launch_rows_to_f16(a, a16, a_scale, m, k, nullptr, 1u, stream);
@@ -597,10 +597,9 @@ hipError_t launch_kquant_f16_gemm(const float* a, const uint8_t* w, uint32_t blo
   _Float16* a16 = static_cast<_Float16*>(workspace);
   float* a_scale = reinterpret_cast<float*>(a16 + static_cast<size_t>(m) * k);
   _Float16* w16 = reinterpret_cast<_Float16*>(a_scale + m + 256);
-  const uint64_t blocks = static_cast<uint64_t>(n) * (k / 256);
   if (block_bytes != 210 && block_bytes != 176) return hipErrorInvalidValue;
-  if (block_bytes == 210) launch_operands_to_f16<6>(a, a16, a_scale, m, k, w, w16, blocks, stream);
-  else launch_operands_to_f16<5>(a, a16, a_scale, m, k, w, w16, blocks, stream);
+  if (block_bytes == 210) launch_operands_to_f16<6>(a, a16, a_scale, m, n, k, w, w16, stream);
+  else launch_operands_to_f16<5>(a, a16, a_scale, m, n, k, w, w16, stream);
   const SharedTiles plan = shared_f16_tiles(m, n, k / 256u, static_cast<uint64_t>(num_cus()), false);
   if (plan.groups != 0u) return launch_shared<F16Weights>(a16, a_scale, w16, c, parts, m, n, k, plan, stream);
   const F16wTiles tiles = f16w_tiles(m, n, k, static_cast<uint32_t>(num_cus()));

@@ -104,16 +104,17 @@ constexpr uint32_t gate_up_large_tiles(uint32_t m, uint32_t n, uint32_t cus) {
 // it was left last.  RowsTwice: rows first and read twice, since a row of more than 6144 held in registers leaves five wavefronts a
 // SIMD also to the weights, where Q5_K's decode wants eight.  Apart: the weights, then the rows in a launch of their own.
 // Sides measured in a whole feed forward of Q4_K gate and up with silu and this product (us, rows x hidden x inter).  Q6_K, first /
-// last: 300 x 5120 x 17408 407-454 / 411, 1024 801 / 775, 2048 1249 / 1244, 2048 x 4096 x 11008 708 / 672; but 2048 x 5120 x 6400
-// 528 / 542, 1024 x 4096 x 8192 282 / 284, and the product of 2048 x 5120 x 5120 135 / 138.  Q5_K, first / twice / apart: 100 x 5120 x 17408 244 / 232 / 235, 300 420 / 413 / 420,
-// 512 563 / 555 / 560, 1024 838 / 834 / 799, 2048 x 4096 x 11008 716 / 725 / 685, 2048 x 5120 x 6400 537 / 542 / 548; the product of 33 x 24576 x 17408 693 / 638 / 638, of
-// 33 x 512 x 12288 31.0 / 31.7 / 34.1.
+// last: 256 x 5120 x 17408 373 / 382 (the product alone, called again and again, 168 / 219), 512 534 / 536, 1024 812 / 783,
+// 2048 x 4096 x 11008 708 / 672; but 2048 x 5120 x 6400 528 / 542, 1024 x 4096 x 8192 282 / 284, and the product of 2048 x 5120 x 5120
+// 135 / 138.  Q5_K, first / twice / apart: 100 x 5120 x 17408 244 / 232 / 235, 256 375 / 380 (the product 168 / 213), 384 464 / 453 (186 /
+// 230), 1024 838 / 834 / 799, 2048 x 4096 x 11008 716 / 725 / 685, 2048 x 5120 x 6400 537 / 542 / 548; the product of 33 x 24576 x 17408
+// 693 / 638 / 638, of 512 x 24576 x 8192 409 / 381 / 378, of 33 x 512 x 12288 31.0 / 31.7 / 34.1: twice where the weights are most of it.
 enum class KquantOperands { RowsFirst, RowsLast, RowsTwice, Apart };
-constexpr KquantOperands kquant_operands(uint32_t m, uint32_t k, uint32_t bits) {
-  if (k <= 6144u || (bits == 6u && k <= 8192u)) return KquantOperands::RowsFirst;
+constexpr KquantOperands kquant_operands(uint32_t m, uint32_t n, uint32_t k, uint32_t bits) {
+  if (k <= 6144u || (bits == 6u && (m <= 512u || k <= 8192u))) return KquantOperands::RowsFirst;
   if (bits == 6u) return KquantOperands::RowsLast;
-  if (m <= 512u) return KquantOperands::RowsTwice;
-  return k < 8192u ? KquantOperands::RowsFirst : KquantOperands::Apart;
+  if (m > 512u && k >= 8192u) return KquantOperands::Apart;
+  return n >= uint64_t{24} * m ? KquantOperands::RowsTwice : KquantOperands::RowsFirst;
 }
 
 // ---- Q5_K and Q6_K from 17 rows: fp16 weights, decoded by the launch before ----------------------------------------------

@@ -1,6 +1,6 @@
 """Q5_K and Q6_K from 17 rows, whose two operands become fp16 in one launch or two: rows of each length a thread's registers are
-laid out for, row counts on both sides of Q5_K's line, and counts of blocks that leave the last workgroup's share short.  One element a row other than zero gives the
-products of an fp16 activation and an fp16 weight, which fp32 holds, times the row's power of two."""
+laid out for, row and column counts on both sides of the lines between these, and counts of blocks that leave the last
+workgroup's share short.  One element a row other than zero gives the products of an fp16 activation and an fp16 weight, which fp32 holds, times the row's power of two."""
 import numpy as np
 import pytest
 
@@ -15,7 +15,7 @@ DECODE = {"q5k": (synth.q5k_weights, oracle.dequantize_q5k), "q6k": (synth.q6k_w
 
 @pytest.mark.parametrize("kind", list(DECODE))
 @pytest.mark.parametrize("k", [256, 2048, 2304, 6144, 6400, 8192, 8448, 18432, 18688])
-@pytest.mark.parametrize("m,n", [(17, 33), (41, 7), (512, 9), (513, 9)])
+@pytest.mark.parametrize("m,n", [(17, 33), (17, 409), (41, 7), (512, 9), (513, 9)])
 def test_one_element_a_row_gives_the_weights(backend, kind, k, m, n):
     g = synth.rng(k + m)
     w = DECODE[kind][0](g, n, k)
