@@ -1,6 +1,7 @@
 """Q5_K and Q6_K from 17 rows, whose two operands become fp16 in one launch or two: rows of each length a thread's registers are
 laid out for, row and column counts on both sides of the lines between these, and counts of blocks that leave the last
-workgroup's share short.  One element a row other than zero gives the products of an fp16 activation and an fp16 weight, which fp32 holds, times the row's power of two."""
+workgroup's share short.  One element a row other than zero gives the products of an fp16 activation and an fp16 weight,
+which fp32 holds, times the row's power of two."""
 import numpy as np
 import pytest
 
